@@ -23,7 +23,7 @@ struct isspa_diff {
     float4 *nb_ld = nullptr;
     float4 *xq = nullptr, *arec = nullptr;
     double *se = nullptr, *ftmp = nullptr, *gatom = nullptr;
-    double *ppart = nullptr, *apart = nullptr;
+    double *ppart = nullptr, *apart = nullptr, *tpart = nullptr;
     float4 *prec = nullptr;
     long long capF = 0, capC = 0;
     // inputs and tiling generation of the last isspa_diff_forces, whose points,
@@ -41,7 +41,7 @@ static void diff_free(isspa_diff *m)
     m->nb = nullptr;
     dfree(m->camp); dfree(m->dtypes); dfree(m->nb_ld); dfree(m->xq); dfree(m->arec);
     dfree(m->se); dfree(m->ftmp); dfree(m->gatom); dfree(m->ppart); dfree(m->apart);
-    dfree(m->prec);
+    dfree(m->prec); dfree(m->tpart);
 }
 
 // partial buffers follow the IS-SPA model's current tiling
@@ -119,6 +119,7 @@ extern "C" int isspa_diff_create(const isspa_diff_desc *d, const isspa_windows *
     if (rc == ISSPA_OK) rc = dalloc(&m->se, 3 * n);
     if (rc == ISSPA_OK) rc = dalloc(&m->ftmp, 3 * n);
     if (rc == ISSPA_OK) rc = dalloc(&m->gatom, 5 * n);
+    if (rc == ISSPA_OK) rc = dalloc(&m->tpart, 5 * (size_t)T * type_reduce_ranges(d->n_atoms));
     if (rc == ISSPA_OK) rc = dalloc(&m->prec, 4 * (size_t)m->im->P);
     if (rc == ISSPA_OK) rc = diff_buffers(m);
     if (rc != ISSPA_OK) {
@@ -306,7 +307,7 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     fa.gq = gq_d;
     fa.gatom = gatom_d ? gatom_d : m->gatom;
     HIPCHK(launch_vjp_finish(fa, s));
-    HIPCHK(launch_type_reduce(fa.gatom, im->itype, m->n, m->T, gtheta_d, s));
+    HIPCHK(launch_type_reduce(fa.gatom, im->itype, m->n, m->T, m->tpart, gtheta_d, s));
     return ISSPA_OK;
 }
 

@@ -18,9 +18,12 @@
 //   k_type_reduce  per type, FP64, fixed order
 // Every accumulation is an FP32 tile sum flushed into FP64, summed over
 // partials in a fixed order: results are deterministic.
+#include <algorithm>
+
 #include "device_common.hpp"
 #include "diff_device.hpp"
 #include "kernels.hpp"
+#include "reduce_device.hpp"
 
 namespace isspa {
 
@@ -95,23 +98,24 @@ __global__ __launch_bounds__(kB) void k_diff_prep_atoms(DiffAtomArgs a)
     r[3] = make_float4((float)l0, (float)l1, (float)l2, 0.0f);
 }
 
-// F_i = -q_i vtot_i S_e - vtot_i S_lj (overwrites f), S_e kept for the adjoint
+// F_i = -q_i vtot_i S_e - vtot_i S_lj (overwrites f), S_e kept for the adjoint.
+// Latency bound: a block of 32 atoms x 8 chunk slices (reduce_device.hpp) with
+// six chunks' entries in flight a slice.  One lane per atom over all chunks
+// took 53.9 us at 550 atoms (3 blocks, 181 dependent rounds) and 121 us for
+// 32 x 1,100 atoms; now 7.4 and 81 us (345 MB, 4.3 TB/s).
 __global__ __launch_bounds__(kB) void k_diff_reduce(DiffReduceArgs a)
 {
-    const int i = blockIdx.x * kB + threadIdx.x;
-    if (i >= a.n) return;
-    const WinDesc W = a.wins[a.atom_win[i]];
-    const int il = i - W.a0;
+    __shared__ double red[kSumSlices][6][kSumAtoms];
+    const int al = threadIdx.x % kSumAtoms, sl = threadIdx.x / kSumAtoms;
+    const int i = blockIdx.x * kSumAtoms + al;
+    const bool valid = i < a.n;
     double s[6] = {0, 0, 0, 0, 0, 0};
-    for (int c = 0; c < W.chunks; ++c) {
-        const long long o = W.ppo + (long long)c * W.n + il;
-        const double2 *e = reinterpret_cast<const double2 *>(a.part + o * force_part_stride(false));
-        for (int h = 0; h < 3; ++h) {
-            const double2 d = e[h];
-            s[2 * h] += d.x;
-            s[2 * h + 1] += d.y;
-        }
+    if (valid) {
+        const WinDesc W = a.wins[a.atom_win[i]];
+        force_slice_sum<6>(W, a.part, i, sl, s);
     }
+    combine_slices<6>(red, al, sl, s);
+    if (sl != 0 || !valid) return;
     const double vt = a.vtot[a.itype[i]];
     const double qv = -a.q[i] * vt;
     for (int c = 0; c < 3; ++c) {
@@ -488,48 +492,71 @@ __global__ __launch_bounds__(kB) void k_vjp_nonbond(VjpNbArgs a)
     a.part[2 * a.B + o] = eacc;
 }
 
-// per atom: chunk partials in order + the direct charge term
+// Sums of NC component-major partials [NC][stride], entries c = sl,
+// sl + kSumSlices, ... of atom slot `base`, B entries' loads in flight.
+template <int NC, int B>
+__device__ __forceinline__ void planar_slice_sum(const double *__restrict__ part, long long stride,
+                                                 long long base, int step, int n, int sl,
+                                                 double *s)
+{
+    int c = sl;
+    for (; c + (B - 1) * kSumSlices < n; c += B * kSumSlices) {
+        double v[B][NC];
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+#pragma unroll
+            for (int k = 0; k < NC; ++k)
+                v[u][k] = part[k * stride + base + (long long)(c + u * kSumSlices) * step];
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+#pragma unroll
+            for (int k = 0; k < NC; ++k) s[k] += v[u][k];
+    }
+    for (; c < n; c += kSumSlices)
+#pragma unroll
+        for (int k = 0; k < NC; ++k) s[k] += part[k * stride + base + (long long)c * step];
+}
+
+// Per atom: the chunk partials + the direct charge term.  Latency bound like
+// k_diff_reduce and split the same way (32 atoms x 8 slices a block, four
+// chunks in flight a slice): one lane per atom took 74.7 us at 550 atoms and
+// 133 us for 32 x 1,100 atoms; now 9.2 and 81 us.
 __global__ __launch_bounds__(kB) void k_vjp_finish(VjpFinishArgs a)
 {
-    const int i = blockIdx.x * kB + threadIdx.x;
-    if (i >= a.n) return;
-    const WinDesc W = a.wins[a.atom_win[i]];
-    const WinDesc Wn = a.nb_wins[a.atom_win[i]];
-    const int il = i - W.a0;
-    double q = 0.0, t[5] = {0, 0, 0, 0, 0};
-    for (int c = 0; c < W.chunks; ++c) {
-        const long long o = W.ppo + (long long)c * W.n + il;
-        q += a.apart[o];
-        for (int k = 0; k < 5; ++k) t[k] += a.apart[(1 + k) * a.C + o];
+    __shared__ double red[kSumSlices][9][kSumAtoms];
+    const int al = threadIdx.x % kSumAtoms, sl = threadIdx.x / kSumAtoms;
+    const int i = blockIdx.x * kSumAtoms + al;
+    const bool valid = i < a.n;
+    double s[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};  // q, theta(5); nonbond q, sigma, eps
+    if (valid) {
+        const int w = a.atom_win[i];
+        const WinDesc W = a.wins[w];
+        const WinDesc Wn = a.nb_wins[w];
+        const int il = i - W.a0;
+        planar_slice_sum<6, 4>(a.apart, a.C, W.ppo + il, W.n, W.chunks, sl, s);
+        planar_slice_sum<3, 4>(a.nbpart, a.B, Wn.npo + il, Wn.n, Wn.nbc, sl, s + 6);
     }
-    double nq = 0.0, ns = 0.0, ne = 0.0;
-    for (int c = 0; c < Wn.nbc; ++c) {
-        const long long o = Wn.npo + (long long)c * Wn.n + il;
-        nq += a.nbpart[o];
-        ns += a.nbpart[a.B + o];
-        ne += a.nbpart[2 * a.B + o];
-    }
+    combine_slices<9>(red, al, sl, s);
+    if (sl != 0 || !valid) return;
     const int ti = a.itype[i];
     const double vt = a.vtot[ti];
     const double direct = -vt * (a.lam[3 * i] * a.se[3 * i] + a.lam[3 * i + 1] * a.se[3 * i + 1] +
                                  a.lam[3 * i + 2] * a.se[3 * i + 2]);
-    a.gq[i] = q + nq + direct;
-    a.gatom[5 * i + 0] = t[0] + ns;
-    a.gatom[5 * i + 1] = t[1] + ne / (2.0 * a.theta[5 * ti + 1]);
-    for (int k = 2; k < 5; ++k) a.gatom[5 * i + k] = t[k];
+    a.gq[i] = s[0] + s[6] + direct;
+    a.gatom[5 * i + 0] = s[1] + s[7];
+    a.gatom[5 * i + 1] = s[2] + s[8] / (2.0 * a.theta[5 * ti + 1]);
+    for (int k = 2; k < 5; ++k) a.gatom[5 * i + k] = s[1 + k];
 }
 
-// per-type sums of the per-atom bars, FP64, fixed order (one block per type)
-__global__ __launch_bounds__(kB) void k_type_reduce(const double *__restrict__ gatom,
-                                                    const int *__restrict__ itype, int n,
-                                                    double *gtheta)
+// Per-type sums of the per-atom bars, FP64, fixed order: one block per type
+// and atom range [kTypeRange b, kTypeRange (b + 1)), then, with more than one
+// range, one block per type over the ranges.  Latency bound: a block that
+// walks all 35,200 atoms of 32 x 1,100 alone takes 137 dependent rounds
+// (81.6 us); in ranges it takes 7.7 + 4.6 us.
+constexpr int kTypeRange = 2048;
+
+__device__ __forceinline__ void type_tree(double (&red)[5][kB], const double (&s)[5])
 {
-    __shared__ double red[5][kB];
-    const int t = blockIdx.x;
-    double s[5] = {0, 0, 0, 0, 0};
-    for (int i = threadIdx.x; i < n; i += kB)
-        if (itype[i] == t)
-            for (int k = 0; k < 5; ++k) s[k] += gatom[5 * i + k];
     for (int k = 0; k < 5; ++k) red[k][threadIdx.x] = s[k];
     __syncthreads();
     for (int w = kB / 2; w > 0; w >>= 1) {
@@ -537,6 +564,37 @@ __global__ __launch_bounds__(kB) void k_type_reduce(const double *__restrict__ g
             for (int k = 0; k < 5; ++k) red[k][threadIdx.x] += red[k][threadIdx.x + w];
         __syncthreads();
     }
+}
+
+// out[(type * gridDim.y + range) * 5 + k]
+__global__ __launch_bounds__(kB) void k_type_reduce(const double *__restrict__ gatom,
+                                                    const int *__restrict__ itype, int n,
+                                                    double *out)
+{
+    __shared__ double red[5][kB];
+    const int t = blockIdx.x;
+    double s[5] = {0, 0, 0, 0, 0};
+    const int i0 = blockIdx.y * kTypeRange + threadIdx.x;
+#pragma unroll
+    for (int u = 0; u < kTypeRange / kB; ++u) {
+        const int i = i0 + u * kB;
+        if (i < n && itype[i] == t)
+            for (int k = 0; k < 5; ++k) s[k] += gatom[5 * (size_t)i + k];
+    }
+    type_tree(red, s);
+    if (threadIdx.x < 5)
+        out[5 * ((size_t)t * gridDim.y + blockIdx.y) + threadIdx.x] = red[threadIdx.x][0];
+}
+
+__global__ __launch_bounds__(kB) void k_type_sum(const double *__restrict__ part, int ranges,
+                                                 double *gtheta)
+{
+    __shared__ double red[5][kB];
+    const int t = blockIdx.x;
+    double s[5] = {0, 0, 0, 0, 0};
+    for (int r = threadIdx.x; r < ranges; r += kB)
+        for (int k = 0; k < 5; ++k) s[k] += part[5 * ((size_t)t * ranges + r) + k];
+    type_tree(red, s);
     if (threadIdx.x < 5) gtheta[5 * t + threadIdx.x] = red[threadIdx.x][0];
 }
 
@@ -559,7 +617,7 @@ hipError_t launch_diff_prep_atoms(const DiffAtomArgs &a, hipStream_t s)
 hipError_t launch_diff_reduce(const DiffReduceArgs &a, hipStream_t s)
 {
     if (a.n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_diff_reduce, dim3(nblk(a.n)), dim3(kB), 0, s, a);
+    hipLaunchKernelGGL(k_diff_reduce, dim3((a.n + kSumAtoms - 1) / kSumAtoms), dim3(kB), 0, s, a);
     return hipGetLastError();
 }
 
@@ -599,15 +657,21 @@ hipError_t launch_vjp_nonbond(const VjpNbArgs &a, int nblocks, hipStream_t s)
 hipError_t launch_vjp_finish(const VjpFinishArgs &a, hipStream_t s)
 {
     if (a.n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_vjp_finish, dim3(nblk(a.n)), dim3(kB), 0, s, a);
+    hipLaunchKernelGGL(k_vjp_finish, dim3((a.n + kSumAtoms - 1) / kSumAtoms), dim3(kB), 0, s, a);
     return hipGetLastError();
 }
 
-hipError_t launch_type_reduce(const double *gatom, const int *itype, int n, int T,
+int type_reduce_ranges(int n) { return std::max(1, (n + kTypeRange - 1) / kTypeRange); }
+
+hipError_t launch_type_reduce(const double *gatom, const int *itype, int n, int T, double *part,
                               double *gtheta, hipStream_t s)
 {
     if (T == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_type_reduce, dim3(T), dim3(kB), 0, s, gatom, itype, n, gtheta);
+    const int ranges = type_reduce_ranges(n);
+    hipLaunchKernelGGL(k_type_reduce, dim3(T, ranges), dim3(kB), 0, s, gatom, itype, n,
+                       ranges > 1 ? part : gtheta);
+    if (ranges > 1)
+        hipLaunchKernelGGL(k_type_sum, dim3(T), dim3(kB), 0, s, part, ranges, gtheta);
     return hipGetLastError();
 }
 

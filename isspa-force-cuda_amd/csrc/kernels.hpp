@@ -400,7 +400,9 @@ hipError_t launch_vjp_epilogue(const VjpArgs &a, hipStream_t s);
 hipError_t launch_vjp_atoms(const VjpArgs &a, int nblocks, hipStream_t s);
 hipError_t launch_vjp_nonbond(const VjpNbArgs &a, int nblocks, hipStream_t s);
 hipError_t launch_vjp_finish(const VjpFinishArgs &a, hipStream_t s);
-hipError_t launch_type_reduce(const double *gatom, const int *itype, int n, int T,
+// part: scratch of 5 T type_reduce_ranges(n) doubles
+int type_reduce_ranges(int n);
+hipError_t launch_type_reduce(const double *gatom, const int *itype, int n, int T, double *part,
                               double *gtheta, hipStream_t s);
 
 // ---- integrator / restraint / utilities ----

@@ -64,16 +64,16 @@ __device__ __forceinline__ void load_force_entry(const double *part, long long o
 }
 
 template <int COMPS>
-__device__ inline void isspa_slice_sum(const ReduceArgs &a, int i, int sl, double (&s)[COMPS])
+__device__ inline void force_slice_sum(const WinDesc &W, const double *part, int i, int sl,
+                                       double (&s)[COMPS])
 {
-    const WinDesc W = a.wins[a.atom_win[i]];
     const long long base = W.ppo + (i - W.a0);
     int c = sl;
     for (; c + (kSumBatch - 1) * kSumSlices < W.chunks; c += kSumBatch * kSumSlices) {
         double v[kSumBatch][COMPS];
 #pragma unroll
         for (int u = 0; u < kSumBatch; ++u)
-            load_force_entry<COMPS>(a.part, base + (long long)(c + u * kSumSlices) * W.n, v[u]);
+            load_force_entry<COMPS>(part, base + (long long)(c + u * kSumSlices) * W.n, v[u]);
 #pragma unroll
         for (int u = 0; u < kSumBatch; ++u)
 #pragma unroll
@@ -81,10 +81,17 @@ __device__ inline void isspa_slice_sum(const ReduceArgs &a, int i, int sl, doubl
     }
     for (; c < W.chunks; c += kSumSlices) {
         double v[COMPS];
-        load_force_entry<COMPS>(a.part, base + (long long)c * W.n, v);
+        load_force_entry<COMPS>(part, base + (long long)c * W.n, v);
 #pragma unroll
         for (int k = 0; k < COMPS; ++k) s[k] += v[k];
     }
+}
+
+template <int COMPS>
+__device__ inline void isspa_slice_sum(const ReduceArgs &a, int i, int sl, double (&s)[COMPS])
+{
+    const WinDesc W = a.wins[a.atom_win[i]];
+    force_slice_sum<COMPS>(W, a.part, i, sl, s);
 }
 
 // F_i = -q_i vtot_i S_e - vtot_i S_lj from the summed IS-SPA partials
