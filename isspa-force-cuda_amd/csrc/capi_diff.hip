@@ -25,7 +25,7 @@ struct isspa_diff {
     double *se = nullptr, *ftmp = nullptr, *gatom = nullptr;
     double *ppart = nullptr, *apart = nullptr, *tpart = nullptr;
     float4 *prec = nullptr;
-    long long capF = 0, capC = 0;
+    long long capF = 0, capV = 0;
     // inputs and tiling generation of the last isspa_diff_forces, whose points,
     // records and S_e isspa_diff_vjp_after_forces reuses
     const void *fwd_x = nullptr, *fwd_q = nullptr, *fwd_theta = nullptr;
@@ -53,10 +53,10 @@ static int diff_buffers(isspa_diff *m)
         CHK(dalloc(&m->ppart, (size_t)10 * im->F));
         m->capF = im->F;
     }
-    if (im->C > m->capC) {
+    if (im->V > m->capV) {
         dfree(m->apart);
-        CHK(dalloc(&m->apart, (size_t)6 * im->C));
-        m->capC = im->C;
+        CHK(dalloc(&m->apart, (size_t)6 * im->V));
+        m->capV = im->V;
     }
     return ISSPA_OK;
 }
@@ -245,7 +245,7 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     va.wins = im->wins;
     va.atom_win = im->atom_win;
     va.fblk = im->fblk;
-    va.pblk = im->pblk;
+    va.vblk = im->vblk;
     va.nmc = im->d.n_mc;
     va.Ptot = im->P;
     va.pts = im->pts;
@@ -269,10 +269,10 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     va.F = im->F;
     va.prec = m->prec;
     va.apart = m->apart;
-    va.C = im->C;
+    va.C = im->V;
     HIPCHK(launch_vjp_points(va, im->nfblk, s));
     HIPCHK(launch_vjp_epilogue(va, s));
-    HIPCHK(launch_vjp_atoms(va, im->npblk, s));
+    HIPCHK(launch_vjp_atoms(va, im->nvblk, s));
     HIPCHK(launch_pbc_flag(nb->wins, nb->lay.W, m->xq, 0.0f, nb->pbc_flag, s));
     VjpNbArgs na{};
     na.wins = nb->wins;
@@ -296,7 +296,7 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     fa.nb_wins = nb->wins;
     fa.atom_win = im->atom_win;
     fa.apart = m->apart;
-    fa.C = im->C;
+    fa.C = im->V;
     fa.nbpart = nb->part;
     fa.B = nb->B;
     fa.itype = im->itype;

@@ -99,7 +99,7 @@ static void isspa_free(isspa_model *m)
     dfree(m->g); dfree(m->e); dfree(m->f);
     dfree(m->pts); dfree(m->rec); dfree(m->g_out); dfree(m->E_out); dfree(m->E0_out);
     dfree(m->cnt_out); dfree(m->pbc_flag); dfree(m->wins); dfree(m->fblk); dfree(m->gblk);
-    dfree(m->pblk);
+    dfree(m->pblk); dfree(m->vblk);
     dfree(m->part_g); dfree(m->part_cnt); dfree(m->part_s0); dfree(m->part_ein); dfree(m->part_f);
     dfree(m->prof_f);
 }
@@ -118,11 +118,10 @@ static int isspa_tile(isspa_model *m)
             : (double)std::min(kMaxAutoWaves,
                                std::max(kMinAutoWaves, (long)(m->P / kPointsPerWave)));
     m->wins_h.assign(L.W, WinDesc{});
-    m->max_win_atoms = m->max_chunk_pts = 0;
+    m->max_win_atoms = m->max_group_pts = 0;
     m->max_fg = 1;
-    m->min_win_atoms = 1 << 30;
-    long long F = 0, C = 0;
-    std::vector<std::pair<long long, int4>> fb, gb, pb;
+    long long F = 0, C = 0, V = 0;
+    std::vector<std::pair<long long, int4>> fb, gb, pb, vb;
     for (int w = 0; w < L.W; ++w) {
         WinDesc d = base_desc(L, w);
         const long long n = L.n[w], P = n * nmc;
@@ -134,21 +133,25 @@ static int isspa_tile(isspa_model *m)
         if (m->user_splits <= 0 && s >= 4) s -= s % 4;
         d.aps = (int)((n + s - 1) / s);
         d.splits = (int)((n + d.aps - 1) / d.aps);
-        // a chunk keeps kMinChunkPoints points for each receiver replica
+        // a chunk keeps kMinChunkPoints points for each of its shares
         int c = m->user_chunks > 0
                     ? m->user_chunks
-                    : auto_pieces(n, P, kMinChunkPoints * force_replicas((int)n), tgt);
+                    : auto_pieces(n, P, kMinChunkPoints * force_shares((int)n), tgt);
         c = (int)std::max(1LL, std::min((long long)c, P));
         d.ppc = (int)((P + c - 1) / c);
         d.chunks = (int)((P + d.ppc - 1) / d.ppc);
         m->max_win_atoms = std::max(m->max_win_atoms, (int)n);
-        m->min_win_atoms = std::min(m->min_win_atoms, (int)n);
-        m->max_chunk_pts = std::max(m->max_chunk_pts, d.ppc);
+        const int group = force_group((int)n), shares = force_shares((int)n);
+        m->max_group_pts = std::max(m->max_group_pts, (int)std::min(P, (long long)group * d.ppc));
+        d.fents = (d.chunks + group - 1) / group;
+        d.vents = (d.chunks + 3) / 4;
         d.fpo = F;
         d.ppo = C;
+        d.vpo = V;
         F += (long long)d.splits * P;
-        C += (long long)d.chunks * n;
-        const int pblocks = (int)((P + 255) / 256), rblocks = (int)((n + 255) / 256);
+        C += (long long)d.fents * n;
+        V += (long long)d.vents * n;
+        const int pblocks = (int)((P + 255) / 256), rblocks = (int)((n + 63) / 64);
         for (int b = 0; b < pblocks; ++b)
             for (int sp = 0; sp < d.splits; ++sp) fb.push_back({(long long)d.aps, make_int4(w, b, sp, 0)});
         // the field pass: fg splits of the same 256 / fg points a block
@@ -158,11 +161,14 @@ static int isspa_tile(isspa_model *m)
         for (int b = 0; b < gblocks; ++b)
             for (int gr = 0; gr < d.splits / d.fg; ++gr)
                 gb.push_back({(long long)d.aps, make_int4(w, b, gr, 0)});
-        // chunk-major: the receiver blocks of one point chunk are consecutive,
-        // so the round-robin dispatch over the 8 XCDs gives each XCD's L2 a
-        // share of them that reuses the chunk's records
-        for (int ch = 0; ch < d.chunks; ++ch)
-            for (int b = 0; b < rblocks; ++b) pb.push_back({(long long)d.ppc, make_int4(w, b, ch, 0)});
+        // chunk-major: the receiver blocks of one group of point chunks are
+        // consecutive, so the round-robin dispatch over the 8 XCDs gives each
+        // XCD's L2 a share of them that reuses the group's records
+        for (int gr = 0; gr < d.fents; ++gr)
+            for (int b = 0; b < rblocks; ++b)
+                pb.push_back({(long long)(d.ppc + shares - 1) / shares, make_int4(w, b, gr, 0)});
+        for (int gr = 0; gr < d.vents; ++gr)
+            for (int b = 0; b < rblocks; ++b) vb.push_back({(long long)d.ppc, make_int4(w, b, gr, 0)});
         m->wins_h[w] = d;
     }
     auto by_work = [](const std::pair<long long, int4> &a, const std::pair<long long, int4> &b) {
@@ -171,20 +177,25 @@ static int isspa_tile(isspa_model *m)
     std::stable_sort(fb.begin(), fb.end(), by_work);
     std::stable_sort(gb.begin(), gb.end(), by_work);
     std::stable_sort(pb.begin(), pb.end(), by_work);
-    std::vector<int4> fbv, gbv, pbv;
+    std::stable_sort(vb.begin(), vb.end(), by_work);
+    std::vector<int4> fbv, gbv, pbv, vbv;
     for (auto &x : fb) fbv.push_back(x.second);
     for (auto &x : gb) gbv.push_back(x.second);
     for (auto &x : pb) pbv.push_back(x.second);
-    dfree(m->wins); dfree(m->fblk); dfree(m->gblk); dfree(m->pblk);
+    for (auto &x : vb) vbv.push_back(x.second);
+    dfree(m->wins); dfree(m->fblk); dfree(m->gblk); dfree(m->pblk); dfree(m->vblk);
     CHK(upload(&m->wins, m->wins_h.data(), m->wins_h.size()));
     CHK(upload(&m->fblk, fbv.data(), fbv.size()));
     CHK(upload(&m->gblk, gbv.data(), gbv.size()));
     CHK(upload(&m->pblk, pbv.data(), pbv.size()));
+    CHK(upload(&m->vblk, vbv.data(), vbv.size()));
     m->nfblk = (int)fbv.size();
     m->ngblk = (int)gbv.size();
     m->npblk = (int)pbv.size();
+    m->nvblk = (int)vbv.size();
     m->F = F;
     m->C = C;
+    m->V = V;
     m->generation++;
     if (F > m->cap_field) {
         dfree(m->part_g); dfree(m->part_cnt); dfree(m->part_s0); dfree(m->part_ein);
@@ -372,7 +383,6 @@ ForceArgs force_args(isspa_model *m, const float4 *x)
     // one system: every block has the same work, so each XCD may take a
     // contiguous run of chunks (batches keep their longest-first order)
     fa.xcd_runs = m->lay.W == 1;
-    fa.replicas = force_replicas(m->min_win_atoms);
     return fa;
 }
 
@@ -1263,7 +1273,7 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
         }
         HIPCHK(launch_field(fa, m->ngblk, s));
         const ForceArgs fo = force_args(m, x4);
-        if (!fo.dtypes && force_epi_fits(fo.tab, m->max_win_atoms, m->max_chunk_pts, m->npblk)) {
+        if (!fo.dtypes && force_epi_fits(fo.tab, m->max_win_atoms, m->max_group_pts, m->npblk)) {
             // small windows: the epilogue inside the force launch
             HIPCHK(launch_force_epi(fo, epilogue_args(m, false), m->npblk, s));
         } else {

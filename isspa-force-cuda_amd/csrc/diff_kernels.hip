@@ -102,7 +102,7 @@ __global__ __launch_bounds__(kB) void k_diff_prep_atoms(DiffAtomArgs a)
 // Latency bound: a block of 32 atoms x 8 chunk slices (reduce_device.hpp) with
 // six chunks' entries in flight a slice.  One lane per atom over all chunks
 // took 53.9 us at 550 atoms (3 blocks, 181 dependent rounds) and 121 us for
-// 32 x 1,100 atoms; now 7.4 and 81 us (345 MB, 4.3 TB/s).
+// 32 x 1,100 atoms; now 7.4 and 16 us (86 MB, 5.4 TB/s).
 __global__ __launch_bounds__(kB) void k_diff_reduce(DiffReduceArgs a)
 {
     __shared__ double red[kSumSlices][6][kSumAtoms];
@@ -372,16 +372,24 @@ __device__ __forceinline__ void vjp_atoms_tile(const VjpArgs &a, const float4 *_
     }
 }
 
+// A block's four waves take the same 64 atoms and one chunk each, and add
+// their FP64 sums in chunk order through LDS (as the force pass): a quarter of
+// the partials to write and to sum, and no idle wave in a window's last block.
+// 32 x 1,100 atoms: 1,016 -> 989 us, and k_vjp_finish behind it 81 -> 24 us.
 __global__ __launch_bounds__(kB) void k_vjp_atoms(VjpArgs a)
 {
-    const int4 bt = a.pblk[blockIdx.x];
+    __shared__ double red[3][6][kWave];
+    const int4 bt = a.vblk[blockIdx.x];
     const WinDesc W = a.wins[bt.x];
-    const int il = bt.y * kB + threadIdx.x;
-    const int chunk = bt.z;
+    const int lane = threadIdx.x % kWave;
+    // read from the first lane so the compiler knows it is wave-uniform
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int il = bt.y * kWave + lane;
     const long long pbase = (long long)W.a0 * a.nmc;
     const float4 *__restrict__ pr = a.prec + 4 * pbase;  // this window's point bars
-    const int m0 = chunk * W.ppc;                        // window-local point range
-    const int m1 = min(W.n * a.nmc, m0 + W.ppc);
+    const int P = W.n * a.nmc;
+    const int m0 = min(P, (4 * bt.z + wv) * W.ppc);  // window-local point range
+    const int m1 = min(P, m0 + W.ppc);
     const bool valid = il < W.n;
     const int j = W.a0 + (valid ? il : 0);
     const float4 xj = a.xq[j];
@@ -390,9 +398,8 @@ __global__ __launch_bounds__(kB) void k_vjp_atoms(VjpArgs a)
     const float4 lp = a.arec[4 * (size_t)j + 2];  // Lambda' = -vtot lambda
     const bool pbc = a.pbc_flag[bt.x] != 0;
     const DiffType &Tj = stage_dtypes(a)[tj];
-    // a wave with no atom of the window stops after the block's barrier
-    if (bt.y * kB + (int)(threadIdx.x & ~(kWave - 1)) >= W.n) return;
-    double qacc = 0.0, tb[5] = {0, 0, 0, 0, 0};
+    double acc[6] = {0, 0, 0, 0, 0, 0};  // q, theta(5)
+    double tb[5] = {0, 0, 0, 0, 0};
     for (int mt = m0; mt < m1; mt += kTile) {
         const int me = min(m1, mt + kTile);
         float qb = 0.0f;
@@ -400,12 +407,18 @@ __global__ __launch_bounds__(kB) void k_vjp_atoms(VjpArgs a)
             vjp_atoms_tile<true>(a, pr, Tj, mt, me, W.L, W.h, xj, R2j, lp.x, lp.y, lp.z, qb, tb);
         else
             vjp_atoms_tile<false>(a, pr, Tj, mt, me, W.L, W.h, xj, R2j, lp.x, lp.y, lp.z, qb, tb);
-        qacc += (double)qb;
+        acc[0] += (double)qb;
     }
-    if (!valid) return;
-    const long long o = W.ppo + (long long)chunk * W.n + il;
-    a.apart[o] = qacc;
-    for (int k = 0; k < 5; ++k) a.apart[(1 + k) * a.C + o] = tb[k];
+    for (int k = 0; k < 5; ++k) acc[1 + k] = tb[k];
+    if (wv > 0)
+        for (int k = 0; k < 6; ++k) red[wv - 1][k][lane] = acc[k];
+    __syncthreads();
+    if (wv > 0 || !valid) return;
+    const long long o = W.vpo + (long long)bt.z * W.n + il;
+    for (int k = 0; k < 6; ++k) {
+        for (int w = 0; w < 3; ++w) acc[k] += red[w][k][lane];
+        a.apart[k * a.C + o] = acc[k];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -520,7 +533,7 @@ __device__ __forceinline__ void planar_slice_sum(const double *__restrict__ part
 // Per atom: the chunk partials + the direct charge term.  Latency bound like
 // k_diff_reduce and split the same way (32 atoms x 8 slices a block, four
 // chunks in flight a slice): one lane per atom took 74.7 us at 550 atoms and
-// 133 us for 32 x 1,100 atoms; now 9.2 and 81 us.
+// 133 us for 32 x 1,100 atoms; now 9.2 and 24 us.
 __global__ __launch_bounds__(kB) void k_vjp_finish(VjpFinishArgs a)
 {
     __shared__ double red[kSumSlices][9][kSumAtoms];
@@ -533,7 +546,7 @@ __global__ __launch_bounds__(kB) void k_vjp_finish(VjpFinishArgs a)
         const WinDesc W = a.wins[w];
         const WinDesc Wn = a.nb_wins[w];
         const int il = i - W.a0;
-        planar_slice_sum<6, 4>(a.apart, a.C, W.ppo + il, W.n, W.chunks, sl, s);
+        planar_slice_sum<6, 4>(a.apart, a.C, W.vpo + il, W.n, W.vents, sl, s);
         planar_slice_sum<3, 4>(a.nbpart, a.B, Wn.npo + il, Wn.n, Wn.nbc, sl, s + 6);
     }
     combine_slices<9>(red, al, sl, s);

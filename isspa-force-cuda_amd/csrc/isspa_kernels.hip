@@ -658,25 +658,23 @@ __device__ __forceinline__ void force_chunk(const ForceArgs &a, const float4 *__
     }
 }
 
-// Replicas 1..r-1 of the block's receivers leave their sums in LDS; replica
-// 0 adds them in replica order.  Every wave of the block reaches the barrier
-// (with r > 1 every wave holds receivers).  Returns false on the waves whose
-// sums were handed over.
+// Waves 1..3 leave their shares' sums in LDS; wave 0 adds them in share
+// order.  Every wave of the block reaches the barrier.  Returns false on the
+// waves whose sums were handed over.
 template <bool SPLIT>
-__device__ __forceinline__ bool replica_sum(double *red, int r, int q, int slot, int nslots,
-                                            ForceAcc &acc)
+__device__ __forceinline__ bool share_sum(double *red, int wv, int lane, ForceAcc &acc)
 {
     constexpr int nc = SPLIT ? 9 : 6;
-    if (q > 0) {
-        double *d = red + ((long long)(q - 1) * nslots + slot) * nc;
+    if (wv > 0) {
+        double *d = red + ((wv - 1) * kWave + lane) * nc;
         d[0] = acc.ex; d[1] = acc.ey; d[2] = acc.ez;
         d[3] = acc.lx; d[4] = acc.ly; d[5] = acc.lz;
         if (SPLIT) { d[6] = acc.cx; d[7] = acc.cy; d[8] = acc.cz; }
     }
     __syncthreads();
-    if (q > 0) return false;
-    for (int k = 1; k < r; ++k) {
-        const double *d = red + ((long long)(k - 1) * nslots + slot) * nc;
+    if (wv > 0) return false;
+    for (int k = 0; k < 3; ++k) {
+        const double *d = red + (k * kWave + lane) * nc;
         acc.ex += d[0]; acc.ey += d[1]; acc.ez += d[2];
         acc.lx += d[3]; acc.ly += d[4]; acc.lz += d[5];
         if (SPLIT) { acc.cx += d[6]; acc.cy += d[7]; acc.cz += d[8]; }
@@ -684,47 +682,66 @@ __device__ __forceinline__ bool replica_sum(double *red, int r, int q, int slot,
     return true;
 }
 
-// REP: some window of the launch has receiver replicas (the replica code is
-// compiled only into that instantiation, so the large-system kernel keeps its
-// registers)
-template <bool SPLIT, bool AN, bool REP>
+// the window-local points [ms, me) of wave wv's share of chunk group gr
+__device__ __forceinline__ void share_range(const WinDesc &W, int P, int gr, int wv, int &ms,
+                                            int &me)
+{
+    const int shares = force_shares(W.n), group = force_group(W.n);
+    const int ch = gr * group + wv / shares, part = wv % shares;
+    const int c0 = min(P, ch * W.ppc), c1 = min(P, c0 + W.ppc);
+    const int sub = (c1 - c0 + shares - 1) / shares;
+    ms = min(c1, c0 + part * sub);
+    me = min(c1, ms + sub);
+}
+
+template <bool SPLIT>
+__device__ __forceinline__ void write_force_entry(const ForceArgs &a, const WinDesc &W, int gr,
+                                                  int il, const ForceAcc &acc)
+{
+    const long long o = W.ppo + (long long)gr * W.n + il;
+    double2 *e = reinterpret_cast<double2 *>(a.part + o * force_part_stride(SPLIT));
+    e[0] = make_double2(acc.ex, acc.ey);
+    e[1] = make_double2(acc.ez, acc.lx);
+    e[2] = make_double2(acc.ly, acc.lz);
+    if (SPLIT) {
+        e[3] = make_double2(acc.cx, acc.cy);
+        e[4] = make_double2(acc.cz, 0.0);
+    }
+}
+
+template <bool SPLIT, bool AN>
 __global__ __launch_bounds__(kBlock) void k_force(ForceArgs a)
 {
     const int4 bt = a.blocks[a.xcd_runs ? xcd_run_entry(blockIdx.x, gridDim.x) : blockIdx.x];
     const WinDesc W = a.wins[bt.x];
-    // receiver replicas: wave wv serves receivers (wv % nrw) * 64 + lane of
-    // the block on the q-th share of the chunk's points
-    const int r = REP ? force_replicas(W.n) : 1, nrw = 4 / r;
+    const int lane = (int)threadIdx.x % kWave;
     // the wave index read from the first lane, so the compiler knows it is
-    // wave-uniform and the replica's point range stays on scalar loads
-    const int wv = REP ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave) : 0;
-    const int q = REP ? wv / nrw : 0;
-    const int slot = REP ? (wv % nrw) * kWave + (int)threadIdx.x % kWave : (int)threadIdx.x;
-    const int il = bt.y * kBlock + slot;  // receiver within the window
-    const int chunk = bt.z;
+    // wave-uniform and the share's point range stays on scalar loads
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int il = bt.y * kWave + lane;  // receiver within the window
+    const int P = W.n * a.nmc;
     const long long pbase = (long long)W.a0 * a.nmc;
     const float4 *__restrict__ rec = a.rec4 + 4 * pbase;  // this window's records
     const float4 *__restrict__ aux = a.aux4 + pbase;
-    const int m0 = chunk * W.ppc;                        // window-local point range
-    const int m1 = min(W.n * a.nmc, m0 + W.ppc);
-    const int sub = (m1 - m0 + r - 1) / r;               // this replica's share
-    const int ms = min(m1, m0 + q * sub), me = min(m1, ms + sub);
+    int ms, me;
+    share_range(W, P, bt.z, wv, ms, me);
     const bool valid = il < W.n;
     const int i = W.a0 + (valid ? il : 0);
     const float4 xi = a.xyzq[i];
     const int ti = a.itype[i];
     const float R2 = valid ? a.rmax2[ti] : -1.0f;
-    // Warm-up: the chunk's records and aux entries are requested at block
+    // Warm-up: the group's records and aux entries are requested at block
     // start, one 128-byte line per work-item, the lines dealt over the
-    // chunk's receiver blocks, so that all of them are in flight at once.
+    // group's receiver blocks, so that all of them are in flight at once.
     // Right after the epilogue has written the records they sit in another
     // XCD's L2 or in memory, and the loop's one-record-ahead scalar loads
     // would otherwise wait for each line in turn.  The loaded values are only
     // kept alive (an empty asm takes them after the loop), never used.
     float w0 = 0.0f, w1 = 0.0f;
     {
-        const int nrb = (W.n + kBlock - 1) / kBlock;  // receiver blocks of the chunk
-        const int np = m1 - m0;
+        const int nrb = (W.n + kWave - 1) / kWave;    // receiver blocks of the group
+        const int span = force_group(W.n) * W.ppc;
+        const int m0 = min(P, bt.z * span), np = min(P, m0 + span) - m0;
         const int nrl = (16 * np + 31) / 32;          // record lines, then aux lines
         const int nl = nrl + (4 * np + 31) / 32;
         const float *rb = reinterpret_cast<const float *>(rec + 4 * m0);
@@ -748,44 +765,25 @@ __global__ __launch_bounds__(kBlock) void k_force(ForceArgs a)
     ForceAcc acc{0, 0, 0, 0, 0, 0, 0, 0, 0};
     // two call sites, so the table pointer of each has one address space and
     // the LDS one compiles to LDS reads
-    // a wave with no receiver of the window (small windows) stops after the
-    // block's one barrier instead of running the point loop for nothing
-    // (with replicas every wave holds receivers, so none leaves before the
-    // replica barrier)
-    const bool wave_idle = bt.y * kBlock + (slot & ~(kWave - 1)) >= W.n;
     if (!AN && force_tab_floats(a.tab) <= kTabLdsFloats) {
         stage_lds(lds_tab, a.tab.f, force_tab_floats(a.tab));
         __syncthreads();
-        if (wave_idle) return;
         force_chunk<SPLIT, AN>(a, rec, aux, ms, me, W, pbc, xi, R2, lds_tab + ti * a.tab.ld_f, fp,
                                acc);
     } else {
-        if (wave_idle) return;
         force_chunk<SPLIT, AN>(a, rec, aux, ms, me, W, pbc, xi, R2,
                                AN ? nullptr : a.tab.f + ti * a.tab.ld_f, fp, acc);
     }
     asm volatile("" ::"v"(w0), "v"(w1));
-    if (REP && r > 1 &&
-        !replica_sum<SPLIT>(reinterpret_cast<double *>(lds_tab + a.red_off), r, q, slot,
-                            nrw * kWave, acc))
-        return;
-    if (!valid) return;
-    const long long o = W.ppo + (long long)chunk * W.n + il;
-    double2 *e = reinterpret_cast<double2 *>(a.part + o * force_part_stride(SPLIT));
-    e[0] = make_double2(acc.ex, acc.ey);
-    e[1] = make_double2(acc.ez, acc.lx);
-    e[2] = make_double2(acc.ly, acc.lz);
-    if (SPLIT) {
-        e[3] = make_double2(acc.cx, acc.cy);
-        e[4] = make_double2(acc.cz, 0.0);
-    }
+    if (!share_sum<SPLIT>(reinterpret_cast<double *>(lds_tab + a.red_off), wv, lane, acc)) return;
+    if (valid) write_force_entry<SPLIT>(a, W, bt.z, il, acc);
 }
 
-// Small systems (every window within one receiver block, at most
-// kFuseMaxPts points a chunk, at most kFuseMaxBlocks blocks): the epilogue
-// and the force pass in one launch.  The block runs the epilogue of its
-// chunk's points (no other block needs them: the chunk has one receiver
-// block) into LDS, then the force loop reads the records from there.
+// Small systems (windows of at most kBlock atoms, at most kFuseMaxPts points a
+// chunk group, at most kFuseMaxBlocks blocks): the epilogue and the force pass
+// in one launch.  The block runs the epilogue of its group's points (windows
+// above 64 atoms repeat it in each of their two to four receiver blocks) into
+// LDS, then the force loop reads the records from there.
 // Records and force sums are those of the two launches bit for bit; the
 // records are not written to memory.  The epilogue keeps all (up to eight)
 // split groups' partial loads in flight, and its FP64 registers then allow one
@@ -803,18 +801,17 @@ __global__ __launch_bounds__(kBlock) void k_force_epi(ForceArgs a, EpilogueArgs 
 {
     const int4 bt = a.blocks[a.xcd_runs ? xcd_run_entry(blockIdx.x, gridDim.x) : blockIdx.x];
     const WinDesc W = a.wins[bt.x];
-    const int r = force_replicas(W.n), nrw = 4 / r;
+    const int lane = (int)threadIdx.x % kWave;
     // the wave index read from the first lane, so the compiler knows it is
-    // wave-uniform and the replica's point range stays on scalar loads
-    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave), q = wv / nrw;
-    const int slot = (wv % nrw) * kWave + (int)threadIdx.x % kWave;
-    const int il = bt.y * kBlock + slot;
-    const int chunk = bt.z;
+    // wave-uniform and the share's point range stays on scalar loads
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int il = bt.y * kWave + lane;
+    const int P = W.n * a.nmc;
     const long long pbase = (long long)W.a0 * a.nmc;
-    const int m0 = chunk * W.ppc;
-    const int np = min(W.n * a.nmc, m0 + W.ppc) - m0;
-    const int sub = (np + r - 1) / r;
-    const int ms = min(np, q * sub), me = min(np, ms + sub);  // chunk-local
+    const int span = force_group(W.n) * W.ppc;
+    const int m0 = min(P, bt.z * span), np = min(P, m0 + span) - m0;
+    int ms, me;
+    share_range(W, P, bt.z, wv, ms, me);
     const bool valid = il < W.n;
     const int i = W.a0 + (valid ? il : 0);
     const float4 xi = a.xyzq[i];
@@ -832,22 +829,13 @@ __global__ __launch_bounds__(kBlock) void k_force_epi(ForceArgs a, EpilogueArgs 
     }
     stage_lds(lds_tab, a.tab.f, nt);
     __syncthreads();
-    const bool wave_idle = bt.y * kBlock + (wv % nrw) * kWave >= W.n;
-    if (wave_idle) return;
     const bool pbc = a.pbc_flag[bt.x] != 0;
     const DiffFParams fp{0.0f, 0.0f, 0.0f, 0.0f};
     ForceAcc acc{0, 0, 0, 0, 0, 0, 0, 0, 0};
-    force_chunk<false, false>(a, lrec, laux, ms, me, W, pbc, xi, R2, lds_tab + ti * a.tab.ld_f,
-                              fp, acc);
-    if (r > 1 && !replica_sum<false>(reinterpret_cast<double *>(lds_tab + a.red_off), r, q, slot,
-                                     nrw * kWave, acc))
-        return;
-    if (!valid) return;
-    const long long o = W.ppo + (long long)chunk * W.n + il;
-    double2 *e = reinterpret_cast<double2 *>(a.part + o * force_part_stride(false));
-    e[0] = make_double2(acc.ex, acc.ey);
-    e[1] = make_double2(acc.ez, acc.lx);
-    e[2] = make_double2(acc.ly, acc.lz);
+    force_chunk<false, false>(a, lrec, laux, ms - m0, me - m0, W, pbc, xi, R2,
+                              lds_tab + ti * a.tab.ld_f, fp, acc);
+    if (!share_sum<false>(reinterpret_cast<double *>(lds_tab + a.red_off), wv, lane, acc)) return;
+    if (valid) write_force_entry<false>(a, W, bt.z, il, acc);
 }
 
 // F_i = -q_i vtot_i S_e - vtot_i S_lj over the chunk partials, summed in the
@@ -942,9 +930,9 @@ hipError_t launch_epilogue(const EpilogueArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
-bool force_epi_fits(const TableView &t, int max_window_atoms, int max_chunk_points, int nblocks)
+bool force_epi_fits(const TableView &t, int max_window_atoms, int max_group_points, int nblocks)
 {
-    return max_window_atoms <= kBlock && max_chunk_points <= kFuseMaxPts &&
+    return max_window_atoms <= kBlock && max_group_points <= kFuseMaxPts &&
            nblocks <= kFuseMaxBlocks && force_tab_floats(t) <= kTabLdsFloats;
 }
 
@@ -953,8 +941,7 @@ hipError_t launch_force_epi(const ForceArgs &a, const EpilogueArgs &ea, int nblo
     if (nblocks == 0) return hipSuccess;
     ForceArgs b = a;
     b.red_off = fused_lds_floats(a.tab);  // a multiple of 4 floats
-    const int red = a.replicas > 1 ? 2 * force_replica_doubles(false) : 0;
-    const size_t lds = (size_t)(b.red_off + red) * sizeof(float);
+    const size_t lds = (size_t)(b.red_off + 2 * force_share_doubles(false)) * sizeof(float);
     hipLaunchKernelGGL(k_force_epi, dim3(nblocks), dim3(kBlock), lds, s, b, ea);
     return hipGetLastError();
 }
@@ -963,23 +950,17 @@ hipError_t launch_force(const ForceArgs &a, int nblocks, bool split, hipStream_t
 {
     if (nblocks == 0) return hipSuccess;
     // dynamic LDS: the F table when it fits (table model), then the
-    // replica-sum area when some window has receiver replicas
+    // share-sum area
     ForceArgs b = a;
     const int nt = force_tab_floats(a.tab);
     b.red_off = (!a.dtypes && nt <= kTabLdsFloats) ? (nt + 3) & ~3 : 0;
-    const int red = a.replicas > 1 ? 2 * force_replica_doubles(split) : 0;
-    const size_t lds = (size_t)(b.red_off + red) * sizeof(float);
+    const size_t lds = (size_t)(b.red_off + 2 * force_share_doubles(split)) * sizeof(float);
     const dim3 g(nblocks), t(kBlock);
-    const int v = (a.dtypes ? 4 : 0) + (split ? 2 : 0) + (a.replicas > 1 ? 1 : 0);
-    switch (v) {
-    case 0: hipLaunchKernelGGL((k_force<false, false, false>), g, t, lds, s, b); break;
-    case 1: hipLaunchKernelGGL((k_force<false, false, true>), g, t, lds, s, b); break;
-    case 2: hipLaunchKernelGGL((k_force<true, false, false>), g, t, lds, s, b); break;
-    case 3: hipLaunchKernelGGL((k_force<true, false, true>), g, t, lds, s, b); break;
-    case 4: hipLaunchKernelGGL((k_force<false, true, false>), g, t, lds, s, b); break;
-    case 5: hipLaunchKernelGGL((k_force<false, true, true>), g, t, lds, s, b); break;
-    case 6: hipLaunchKernelGGL((k_force<true, true, false>), g, t, lds, s, b); break;
-    default: hipLaunchKernelGGL((k_force<true, true, true>), g, t, lds, s, b); break;
+    switch ((a.dtypes ? 2 : 0) + (split ? 1 : 0)) {
+    case 0: hipLaunchKernelGGL((k_force<false, false>), g, t, lds, s, b); break;
+    case 1: hipLaunchKernelGGL((k_force<true, false>), g, t, lds, s, b); break;
+    case 2: hipLaunchKernelGGL((k_force<false, true>), g, t, lds, s, b); break;
+    default: hipLaunchKernelGGL((k_force<true, true>), g, t, lds, s, b); break;
     }
     return hipGetLastError();
 }

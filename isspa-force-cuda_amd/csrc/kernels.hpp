@@ -22,7 +22,7 @@ struct WinDesc {
     int chunks, ppc;    // force pass: point chunks, points per chunk
     int nbc, apc;       // nonbond: partner chunks, atoms per chunk
     long long fpo;      // field partial offset:  sum over earlier windows of splits * P
-    long long ppo;      // force partial offset:  sum of chunks * n
+    long long ppo;      // force partial offset:  sum of fents * n
     long long npo;      // nonbond partial offset: sum of nbc * n
     uint32_t sys;       // Philox counter word 3
     float L, h;         // box length and half length
@@ -31,8 +31,10 @@ struct WinDesc {
     int fg;             // field pass: splits per block (1, 2 or 4; divides splits);
                         // the block's waves take fg splits of 256 / fg points
                         // and leave one partial per group of fg splits
-    int fgpad;
+    int fents;          // force pass: partial entries per atom, ceil(chunks / force_group(n))
     long long spo;      // nonbond total-force partial offset: sum of nte * n
+    long long vpo;      // adjoint atom-pass partial offset: sum of vents * n
+    int vents, vpad;    // adjoint atom pass: entries per atom, ceil(chunks / 4)
 };
 
 // splits per field block for a window of `splits` splits
@@ -143,7 +145,7 @@ struct EpilogueArgs {
 
 struct ForceArgs {
     const WinDesc *wins;
-    const int4 *blocks;   // {w, receiver block, chunk, -}
+    const int4 *blocks;   // {w, receiver block (64 atoms), chunk group, -}
     const float4 *rec4;   // [P][4] float4 view of the records
     const float4 *aux4;   // [P] {cp E0, A1}
     const float4 *xyzq;
@@ -156,19 +158,23 @@ struct ForceArgs {
     double *part;         // [C][stride]: (S_e, S_lj), or (pol, lj, cdd, pad) split
     long long C;
     int xcd_runs;         // 1: each XCD takes a contiguous run of the table (equal work items)
-    int replicas;         // most receiver replicas of any window (force_replicas of the smallest)
-    int red_off;          // float offset of the replica-sum area in the dynamic LDS (set at launch)
+    int red_off;          // float offset of the share-sum area in the dynamic LDS (set at launch)
 };
 
-// Windows of at most 128 atoms fill only one or two of a 256-thread force
-// block's four waves with receivers.  The other waves then take a share of
-// the chunk's points for the same receivers (4 replicas of the receivers at
-// <= 64 atoms, 2 at <= 128), and the block adds the replicas' sums in replica
-// order before it writes the chunk's partial: the same parallelism with a
-// quarter (or half) of the chunks, so a quarter of the partials to reduce.
-__host__ __device__ constexpr int force_replicas(int n) { return n <= 64 ? 4 : (n <= 128 ? 2 : 1); }
-// doubles of the replica-sum area: replicas 1..r-1 of 64 * (4 / r) receivers
-__host__ __device__ constexpr int force_replica_doubles(bool split)
+// A force block's four waves serve the same 64 receivers, each with its own
+// share of the MC points, and the block adds the shares' sums in order before
+// it writes one partial: a quarter of the partials of a block that gives each
+// wave its own receivers, at the same number of waves, and no idle wave in
+// the last receiver block.  A share is a whole chunk, or, in windows of at
+// most 128 (64) atoms, a half (quarter) of one; the block takes force_group
+// consecutive chunks.  Against 256 receivers a block: the force assembly, which
+// reads the partials, 78 -> 38 us at 19,998 atoms and 13.9 -> 10.4 us at
+// 1,100, the force pass there 43.0 -> 40.9 us, the differentiable model's
+// reduction of 32 x 1,100 atoms 81 -> 16 us.
+__host__ __device__ constexpr int force_shares(int n) { return n <= 64 ? 4 : (n <= 128 ? 2 : 1); }
+__host__ __device__ constexpr int force_group(int n) { return 4 / force_shares(n); }
+// doubles of the share-sum area: shares 1..3 of 64 receivers
+__host__ __device__ constexpr int force_share_doubles(bool split)
 {
     return 3 * 64 * (split ? 9 : 6);
 }
@@ -183,8 +189,8 @@ __device__ __forceinline__ int xcd_run_entry(int b, int nb)
     return x * q + (x < r ? x : r) + k;
 }
 
-// The force pass's chunk partials are stored entry by entry, entry
-// (chunk, atom) holding its components together: 6 doubles (S_e, S_lj), or
+// The force pass's partials are stored entry by entry, entry
+// (chunk group, atom) holding its components together: 6 doubles (S_e, S_lj), or
 // 10 in split mode (pol, lj, cdd and a pad, so every entry stays 16-byte
 // aligned), read and written as double2.
 __host__ __device__ constexpr int force_part_stride(bool split) { return split ? 10 : 6; }
@@ -225,9 +231,9 @@ hipError_t launch_mc_points(const WinDesc *wins, const int *atom_win, const floa
 hipError_t launch_field(const FieldArgs &a, int nblocks, hipStream_t s);
 hipError_t launch_epilogue(const EpilogueArgs &a, hipStream_t s);
 // the epilogue and the force pass in one launch, for models whose windows all
-// fit one receiver block, whose chunks hold at most 256 points and whose force
-// grid has at most 256 blocks (table model, total force only)
-bool force_epi_fits(const TableView &t, int max_window_atoms, int max_chunk_points, int nblocks);
+// have at most 256 atoms, whose chunk groups hold at most 256 points and whose
+// force grid has at most 256 blocks (table model, total force only)
+bool force_epi_fits(const TableView &t, int max_window_atoms, int max_group_points, int nblocks);
 hipError_t launch_force_epi(const ForceArgs &a, const EpilogueArgs &ea, int nblocks, hipStream_t s);
 hipError_t launch_force(const ForceArgs &a, int nblocks, bool split, hipStream_t s);
 hipError_t launch_force_reduce(const ReduceArgs &a, bool split, hipStream_t s);
@@ -347,7 +353,7 @@ struct DiffReduceArgs {
 struct VjpArgs {
     const WinDesc *wins;
     const int *atom_win;
-    const int4 *fblk, *pblk;   // point-lane and atom-lane block tables
+    const int4 *fblk, *vblk;   // point-lane and atom-lane block tables
     int nmc;
     long long Ptot;
     const float4 *pts, *rec4, *aux4, *arec, *xq;
@@ -363,7 +369,7 @@ struct VjpArgs {
     long long F;
     float4 *prec;              // [P][4] {p, R2}, {dL/dE, g dL/dg}, {dL/dE0, w}, -
     double *apart;             // [6][C] atom bars: q, theta(5)
-    long long C;
+    long long C;               // sum of vents * n
 };
 struct VjpNbArgs {
     const WinDesc *wins;

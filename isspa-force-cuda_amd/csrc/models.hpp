@@ -53,14 +53,15 @@ struct isspa_model {
     // split a block, the adjoint's point pass)
     int4 *fblk = nullptr, *pblk = nullptr, *gblk = nullptr;
     int nfblk = 0, npblk = 0, ngblk = 0;
+    int4 *vblk = nullptr;  // the adjoint's atom pass: {w, 64 atoms, four chunks, -}
+    int nvblk = 0;
     int max_fg = 1;  // the largest splits-per-field-block of the windows
-    int max_win_atoms = 0, max_chunk_pts = 0;  // over the windows, for the fused force launch
-    int min_win_atoms = 0;                     // the smallest window: receiver replicas
+    int max_win_atoms = 0, max_group_pts = 0;  // over the windows, for the fused force launch
     double *part_g = nullptr;
     int *part_cnt = nullptr;
     double *part_s0 = nullptr, *part_ein = nullptr;
     double *part_f = nullptr;
-    long long F = 0, C = 0, cap_field = 0, cap_force = 0;
+    long long F = 0, C = 0, V = 0, cap_field = 0, cap_force = 0;
     float4 *prof_f = nullptr;  // force sink of isspa_model_profile
     TableView tv{};
     // bumped whenever the launch tables are rebuilt; a graph captured under

@@ -69,7 +69,7 @@ __device__ inline void force_slice_sum(const WinDesc &W, const double *part, int
 {
     const long long base = W.ppo + (i - W.a0);
     int c = sl;
-    for (; c + (kSumBatch - 1) * kSumSlices < W.chunks; c += kSumBatch * kSumSlices) {
+    for (; c + (kSumBatch - 1) * kSumSlices < W.fents; c += kSumBatch * kSumSlices) {
         double v[kSumBatch][COMPS];
 #pragma unroll
         for (int u = 0; u < kSumBatch; ++u)
@@ -79,7 +79,7 @@ __device__ inline void force_slice_sum(const WinDesc &W, const double *part, int
 #pragma unroll
             for (int k = 0; k < COMPS; ++k) s[k] += v[u][k];
     }
-    for (; c < W.chunks; c += kSumSlices) {
+    for (; c < W.fents; c += kSumSlices) {
         double v[COMPS];
         load_force_entry<COMPS>(part, base + (long long)c * W.n, v);
 #pragma unroll
