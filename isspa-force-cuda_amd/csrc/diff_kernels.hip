@@ -155,7 +155,7 @@ struct PointBar {
 
 template <bool PBC>
 __device__ __forceinline__ void vjp_points_tile(const VjpArgs &a, const DiffType *dtypes, int j0,
-                                                int j1, float L, float h, float px, float py,
+                                                int j1, const MinImage &mi, float px, float py,
                                                 float pz, float Ex, float Ey, float Ez, float A1,
                                                 float A2, float A3, PointBar &b)
 {
@@ -166,9 +166,9 @@ __device__ __forceinline__ void vjp_points_tile(const VjpArgs &a, const DiffType
         const float4 r2 = ar[4 * j + 2];
         float rx = px - r0.x, ry = py - r0.y, rz = pz - r0.z;
         if (PBC) {
-            rx = min_image1(rx, L, h);
-            ry = min_image1(ry, L, h);
-            rz = min_image1(rz, L, h);
+            rx = min_image1(rx, mi);
+            ry = min_image1(ry, mi);
+            rz = min_image1(rz, mi);
         }
         const float d2 = dist2_f32(rx, ry, rz);
         const float rinv = rsqrt_f32(d2);
@@ -227,15 +227,16 @@ __global__ __launch_bounds__(kB) void k_vjp_points(VjpArgs a)
     const float A1 = a.aux4[gp].w;
     const bool pbc = a.pbc_flag[bt.x] != 0;
     const DiffType *dtypes = stage_dtypes(a);
+    const MinImage mi = min_image_of(W.L, W.h);
     double acc[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     for (int jt = j0; jt < j1; jt += kTile) {
         const int je = min(j1, jt + kTile);
         PointBar b{0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         if (pbc)
-            vjp_points_tile<true>(a, dtypes, jt, je, W.L, W.h, q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, A1,
+            vjp_points_tile<true>(a, dtypes, jt, je, mi, q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, A1,
                                   q3.x, q3.z, b);
         else
-            vjp_points_tile<false>(a, dtypes, jt, je, W.L, W.h, q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, A1,
+            vjp_points_tile<false>(a, dtypes, jt, je, mi, q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, A1,
                                    q3.x, q3.z, b);
         acc[0] += b.hx; acc[1] += b.hy; acc[2] += b.hz;
         acc[3] += b.a1; acc[4] += b.a2; acc[5] += b.a3;
@@ -331,8 +332,8 @@ __global__ __launch_bounds__(kB) void k_vjp_epilogue(VjpArgs a)
 // ---------------------------------------------------------------------------
 template <bool PBC>
 __device__ __forceinline__ void vjp_atoms_tile(const VjpArgs &a, const float4 *__restrict__ pr,
-                                               const DiffType &Tj, int m0, int m1, float L,
-                                               float h, float4 xj, float R2j, float lpx,
+                                               const DiffType &Tj, int m0, int m1,
+                                               const MinImage &mi, float4 xj, float R2j, float lpx,
                                                float lpy, float lpz, float &qb, double tb[5])
 {
     const float e0 = a.e0;
@@ -342,9 +343,9 @@ __device__ __forceinline__ void vjp_atoms_tile(const VjpArgs &a, const float4 *_
         const float4 e0b = pr[4 * m + 2];
         float rx = p.x - xj.x, ry = p.y - xj.y, rz = p.z - xj.z;
         if (PBC) {
-            rx = min_image1(rx, L, h);
-            ry = min_image1(ry, L, h);
-            rz = min_image1(rz, L, h);
+            rx = min_image1(rx, mi);
+            ry = min_image1(ry, mi);
+            rz = min_image1(rz, mi);
         }
         const float d2 = dist2_f32(rx, ry, rz);
         const float rinv = rsqrt_f32(d2);
@@ -398,15 +399,16 @@ __global__ __launch_bounds__(kB) void k_vjp_atoms(VjpArgs a)
     const float4 lp = a.arec[4 * (size_t)j + 2];  // Lambda' = -vtot lambda
     const bool pbc = a.pbc_flag[bt.x] != 0;
     const DiffType &Tj = stage_dtypes(a)[tj];
+    const MinImage mi = min_image_of(W.L, W.h);
     double acc[6] = {0, 0, 0, 0, 0, 0};  // q, theta(5)
     double tb[5] = {0, 0, 0, 0, 0};
     for (int mt = m0; mt < m1; mt += kTile) {
         const int me = min(m1, mt + kTile);
         float qb = 0.0f;
         if (pbc)
-            vjp_atoms_tile<true>(a, pr, Tj, mt, me, W.L, W.h, xj, R2j, lp.x, lp.y, lp.z, qb, tb);
+            vjp_atoms_tile<true>(a, pr, Tj, mt, me, mi, xj, R2j, lp.x, lp.y, lp.z, qb, tb);
         else
-            vjp_atoms_tile<false>(a, pr, Tj, mt, me, W.L, W.h, xj, R2j, lp.x, lp.y, lp.z, qb, tb);
+            vjp_atoms_tile<false>(a, pr, Tj, mt, me, mi, xj, R2j, lp.x, lp.y, lp.z, qb, tb);
         acc[0] += (double)qb;
     }
     for (int k = 0; k < 5; ++k) acc[1 + k] = tb[k];
@@ -443,7 +445,7 @@ __global__ __launch_bounds__(kB) void k_vjp_nonbond(VjpNbArgs a)
     uint32_t ex[4];
     for (int k = 0; k < 4; ++k) ex[k] = a.excl[4 * i + k];
     const bool pbc = a.pbc_flag[bt.x] != 0;
-    const float L = W.L, h = W.h;
+    const MinImage mi = min_image_of(W.L, W.h);
     const int wave_lo = W.a0 + bt.y * kB + (threadIdx.x & ~(kWave - 1));
     const float4 *ldrow = lds_ld + ti * a.T;
     double qacc = 0.0, sacc = 0.0, eacc = 0.0;
@@ -457,9 +459,9 @@ __global__ __launch_bounds__(kB) void k_vjp_nonbond(VjpNbArgs a)
             const float4 lj4 = a.arec[4 * (size_t)j + 3];
             float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
             if (pbc) {
-                rx = min_image1(rx, L, h);
-                ry = min_image1(ry, L, h);
-                rz = min_image1(rz, L, h);
+                rx = min_image1(rx, mi);
+                ry = min_image1(ry, mi);
+                rz = min_image1(rz, mi);
             }
             const float d2 = dist2_f32(rx, ry, rz);
             const float inv = rsqrt_f32(d2);

@@ -147,7 +147,7 @@ __device__ __forceinline__ void field_in_sphere_an(const DiffType &T, float d2, 
 template <bool PBC, bool AN>
 __device__ __forceinline__ void field_tile(const FieldArgs &a, const float *Gtab,
                                            const float *Etab, const DiffType *dtypes, int j0,
-                                           int j1, float L, float h,
+                                           int j1, const MinImage &mi,
                                            float px, float py, float pz, float R2, float &ax,
                                            float &ay, float &az, FieldRare &st)
 {
@@ -162,9 +162,9 @@ __device__ __forceinline__ void field_tile(const FieldArgs &a, const float *Gtab
         const float4 q = make_float4(xq[0], xq[1], xq[2], xq[3]);
         float rx = px - q.x, ry = py - q.y, rz = pz - q.z;
         if (PBC) {
-            rx = min_image1(rx, L, h);
-            ry = min_image1(ry, L, h);
-            rz = min_image1(rz, L, h);
+            rx = min_image1(rx, mi);
+            ry = min_image1(ry, mi);
+            rz = min_image1(rz, mi);
         }
         const float d2 = dist2_f32(rx, ry, rz);
         const float inv = rsqrt_f32(d2);
@@ -197,15 +197,16 @@ __device__ __forceinline__ void field_span(const FieldArgs &a, const float *Gtab
                                            FieldSums &fs)
 {
     FieldRare &st = fs.st;
+    const MinImage mi = min_image_of(W.L, W.h);
     for (int jt = j0; jt < j1; jt += kFieldTile) {
         const int je = min(j1, jt + kFieldTile);
         float ax = 0.0f, ay = 0.0f, az = 0.0f;
         st.ex = st.ey = st.ez = 0.0f;
         if (pbc)
-            field_tile<true, AN>(a, Gtab, Etab, dtypes, jt, je, W.L, W.h, p.x, p.y, p.z, p.w, ax,
+            field_tile<true, AN>(a, Gtab, Etab, dtypes, jt, je, mi, p.x, p.y, p.z, p.w, ax,
                                  ay, az, st);
         else
-            field_tile<false, AN>(a, Gtab, Etab, dtypes, jt, je, W.L, W.h, p.x, p.y, p.z, p.w, ax,
+            field_tile<false, AN>(a, Gtab, Etab, dtypes, jt, je, mi, p.x, p.y, p.z, p.w, ax,
                                   ay, az, st);
         fs.sx += (double)ax;
         fs.sy += (double)ay;
@@ -527,7 +528,7 @@ struct TileSums {
 template <bool PBC, bool SPLIT, bool AN>
 __device__ __forceinline__ void force_tile(const ForceArgs &a, const float4 *__restrict__ rec,
                                            const float4 *__restrict__ aux, int m0, int m1,
-                                           float L, float h, float xi, float yi, float zi,
+                                           const MinImage &mi, float xi, float yi, float zi,
                                            float R2, const float *Ftab,
                                            const DiffFParams &fp, TileSums &ts, ForceAcc &acc)
 {
@@ -559,9 +560,9 @@ __device__ __forceinline__ void force_tile(const ForceArgs &a, const float4 *__r
         const float A2 = q3.x, A2x3 = q3.y, A3 = q3.z, w = q3.w;
         float rx = q0.x - xi, ry = q0.y - yi, rz = q0.z - zi;
         if (PBC) {
-            rx = min_image1(rx, L, h);
-            ry = min_image1(ry, L, h);
-            rz = min_image1(rz, L, h);
+            rx = min_image1(rx, mi);
+            ry = min_image1(ry, mi);
+            rz = min_image1(rz, mi);
         }
         const float d2 = dist2_f32(rx, ry, rz);
         const float rinv = rsqrt_f32(d2);
@@ -639,15 +640,16 @@ __device__ __forceinline__ void force_chunk(const ForceArgs &a, const float4 *__
                                             const float *Ftab, const DiffFParams &fp,
                                             ForceAcc &acc)
 {
+    const MinImage mi = min_image_of(W.L, W.h);
     for (int mt = m0; mt < m1; mt += kForceTile) {
         const int me = min(m1, mt + kForceTile);
         TileSums ts{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
         // tile-local point indices from the tile's first record
         if (pbc)
-            force_tile<true, SPLIT, AN>(a, rec + 4 * mt, aux + mt, 0, me - mt, W.L, W.h, xi.x,
+            force_tile<true, SPLIT, AN>(a, rec + 4 * mt, aux + mt, 0, me - mt, mi, xi.x,
                                         xi.y, xi.z, R2, Ftab, fp, ts, acc);
         else
-            force_tile<false, SPLIT, AN>(a, rec + 4 * mt, aux + mt, 0, me - mt, W.L, W.h, xi.x,
+            force_tile<false, SPLIT, AN>(a, rec + 4 * mt, aux + mt, 0, me - mt, mi, xi.x,
                                          xi.y, xi.z, R2, Ftab, fp, ts, acc);
         acc.ex += (double)ts.sx;
         acc.ey += (double)ts.sy;

@@ -26,7 +26,7 @@ constexpr int kNbNear = 0, kNbFar = 1, kNbFast = 2;
 
 template <bool PBC, bool SPLIT, int KIND>
 __device__ __forceinline__ void nonbond_tile(const NonbondArgs &a, int i, int j0, int j1,
-                                             float L, float h, float4 xi, const uint32_t *ex,
+                                             const MinImage &mi, float4 xi, const uint32_t *ex,
                                              const float2 *__restrict__ ljrow, double *acc)
 {
     static_assert(KIND != kNbFast || !SPLIT, "the fast tile sums the total force only");
@@ -48,9 +48,9 @@ __device__ __forceinline__ void nonbond_tile(const NonbondArgs &a, int i, int j0
         nlj = ljrow[__float_as_int(na.w)];
         float rx = xi.x - xj.x, ry = xi.y - xj.y, rz = xi.z - xj.z;
         if (PBC) {
-            rx = min_image1(rx, L, h);
-            ry = min_image1(ry, L, h);
-            rz = min_image1(rz, L, h);
+            rx = min_image1(rx, mi);
+            ry = min_image1(ry, mi);
+            rz = min_image1(rz, mi);
         }
         const float d2 = dist2_f32(rx, ry, rz);
         const float inv = rsqrt_f32(d2);
@@ -177,7 +177,8 @@ __device__ __forceinline__ float row_rot(float v)
 
 struct SymLane {
     float xi, yi, zi, qi, ri2, cai, cbi;  // the lane's receiver
-    float cfar, cfar1, L, h;              // in VGPRs
+    float cfar, cfar1;                    // in VGPRs
+    MinImage mi;
     const char *ljrow;                    // receiver's LJ row in LDS
     float px, py, pz, pq, pr2, pca, pcb;  // the lane's partner of this round
     int pt8;                              // its LJ column, in bytes
@@ -199,9 +200,9 @@ __device__ __forceinline__ void sym_step(SymLane &l)
     float ry = l.yi - row_rot<S>(l.py);
     float rz = l.zi - row_rot<S>(l.pz);
     if (PBC) {
-        rx = min_image1(rx, l.L, l.h);
-        ry = min_image1(ry, l.L, l.h);
-        rz = min_image1(rz, l.L, l.h);
+        rx = min_image1(rx, l.mi);
+        ry = min_image1(ry, l.mi);
+        rz = min_image1(rz, l.mi);
     }
     const float d2 = dist2_f32(rx, ry, rz);
     const float inv = rsqrt_f32(d2);
@@ -270,8 +271,9 @@ __device__ __forceinline__ void nonbond_supertile(const NonbondArgs &a, const Wi
     // multiplies by them read VGPRs (a wave-uniform SGPR operand halves the
     // issue rate of an FP32 operation)
     asm volatile("v_mov_b32 %0, %1" : "=v"(l.cfar) : "s"(a.cfar));
-    asm volatile("v_mov_b32 %0, %1" : "=v"(l.L) : "s"(W.L));
-    asm volatile("v_mov_b32 %0, %1" : "=v"(l.h) : "s"(W.h));
+    float L;
+    asm volatile("v_mov_b32 %0, %1" : "=v"(L) : "s"(W.L));
+    l.mi = min_image_of(L, 0.5f * L);
     l.cfar1 = 1.0f + l.cfar;
     l.ljrow = reinterpret_cast<const char *>(lds_lj + __float_as_int(ai.w) * a.T);
     const int pbase = W.a0 + pb * kNbBlock, pend = W.a0 + W.n;
@@ -355,6 +357,7 @@ __device__ __forceinline__ void nonbond_block(const NonbondArgs &a, int blk, flo
     uint32_t ex[4];
     for (int k = 0; k < 4; ++k) ex[k] = a.excl[4 * i + k];
     const bool pbc = a.pbc_flag[bt.x] != 0;
+    const MinImage mi = min_image_of(W.L, W.h);
     // first receiver of this wave, for the near-diagonal test
     const int wave_lo = W.a0 + bt.y * kNbBlock + (threadIdx.x & ~(kWave - 1));
     double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -365,20 +368,20 @@ __device__ __forceinline__ void nonbond_block(const NonbondArgs &a, int blk, flo
         const bool near = (jt < wave_lo + kWave + 64) && (je > wave_lo - 64);
         if (near) {
             if (pbc)
-                nonbond_tile<true, SPLIT, kNbNear>(a, i, jt, je, W.L, W.h, xi, ex, ljrow, acc);
+                nonbond_tile<true, SPLIT, kNbNear>(a, i, jt, je, mi, xi, ex, ljrow, acc);
             else
-                nonbond_tile<false, SPLIT, kNbNear>(a, i, jt, je, W.L, W.h, xi, ex, ljrow, acc);
+                nonbond_tile<false, SPLIT, kNbNear>(a, i, jt, je, mi, xi, ex, ljrow, acc);
         } else if (SPLIT || a.excl_ptr) {
             if (pbc)
-                nonbond_tile<true, SPLIT, kNbFar>(a, i, jt, je, W.L, W.h, xi, ex, ljrow, acc);
+                nonbond_tile<true, SPLIT, kNbFar>(a, i, jt, je, mi, xi, ex, ljrow, acc);
             else
-                nonbond_tile<false, SPLIT, kNbFar>(a, i, jt, je, W.L, W.h, xi, ex, ljrow, acc);
+                nonbond_tile<false, SPLIT, kNbFar>(a, i, jt, je, mi, xi, ex, ljrow, acc);
         } else {
             constexpr int kFast = SPLIT ? kNbFar : kNbFast;
             if (pbc)
-                nonbond_tile<true, SPLIT, kFast>(a, i, jt, je, W.L, W.h, xi, ex, ljrow, acc);
+                nonbond_tile<true, SPLIT, kFast>(a, i, jt, je, mi, xi, ex, ljrow, acc);
             else
-                nonbond_tile<false, SPLIT, kFast>(a, i, jt, je, W.L, W.h, xi, ex, ljrow, acc);
+                nonbond_tile<false, SPLIT, kFast>(a, i, jt, je, mi, xi, ex, ljrow, acc);
         }
     }
     if (!valid) return;
