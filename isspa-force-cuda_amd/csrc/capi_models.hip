@@ -99,7 +99,7 @@ static void isspa_free(isspa_model *m)
     dfree(m->g); dfree(m->e); dfree(m->f);
     dfree(m->pts); dfree(m->rec); dfree(m->g_out); dfree(m->E_out); dfree(m->E0_out);
     dfree(m->cnt_out); dfree(m->pbc_flag); dfree(m->wins); dfree(m->fblk); dfree(m->gblk);
-    dfree(m->pblk); dfree(m->vblk);
+    dfree(m->pblk); dfree(m->vblk); dfree(m->wblk);
     dfree(m->part_g); dfree(m->part_cnt); dfree(m->part_s0); dfree(m->part_ein); dfree(m->part_f);
     dfree(m->prof_f);
 }
@@ -121,7 +121,7 @@ static int isspa_tile(isspa_model *m)
     m->max_win_atoms = m->max_group_pts = 0;
     m->max_fg = 1;
     long long F = 0, C = 0, V = 0;
-    std::vector<std::pair<long long, int4>> fb, gb, pb, vb;
+    std::vector<std::pair<long long, int4>> fb, gb, pb, vb, wb;
     for (int w = 0; w < L.W; ++w) {
         WinDesc d = base_desc(L, w);
         const long long n = L.n[w], P = n * nmc;
@@ -167,6 +167,9 @@ static int isspa_tile(isspa_model *m)
         for (int gr = 0; gr < d.fents; ++gr)
             for (int b = 0; b < rblocks; ++b)
                 pb.push_back({(long long)(d.ppc + shares - 1) / shares, make_int4(w, b, gr, 0)});
+        // k_window: a group of a window's points, by its work
+        for (int gr = 0; gr < d.fents; ++gr)
+            wb.push_back({n * std::min(P, (long long)group * d.ppc), make_int4(w, 0, gr, 0)});
         for (int gr = 0; gr < d.vents; ++gr)
             for (int b = 0; b < rblocks; ++b) vb.push_back({(long long)d.ppc, make_int4(w, b, gr, 0)});
         m->wins_h[w] = d;
@@ -178,21 +181,26 @@ static int isspa_tile(isspa_model *m)
     std::stable_sort(gb.begin(), gb.end(), by_work);
     std::stable_sort(pb.begin(), pb.end(), by_work);
     std::stable_sort(vb.begin(), vb.end(), by_work);
-    std::vector<int4> fbv, gbv, pbv, vbv;
+    std::stable_sort(wb.begin(), wb.end(), by_work);
+    std::vector<int4> fbv, gbv, pbv, vbv, wbv;
     for (auto &x : fb) fbv.push_back(x.second);
     for (auto &x : gb) gbv.push_back(x.second);
     for (auto &x : pb) pbv.push_back(x.second);
     for (auto &x : vb) vbv.push_back(x.second);
+    for (auto &x : wb) wbv.push_back(x.second);
+    dfree(m->wblk);
     dfree(m->wins); dfree(m->fblk); dfree(m->gblk); dfree(m->pblk); dfree(m->vblk);
     CHK(upload(&m->wins, m->wins_h.data(), m->wins_h.size()));
     CHK(upload(&m->fblk, fbv.data(), fbv.size()));
     CHK(upload(&m->gblk, gbv.data(), gbv.size()));
     CHK(upload(&m->pblk, pbv.data(), pbv.size()));
     CHK(upload(&m->vblk, vbv.data(), vbv.size()));
+    CHK(upload(&m->wblk, wbv.data(), wbv.size()));
     m->nfblk = (int)fbv.size();
     m->ngblk = (int)gbv.size();
     m->npblk = (int)pbv.size();
     m->nvblk = (int)vbv.size();
+    m->nwblk = (int)wbv.size();
     m->F = F;
     m->C = C;
     m->V = V;
@@ -396,6 +404,22 @@ ReduceArgs reduce_args(isspa_model *m, const float4 *x, float4 *f, double *flj, 
     return ra;
 }
 
+// whether the total force runs as k_window (small windows)
+bool isspa_is_small(const isspa_model *m)
+{
+    return window_fits(m->tv, m->max_win_atoms, m->max_group_pts, m->nwblk);
+}
+
+WindowArgs window_args(isspa_model *m, const float4 *x, uint32_t step, const uint32_t *step_d)
+{
+    WindowArgs a{};
+    a.wins = m->wins; a.blocks = m->wblk; a.nblocks = m->nwblk; a.xyzq = x; a.itype = m->itype;
+    a.rmax = m->rmax; a.rmax2 = m->rmax2; a.rmax_all = m->rmax_all; a.tab = m->tv;
+    a.nmc = m->d.n_mc; a.e0 = m->d.e0; a.p0 = m->d.p0; a.q0 = m->d.q0; a.o0 = m->d.o0;
+    a.seed = m->d.seed; a.step = step; a.step_d = step_d; a.pts = m->pts; a.part = m->part_f;
+    return a;
+}
+
 // points + field + epilogue (shared by the total and component entry points)
 static int isspa_field_pass(isspa_model *m, const float *xyzq4_d, uint32_t step,
                             const uint32_t *step_d, hipStream_t s, bool inspect = false)
@@ -409,15 +433,21 @@ static int isspa_field_pass(isspa_model *m, const float *xyzq4_d, uint32_t step,
     return ISSPA_OK;
 }
 
-static int isspa_force_pass(isspa_model *m, const float *xyzq4_d, bool split, float4 *f,
-                            double *flj, double *fpol, double *fcdd, hipStream_t s,
-                            float4 *f_alone = nullptr)
+// the total force: partials by the small-window launch or by the separate
+// passes, then their sum
+static int isspa_total(isspa_model *m, const float *xyzq4_d, float *f4_d, float *f_isspa4_d,
+                       uint32_t step, const uint32_t *step_d, hipStream_t s)
 {
     const float4 *x = reinterpret_cast<const float4 *>(xyzq4_d);
-    HIPCHK(launch_force(force_args(m, x), m->npblk, split, s));
-    ReduceArgs ra = reduce_args(m, x, f, flj, fpol, fcdd);
-    ra.f_alone = f_alone;
-    HIPCHK(launch_force_reduce(ra, split, s));
+    if (isspa_is_small(m)) {
+        HIPCHK(launch_window(window_args(m, x, step, step_d), m->max_win_atoms, m->max_group_pts, s));
+    } else {
+        CHK(isspa_field_pass(m, xyzq4_d, step, step_d, s));
+        HIPCHK(launch_force(force_args(m, x), m->npblk, false, s));
+    }
+    ReduceArgs ra = reduce_args(m, x, reinterpret_cast<float4 *>(f4_d), nullptr, nullptr, nullptr);
+    ra.f_alone = reinterpret_cast<float4 *>(f_isspa4_d);
+    HIPCHK(launch_force_reduce(ra, false, s));
     return ISSPA_OK;
 }
 
@@ -425,9 +455,7 @@ extern "C" int isspa_model_force(isspa_model *m, const float *xyzq4_d, float *f4
                                  uint32_t step, const uint32_t *step_d, void *stream)
 {
     if (!m || !xyzq4_d || !f4_d) return fail(ISSPA_ERR_ARG, "isspa_model_force: null argument");
-    CHK(isspa_field_pass(m, xyzq4_d, step, step_d, S(stream)));
-    return isspa_force_pass(m, xyzq4_d, false, reinterpret_cast<float4 *>(f4_d), nullptr, nullptr,
-                            nullptr, S(stream));
+    return isspa_total(m, xyzq4_d, f4_d, nullptr, step, step_d, S(stream));
 }
 
 extern "C" int isspa_model_force_keep(isspa_model *m, const float *xyzq4_d, float *f4_d,
@@ -436,9 +464,7 @@ extern "C" int isspa_model_force_keep(isspa_model *m, const float *xyzq4_d, floa
 {
     if (!m || !xyzq4_d || !f4_d || !f_isspa4_d)
         return fail(ISSPA_ERR_ARG, "isspa_model_force_keep: null argument");
-    CHK(isspa_field_pass(m, xyzq4_d, step, step_d, S(stream)));
-    return isspa_force_pass(m, xyzq4_d, false, reinterpret_cast<float4 *>(f4_d), nullptr, nullptr,
-                            nullptr, S(stream), reinterpret_cast<float4 *>(f_isspa4_d));
+    return isspa_total(m, xyzq4_d, f4_d, f_isspa4_d, step, step_d, S(stream));
 }
 
 extern "C" int isspa_model_force_components(isspa_model *m, const float *xyzq4_d,
@@ -447,8 +473,11 @@ extern "C" int isspa_model_force_components(isspa_model *m, const float *xyzq4_d
 {
     if (!m || !xyzq4_d || !f_lj_d || !f_pol_d || !f_cdd_d)
         return fail(ISSPA_ERR_ARG, "isspa_model_force_components: null argument");
+    const float4 *x = reinterpret_cast<const float4 *>(xyzq4_d);
     CHK(isspa_field_pass(m, xyzq4_d, step, nullptr, S(stream), true));
-    return isspa_force_pass(m, xyzq4_d, true, nullptr, f_lj_d, f_pol_d, f_cdd_d, S(stream));
+    HIPCHK(launch_force(force_args(m, x), m->npblk, true, S(stream)));
+    HIPCHK(launch_force_reduce(reduce_args(m, x, nullptr, f_lj_d, f_pol_d, f_cdd_d), true, S(stream)));
+    return ISSPA_OK;
 }
 
 extern "C" int isspa_model_profile(isspa_model *m, const float *xyzq4_d, int reps, float *ms,
@@ -1230,61 +1259,65 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
         CHK(nonbond_partials(e->nb, e->x, false, e->side));
         HIPCHK(hipEventRecord(e->ev_join, e->side));
     }
-    PrologueArgs p{};
     AssembleArgs a{};
     a.n = e->n;
     a.f = reinterpret_cast<float4 *>(e->f);
     isspa_model *m = e->isspa;
-    if (m) {
-        p.nflag = m->lay.W;
-        p.rmax_all = m->rmax_all;
-        p.flag = m->pbc_flag;
-        p.pts = PointsArgs{m->wins, m->atom_win, x4, m->itype, m->rmax, m->rmax2, m->d.n_atoms,
-                           m->d.n_mc, m->d.seed, 0u, e->step_d, m->pts};
-    }
+    BondedArgs bonded{};
+    RestraintArgs us{};
     if (e->bonded) {
-        p.bonded = bonded_args(e->bonded, ISSPA_TERM_ALL, e->x);
+        bonded = bonded_args(e->bonded, ISSPA_TERM_ALL, e->x);
         a.contrib = e->bonded->contrib;
         a.gptr = e->bonded->gptr;
         a.gidx = e->bonded->gidx;
     }
     if (e->us) {
-        p.nres = e->us->nres;
-        p.boff = e->us->boff;
-        p.us_atoms = e->us->atoms;
-        p.us_mass = e->us->mass;
-        p.kx = e->us->kx;
-        p.Ls = e->us->L;
-        p.fus = e->fus;
-        p.com = e->com_d;
+        us = RestraintArgs{e->us->nres, e->us->boff, e->us->atoms, e->us->mass, e->us->kx,
+                           e->us->L, e->fus, e->com_d};
         a.fus = e->fus;
     }
-    HIPCHK(launch_step_prologue(p, s));
-    // without the side stream the all-pairs blocks ride on the field launch,
-    // reusing the prologue's IS-SPA minimum-image flags (the field kernel
-    // carries partner-chunk blocks only: windows large enough for super-tiles
-    // always have the side stream)
-    const bool nb_in_field = m && e->nb && !fork && !e->nb->any_sym;
-    if (m) {
-        FieldArgs fa = field_args(m, x4);
-        if (nb_in_field) {
-            fa.nb = nonbond_args(e->nb, x4, m->pbc_flag, false);
-            fa.nb_blocks = e->nb->nblk_tot;
+    // without the side stream the all-pairs blocks ride on the small-window or
+    // the field launch (which carry partner-chunk blocks only: windows large
+    // enough for super-tiles always have the side stream)
+    const bool nb_rides = m && e->nb && !fork && !e->nb->any_sym;
+    if (m && isspa_is_small(m)) {
+        WindowArgs w = window_args(m, x4, 0u, e->step_d);
+        w.bonded = bonded;
+        w.us = us;
+        if (nb_rides) {
+            w.nb = nonbond_args(e->nb, x4, nullptr, false);
+            w.nb_blocks = e->nb->nblk_tot;
         }
-        HIPCHK(launch_field(fa, m->ngblk, s));
-        const ForceArgs fo = force_args(m, x4);
-        if (!fo.dtypes && force_epi_fits(fo.tab, m->max_win_atoms, m->max_group_pts, m->npblk)) {
-            // small windows: the epilogue inside the force launch
-            HIPCHK(launch_force_epi(fo, epilogue_args(m, false), m->npblk, s));
-        } else {
+        HIPCHK(launch_window(w, m->max_win_atoms, m->max_group_pts, s));
+    } else {
+        PrologueArgs p{};
+        p.bonded = bonded;
+        p.us = us;
+        p.pts.xyzq = x4;
+        if (m) {
+            p.nflag = m->lay.W;
+            p.rmax_all = m->rmax_all;
+            p.flag = m->pbc_flag;
+            p.pts = PointsArgs{m->wins, m->atom_win, x4, m->itype, m->rmax, m->rmax2,
+                               m->d.n_atoms, m->d.n_mc, m->d.seed, 0u, e->step_d, m->pts};
+        }
+        HIPCHK(launch_step_prologue(p, s));
+        if (m) {
+            FieldArgs fa = field_args(m, x4);
+            if (nb_rides) {
+                // with the prologue's IS-SPA minimum-image flags
+                fa.nb = nonbond_args(e->nb, x4, m->pbc_flag, false);
+                fa.nb_blocks = e->nb->nblk_tot;
+            }
+            HIPCHK(launch_field(fa, m->ngblk, s));
             HIPCHK(launch_epilogue(epilogue_args(m, false), s));
-            HIPCHK(launch_force(fo, m->npblk, false, s));
+            HIPCHK(launch_force(force_args(m, x4), m->npblk, false, s));
         }
-        a.isspa = reduce_args(m, x4, nullptr, nullptr, nullptr, nullptr);
     }
+    if (m) a.isspa = reduce_args(m, x4, nullptr, nullptr, nullptr, nullptr);
     if (fork)
         HIPCHK(hipStreamWaitEvent(s, e->ev_join, 0));
-    else if (e->nb && !nb_in_field)
+    else if (e->nb && !nb_rides)
         CHK(nonbond_partials(e->nb, e->x, false, s));
     if (e->nb) {
         a.nb_wins = e->nb->wins;

@@ -100,34 +100,40 @@ extern "C" int isspa_model_force_noalloc(isspa_model *m, const float *xyzq4_d, f
 
     hipStream_t s = S(stream);
     const float4 *x = reinterpret_cast<const float4 *>(xyzq4_d);
-    // the launches of isspa_model_force (isspa_field_pass, isspa_force_pass)
-    // with the buffers above
-    HIPCHK(launch_mc_points(m->wins, m->atom_win, x, m->itype, m->rmax, m->rmax2, m->d.n_atoms,
-                            m->d.n_mc, m->d.seed, step, step_d, pts, s, m->lay.W, m->rmax_all,
-                            flag));
-    FieldArgs fa = field_args(m, x);
-    fa.pts = pts;
-    fa.pbc_flag = flag;
-    fa.part_g = part_g;
-    fa.part_cnt = part_cnt;
-    fa.part_s0 = part_s0;
-    fa.part_ein = part_ein;
-    HIPCHK(launch_field(fa, m->ngblk, s));
-    EpilogueArgs ea = epilogue_args(m, false);
-    ea.pts = pts;
-    ea.part_g = part_g;
-    ea.part_cnt = part_cnt;
-    ea.part_s0 = part_s0;
-    ea.part_ein = part_ein;
-    ea.rec = rec;
-    ea.aux = aux;
-    HIPCHK(launch_epilogue(ea, s));
-    ForceArgs fo = force_args(m, x);
-    fo.rec4 = reinterpret_cast<const float4 *>(rec);
-    fo.aux4 = aux;
-    fo.pbc_flag = flag;
-    fo.part = part_f;
-    HIPCHK(launch_force(fo, m->npblk, false, s));
+    // the launches of isspa_model_force with the buffers above
+    if (isspa_is_small(m)) {
+        WindowArgs wa = window_args(m, x, step, step_d);
+        wa.pts = pts;
+        wa.part = part_f;
+        HIPCHK(launch_window(wa, m->max_win_atoms, m->max_group_pts, s));
+    } else {
+        HIPCHK(launch_mc_points(m->wins, m->atom_win, x, m->itype, m->rmax, m->rmax2, m->d.n_atoms,
+                                m->d.n_mc, m->d.seed, step, step_d, pts, s, m->lay.W, m->rmax_all,
+                                flag));
+        FieldArgs fa = field_args(m, x);
+        fa.pts = pts;
+        fa.pbc_flag = flag;
+        fa.part_g = part_g;
+        fa.part_cnt = part_cnt;
+        fa.part_s0 = part_s0;
+        fa.part_ein = part_ein;
+        HIPCHK(launch_field(fa, m->ngblk, s));
+        EpilogueArgs ea = epilogue_args(m, false);
+        ea.pts = pts;
+        ea.part_g = part_g;
+        ea.part_cnt = part_cnt;
+        ea.part_s0 = part_s0;
+        ea.part_ein = part_ein;
+        ea.rec = rec;
+        ea.aux = aux;
+        HIPCHK(launch_epilogue(ea, s));
+        ForceArgs fo = force_args(m, x);
+        fo.rec4 = reinterpret_cast<const float4 *>(rec);
+        fo.aux4 = aux;
+        fo.pbc_flag = flag;
+        fo.part = part_f;
+        HIPCHK(launch_force(fo, m->npblk, false, s));
+    }
     ReduceArgs ra = reduce_args(m, x, reinterpret_cast<float4 *>(f4_d), nullptr, nullptr, nullptr);
     ra.part = part_f;
     HIPCHK(launch_force_reduce(ra, false, s));

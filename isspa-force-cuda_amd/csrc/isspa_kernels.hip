@@ -30,6 +30,7 @@
 #include "pbc_device.hpp"
 #include "points_device.hpp"
 #include "nonbond_device.hpp"
+#include "bonded_device.hpp"
 #include "reduce_device.hpp"
 
 namespace isspa {
@@ -55,19 +56,20 @@ __host__ __device__ inline int diff_tab_floats(const TableView &t)
 // copy n floats into LDS with the whole block (n is block-uniform); eight
 // loads per thread are issued before their stores, so a small system's
 // kernel waits for the table once rather than once per 256 floats
+template <int NT = kBlock>
 __device__ __forceinline__ void stage_lds(float *dst, const float *__restrict__ src, int n)
 {
     constexpr int kU = 8;
-    for (int t0 = threadIdx.x; t0 < n; t0 += kU * kBlock) {
+    for (int t0 = threadIdx.x; t0 < n; t0 += kU * NT) {
         float v[kU];
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            const int t = t0 + u * kBlock;
+            const int t = t0 + u * NT;
             v[u] = t < n ? src[t] : 0.0f;
         }
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            const int t = t0 + u * kBlock;
+            const int t = t0 + u * NT;
             if (t < n) dst[t] = v[u];
         }
     }
@@ -144,6 +146,36 @@ __device__ __forceinline__ void field_in_sphere_an(const DiffType &T, float d2, 
     st.ez = __builtin_fmaf(c, rz, st.ez);
 }
 
+// One (point, atom) pair; type: where the atom's type is read, if it is needed
+template <bool PBC, bool AN, typename TypePtr>
+__device__ __forceinline__ void field_pair(const TableView &tab, float e0, const float *Gtab,
+                                           const float *Etab, const DiffType *dtypes, float4 q,
+                                           TypePtr type, const MinImage &mi, float px, float py,
+                                           float pz, float R2, float &ax, float &ay, float &az,
+                                           FieldRare &st)
+{
+    float rx = px - q.x, ry = py - q.y, rz = pz - q.z;
+    if (PBC) {
+        rx = min_image1(rx, mi);
+        ry = min_image1(ry, mi);
+        rz = min_image1(rz, mi);
+    }
+    const float d2 = dist2_f32(rx, ry, rz);
+    const float inv = rsqrt_f32(d2);
+    const float s = q.w * (inv * inv * inv);
+    const bool in = d2 <= R2;
+    const float so = in ? 0.0f : s;
+    ax = __builtin_fmaf(so, rx, ax);
+    ay = __builtin_fmaf(so, ry, ay);
+    az = __builtin_fmaf(so, rz, az);
+    if (in) {
+        if (AN)
+            field_in_sphere_an(dtypes[*type], d2, inv, s, rx, ry, rz, e0, st);
+        else
+            field_in_sphere(tab, Gtab, Etab, *type, d2, inv, s, rx, ry, rz, e0, st);
+    }
+}
+
 template <bool PBC, bool AN>
 __device__ __forceinline__ void field_tile(const FieldArgs &a, const float *Gtab,
                                            const float *Etab, const DiffType *dtypes, int j0,
@@ -157,31 +189,9 @@ __device__ __forceinline__ void field_tile(const FieldArgs &a, const float *Gtab
     const auto *xq = read_only(reinterpret_cast<const float *>(a.xyzq + j0));
     const auto *ity = read_only(a.itype);
 #pragma unroll 2
-    for (int j = j0; j < j1; ++j, xq += 4) {
-        // wave-uniform
-        const float4 q = make_float4(xq[0], xq[1], xq[2], xq[3]);
-        float rx = px - q.x, ry = py - q.y, rz = pz - q.z;
-        if (PBC) {
-            rx = min_image1(rx, mi);
-            ry = min_image1(ry, mi);
-            rz = min_image1(rz, mi);
-        }
-        const float d2 = dist2_f32(rx, ry, rz);
-        const float inv = rsqrt_f32(d2);
-        const float s = q.w * (inv * inv * inv);
-        const bool in = d2 <= R2;
-        const float so = in ? 0.0f : s;
-        ax = __builtin_fmaf(so, rx, ax);
-        ay = __builtin_fmaf(so, ry, ay);
-        az = __builtin_fmaf(so, rz, az);
-        if (in) {
-            if (AN)
-                field_in_sphere_an(dtypes[ity[j]], d2, inv, s, rx, ry, rz, a.e0, st);
-            else
-                field_in_sphere(a.tab, Gtab, Etab, ity[j], d2, inv, s, rx, ry, rz, a.e0,
-                                st);
-        }
-    }
+    for (int j = j0; j < j1; ++j, xq += 4)  // wave-uniform
+        field_pair<PBC, AN>(a.tab, a.e0, Gtab, Etab, dtypes, make_float4(xq[0], xq[1], xq[2], xq[3]),
+                            ity + j, mi, px, py, pz, R2, ax, ay, az, st);
 }
 
 // a point's sums over atoms [j0, j1) of its split
@@ -233,10 +243,10 @@ constexpr int kFieldXchgBytes = 3 * 64 * (int)sizeof(FieldXchg);  // fg = 4: 3 s
 template <bool AN, bool NB>
 __global__ __launch_bounds__(kBlock) void k_field(FieldArgs a)
 {
-    extern __shared__ float lds_tab[];
+    extern __shared__ __align__(16) float lds_tab[];
     if (NB && (int)blockIdx.x >= a.nfield) {
         // an all-pairs block riding on this launch (its LJ table in the LDS)
-        nonbond_block<false, false>(a.nb, blockIdx.x - a.nfield, reinterpret_cast<float2 *>(lds_tab));
+        nonbond_block<false, false, false>(a.nb, blockIdx.x - a.nfield, reinterpret_cast<float2 *>(lds_tab));
         return;
     }
     const int4 bt = a.blocks[blockIdx.x];
@@ -369,8 +379,8 @@ __device__ __forceinline__ void langevin_moments(double x, double inv_x, double 
 // summed in group order (B groups' loads in flight at a time), then the FP64
 // Langevin moments, the 16-float force record {p, Ehat, V, D, A2, 3 A2, A3,
 // w} and the aux entry {cp E0, A1}.  The epilogue kernel writes them to
-// memory; the fused force kernel of small systems keeps them in LDS.  Both
-// run this same code, so the records are the same bit for bit.
+// memory; the small-window kernel keeps them in LDS.  Both run this same
+// code, so the records are the same bit for bit.
 struct PointRecord {
     float4 r[4];
     float4 aux;
@@ -378,6 +388,48 @@ struct PointRecord {
     int cnt;
     double E[3], E0[3];
 };
+
+// the record of point p from its summed field
+__device__ __forceinline__ void point_record(float fe0, float fp0, float fq0, float fo0, float4 p,
+                                             double g, int cnt, const double *s0, const double *ei,
+                                             PointRecord &out)
+{
+    double E0[3], E[3];
+    for (int c = 0; c < 3; ++c) {
+        E0[c] = -(double)fe0 * s0[c];
+        E[c] = E0[c] + ei[c];
+    }
+    const double x = sqrt(E[0] * E[0] + E[1] * E[1] + E[2] * E[2]);
+    const double inv_x = x > 0.0 ? 1.0 / x : 0.0;
+    double eh[3];
+    for (int c = 0; c < 3; ++c) eh[c] = E[c] * inv_x;
+    double m1, m2, m3;
+    langevin_moments(x, inv_x, m1, m2, m3);
+    // cnt >= 1 always: the owner atom lies inside its own sphere
+    const double inv_cnt = 1.0 / (double)(cnt > 0 ? cnt : 1);
+    const double w = g * inv_cnt;
+    const double cp = (double)fp0 * inv_cnt;
+    const double A1 = (double)fp0 * m1 * w;
+    const double A2 = (double)fq0 * m2 * w;
+    const double A3 = (double)fo0 * m3 * w;
+    double c3[3];  // cp E0 / 3
+    for (int c = 0; c < 3; ++c) c3[c] = cp * E0[c] * (1.0 / 3.0);
+    out.r[0] = make_float4(p.x, p.y, p.z, (float)eh[0]);
+    out.r[1] = make_float4((float)eh[1], (float)eh[2], (float)(A1 * eh[0] + c3[0]),
+                           (float)(A1 * eh[1] + c3[1]));
+    out.r[2] = make_float4((float)(A1 * eh[2] + c3[2]),
+                           (float)(3.0 * A1 * eh[0] + cp * E0[0]),
+                           (float)(3.0 * A1 * eh[1] + cp * E0[1]),
+                           (float)(3.0 * A1 * eh[2] + cp * E0[2]));
+    out.r[3] = make_float4((float)A2, (float)(3.0 * A2), (float)A3, (float)w);
+    out.aux = make_float4((float)(cp * E0[0]), (float)(cp * E0[1]), (float)(cp * E0[2]), (float)A1);
+    out.g = g;
+    out.cnt = cnt;
+    for (int c = 0; c < 3; ++c) {
+        out.E[c] = E[c];
+        out.E0[c] = E0[c];
+    }
+}
 
 template <int B>
 __device__ __forceinline__ void epilogue_point(const EpilogueArgs &a, const WinDesc &W,
@@ -421,41 +473,7 @@ __device__ __forceinline__ void epilogue_point(const EpilogueArgs &a, const WinD
             }
         }
     }
-    double E0[3], E[3];
-    for (int c = 0; c < 3; ++c) {
-        E0[c] = -(double)a.e0 * s0[c];
-        E[c] = E0[c] + ei[c];
-    }
-    const double x = sqrt(E[0] * E[0] + E[1] * E[1] + E[2] * E[2]);
-    const double inv_x = x > 0.0 ? 1.0 / x : 0.0;
-    double eh[3];
-    for (int c = 0; c < 3; ++c) eh[c] = E[c] * inv_x;
-    double m1, m2, m3;
-    langevin_moments(x, inv_x, m1, m2, m3);
-    // cnt >= 1 always: the owner atom lies inside its own sphere
-    const double inv_cnt = 1.0 / (double)(cnt > 0 ? cnt : 1);
-    const double w = g * inv_cnt;
-    const double cp = (double)a.p0 * inv_cnt;
-    const double A1 = (double)a.p0 * m1 * w;
-    const double A2 = (double)a.q0 * m2 * w;
-    const double A3 = (double)a.o0 * m3 * w;
-    double c3[3];  // cp E0 / 3
-    for (int c = 0; c < 3; ++c) c3[c] = cp * E0[c] * (1.0 / 3.0);
-    out.r[0] = make_float4(p.x, p.y, p.z, (float)eh[0]);
-    out.r[1] = make_float4((float)eh[1], (float)eh[2], (float)(A1 * eh[0] + c3[0]),
-                           (float)(A1 * eh[1] + c3[1]));
-    out.r[2] = make_float4((float)(A1 * eh[2] + c3[2]),
-                           (float)(3.0 * A1 * eh[0] + cp * E0[0]),
-                           (float)(3.0 * A1 * eh[1] + cp * E0[1]),
-                           (float)(3.0 * A1 * eh[2] + cp * E0[2]));
-    out.r[3] = make_float4((float)A2, (float)(3.0 * A2), (float)A3, (float)w);
-    out.aux = make_float4((float)(cp * E0[0]), (float)(cp * E0[1]), (float)(cp * E0[2]), (float)A1);
-    out.g = g;
-    out.cnt = cnt;
-    for (int c = 0; c < 3; ++c) {
-        out.E[c] = E[c];
-        out.E0[c] = E0[c];
-    }
+    point_record(a.e0, a.p0, a.q0, a.o0, p, g, cnt, s0, ei, out);
 }
 
 // B groups' loads in flight at a time: 8 for launches with fewer blocks than
@@ -760,7 +778,7 @@ __global__ __launch_bounds__(kBlock) void k_force(ForceArgs a)
     }
     // the receiver type's F table for the in-sphere branch: LDS when it fits;
     // the analytic model keeps its four F constants in registers
-    extern __shared__ float lds_tab[];
+    extern __shared__ __align__(16) float lds_tab[];
     DiffFParams fp{0.0f, 0.0f, 0.0f, 0.0f};
     if (AN) fp = diff_f_params(a.dtypes[ti]);
     const bool pbc = a.pbc_flag[bt.x] != 0;
@@ -781,63 +799,228 @@ __global__ __launch_bounds__(kBlock) void k_force(ForceArgs a)
     if (valid) write_force_entry<SPLIT>(a, W, bt.z, il, acc);
 }
 
-// Small systems (windows of at most kBlock atoms, at most kFuseMaxPts points a
-// chunk group, at most kFuseMaxBlocks blocks): the epilogue and the force pass
-// in one launch.  The block runs the epilogue of its group's points (windows
-// above 64 atoms repeat it in each of their two to four receiver blocks) into
-// LDS, then the force loop reads the records from there.
-// Records and force sums are those of the two launches bit for bit; the
-// records are not written to memory.  The epilogue keeps all (up to eight)
-// split groups' partial loads in flight, and its FP64 registers then allow one
-// block per CU, so the launch is fused only when its blocks fit one round of
-// them: beyond that the separate launches are faster.
-constexpr int kFuseMaxPts = 256;
-constexpr int kFuseMaxBlocks = 256;
+// ---------------------------------------------------------------------------
+// Models of small windows (at most kWinMaxAtoms atoms each): the whole IS-SPA
+// pass of a chunk group -- its points, their field over all atoms, the
+// epilogue and the force on every receiver -- in one block, with everything
+// in LDS: no other block needs a group's points or fields.  Bounded by
+// latency: each phase is one short chain per wave, so a block has eight waves
+// (one wave alone issues a VALU operation every 8 cycles, two on a SIMD one
+// every 2.7), the draws of a point's rejection loop are tried by several
+// lanes at once, and all field splits of 64 points run side by side.
+// Splits, FP32 tiles, shares and the order of every sum are those of the
+// separate launches, so the forces are the same bit for bit.
+// Whole step of 44 atoms, nMC = 100: 38.7 -> 31.1 us (prologue 6.1, field 6.5
+// and epilogue + force 10.0 us before, 17.5 us now); 22 atoms 36.1 -> 28.7 us.
+// The step's all-pairs, bonded and restraint blocks, which depend on the
+// coordinates alone, ride on the launch (work-items from 256 up leave).
+// ---------------------------------------------------------------------------
+constexpr int kWinThreads = 512;
+constexpr int kWinWaves = kWinThreads / kWave;
+constexpr int kWinMaxAtoms = 256;
+constexpr int kWinMaxPts = 256;
+// More blocks than this are throughput, not latency, and the separate
+// launches do that better: 339 blocks (22 atoms, nMC = 1,000) take 28.3
+// against 34.5 us, 303 (242 atoms, nMC = 100) 49.7 against 71.6 us, but 677
+// (44 atoms, nMC = 1,000) 50.5 against 47.5 us.
+constexpr int kWinMaxBlocks = 512;
 
-__host__ __device__ inline int fused_lds_floats(const TableView &t)
+struct WindowLds {
+    const float4 *atoms;
+    const int *types;
+    const float *G, *E;
+};
+
+template <bool PBC>
+__device__ __forceinline__ void window_field_span(const WindowArgs &a, const WindowLds &l, int j0,
+                                                  int j1, const MinImage &mi, float4 p,
+                                                  FieldSums &fs)
 {
-    return ((force_tab_floats(t) + 3) & ~3) + kFuseMaxPts * (kRecFloats + 4);
+    FieldRare &st = fs.st;
+    for (int jt = j0; jt < j1; jt += kFieldTile) {
+        const int je = min(j1, jt + kFieldTile);
+        float ax = 0.0f, ay = 0.0f, az = 0.0f;
+        st.ex = st.ey = st.ez = 0.0f;
+#pragma unroll 2
+        for (int j = jt; j < je; ++j)
+            field_pair<PBC, false>(a.tab, a.e0, l.G, l.E, nullptr, l.atoms[j], l.types + j, mi, p.x,
+                                   p.y, p.z, p.w, ax, ay, az, st);
+        fs.sx += (double)ax;
+        fs.sy += (double)ay;
+        fs.sz += (double)az;
+        fs.ex += (double)st.ex;
+        fs.ey += (double)st.ey;
+        fs.ez += (double)st.ez;
+    }
 }
 
-__global__ __launch_bounds__(kBlock) void k_force_epi(ForceArgs a, EpilogueArgs ea)
+// the points [m0, m0 + np) of window W into LDS and memory; D lanes a point
+// try D consecutive draws at a time, the first accepted one counts
+__device__ __forceinline__ void window_points(const WindowArgs &a, const WinDesc &W, int m0, int np,
+                                              int lt, int sub, int D, const float4 *atoms,
+                                              const int *types, float4 *lrec, int *best)
 {
-    const int4 bt = a.blocks[a.xcd_runs ? xcd_run_entry(blockIdx.x, gridDim.x) : blockIdx.x];
-    const WinDesc W = a.wins[bt.x];
-    const int lane = (int)threadIdx.x % kWave;
-    // the wave index read from the first lane, so the compiler knows it is
-    // wave-uniform and the share's point range stays on scalar loads
-    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
-    const int il = bt.y * kWave + lane;
-    const int P = W.n * a.nmc;
-    const long long pbase = (long long)W.a0 * a.nmc;
-    const int span = force_group(W.n) * W.ppc;
-    const int m0 = min(P, bt.z * span), np = min(P, m0 + span) - m0;
-    int ms, me;
-    share_range(W, P, bt.z, wv, ms, me);
-    const bool valid = il < W.n;
-    const int i = W.a0 + (valid ? il : 0);
-    const float4 xi = a.xyzq[i];
-    const int ti = a.itype[i];
-    const float R2 = valid ? a.rmax2[ti] : -1.0f;
-    extern __shared__ float lds_tab[];
-    const int nt = force_tab_floats(a.tab);
-    float4 *lrec = reinterpret_cast<float4 *>(lds_tab + ((nt + 3) & ~3));
-    float4 *laux = lrec + 4 * kFuseMaxPts;
-    for (int t = threadIdx.x; t < np; t += kBlock) {
-        PointRecord pr;
-        epilogue_point<8>(ea, W, pbase + m0 + t, pr);
-        for (int k = 0; k < 4; ++k) lrec[4 * t + k] = pr.r[k];
-        laux[t] = pr.aux;
-    }
-    stage_lds(lds_tab, a.tab.f, nt);
+    const uint32_t step = a.step_d ? *a.step_d : a.step;
+    const bool mine = lt < np && sub < D;
+    const int il = mine ? (m0 + lt) / a.nmc : 0;
+    if (mine && sub == 0) best[lt] = kMcMaxAttempts;
     __syncthreads();
-    const bool pbc = a.pbc_flag[bt.x] != 0;
+    for (int base = 0;; base += D) {
+        int c0 = 0, c1 = 0, c2 = 0;
+        const int d = base + sub;
+        const bool open = mine && d < kMcMaxAttempts && best[lt] > d;
+        const bool ok = open && mc_draw(a.seed, (uint32_t)(m0 + lt), (uint32_t)d, step, W.sys, c0, c1, c2);
+        if (ok) atomicMin(best + lt, d);
+        __syncthreads();
+        const int b = mine ? best[lt] : 0;
+        const bool last = base + D >= kMcMaxAttempts;
+        // the winner, or, after the last draw, the point at its atom
+        const bool none = mine && last && sub == 0 && b == kMcMaxAttempts;
+        if ((ok && b == d) || none) {
+            const int t = types[il];
+            const float4 p = none ? mc_place(atoms[il], a.rmax[t], a.rmax2[t], 0, 0, 0)
+                                  : mc_place(atoms[il], a.rmax[t], a.rmax2[t], c0, c1, c2);
+            lrec[4 * lt] = p;
+            a.pts[(long long)W.a0 * a.nmc + m0 + lt] = p;
+        }
+        // every work-item of the block sees the same answer
+        if (!__syncthreads_or(mine && b == kMcMaxAttempts) || last) break;
+    }
+}
+
+__global__ __launch_bounds__(kWinThreads, 4) void k_window(WindowArgs a)
+{
+    extern __shared__ __align__(16) float lds_tab[];
+    int b = blockIdx.x;
+    if (b >= a.nblocks) {
+        // a riding block
+        b -= a.nblocks;
+        if (threadIdx.x >= (unsigned)kBlock) return;
+        if (b < a.nb_blocks) {
+            nonbond_block<false, false, true>(a.nb, b, reinterpret_cast<float2 *>(lds_tab));
+            return;
+        }
+        b -= a.nb_blocks;
+        if (b < a.bonded_blocks) {
+            bonded_one(a.bonded, b * kBlock + (int)threadIdx.x);
+            return;
+        }
+        b -= a.bonded_blocks;
+        us_block(b, a.us.boff, a.us.us_atoms, a.us.us_mass, a.us.kx, a.us.Ls, a.xyzq, a.us.fus,
+                 a.us.com, true, reinterpret_cast<double (*)[kTermBlock]>(lds_tab));
+        return;
+    }
+    const int4 bt = a.blocks[b];
+    const WinDesc W = a.wins[bt.x];
+    const int tid = threadIdx.x, lane = tid % kWave;
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int n = W.n, P = n * a.nmc;
+    const int span = force_group(n) * W.ppc;
+    const int m0 = min(P, bt.z * span), np = min(P, m0 + span) - m0;
+    // LDS: F table, atoms and types, point records (until they are written the
+    // points, in each record's first entry, and the draws' counters), then an
+    // area that holds the g and E tables and the splits' field sums, later the
+    // shares' force sums
+    const int nf = force_tab_floats(a.tab), ng = a.tab.ntypes * a.tab.ld_g;
+    const int ne = a.tab.ntypes * a.tab.ld_e;
+    float4 *atoms = reinterpret_cast<float4 *>(lds_tab + a.off_atoms);
+    int *types = reinterpret_cast<int *>(atoms + kWinMaxAtoms);
+    float4 *lrec = reinterpret_cast<float4 *>(lds_tab + a.off_pts);
+    float4 *laux = lrec + 4 * a.cap_pts;
+    int *best = reinterpret_cast<int *>(laux);
+    float *area = lds_tab + a.off_x;
+    FieldXchg *xc = reinterpret_cast<FieldXchg *>(area + ((ng + ne + 3) & ~3));
+    for (int i = tid; i < n; i += kWinThreads) {
+        atoms[i] = a.xyzq[W.a0 + i];
+        types[i] = a.itype[W.a0 + i];
+    }
+    stage_lds<kWinThreads>(lds_tab, a.tab.f, nf);
+    stage_lds<kWinThreads>(area, a.tab.g, ng);
+    stage_lds<kWinThreads>(area + ng, a.tab.e, ne);
+    // (its barrier also publishes the staged data)
+    const bool pbc = needs_image<kWinThreads>(W, a.xyzq, a.rmax_all);
+    const MinImage mi = min_image_of(W.L, W.h);
+    // lt: the work-item's point, sub: its draw or field split, wave-uniform
+    const int npr = (np + kWave - 1) & ~(kWave - 1);
+    const int D = kWinThreads / npr;
+    const int sub = __builtin_amdgcn_readfirstlane(tid / npr);
+    const int lt = tid - sub * npr;
+    window_points(a, W, m0, np, lt, sub, D, atoms, types, lrec, best);
+    // field: D splits side by side, added in order, groups of W.fg at a time
+    const WindowLds l{atoms, types, area, area + ng};
+    const float4 p = lt < np ? lrec[4 * lt] : make_float4(0.0f, 0.0f, 0.0f, -1.0f);
+    double g = 1.0, s0[3] = {0, 0, 0}, ei[3] = {0, 0, 0};
+    double gg = 1.0, gs[3] = {0, 0, 0}, ge[3] = {0, 0, 0};
+    int cnt = 0;
+    for (int sp = 0; sp < W.splits; sp += D) {
+        const int split = sp + sub;
+        if (sub < D && split < W.splits) {
+            const int j0 = split * W.aps, j1 = min(n, j0 + W.aps);
+            FieldSums fs;
+            if (pbc)
+                window_field_span<true>(a, l, j0, j1, mi, p, fs);
+            else
+                window_field_span<false>(a, l, j0, j1, mi, p, fs);
+            FieldXchg &e = xc[tid];
+            e.s[0] = fs.sx; e.s[1] = fs.sy; e.s[2] = fs.sz;
+            e.s[3] = fs.ex; e.s[4] = fs.ey; e.s[5] = fs.ez;
+            e.g = fs.st.g;
+            e.cnt = fs.st.cnt;
+        }
+        __syncthreads();
+        if (tid < np)
+            for (int k = 0; k < D && sp + k < W.splits; ++k) {
+                const FieldXchg &e = xc[k * npr + tid];
+                cnt += e.cnt;
+                if ((sp + k) % W.fg == 0) {
+                    gg = (double)e.g;
+                    for (int c = 0; c < 3; ++c) { gs[c] = e.s[c]; ge[c] = e.s[3 + c]; }
+                } else {
+                    gg *= (double)e.g;
+                    for (int c = 0; c < 3; ++c) { gs[c] += e.s[c]; ge[c] += e.s[3 + c]; }
+                }
+                if ((sp + k) % W.fg == W.fg - 1) {
+                    g *= gg;
+                    for (int c = 0; c < 3; ++c) { s0[c] += gs[c]; ei[c] += ge[c]; }
+                }
+            }
+        __syncthreads();
+    }
+    if (tid < np) {
+        PointRecord pr;
+        point_record(a.e0, a.p0, a.q0, a.o0, lrec[4 * tid], g, cnt, s0, ei, pr);
+        for (int k = 0; k < 4; ++k) lrec[4 * tid + k] = pr.r[k];
+        laux[tid] = pr.aux;
+    }
+    __syncthreads();
+    // force: units of 64 receivers and one share, over the eight waves
+    ForceArgs fa{};
+    fa.tab = a.tab;
+    fa.part = a.part;
+    const int nrw = (n + kWave - 1) / kWave;
+    double *sh = reinterpret_cast<double *>(area);  // [share][receiver][6]
     const DiffFParams fp{0.0f, 0.0f, 0.0f, 0.0f};
-    ForceAcc acc{0, 0, 0, 0, 0, 0, 0, 0, 0};
-    force_chunk<false, false>(a, lrec, laux, ms - m0, me - m0, W, pbc, xi, R2,
-                              lds_tab + ti * a.tab.ld_f, fp, acc);
-    if (!share_sum<false>(reinterpret_cast<double *>(lds_tab + a.red_off), wv, lane, acc)) return;
-    if (valid) write_force_entry<false>(a, W, bt.z, il, acc);
+    for (int u = wv; u < 4 * nrw; u += kWinWaves) {
+        const int share = u & 3, il = (u >> 2) * kWave + lane;
+        int ms, me;
+        share_range(W, P, bt.z, share, ms, me);
+        const float4 xi = atoms[min(il, n - 1)];
+        const int ti = types[min(il, n - 1)];
+        const float R2 = il < n ? a.rmax2[ti] : -1.0f;
+        ForceAcc acc{0, 0, 0, 0, 0, 0, 0, 0, 0};
+        force_chunk<false, false>(fa, lrec, laux, ms - m0, me - m0, W, pbc, xi, R2,
+                                  lds_tab + ti * a.tab.ld_f, fp, acc);
+        double *d = sh + 6 * ((size_t)share * nrw * kWave + il);
+        d[0] = acc.ex; d[1] = acc.ey; d[2] = acc.ez;
+        d[3] = acc.lx; d[4] = acc.ly; d[5] = acc.lz;
+    }
+    __syncthreads();
+    if (tid >= n) return;
+    double f[6];
+    for (int k = 0; k < 6; ++k) f[k] = sh[6 * tid + k];
+    for (int q = 1; q < 4; ++q)
+        for (int k = 0; k < 6; ++k) f[k] += sh[6 * ((size_t)q * nrw * kWave + tid) + k];
+    write_force_entry<false>(fa, W, bt.z, tid, ForceAcc{f[0], f[1], f[2], f[3], f[4], f[5], 0, 0, 0});
 }
 
 // F_i = -q_i vtot_i S_e - vtot_i S_lj over the chunk partials, summed in the
@@ -932,19 +1115,40 @@ hipError_t launch_epilogue(const EpilogueArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
-bool force_epi_fits(const TableView &t, int max_window_atoms, int max_group_points, int nblocks)
+// LDS of k_window in floats: F table, atoms, points; then the shared area
+static int window_lds(const TableView &t, int max_atoms, int max_points, WindowArgs *a)
 {
-    return max_window_atoms <= kBlock && max_group_points <= kFuseMaxPts &&
-           nblocks <= kFuseMaxBlocks && force_tab_floats(t) <= kTabLdsFloats;
+    const int off_atoms = (force_tab_floats(t) + 3) & ~3;
+    const int off_pts = off_atoms + 5 * kWinMaxAtoms;
+    const int cap_pts = (max_points + kWave - 1) / kWave * kWave;
+    const int off_x = off_pts + (kRecFloats + kAuxFloats) * cap_pts;
+    const int nxc = ((field_tab_floats(t) + 3) & ~3) + kWinThreads * (int)(sizeof(FieldXchg) / 4);
+    const int nsh = 4 * 6 * 2 * ((max_atoms + kWave - 1) / kWave) * kWave;
+    if (a) {
+        a->off_atoms = off_atoms;
+        a->off_pts = off_pts;
+        a->off_x = off_x;
+        a->cap_pts = cap_pts;
+    }
+    return off_x + std::max(nxc, nsh);
 }
 
-hipError_t launch_force_epi(const ForceArgs &a, const EpilogueArgs &ea, int nblocks, hipStream_t s)
+bool window_fits(const TableView &t, int max_atoms, int max_points, int nblocks)
 {
-    if (nblocks == 0) return hipSuccess;
-    ForceArgs b = a;
-    b.red_off = fused_lds_floats(a.tab);  // a multiple of 4 floats
-    const size_t lds = (size_t)(b.red_off + 2 * force_share_doubles(false)) * sizeof(float);
-    hipLaunchKernelGGL(k_force_epi, dim3(nblocks), dim3(kBlock), lds, s, b, ea);
+    return max_atoms <= kWinMaxAtoms && max_points <= kWinMaxPts && nblocks <= kWinMaxBlocks &&
+           field_tab_floats(t) <= kTabLdsFloats && force_tab_floats(t) <= kTabLdsFloats;
+}
+
+hipError_t launch_window(const WindowArgs &a0, int max_atoms, int max_points, hipStream_t s)
+{
+    WindowArgs a = a0;
+    size_t lds = sizeof(float) * window_lds(a.tab, max_atoms, max_points, &a);
+    if (a.nb_blocks) lds = std::max(lds, nonbond_lds_bytes(a.nb.T, false));
+    const long terms = (long)a.bonded.nb + a.bonded.na + a.bonded.nd;
+    a.bonded_blocks = a.bonded.contrib ? blocks_for(terms) : 0;
+    const int grid = a.nblocks + a.nb_blocks + a.bonded_blocks + a.us.nres;
+    if (grid == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_window, dim3(grid), dim3(kWinThreads), lds, s, a);
     return hipGetLastError();
 }
 

@@ -223,6 +223,65 @@ struct PointsArgs {
     float4 *pts;
 };
 
+// bonded terms (window-agnostic: they carry global atom indices)
+struct BondedArgs {
+    const float4 *xyzq;
+    float L, h;
+    int nb, na, nd;
+    const int4 *bond_atoms;
+    const float2 *bond_params;
+    const int4 *angle_atoms;
+    const float2 *angle_params;
+    const int4 *dih_atoms;
+    const int *dih_types;
+    const float4 *dih_params;
+    const float2 *sc14;
+    const int *ityp;
+    const float2 *lj;      // [T*T] {A, B}
+    int T;
+    float4 *contrib;       // [2 nb + 3 na + 6 nd]
+    double *energy;        // per-term energies (3 per dihedral: torsion, 1-4 Coulomb, 1-4 LJ)
+    int terms;
+};
+// umbrella restraints: nres blocks, bias entries [boff[r], boff[r+1])
+struct RestraintArgs {
+    int nres;
+    const int *boff;
+    const int2 *us_atoms;
+    const float *us_mass;
+    const float2 *kx;
+    const float *Ls;
+    float4 *fus;  // bias forces stored (w = 1)
+    double *com;
+};
+
+// The IS-SPA pass of a model of small windows in one launch (k_window), with
+// the all-pairs, bonded and restraint blocks of an engine step riding on it
+// (each part skipped when empty).
+struct WindowArgs {
+    const WinDesc *wins;
+    const int4 *blocks;   // {w, -, chunk group, -}
+    int nblocks;
+    const float4 *xyzq;
+    const int *itype;
+    const float *rmax, *rmax2;
+    float rmax_all;
+    TableView tab;
+    int nmc;
+    float e0, p0, q0, o0;
+    uint64_t seed;
+    uint32_t step;
+    const uint32_t *step_d;
+    float4 *pts;
+    double *part;         // force partials, as k_force leaves them
+    NonbondArgs nb;
+    int nb_blocks;
+    BondedArgs bonded;
+    int bonded_blocks;    // set by the launcher
+    RestraintArgs us;
+    int off_atoms, off_pts, off_x, cap_pts;  // LDS layout in floats (set by the launcher)
+};
+
 hipError_t launch_mc_points(const WinDesc *wins, const int *atom_win, const float4 *xyzq,
                             const int *itype, const float *rmax, const float *rmax2, int ntot,
                             int nmc, uint64_t seed, uint32_t step, const uint32_t *step_d,
@@ -230,11 +289,10 @@ hipError_t launch_mc_points(const WinDesc *wins, const int *atom_win, const floa
                             int *flag = nullptr);
 hipError_t launch_field(const FieldArgs &a, int nblocks, hipStream_t s);
 hipError_t launch_epilogue(const EpilogueArgs &a, hipStream_t s);
-// the epilogue and the force pass in one launch, for models whose windows all
-// have at most 256 atoms, whose chunk groups hold at most 256 points and whose
-// force grid has at most 256 blocks (table model, total force only)
-bool force_epi_fits(const TableView &t, int max_window_atoms, int max_group_points, int nblocks);
-hipError_t launch_force_epi(const ForceArgs &a, const EpilogueArgs &ea, int nblocks, hipStream_t s);
+// k_window: whether a model's windows, chunk groups and tables fit it, and the
+// launch (max_atoms, max_points: of the largest window and chunk group)
+bool window_fits(const TableView &t, int max_atoms, int max_points, int nblocks);
+hipError_t launch_window(const WindowArgs &a, int max_atoms, int max_points, hipStream_t s);
 hipError_t launch_force(const ForceArgs &a, int nblocks, bool split, hipStream_t s);
 hipError_t launch_force_reduce(const ReduceArgs &a, bool split, hipStream_t s);
 
@@ -271,46 +329,20 @@ hipError_t launch_chunk_reduce3(const WinDesc *wins, const int *atom_win, const 
                                 long long B, int ntot, int comps, float4 *f, double *o0,
                                 double *o1, double *o2, hipStream_t s);
 
-// ---- bonded (window-agnostic: terms carry global atom indices) ----
-struct BondedArgs {
-    const float4 *xyzq;
-    float L, h;
-    int nb, na, nd;
-    const int4 *bond_atoms;
-    const float2 *bond_params;
-    const int4 *angle_atoms;
-    const float2 *angle_params;
-    const int4 *dih_atoms;
-    const int *dih_types;
-    const float4 *dih_params;
-    const float2 *sc14;
-    const int *ityp;
-    const float2 *lj;      // [T*T] {A, B}
-    int T;
-    float4 *contrib;       // [2 nb + 3 na + 6 nd]
-    double *energy;        // per-term energies (3 per dihedral: torsion, 1-4 Coulomb, 1-4 LJ)
-    int terms;
-};
+// ---- bonded ----
 hipError_t launch_bonded_terms(const BondedArgs &a, hipStream_t s);
 hipError_t launch_bonded_gather(const float4 *contrib, const int *ptr, const int *idx, int n,
                                 float4 *f, hipStream_t s);
 // The MD engine's step prologue: every launch of a step that depends only on
 // the coordinates, in one grid.  Each part is skipped when empty (nflag 0,
-// bonded.contrib null, nres 0, pts.ntot 0).
+// bonded.contrib null, us.nres 0, pts.ntot 0).
 struct PrologueArgs {
     int nflag;              // minimum-image flags of the IS-SPA windows
     float rmax_all;
     int *flag;
     BondedArgs bonded;      // bonded terms into their contribution slots
     int bonded_blocks;      // set by the launcher
-    int nres;               // restraints: bias forces stored into fus (w = 1)
-    const int *boff;
-    const int2 *us_atoms;
-    const float *us_mass;
-    const float2 *kx;
-    const float *Ls;
-    float4 *fus;
-    double *com;
+    RestraintArgs us;       // bias forces stored into fus
     PointsArgs pts;         // MC points (pts.wins also serves the flags)
 };
 hipError_t launch_step_prologue(PrologueArgs a, hipStream_t s);

@@ -55,6 +55,8 @@ struct isspa_model {
     int nfblk = 0, npblk = 0, ngblk = 0;
     int4 *vblk = nullptr;  // the adjoint's atom pass: {w, 64 atoms, four chunks, -}
     int nvblk = 0;
+    int4 *wblk = nullptr;  // k_window: {w, -, chunk group, -}
+    int nwblk = 0;
     int max_fg = 1;  // the largest splits-per-field-block of the windows
     int max_win_atoms = 0, max_group_pts = 0;  // over the windows, for the fused force launch
     double *part_g = nullptr;
@@ -102,6 +104,8 @@ inline float4 *rec_aux(isspa_model *m)
 FieldArgs field_args(isspa_model *m, const float4 *x);
 EpilogueArgs epilogue_args(isspa_model *m, bool inspect);
 ForceArgs force_args(isspa_model *m, const float4 *x);
+bool isspa_is_small(const isspa_model *m);
+WindowArgs window_args(isspa_model *m, const float4 *x, uint32_t step, const uint32_t *step_d);
 ReduceArgs reduce_args(isspa_model *m, const float4 *x, float4 *f, double *flj, double *fpol,
                        double *fcdd);
 // the all-pairs term for positions x: split -> three FP64 component outputs;

@@ -5,6 +5,7 @@
 
 #include "device_common.hpp"
 #include "kernels.hpp"
+#include "pbc_device.hpp"
 
 namespace isspa {
 
@@ -325,7 +326,10 @@ __device__ __forceinline__ void nonbond_supertile(const NonbondArgs &a, const Wi
 // force writes the total-mode layout (spo, nte entries per atom).  SYM
 // compiles the super-tile kinds in (the field launch that carries the
 // all-pairs blocks of small systems has none).
-template <bool SPLIT, bool SYM>
+//
+// OWN: no minimum-image flags are there yet (the small-window launch, whose
+// windows the block reads in one pass): the block decides for itself.
+template <bool SPLIT, bool SYM, bool OWN>
 __device__ __forceinline__ void nonbond_block(const NonbondArgs &a, int blk, float2 *lds_lj)
 {
     static_assert(!(SPLIT && SYM), "the split components take every pair in both orders");
@@ -342,7 +346,13 @@ __device__ __forceinline__ void nonbond_block(const NonbondArgs &a, int blk, flo
             nonbond_supertile<false>(a, W, bt.y, bt.z, lds_lj, jl);
         return;
     }
-    __syncthreads();
+    bool pbc;
+    if (OWN) {
+        pbc = needs_image<kNbBlock>(W, a.xyzq, 0.0f);  // and the barrier for the table
+    } else {
+        __syncthreads();
+        pbc = a.pbc_flag[bt.x] != 0;
+    }
     const bool near_kind = SYM && bt.w == kNbKindNear;
     // partners: a chunk, or (near kind) 256-atom block bt.z, the receivers'
     // own block or a neighbour; both write entry bt.z
@@ -356,7 +366,6 @@ __device__ __forceinline__ void nonbond_block(const NonbondArgs &a, int blk, flo
     const int ti = __float_as_int(a.aux[i].w);
     uint32_t ex[4];
     for (int k = 0; k < 4; ++k) ex[k] = a.excl[4 * i + k];
-    const bool pbc = a.pbc_flag[bt.x] != 0;
     const MinImage mi = min_image_of(W.L, W.h);
     // first receiver of this wave, for the near-diagonal test
     const int wave_lo = W.a0 + bt.y * kNbBlock + (threadIdx.x & ~(kWave - 1));

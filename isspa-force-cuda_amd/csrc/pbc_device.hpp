@@ -44,4 +44,28 @@ __device__ inline void pbc_flag_block(const WinDesc &W, const float4 *__restrict
     }
 }
 
+// The same decision taken by a block's first NT work-items for its own use,
+// with two barriers and no memory: false only if every atom lies within
+// (L/2 - rmax - margin) / 2 of the first one on every axis.  It may say true
+// where the flag says 0; the image loop then shifts nothing.
+template <int NT>
+__device__ __forceinline__ bool needs_image(const WinDesc &W, const float4 *__restrict__ xyzq,
+                                            float rmax_all)
+{
+    const float lim = 0.5f * (W.h - rmax_all - 1.0e-2f);
+    const float4 o = xyzq[W.a0];
+    int far = 0;
+    for (int i = threadIdx.x; i < W.n; i += NT) {
+        const float4 x = xyzq[W.a0 + i];
+        // NaN -> far
+        far |= !(fabsf(x.x - o.x) < lim && fabsf(x.y - o.y) < lim && fabsf(x.z - o.z) < lim);
+    }
+    __shared__ int need;
+    if (threadIdx.x == 0) need = 0;
+    __syncthreads();
+    if (far) need = 1;
+    __syncthreads();
+    return need != 0;
+}
+
 }  // namespace isspa

@@ -19,6 +19,26 @@ __device__ __forceinline__ float point_coord(float x, float R, int v)
     return x + du;
 }
 
+// Draw d of point m (window-local index): true if its 24-bit signed lattice
+// vector lies in the unit ball.
+__device__ __forceinline__ bool mc_draw(uint64_t seed, uint32_t m, uint32_t d, uint32_t step,
+                                        uint32_t sys, int &c0, int &c1, int &c2)
+{
+    const uint4 o = philox_draw(seed, m, kStreamPoints, d, step, sys);
+    c0 = 2 * (int)(o.x >> 8) - (1 << 24);
+    c1 = 2 * (int)(o.y >> 8) - (1 << 24);
+    c2 = 2 * (int)(o.z >> 8) - (1 << 24);
+    const uint64_t r2 = (uint64_t)((int64_t)c0 * c0 + (int64_t)c1 * c1 + (int64_t)c2 * c2);
+    return r2 <= kMcAcceptMax;
+}
+
+// the point of owner x at lattice vector (v0, v1, v2); .w is the owner's rmax^2
+__device__ __forceinline__ float4 mc_place(float4 x, float R, float R2, int v0, int v1, int v2)
+{
+    return make_float4(point_coord(x.x, R, v0), point_coord(x.y, R, v1), point_coord(x.z, R, v2),
+                       R2);
+}
+
 // Point gp (global index; window w owns points [a0_w nMC, (a0_w + n_w) nMC),
 // point m of the window belongs to atom m / nMC) is drawn with counter
 // {m, draw, step, sys_w}: the first draw whose 24-bit signed lattice vector
@@ -32,24 +52,13 @@ __device__ __forceinline__ void mc_point(const PointsArgs &a, long long gp)
     const int t = a.itype[k];
     int v0 = 0, v1 = 0, v2 = 0;
     for (int d = 0; d < kMcMaxAttempts; ++d) {
-        const uint4 o = philox_draw(a.seed, m, kStreamPoints, (uint32_t)d, step, W.sys);
-        const int c0 = 2 * (int)(o.x >> 8) - (1 << 24);
-        const int c1 = 2 * (int)(o.y >> 8) - (1 << 24);
-        const int c2 = 2 * (int)(o.z >> 8) - (1 << 24);
-        const uint64_t r2 = (uint64_t)((int64_t)c0 * c0 + (int64_t)c1 * c1 + (int64_t)c2 * c2);
-        if (r2 <= kMcAcceptMax) {
+        int c0, c1, c2;
+        if (mc_draw(a.seed, m, (uint32_t)d, step, W.sys, c0, c1, c2)) {
             v0 = c0; v1 = c1; v2 = c2;
             break;
         }
     }
-    const float R = a.rmax[t];
-    const float4 x = a.xyzq[k];
-    float4 p;
-    p.x = point_coord(x.x, R, v0);
-    p.y = point_coord(x.y, R, v1);
-    p.z = point_coord(x.z, R, v2);
-    p.w = a.rmax2[t];
-    a.pts[gp] = p;
+    a.pts[gp] = mc_place(a.xyzq[k], a.rmax[t], a.rmax2[t], v0, v1, v2);
 }
 
 }  // namespace isspa
