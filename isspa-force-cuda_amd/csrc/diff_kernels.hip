@@ -248,28 +248,27 @@ __global__ __launch_bounds__(kB) void k_vjp_points(VjpArgs a)
     for (int k = 0; k < 10; ++k) a.ppart[k * a.F + o] = acc[k];
 }
 
-// Langevin moments and their derivatives in FP64 (series ratio below 5, coth
-// recurrence above), as the forward epilogue
-__device__ void moments_derivs(double x, double m[3], double dm[3])
+// Langevin moments and their derivatives, as the forward epilogue
+__device__ __forceinline__ void moments_derivs(double x, double m[3], double dm[3])
 {
     if (x < 5.0) {
         const double h = 0.5 * x * x;
-        double s[4], ds[4];
+        double s[4], ds[4];  // the series and their derivatives by h
+#pragma unroll
         for (int l = 0; l < 4; ++l) {
-            // terms T_0 = 1/(2l+1)!!, T_(k+1) = T_k h / ((k+1)(2l+2k+3)), so
-            // d T_(k+1) / dh = T_k / (2l+2k+3); stop once a term is below
-            // 1e-17 of the sum
-            double t = kLangevin.first[l], sum = t, dsum = 0.0;
-            for (int k = 0; k < kLgTerms && t > 1e-17 * sum; ++k) {
-                dsum += t * kLangevin.inv[l][k];
-                t *= h * kLangevin.step[l][k];
-                sum += t;
-            }
-            s[l] = sum;
-            ds[l] = dsum;
+            s[l] = kLangevin.a[l][kLgTerms - 1];
+            ds[l] = 0.0;
         }
+#pragma unroll
+        for (int k = kLgTerms - 2; k >= 0; --k)
+#pragma unroll
+            for (int l = 0; l < 4; ++l) {
+                ds[l] = __builtin_fma(ds[l], h, s[l]);
+                s[l] = __builtin_fma(s[l], h, kLangevin.a[l][k]);
+            }
         const double s0 = s[0];
         double xl = 1.0;
+#pragma unroll
         for (int l = 1; l <= 3; ++l) {
             const double xl1 = xl;  // x^(l-1)
             xl *= x;                // x^l
@@ -278,7 +277,7 @@ __device__ void moments_derivs(double x, double m[3], double dm[3])
         }
         return;
     }
-    const double coth = 1.0 / tanh(x);
+    const double coth = coth_large(x);
     const double sh = sinh(x);
     m[0] = coth - 1.0 / x;
     m[1] = 1.0 - 3.0 * m[0] / x;

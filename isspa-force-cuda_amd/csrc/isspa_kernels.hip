@@ -335,42 +335,28 @@ __global__ __launch_bounds__(kBlock) void k_field(FieldArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// per-point epilogue in FP64: Langevin moments <P1>,<P2>,<P3>
-// (= c1, 1.5 c2 - 0.5, 2.5 c3 - 1.5 c1 of src/isspa_force_cuda.cu:270-287)
+// per-point epilogue in FP64
 // ---------------------------------------------------------------------------
-// Below x = 5: <P_l> = i_l(x)/i_0(x) from the all-positive power series
-// i_l(x) = x^l sum_k (x^2/2)^k / (k! (2l+2k+1)!!), 30 terms; above 5 the
-// upward recurrence from coth, which then cancels by at most ~3x.
 __device__ __forceinline__ void langevin_moments(double x, double inv_x, double &m1, double &m2,
                                                  double &m3)
 {
     if (x < 5.0) {
-        // all 30 terms of the four series, advanced together as four
-        // independent FP64 chains with compile-time coefficients: past the
-        // first few terms they add nothing (below 1e-17 of the sum for small
-        // x), but a fixed count keeps the loop free of branches and loads
+        // the four series advance together: independent FP64 chains
         const double h = 0.5 * x * x;
-        double t[4], s[4];
+        double s[4];
 #pragma unroll
-        for (int l = 0; l < 4; ++l) {
-            t[l] = kLangevin.first[l];
-            s[l] = t[l];
-        }
+        for (int l = 0; l < 4; ++l) s[l] = kLangevin.a[l][kLgTerms - 1];
 #pragma unroll
-        for (int k = 0; k < kLgTerms; ++k)
+        for (int k = kLgTerms - 2; k >= 0; --k)
 #pragma unroll
-            for (int l = 0; l < 4; ++l) {
-                t[l] *= h * kLangevin.step[l][k];
-                s[l] += t[l];
-            }
+            for (int l = 0; l < 4; ++l) s[l] = __builtin_fma(s[l], h, kLangevin.a[l][k]);
         const double r = 1.0 / s[0];
         m1 = x * s[1] * r;
         m2 = x * x * s[2] * r;
         m3 = x * x * x * s[3] * r;
         return;
     }
-    const double coth = 1.0 / tanh(x);
-    m1 = coth - inv_x;
+    m1 = coth_large(x) - inv_x;
     m2 = 1.0 - 3.0 * m1 * inv_x;
     m3 = m1 - 5.0 * m2 * inv_x;
 }
