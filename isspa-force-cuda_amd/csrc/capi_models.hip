@@ -96,7 +96,7 @@ static int auto_pieces(long long lanes, long long work, long long min_work, doub
 static void isspa_free(isspa_model *m)
 {
     dfree(m->itype); dfree(m->atom_win); dfree(m->rmax); dfree(m->rmax2); dfree(m->vtot);
-    dfree(m->g); dfree(m->e); dfree(m->f);
+    dfree(m->ge); dfree(m->f);
     dfree(m->pts); dfree(m->rec); dfree(m->g_out); dfree(m->E_out); dfree(m->E0_out);
     dfree(m->cnt_out); dfree(m->pbc_flag); dfree(m->wins); dfree(m->fblk); dfree(m->gblk);
     dfree(m->pblk); dfree(m->vblk); dfree(m->wblk);
@@ -271,10 +271,13 @@ extern "C" int isspa_model_create_batch(const isspa_model_desc *d, const isspa_w
                         (double)(float)d->n_mc);
         m->rmax_all = std::max(m->rmax_all, rmax[t]);
     }
-    std::vector<float> gp, ep, fp;
-    pad_table(g, T, d->n_g, gp);
-    pad_table(e, T, d->n_e, ep);
+    std::vector<float> fp;
     pad_table(f, T, d->n_f, fp);
+    std::vector<float2> ge((size_t)T * (d->n_g + 1), make_float2(0.0f, 0.0f));
+    for (int t = 0; t < T; ++t)
+        for (int b = 0; b < d->n_g; ++b)
+            ge[(size_t)t * (d->n_g + 1) + b] =
+                make_float2(g[(size_t)t * d->n_g + b], e[(size_t)t * d->n_e + b]);
 #define TRY(x)                      \
     if ((rc = (x)) != ISSPA_OK) {   \
         isspa_free(m);              \
@@ -286,8 +289,7 @@ extern "C" int isspa_model_create_batch(const isspa_model_desc *d, const isspa_w
     TRY(upload(&m->rmax, rmax, T));
     TRY(upload(&m->rmax2, r2.data(), T));
     TRY(upload(&m->vtot, vt.data(), T));
-    TRY(upload(&m->g, gp.data(), gp.size()));
-    TRY(upload(&m->e, ep.data(), ep.size()));
+    TRY(upload(&m->ge, ge.data(), ge.size()));
     TRY(upload(&m->f, fp.data(), fp.size()));
     TRY(dalloc(&m->pts, m->P));
     TRY(dalloc(&m->rec, (size_t)m->P * (kRecFloats + kAuxFloats)));  // records, then aux
@@ -299,9 +301,9 @@ extern "C" int isspa_model_create_batch(const isspa_model_desc *d, const isspa_w
     TRY(isspa_tile(m));
 #undef TRY
     TableView &tv = m->tv;
-    tv.g = m->g; tv.e = m->e; tv.f = m->f;
-    tv.n_g = d->n_g; tv.n_e = d->n_e; tv.n_f = d->n_f;
-    tv.ld_g = d->n_g + 1; tv.ld_e = d->n_e + 1; tv.ld_f = d->n_f + 1;
+    tv.ge = m->ge; tv.f = m->f;
+    tv.n_g = d->n_g; tv.n_f = d->n_f;
+    tv.ld_g = d->n_g + 1; tv.ld_f = d->n_f + 1;
     tv.ntypes = d->n_types;
     tv.g_r0 = d->g_r0; tv.g_dr = d->g_dr; tv.g_inv = 1.0f / d->g_dr;
     tv.e_r0 = d->e_r0; tv.e_dr = d->e_dr; tv.e_inv = 1.0f / d->e_dr;

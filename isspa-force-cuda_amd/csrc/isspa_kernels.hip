@@ -44,7 +44,7 @@ constexpr int kTabLdsFloats = 4096;
 
 __host__ __device__ inline int field_tab_floats(const TableView &t)
 {
-    return t.ntypes * (t.ld_g + t.ld_e);
+    return 2 * t.ntypes * t.ld_g;
 }
 __host__ __device__ inline int force_tab_floats(const TableView &t) { return t.ntypes * t.ld_f; }
 // per-type records of the analytic model (one DiffType per type)
@@ -105,25 +105,28 @@ struct FieldRare {
     float ex, ey, ez;
 };
 
-__device__ __forceinline__ void field_in_sphere(const TableView &tb, const float *Gtab,
-                                                const float *Etab, int tj, float d2, float inv,
-                                                float s, float rx, float ry, float rz, float e0,
-                                                FieldRare &st)
+// GE: {g, E} rows, [type][ld_g].  No branch (each costs a lone wave some 30
+// cycles): a lane outside the table reads the nearest row and drops it.  With
+// one paired read and no nested branches here and in table_force the step of
+// 44 atoms went from 30.2 to 29.3 us, of 1,100 atoms from 94.7 to 93.4 us.
+__device__ __forceinline__ void field_in_sphere(const TableView &tb, const float2 *GE, int tj,
+                                                float d2, float inv, float s, float rx, float ry,
+                                                float rz, float e0, FieldRare &st)
 {
+    // every rounding spelt out: the bin from a fused d2 inv - r0, the phases
+    // from the rounded distance
+#pragma clang fp contract(off)
     const float d = d2 * inv;
-    const float x = (d - tb.g_r0) * tb.g_inv;
-    const int b = (int)x;  // truncation, as the reference's int()
-    float fac = 1.0f, et = 0.0f;
-    if (b < 0) {
-        fac = 0.0f;
-    } else if (b < tb.n_g - 1) {
-        const float ph = (d - (tb.g_r0 + (float)b * tb.g_dr)) * tb.g_inv;
-        const float *G = Gtab + tj * tb.ld_g;
-        fac = __builtin_fmaf(G[b + 1], ph, G[b] * (1.0f - ph));
-        const float phe = (d - (tb.e_r0 + (float)b * tb.e_dr)) * tb.e_inv;
-        const float *Et = Etab + tj * tb.ld_e;
-        et = __builtin_fmaf(Et[b + 1], phe, Et[b] * (1.0f - phe));
-    }
+    // truncation, as the reference's int()
+    const int b = (int)(__builtin_fmaf(d2, inv, -tb.g_r0) * tb.g_inv);
+    const int row = max(0, min(b, tb.n_g - 2));
+    const float2 t0 = GE[tj * tb.ld_g + row], t1 = GE[tj * tb.ld_g + row + 1];
+    const float og = d - __builtin_fmaf(tb.g_dr, (float)row, tb.g_r0);
+    const float oe = d - __builtin_fmaf(tb.e_dr, (float)row, tb.e_r0);
+    float fac = __builtin_fmaf(t1.x, og * tb.g_inv, t0.x * __builtin_fmaf(-tb.g_inv, og, 1.0f));
+    float et = __builtin_fmaf(t1.y, oe * tb.e_inv, t0.y * __builtin_fmaf(-tb.e_inv, oe, 1.0f));
+    fac = b < 0 ? 0.0f : (b < tb.n_g - 1 ? fac : 1.0f);
+    et = b == row ? et : 0.0f;
     st.g *= fac;
     st.cnt += 1;
     const float c = __builtin_fmaf(-e0, s, et * inv);
@@ -146,12 +149,12 @@ __device__ __forceinline__ void field_in_sphere_an(const DiffType &T, float d2, 
     st.ez = __builtin_fmaf(c, rz, st.ez);
 }
 
-// One (point, atom) pair; type: where the atom's type is read, if it is needed
-template <bool PBC, bool AN, typename TypePtr>
-__device__ __forceinline__ void field_pair(const TableView &tab, float e0, const float *Gtab,
-                                           const float *Etab, const DiffType *dtypes, float4 q,
-                                           TypePtr type, const MinImage &mi, float px, float py,
-                                           float pz, float R2, float &ax, float &ay, float &az,
+// One (point, atom) pair; type(): the atom's type, asked for only in a sphere
+template <bool PBC, bool AN, typename Type>
+__device__ __forceinline__ void field_pair(const TableView &tab, float e0, const float2 *GE,
+                                           const DiffType *dtypes, float4 q, Type type,
+                                           const MinImage &mi, float px, float py, float pz,
+                                           float R2, float &ax, float &ay, float &az,
                                            FieldRare &st)
 {
     float rx = px - q.x, ry = py - q.y, rz = pz - q.z;
@@ -170,18 +173,18 @@ __device__ __forceinline__ void field_pair(const TableView &tab, float e0, const
     az = __builtin_fmaf(so, rz, az);
     if (in) {
         if (AN)
-            field_in_sphere_an(dtypes[*type], d2, inv, s, rx, ry, rz, e0, st);
+            field_in_sphere_an(dtypes[type()], d2, inv, s, rx, ry, rz, e0, st);
         else
-            field_in_sphere(tab, Gtab, Etab, *type, d2, inv, s, rx, ry, rz, e0, st);
+            field_in_sphere(tab, GE, type(), d2, inv, s, rx, ry, rz, e0, st);
     }
 }
 
 template <bool PBC, bool AN>
-__device__ __forceinline__ void field_tile(const FieldArgs &a, const float *Gtab,
-                                           const float *Etab, const DiffType *dtypes, int j0,
-                                           int j1, const MinImage &mi,
-                                           float px, float py, float pz, float R2, float &ax,
-                                           float &ay, float &az, FieldRare &st)
+__device__ __forceinline__ void field_tile(const FieldArgs &a, const float2 *GE,
+                                           const DiffType *dtypes, int j0, int j1,
+                                           const MinImage &mi, float px, float py, float pz,
+                                           float R2, float &ax, float &ay, float &az,
+                                           FieldRare &st)
 {
     // the tile's atoms by a pointer that advances 16 bytes an atom (an index
     // recomputed from j costs the scalar unit a sign extension and a shift
@@ -190,8 +193,8 @@ __device__ __forceinline__ void field_tile(const FieldArgs &a, const float *Gtab
     const auto *ity = read_only(a.itype);
 #pragma unroll 2
     for (int j = j0; j < j1; ++j, xq += 4)  // wave-uniform
-        field_pair<PBC, AN>(a.tab, a.e0, Gtab, Etab, dtypes, make_float4(xq[0], xq[1], xq[2], xq[3]),
-                            ity + j, mi, px, py, pz, R2, ax, ay, az, st);
+        field_pair<PBC, AN>(a.tab, a.e0, GE, dtypes, make_float4(xq[0], xq[1], xq[2], xq[3]),
+                            [=]() { return ity[j]; }, mi, px, py, pz, R2, ax, ay, az, st);
 }
 
 // a point's sums over atoms [j0, j1) of its split
@@ -201,10 +204,9 @@ struct FieldSums {
 };
 
 template <bool AN>
-__device__ __forceinline__ void field_span(const FieldArgs &a, const float *Gtab,
-                                           const float *Etab, const DiffType *dtypes, int j0,
-                                           int j1, const WinDesc &W, bool pbc, float4 p,
-                                           FieldSums &fs)
+__device__ __forceinline__ void field_span(const FieldArgs &a, const float2 *GE,
+                                           const DiffType *dtypes, int j0, int j1,
+                                           const WinDesc &W, bool pbc, float4 p, FieldSums &fs)
 {
     FieldRare &st = fs.st;
     const MinImage mi = min_image_of(W.L, W.h);
@@ -213,11 +215,9 @@ __device__ __forceinline__ void field_span(const FieldArgs &a, const float *Gtab
         float ax = 0.0f, ay = 0.0f, az = 0.0f;
         st.ex = st.ey = st.ez = 0.0f;
         if (pbc)
-            field_tile<true, AN>(a, Gtab, Etab, dtypes, jt, je, mi, p.x, p.y, p.z, p.w, ax,
-                                 ay, az, st);
+            field_tile<true, AN>(a, GE, dtypes, jt, je, mi, p.x, p.y, p.z, p.w, ax, ay, az, st);
         else
-            field_tile<false, AN>(a, Gtab, Etab, dtypes, jt, je, mi, p.x, p.y, p.z, p.w, ax,
-                                  ay, az, st);
+            field_tile<false, AN>(a, GE, dtypes, jt, je, mi, p.x, p.y, p.z, p.w, ax, ay, az, st);
         fs.sx += (double)ax;
         fs.sy += (double)ay;
         fs.sz += (double)az;
@@ -282,18 +282,17 @@ __global__ __launch_bounds__(kBlock) void k_field(FieldArgs a)
     // space, so the LDS ones compile to LDS reads.
     FieldSums fs;
     if (!AN && field_tab_floats(a.tab) <= kTabLdsFloats) {
-        const int ng = a.tab.ntypes * a.tab.ld_g;
-        stage_lds(lds_tab, a.tab.g, ng);
-        stage_lds(lds_tab + ng, a.tab.e, a.tab.ntypes * a.tab.ld_e);
+        stage_lds(lds_tab, reinterpret_cast<const float *>(a.tab.ge), field_tab_floats(a.tab));
         __syncthreads();
-        field_span<AN>(a, lds_tab, lds_tab + ng, a.dtypes, j0, j1, W, pbc, p, fs);
+        field_span<AN>(a, reinterpret_cast<const float2 *>(lds_tab), a.dtypes, j0, j1, W, pbc, p,
+                       fs);
     } else if (AN && diff_tab_floats(a.tab) <= kTabLdsFloats) {
         stage_lds(lds_tab, reinterpret_cast<const float *>(a.dtypes), diff_tab_floats(a.tab));
         __syncthreads();
-        field_span<AN>(a, a.tab.g, a.tab.e, reinterpret_cast<const DiffType *>(lds_tab), j0, j1,
-                       W, pbc, p, fs);
+        field_span<AN>(a, a.tab.ge, reinterpret_cast<const DiffType *>(lds_tab), j0, j1, W, pbc, p,
+                       fs);
     } else {
-        field_span<AN>(a, a.tab.g, a.tab.e, a.dtypes, j0, j1, W, pbc, p, fs);
+        field_span<AN>(a, a.tab.ge, a.dtypes, j0, j1, W, pbc, p, fs);
     }
     asm volatile("" ::"v"(w0), "v"(w1));
     FieldRare &st = fs.st;
@@ -522,6 +521,21 @@ __device__ __forceinline__ float3 cdd_term(float4 c, float rx, float ry, float r
                        __builtin_fmaf(ac, rz, -bc * c.z));
 }
 
+// F of the receiver type's table at d = d2 rinv.  No branch: a lane outside the
+// table reads the nearest row and drops it; roundings as in field_in_sphere.
+__device__ __forceinline__ float table_force(const TableView &tb, const float *F, float d2,
+                                             float rinv)
+{
+#pragma clang fp contract(off)
+    const int b =
+        (int)__builtin_fmaf(tb.f_inv, __builtin_fmaf(d2, rinv, -tb.f_r0), 0.5f);
+    const int row = max(0, min(b, tb.n_f - 1));
+    const float o = d2 * rinv - __builtin_fmaf(tb.f_dr, (float)row, tb.f_r0);
+    const float f =
+        __builtin_fmaf(F[row + 1], o * tb.f_inv, F[row] * __builtin_fmaf(-tb.f_inv, o, 1.0f));
+    return b == row ? f : 0.0f;
+}
+
 // FP32 sums of one tile: the electrostatic (or, split, polarisation) sum s and
 // the in-sphere LJ sum l; flushed into the FP64 ForceAcc per tile
 struct TileSums {
@@ -610,16 +624,11 @@ __device__ __forceinline__ void force_tile(const ForceArgs &a, const float4 *__r
             }
         }
         if (in) {
-            const float d = d2 * rinv;
-            float fs = 0.0f;
+            float fs;
             if (AN) {
-                fs = diff_F(fp, d, rinv) * w;
+                fs = diff_F(fp, d2 * rinv, rinv) * w;
             } else {
-                const int b = (int)((d - a.tab.f_r0) * a.tab.f_inv + 0.5f);
-                if (b >= 0 && b < a.tab.n_f) {
-                    const float ph = (d - (a.tab.f_r0 + (float)b * a.tab.f_dr)) * a.tab.f_inv;
-                    fs = __builtin_fmaf(Ftab[b + 1], ph, Ftab[b] * (1.0f - ph)) * w;
-                }
+                fs = table_force(a.tab, Ftab, d2, rinv) * w;
             }
             const float fl = fs * rinv;
             ts.lx = __builtin_fmaf(fl, rx, ts.lx);
@@ -814,7 +823,7 @@ constexpr int kWinMaxBlocks = 512;
 struct WindowLds {
     const float4 *atoms;
     const int *types;
-    const float *G, *E;
+    const float2 *GE;
 };
 
 template <bool PBC>
@@ -829,8 +838,9 @@ __device__ __forceinline__ void window_field_span(const WindowArgs &a, const Win
         st.ex = st.ey = st.ez = 0.0f;
 #pragma unroll 2
         for (int j = jt; j < je; ++j)
-            field_pair<PBC, false>(a.tab, a.e0, l.G, l.E, nullptr, l.atoms[j], l.types + j, mi, p.x,
-                                   p.y, p.z, p.w, ax, ay, az, st);
+            field_pair<PBC, false>(a.tab, a.e0, l.GE, nullptr, l.atoms[j],
+                                   [=]() { return l.types[j]; }, mi, p.x, p.y, p.z, p.w, ax, ay,
+                                   az, st);
         fs.sx += (double)ax;
         fs.sy += (double)ay;
         fs.sz += (double)az;
@@ -907,22 +917,20 @@ __global__ __launch_bounds__(kWinThreads, 4) void k_window(WindowArgs a)
     // points, in each record's first entry, and the draws' counters), then an
     // area that holds the g and E tables and the splits' field sums, later the
     // shares' force sums
-    const int nf = force_tab_floats(a.tab), ng = a.tab.ntypes * a.tab.ld_g;
-    const int ne = a.tab.ntypes * a.tab.ld_e;
+    const int nf = force_tab_floats(a.tab), nge = field_tab_floats(a.tab);
     float4 *atoms = reinterpret_cast<float4 *>(lds_tab + a.off_atoms);
     int *types = reinterpret_cast<int *>(atoms + kWinMaxAtoms);
     float4 *lrec = reinterpret_cast<float4 *>(lds_tab + a.off_pts);
     float4 *laux = lrec + 4 * a.cap_pts;
     int *best = reinterpret_cast<int *>(laux);
     float *area = lds_tab + a.off_x;
-    FieldXchg *xc = reinterpret_cast<FieldXchg *>(area + ((ng + ne + 3) & ~3));
+    FieldXchg *xc = reinterpret_cast<FieldXchg *>(area + ((nge + 3) & ~3));
     for (int i = tid; i < n; i += kWinThreads) {
         atoms[i] = a.xyzq[W.a0 + i];
         types[i] = a.itype[W.a0 + i];
     }
     stage_lds<kWinThreads>(lds_tab, a.tab.f, nf);
-    stage_lds<kWinThreads>(area, a.tab.g, ng);
-    stage_lds<kWinThreads>(area + ng, a.tab.e, ne);
+    stage_lds<kWinThreads>(area, reinterpret_cast<const float *>(a.tab.ge), nge);
     // (its barrier also publishes the staged data)
     const bool pbc = needs_image<kWinThreads>(W, a.xyzq, a.rmax_all);
     const MinImage mi = min_image_of(W.L, W.h);
@@ -933,7 +941,7 @@ __global__ __launch_bounds__(kWinThreads, 4) void k_window(WindowArgs a)
     const int lt = tid - sub * npr;
     window_points(a, W, m0, np, lt, sub, D, atoms, types, lrec, best);
     // field: D splits side by side, added in order, groups of W.fg at a time
-    const WindowLds l{atoms, types, area, area + ng};
+    const WindowLds l{atoms, types, reinterpret_cast<const float2 *>(area)};
     const float4 p = lt < np ? lrec[4 * lt] : make_float4(0.0f, 0.0f, 0.0f, -1.0f);
     double g = 1.0, s0[3] = {0, 0, 0}, ei[3] = {0, 0, 0};
     double gg = 1.0, gs[3] = {0, 0, 0}, ge[3] = {0, 0, 0};

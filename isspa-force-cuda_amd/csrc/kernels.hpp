@@ -43,11 +43,14 @@ inline int field_group(int splits) { return splits % 4 == 0 ? 4 : (splits % 2 ==
 // Per-type tables on the device, each type padded with one trailing zero row
 // so that a lerp at the last row reads 0 (the reference reads the next type's
 // first row there, 0 in every shipped table; quirk Q4).  All windows share the
-// grid; their types are concatenated.
+// grid; their types are concatenated.  The E table is read at the g table's
+// row, so the two are stored as pairs {g, E}: both ends of both lerps are one
+// 16-byte read (E rows beyond the g table are never read).
 struct TableView {
-    const float *g, *e, *f;
-    int n_g, n_e, n_f;     // logical rows
-    int ld_g, ld_e, ld_f;  // padded rows per type
+    const float2 *ge;
+    const float *f;
+    int n_g, n_f;    // logical rows
+    int ld_g, ld_f;  // padded rows per type
     int ntypes;
     float g_r0, g_dr, g_inv;
     float e_r0, e_dr, e_inv;

@@ -38,7 +38,8 @@ struct isspa_model {
     float rmax_all = 0.f;
     int *itype = nullptr, *atom_win = nullptr;
     float *rmax = nullptr, *rmax2 = nullptr, *vtot = nullptr;
-    float *g = nullptr, *e = nullptr, *f = nullptr;
+    float2 *ge = nullptr;
+    float *f = nullptr;
     float4 *pts = nullptr;
     float *rec = nullptr;  // [P][kRecFloats] records, then [P] float4 aux
     double *g_out = nullptr, *E_out = nullptr, *E0_out = nullptr;
