@@ -195,6 +195,7 @@ static int diff_isspa_forward(isspa_diff *m, const double *q_d, double *f_d, hip
     DiffReduceArgs ra{};
     ra.n = m->n;
     ra.wins = im->wins;
+    ra.nwin = im->lay.W;
     ra.atom_win = im->atom_win;
     ra.part = im->part_f;
     ra.C = im->C;
@@ -294,6 +295,7 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     fa.n = m->n;
     fa.wins = im->wins;
     fa.nb_wins = nb->wins;
+    fa.nwin = im->lay.W;
     fa.atom_win = im->atom_win;
     fa.apart = m->apart;
     fa.C = im->V;

@@ -400,7 +400,7 @@ ReduceArgs reduce_args(isspa_model *m, const float4 *x, float4 *f, double *flj, 
                        double *fcdd)
 {
     ReduceArgs ra{};
-    ra.wins = m->wins; ra.atom_win = m->atom_win; ra.part = m->part_f; ra.C = m->C;
+    ra.wins = m->wins; ra.nwin = m->lay.W; ra.atom_win = m->atom_win; ra.part = m->part_f; ra.C = m->C;
     ra.ntot = m->d.n_atoms; ra.xyzq = x; ra.itype = m->itype; ra.vtot = m->vtot; ra.f = f;
     ra.f_lj = flj; ra.f_pol = fpol; ra.f_cdd = fcdd;
     return ra;
@@ -787,7 +787,7 @@ int nonbond_partials(nonbond_model *m, const float *xyzq4_d, bool split, hipStre
 int nonbond_reduce(nonbond_model *m, bool split, float4 *f, double *o0, double *o1, double *o2,
                    hipStream_t s)
 {
-    HIPCHK(launch_chunk_reduce3(m->wins, m->atom_win, m->part, split ? m->B : m->B_tot, m->n,
+    HIPCHK(launch_chunk_reduce3(m->wins, m->lay.W, m->atom_win, m->part, split ? m->B : m->B_tot, m->n,
                                 split ? 9 : 3, f, o0, o1, o2, s));
     return ISSPA_OK;
 }
@@ -1120,8 +1120,9 @@ struct md_engine {
     uint64_t seed = 0;
     uint32_t sys = 0;
     WinDesc *wins = nullptr;   // integrator windows (owned)
+    int nwin = 1;
     int *atom_win = nullptr;
-    uint32_t *step_d = nullptr;  // [2]: step, leap-frog blocks done
+    uint32_t *step_d = nullptr;  // [2]: kStepNext, kStepNow
     double *com_d = nullptr;
     float4 *fus = nullptr;       // restraint bias forces of the step (w = 1: restrained)
     hipGraph_t graph = nullptr;
@@ -1193,9 +1194,9 @@ extern "C" int md_engine_create(isspa_model *isspa, nonbond_model *nb, bonded_mo
     else rc = build_windows(n, nullptr, sys, lbox, lay);
     std::vector<WinDesc> wd;
     for (int w = 0; rc == ISSPA_OK && w < lay.W; ++w) wd.push_back(base_desc(lay, w));
+    e->nwin = (int)wd.size();
     if (rc == ISSPA_OK) rc = upload(&e->wins, wd.data(), wd.size());
     if (rc == ISSPA_OK) rc = upload(&e->atom_win, lay.atom_win.data(), lay.atom_win.size());
-    // {step, leap-frog blocks done}: the leap-frog launch advances the step
     if (rc == ISSPA_OK) rc = dalloc(&e->step_d, 2);
     if (rc == ISSPA_OK) rc = dalloc(&e->com_d, 6 * (size_t)(us ? us->nres : 1));
     if (rc == ISSPA_OK && us) {
@@ -1239,7 +1240,7 @@ extern "C" int md_engine_destroy(md_engine *e)
 extern "C" int md_engine_set_step(md_engine *e, uint32_t step, void *stream)
 {
     if (!e) return fail(ISSPA_ERR_ARG, "null engine");
-    HIPCHK(launch_set_word(e->step_d, step, S(stream)));
+    HIPCHK(launch_set_word(e->step_d + kStepNext, step, S(stream)));
     return ISSPA_OK;
 }
 
@@ -1283,7 +1284,8 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
     // enough for super-tiles always have the side stream)
     const bool nb_rides = m && e->nb && !fork && !e->nb->any_sym;
     if (m && isspa_is_small(m)) {
-        WindowArgs w = window_args(m, x4, 0u, e->step_d);
+        WindowArgs w = window_args(m, x4, 0u, e->step_d + kStepNext);
+        w.step_now = e->step_d + kStepNow;
         w.bonded = bonded;
         w.us = us;
         if (nb_rides) {
@@ -1296,12 +1298,13 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
         p.bonded = bonded;
         p.us = us;
         p.pts.xyzq = x4;
+        p.step_d = e->step_d;
         if (m) {
             p.nflag = m->lay.W;
             p.rmax_all = m->rmax_all;
             p.flag = m->pbc_flag;
             p.pts = PointsArgs{m->wins, m->atom_win, x4, m->itype, m->rmax, m->rmax2,
-                               m->d.n_atoms, m->d.n_mc, m->d.seed, 0u, e->step_d, m->pts};
+                               m->d.n_atoms, m->d.n_mc, m->d.seed, 0u, e->step_d + kStepNext, m->pts};
         }
         HIPCHK(launch_step_prologue(p, s));
         if (m) {
@@ -1323,6 +1326,7 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
         CHK(nonbond_partials(e->nb, e->x, false, s));
     if (e->nb) {
         a.nb_wins = e->nb->wins;
+        a.nb_nwin = e->nb->lay.W;
         a.nb_atom_win = e->nb->atom_win;
         a.nb_part = e->nb->part;
         a.nb_B = e->nb->B_tot;
@@ -1330,6 +1334,7 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
     if (integrate) {
         // the assembly launch also integrates each atom and advances the step
         a.lf.wins = e->wins;
+        a.lf.nwin = e->nwin;
         a.lf.atom_win = e->atom_win;
         a.lf.xyzq = reinterpret_cast<float4 *>(e->x);
         a.lf.vel = reinterpret_cast<float4 *>(e->v);
@@ -1338,7 +1343,6 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
         a.lf.thr = andersen_threshold(e->pnu);
         a.lf.seed = e->seed;
         a.lf.step_d = e->step_d;
-        a.lf.advance = e->step_d;
     }
     HIPCHK(launch_assemble_forces(a, s));
     return ISSPA_OK;

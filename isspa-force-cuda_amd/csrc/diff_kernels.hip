@@ -99,8 +99,8 @@ __global__ __launch_bounds__(kB) void k_diff_prep_atoms(DiffAtomArgs a)
 }
 
 // F_i = -q_i vtot_i S_e - vtot_i S_lj (overwrites f), S_e kept for the adjoint.
-// Latency bound: a block of 32 atoms x 8 chunk slices (reduce_device.hpp) with
-// six chunks' entries in flight a slice.  One lane per atom over all chunks
+// Latency bound: a block of 16 atoms x 16 entry slices (reduce_device.hpp) with
+// eight entries in flight a slice.  One lane per atom over all chunks
 // took 53.9 us at 550 atoms (3 blocks, 181 dependent rounds) and 121 us for
 // 32 x 1,100 atoms; now 7.4 and 16 us (86 MB, 5.4 TB/s).
 __global__ __launch_bounds__(kB) void k_diff_reduce(DiffReduceArgs a)
@@ -111,8 +111,8 @@ __global__ __launch_bounds__(kB) void k_diff_reduce(DiffReduceArgs a)
     const bool valid = i < a.n;
     double s[6] = {0, 0, 0, 0, 0, 0};
     if (valid) {
-        const WinDesc W = a.wins[a.atom_win[i]];
-        force_slice_sum<6>(W, a.part, i, sl, s);
+        const WinDesc W = window_of(a.wins, a.nwin, a.atom_win, i);
+        sum_batches<6, 8>(ForceEntry<6>(W, a.part, i), sl, W.fents, s);
     }
     combine_slices<6>(red, al, sl, s);
     if (sl != 0 || !valid) return;
@@ -506,34 +506,8 @@ __global__ __launch_bounds__(kB) void k_vjp_nonbond(VjpNbArgs a)
     a.part[2 * a.B + o] = eacc;
 }
 
-// Sums of NC component-major partials [NC][stride], entries c = sl,
-// sl + kSumSlices, ... of atom slot `base`, B entries' loads in flight.
-template <int NC, int B>
-__device__ __forceinline__ void planar_slice_sum(const double *__restrict__ part, long long stride,
-                                                 long long base, int step, int n, int sl,
-                                                 double *s)
-{
-    int c = sl;
-    for (; c + (B - 1) * kSumSlices < n; c += B * kSumSlices) {
-        double v[B][NC];
-#pragma unroll
-        for (int u = 0; u < B; ++u)
-#pragma unroll
-            for (int k = 0; k < NC; ++k)
-                v[u][k] = part[k * stride + base + (long long)(c + u * kSumSlices) * step];
-#pragma unroll
-        for (int u = 0; u < B; ++u)
-#pragma unroll
-            for (int k = 0; k < NC; ++k) s[k] += v[u][k];
-    }
-    for (; c < n; c += kSumSlices)
-#pragma unroll
-        for (int k = 0; k < NC; ++k) s[k] += part[k * stride + base + (long long)c * step];
-}
-
 // Per atom: the chunk partials + the direct charge term.  Latency bound like
-// k_diff_reduce and split the same way (32 atoms x 8 slices a block, four
-// chunks in flight a slice): one lane per atom took 74.7 us at 550 atoms and
+// k_diff_reduce and split the same way, four entries in flight a slice: one lane per atom took 74.7 us at 550 atoms and
 // 133 us for 32 x 1,100 atoms; now 9.2 and 24 us.
 __global__ __launch_bounds__(kB) void k_vjp_finish(VjpFinishArgs a)
 {
@@ -543,12 +517,11 @@ __global__ __launch_bounds__(kB) void k_vjp_finish(VjpFinishArgs a)
     const bool valid = i < a.n;
     double s[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};  // q, theta(5); nonbond q, sigma, eps
     if (valid) {
-        const int w = a.atom_win[i];
-        const WinDesc W = a.wins[w];
-        const WinDesc Wn = a.nb_wins[w];
+        const WinDesc W = window_of(a.wins, a.nwin, a.atom_win, i);
+        const WinDesc Wn = window_of(a.nb_wins, a.nwin, a.atom_win, i);
         const int il = i - W.a0;
-        planar_slice_sum<6, 4>(a.apart, a.C, W.vpo + il, W.n, W.vents, sl, s);
-        planar_slice_sum<3, 4>(a.nbpart, a.B, Wn.npo + il, Wn.n, Wn.nbc, sl, s + 6);
+        sum_batches<6, 4>(PlanarEntry<6>{a.apart, a.C, W.vpo + il, W.n}, sl, W.vents, s);
+        sum_batches<3, 4>(PlanarEntry<3>{a.nbpart, a.B, Wn.npo + il, Wn.n}, sl, Wn.nbc, s + 6);
     }
     combine_slices<9>(red, al, sl, s);
     if (sl != 0 || !valid) return;

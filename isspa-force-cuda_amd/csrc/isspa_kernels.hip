@@ -888,6 +888,7 @@ __global__ __launch_bounds__(kWinThreads, 4) void k_window(WindowArgs a)
 {
     extern __shared__ __align__(16) float lds_tab[];
     int b = blockIdx.x;
+    if (a.step_now && b == 0 && threadIdx.x == 0) *a.step_now = a.step_d ? *a.step_d : a.step;
     if (b >= a.nblocks) {
         // a riding block
         b -= a.nblocks;
@@ -1018,7 +1019,7 @@ __global__ __launch_bounds__(kWinThreads, 4) void k_window(WindowArgs a)
 }
 
 // F_i = -q_i vtot_i S_e - vtot_i S_lj over the chunk partials, summed in the
-// fixed slice order of isspa_slice_sum (kSumAtoms atoms x kSumSlices chunk
+// fixed slice order of reduce_device.hpp (kSumAtoms atoms x kSumSlices chunk
 // slices a block).
 template <bool SPLIT>
 __global__ __launch_bounds__(kBlock) void k_force_reduce(ReduceArgs a)
@@ -1030,11 +1031,14 @@ __global__ __launch_bounds__(kBlock) void k_force_reduce(ReduceArgs a)
     const bool valid = i < a.ntot;
     double s[comps];
     for (int k = 0; k < comps; ++k) s[k] = 0.0;
-    if (valid) isspa_slice_sum<comps>(a, i, sl, s);
+    if (valid) {
+        const WinDesc W = window_of(a.wins, a.nwin, a.atom_win, i);
+        sum_batches<comps, 8>(ForceEntry<comps>(W, a.part, i), sl, W.fents, s);
+    }
     combine_slices<comps>(red, al, sl, s);
     if (sl != 0 || !valid) return;
     if (!SPLIT) {
-        const float3 fi = isspa_atom_force(a, i, s);
+        const float3 fi = isspa_atom_force(a.xyzq[i].w, a.vtot[a.itype[i]], s);
         float4 f = a.f[i];
         f.x += fi.x;
         f.y += fi.y;

@@ -200,6 +200,7 @@ __host__ __device__ constexpr int force_part_stride(bool split) { return split ?
 
 struct ReduceArgs {
     const WinDesc *wins;
+    int nwin;
     const int *atom_win;
     const double *part;
     long long C;
@@ -277,6 +278,7 @@ struct WindowArgs {
     const uint32_t *step_d;
     float4 *pts;
     double *part;         // force partials, as k_force leaves them
+    uint32_t *step_now;   // an engine step's kStepNow word, or null
     NonbondArgs nb;
     int nb_blocks;
     BondedArgs bonded;
@@ -309,26 +311,33 @@ struct AssembleArgs {
     const int *gptr, *gidx;
     ReduceArgs isspa;       // IS-SPA chunk partials (isspa.f unused)
     const WinDesc *nb_wins; // all-pairs chunk partials
+    int nb_nwin;
     const int *nb_atom_win;
     const double *nb_part;
     long long nb_B;
     const float4 *fus;      // restraint bias forces (w = 1 marks a restrained atom), added last
     struct {                // leap-frog + Andersen of the assembled atoms (xyzq null: none)
         const WinDesc *wins;    // integrator windows, both required with xyzq
+        int nwin;
         const int *atom_win;
         float4 *xyzq, *vel;
         float kT, dt;
         uint32_t thr;
         uint64_t seed;
-        const uint32_t *step_d;
-        uint32_t *advance;  // {step, blocks done}: the last block moves the step on
+        uint32_t *step_d;   // kStepNext: written step + 1; kStepNow: this step
     } lf;
 };
 hipError_t launch_assemble_forces(const AssembleArgs &a, hipStream_t s);
 
+// The engine's step counter is two words.  The first launch of a step reads
+// kStepNext and copies it to kStepNow; the assembly, its last launch, reads
+// kStepNow and writes kStepNow + 1 to kStepNext.  No launch both reads a word
+// and writes it, so no block waits for or counts the others.
+constexpr int kStepNext = 0, kStepNow = 1;
+
 // ---- nonbond ----
 hipError_t launch_nonbond(const NonbondArgs &a, int nblocks, bool split, hipStream_t s);
-hipError_t launch_chunk_reduce3(const WinDesc *wins, const int *atom_win, const double *part,
+hipError_t launch_chunk_reduce3(const WinDesc *wins, int nwin, const int *atom_win, const double *part,
                                 long long B, int ntot, int comps, float4 *f, double *o0,
                                 double *o1, double *o2, hipStream_t s);
 
@@ -347,6 +356,7 @@ struct PrologueArgs {
     int bonded_blocks;      // set by the launcher
     RestraintArgs us;       // bias forces stored into fus
     PointsArgs pts;         // MC points (pts.wins also serves the flags)
+    uint32_t *step_d;       // the step counter's two words
 };
 hipError_t launch_step_prologue(PrologueArgs a, hipStream_t s);
 
@@ -376,6 +386,7 @@ struct DiffAtomArgs {
 struct DiffReduceArgs {
     int n;
     const WinDesc *wins;
+    int nwin;
     const int *atom_win;
     const double *part;    // force partials [6][C] (S_e, S_lj)
     long long C;
@@ -422,6 +433,7 @@ struct VjpNbArgs {
 struct VjpFinishArgs {
     int n;
     const WinDesc *wins, *nb_wins;
+    int nwin;
     const int *atom_win;
     const double *apart;
     long long C;
@@ -451,7 +463,7 @@ hipError_t launch_type_reduce(const double *gatom, const int *itype, int n, int 
 hipError_t launch_leapfrog(const WinDesc *wins, const int *atom_win, const WinDesc &one,
                            int ntot, float4 *xyzq, float4 *vel, const float4 *f, float kT,
                            float dt, uint32_t thr, uint64_t seed, uint32_t step,
-                           const uint32_t *step_d, hipStream_t s, uint32_t *advance = nullptr);
+                           const uint32_t *step_d, hipStream_t s);
 // one workgroup per restraint; bias entries [boff[r], boff[r+1]) {atom, group}
 hipError_t launch_us(int nres, const int *boff, const int2 *atoms, const float *mass,
                      const float2 *kx /* {k, x0} */, const float *L, const float4 *xyzq,
@@ -460,7 +472,6 @@ hipError_t launch_pbc_flag(const WinDesc *wins, int W, const float4 *xyzq, float
                            int *flag, hipStream_t s);
 hipError_t launch_zero(void *p, size_t bytes, hipStream_t s);
 hipError_t launch_add4(float4 *dst, const float4 *src, int n, hipStream_t s);
-hipError_t launch_step_advance(uint32_t *step_d, hipStream_t s);
 hipError_t launch_set_word(uint32_t *dst, uint32_t v, hipStream_t s);
 
 }  // namespace isspa

@@ -11,11 +11,14 @@ namespace isspa {
 
 // A 256-thread reduction block owns kSumAtoms atoms and kSumSlices slices of
 // each atom's list: slice t takes entries t, t + S, t + 2S, ... in order, and
-// slice 0 then adds slices 1..S-1 in order.  The slices give the kernel S
-// times the waves of one lane per atom, which small systems need to hide the
-// load latency (a 44-atom system has 275 IS-SPA chunk partials per atom).
-constexpr int kSumAtoms = 32;
-constexpr int kSumSlices = 8;
+// slice 0 then adds slices 1..S-1 in order.  The sums are bounded by the
+// latency of a few dependent loads, so the slices are many and short: with 16
+// slices the 60 or so entries of a large system are one batch of loads a
+// slice.  (32 atoms x 8 slices: the reduction of 44 atoms over 677 entries
+// took 16.1 us, the solvent force of which it is a part 45.8, now 40.4 us;
+// the all-pairs force of 2,222 atoms 25.7, now 22.3 us.)
+constexpr int kSumAtoms = 16;
+constexpr int kSumSlices = 16;
 
 // Every slice's sums into slice 0, added in slice order (slice 0's value,
 // then slices 1, 2, ...).  Component k is added up by the work-items of slice
@@ -31,9 +34,12 @@ __device__ __forceinline__ void combine_slices(double (&red)[kSumSlices][NC][kSu
     for (int k = 0; k < NC; ++k) red[sl][k][al] = s[k];
     __syncthreads();
     for (int k = sl; k < NC; k += kSumSlices) {
-        double acc = red[0][k][al];
-#pragma unroll 4
-        for (int t = 1; t < kSumSlices; ++t) acc += red[t][k][al];
+        double v[kSumSlices];
+#pragma unroll
+        for (int t = 0; t < kSumSlices; ++t) v[t] = red[t][k][al];
+        double acc = v[0];
+#pragma unroll
+        for (int t = 1; t < kSumSlices; ++t) acc += v[t];
         red[0][k][al] = acc;
     }
     __syncthreads();
@@ -42,111 +48,131 @@ __device__ __forceinline__ void combine_slices(double (&red)[kSumSlices][NC][kSu
         for (int k = 0; k < NC; ++k) s[k] = red[0][k][al];
 }
 
-// Chunks whose partial loads one slice keeps in flight at a time; the
-// batch only groups the loads, the adds stay in chunk order.
-constexpr int kSumBatch = 6;
-
-// IS-SPA force partials of atom i (COMPS = 6, or 9 in split mode), chunks of
-// slice sl, added in chunk order.
-// the COMPS components of chunk-partial entry o (stored as double2 pairs)
-template <int COMPS>
-__device__ __forceinline__ void load_force_entry(const double *part, long long o,
-                                                 double (&v)[COMPS])
+// the window of atom i; one window needs no lookup
+__device__ __forceinline__ WinDesc window_of(const WinDesc *__restrict__ wins, int nwin,
+                                             const int *__restrict__ atom_win, int i)
 {
-    constexpr int kStride = force_part_stride(COMPS == 9);
-    const double2 *e = reinterpret_cast<const double2 *>(part + o * kStride);
+    return nwin == 1 ? wins[0] : wins[atom_win[i]];
+}
+
+// One batch of a slice's entries: entries c, c + S, ... (B of them, those
+// below n), the loads of all of them issued before the first is used.  The
+// missing ones read entry n - 1 again and count as zero, so the last batch
+// waits once, as every other.  load(entry, v) reads an entry's COMPS values.
+template <int COMPS, int B, typename Load>
+__device__ __forceinline__ void load_batch(Load load, int c, int n, double (&v)[B][COMPS])
+{
 #pragma unroll
-    for (int h = 0; h < (COMPS + 1) / 2; ++h) {
-        const double2 d = e[h];
-        v[2 * h] = d.x;
-        if (2 * h + 1 < COMPS) v[2 * h + 1] = d.y;
+    for (int u = 0; u < B; ++u) load(min(c + u * kSumSlices, n - 1), v[u]);
+}
+template <int COMPS, int B>
+__device__ __forceinline__ void add_batch(int c, int n, const double (&v)[B][COMPS], double *s)
+{
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+        const bool in = c + u * kSumSlices < n;
+#pragma unroll
+        for (int k = 0; k < COMPS; ++k) s[k] += in ? v[u][k] : 0.0;
+    }
+}
+template <int COMPS, int B, typename Load>
+__device__ __forceinline__ void sum_batches(Load load, int c, int n, double *s)
+{
+    for (; c < n; c += B * kSumSlices) {
+        double v[B][COMPS];
+        load_batch<COMPS, B>(load, c, n, v);
+        add_batch<COMPS, B>(c, n, v, s);
     }
 }
 
+// Reads the COMPS components (6, or 9 in split mode) of the force partial of
+// (entry, atom i of window W), stored as double2 pairs.
 template <int COMPS>
-__device__ inline void force_slice_sum(const WinDesc &W, const double *part, int i, int sl,
-                                       double (&s)[COMPS])
-{
-    const long long base = W.ppo + (i - W.a0);
-    int c = sl;
-    for (; c + (kSumBatch - 1) * kSumSlices < W.fents; c += kSumBatch * kSumSlices) {
-        double v[kSumBatch][COMPS];
-#pragma unroll
-        for (int u = 0; u < kSumBatch; ++u)
-            load_force_entry<COMPS>(part, base + (long long)(c + u * kSumSlices) * W.n, v[u]);
-#pragma unroll
-        for (int u = 0; u < kSumBatch; ++u)
-#pragma unroll
-            for (int k = 0; k < COMPS; ++k) s[k] += v[u][k];
+struct ForceEntry {
+    const double2 *part;
+    long long base, n;
+    __device__ __forceinline__ ForceEntry(const WinDesc &W, const double *p, int i)
+        : part(reinterpret_cast<const double2 *>(p)), base(W.ppo + (i - W.a0)), n(W.n)
+    {
     }
-    for (; c < W.fents; c += kSumSlices) {
-        double v[COMPS];
-        load_force_entry<COMPS>(part, base + (long long)c * W.n, v);
+    __device__ __forceinline__ void operator()(int c, double (&v)[COMPS]) const
+    {
+        const double2 *e = part + (base + c * n) * (force_part_stride(COMPS == 9) / 2);
 #pragma unroll
-        for (int k = 0; k < COMPS; ++k) s[k] += v[k];
+        for (int h = 0; h < (COMPS + 1) / 2; ++h) {
+            const double2 d = e[h];
+            v[2 * h] = d.x;
+            if (2 * h + 1 < COMPS) v[2 * h + 1] = d.y;
+        }
     }
-}
+};
 
+// Reads COMPS component-major partials [COMPS][stride] of entry c, n apart.
 template <int COMPS>
-__device__ inline void isspa_slice_sum(const ReduceArgs &a, int i, int sl, double (&s)[COMPS])
+struct PlanarEntry {
+    const double *part;
+    long long stride, base, n;
+    __device__ __forceinline__ void operator()(int c, double (&v)[COMPS]) const
+    {
+#pragma unroll
+        for (int k = 0; k < COMPS; ++k) v[k] = part[k * stride + base + c * n];
+    }
+};
+
+// all-pairs partials of atom i (COMPS = 3: the total force, entries of the
+// total-force layout; 9: the split components, one entry per partner chunk)
+template <int COMPS>
+__device__ __forceinline__ PlanarEntry<COMPS> nonbond_entry(const WinDesc &W, const double *part,
+                                                            long long B, int i)
 {
-    const WinDesc W = a.wins[a.atom_win[i]];
-    force_slice_sum<COMPS>(W, a.part, i, sl, s);
+    return PlanarEntry<COMPS>{part, B, (COMPS == 3 ? W.spo : W.npo) + (i - W.a0), W.n};
 }
 
 // F_i = -q_i vtot_i S_e - vtot_i S_lj from the summed IS-SPA partials
-__device__ inline float3 isspa_atom_force(const ReduceArgs &a, int i, const double s[6])
+__device__ __forceinline__ float3 isspa_atom_force(float q, float vtot, const double *s)
 {
-    const float4 x = a.xyzq[i];
-    const double vt = (double)a.vtot[a.itype[i]];
-    const double qv = -(double)x.w * vt;
+    const double vt = (double)vtot;
+    const double qv = -(double)q * vt;
     return make_float3((float)(qv * s[0] - vt * s[3]), (float)(qv * s[1] - vt * s[4]),
                        (float)(qv * s[2] - vt * s[5]));
 }
 
-// bonded contribution slots of atom i, slots ptr[i] + sl, + kSumSlices, ...
-__device__ inline void bonded_slice_sum(const float4 *__restrict__ contrib,
-                                        const int *__restrict__ ptr, const int *__restrict__ idx,
-                                        int i, int sl, double &sx, double &sy, double &sz)
+// bonded contribution slots [e0, e1) of an atom, slots e0 + sl, + kSumSlices,
+// ...: the indices of a batch, then its contributions
+constexpr int kBondBatch = 4;
+struct BondBatch {
+    int idx[kBondBatch];
+    float4 c[kBondBatch];
+};
+__device__ __forceinline__ void bonded_load_idx(const int *__restrict__ idx, int e, int e1,
+                                                BondBatch &b)
 {
-    for (int e = ptr[i] + sl; e < ptr[i + 1]; e += kSumSlices) {
-        const float4 c = contrib[idx[e]];
-        sx += c.x;
-        sy += c.y;
-        sz += c.z;
+#pragma unroll
+    for (int u = 0; u < kBondBatch; ++u) b.idx[u] = idx[max(0, min(e + u * kSumSlices, e1 - 1))];
+}
+__device__ __forceinline__ void bonded_load(const float4 *__restrict__ contrib, BondBatch &b)
+{
+#pragma unroll
+    for (int u = 0; u < kBondBatch; ++u) b.c[u] = contrib[b.idx[u]];
+}
+__device__ __forceinline__ void bonded_add(int e, int e1, const BondBatch &b, double *s)
+{
+#pragma unroll
+    for (int u = 0; u < kBondBatch; ++u) {
+        const bool in = e + u * kSumSlices < e1;
+        s[0] += in ? (double)b.c[u].x : 0.0;
+        s[1] += in ? (double)b.c[u].y : 0.0;
+        s[2] += in ? (double)b.c[u].z : 0.0;
     }
 }
-
-// all-pairs partials of atom i (COMPS = 3: the total force, entries of the
-// total-force layout; 9: the split components, one entry per partner chunk),
-// entries of slice sl, added in entry order
-template <int COMPS>
-__device__ inline void nonbond_slice_sum(const WinDesc *__restrict__ wins,
-                                         const int *__restrict__ atom_win,
-                                         const double *__restrict__ part, long long B, int i,
-                                         int sl, double (&s)[COMPS])
+__device__ __forceinline__ void bonded_sum(const float4 *__restrict__ contrib,
+                                           const int *__restrict__ idx, int e, int e1, double *s)
 {
-    const WinDesc W = wins[atom_win[i]];
-    const long long base = (COMPS == 3 ? W.spo : W.npo) + (i - W.a0);
-    const int ne = COMPS == 3 ? W.nte : W.nbc;
-    int c = sl;
-    for (; c + (kSumBatch - 1) * kSumSlices < ne; c += kSumBatch * kSumSlices) {
-        double v[kSumBatch][COMPS];
-#pragma unroll
-        for (int u = 0; u < kSumBatch; ++u) {
-            const long long o = base + (long long)(c + u * kSumSlices) * W.n;
-#pragma unroll
-            for (int k = 0; k < COMPS; ++k) v[u][k] = part[k * B + o];
-        }
-#pragma unroll
-        for (int u = 0; u < kSumBatch; ++u)
-#pragma unroll
-            for (int k = 0; k < COMPS; ++k) s[k] += v[u][k];
-    }
-    for (; c < ne; c += kSumSlices) {
-        const long long o = base + (long long)c * W.n;
-#pragma unroll
-        for (int k = 0; k < COMPS; ++k) s[k] += part[k * B + o];
+    for (; e < e1; e += kBondBatch * kSumSlices) {
+        BondBatch b;
+        bonded_load_idx(idx, e, e1, b);
+        bonded_load(contrib, b);
+        bonded_add(e, e1, b, s);
     }
 }
 
