@@ -96,7 +96,7 @@ static int auto_pieces(long long lanes, long long work, long long min_work, doub
 static void isspa_free(isspa_model *m)
 {
     dfree(m->itype); dfree(m->atom_win); dfree(m->rmax); dfree(m->rmax2); dfree(m->vtot);
-    dfree(m->ge); dfree(m->f);
+    dfree(m->ge);
     dfree(m->pts); dfree(m->rec); dfree(m->g_out); dfree(m->E_out); dfree(m->E0_out);
     dfree(m->cnt_out); dfree(m->pbc_flag); dfree(m->wins); dfree(m->fblk); dfree(m->gblk);
     dfree(m->pblk); dfree(m->vblk); dfree(m->wblk);
@@ -118,7 +118,7 @@ static int isspa_tile(isspa_model *m)
             : (double)std::min(kMaxAutoWaves,
                                std::max(kMinAutoWaves, (long)(m->P / kPointsPerWave)));
     m->wins_h.assign(L.W, WinDesc{});
-    m->max_win_atoms = m->max_group_pts = 0;
+    m->max_win_atoms = m->max_group_pts = m->max_group_items = 0;
     m->max_fg = 1;
     long long F = 0, C = 0, V = 0;
     std::vector<std::pair<long long, int4>> fb, gb, pb, vb, wb;
@@ -143,6 +143,9 @@ static int isspa_tile(isspa_model *m)
         m->max_win_atoms = std::max(m->max_win_atoms, (int)n);
         const int group = force_group((int)n), shares = force_shares((int)n);
         m->max_group_pts = std::max(m->max_group_pts, (int)std::min(P, (long long)group * d.ppc));
+        m->max_group_items = std::max<long long>(
+            m->max_group_items,
+            d.splits * ((std::min(P, (long long)group * d.ppc) + 63) / 64 * 64));
         d.fents = (d.chunks + group - 1) / group;
         d.vents = (d.chunks + 3) / 4;
         d.fpo = F;
@@ -273,7 +276,9 @@ extern "C" int isspa_model_create_batch(const isspa_model_desc *d, const isspa_w
     }
     std::vector<float> fp;
     pad_table(f, T, d->n_f, fp);
-    std::vector<float2> ge((size_t)T * (d->n_g + 1), make_float2(0.0f, 0.0f));
+    const size_t nge = (size_t)T * (d->n_g + 1);
+    std::vector<float2> ge(nge + (fp.size() + 1) / 2, make_float2(0.0f, 0.0f));
+    std::memcpy(ge.data() + nge, fp.data(), fp.size() * sizeof(float));
     for (int t = 0; t < T; ++t)
         for (int b = 0; b < d->n_g; ++b)
             ge[(size_t)t * (d->n_g + 1) + b] =
@@ -290,7 +295,6 @@ extern "C" int isspa_model_create_batch(const isspa_model_desc *d, const isspa_w
     TRY(upload(&m->rmax2, r2.data(), T));
     TRY(upload(&m->vtot, vt.data(), T));
     TRY(upload(&m->ge, ge.data(), ge.size()));
-    TRY(upload(&m->f, fp.data(), fp.size()));
     TRY(dalloc(&m->pts, m->P));
     TRY(dalloc(&m->rec, (size_t)m->P * (kRecFloats + kAuxFloats)));  // records, then aux
     TRY(dalloc(&m->g_out, m->P));
@@ -301,7 +305,7 @@ extern "C" int isspa_model_create_batch(const isspa_model_desc *d, const isspa_w
     TRY(isspa_tile(m));
 #undef TRY
     TableView &tv = m->tv;
-    tv.ge = m->ge; tv.f = m->f;
+    tv.ge = m->ge; tv.f = reinterpret_cast<const float *>(m->ge + nge);
     tv.n_g = d->n_g; tv.n_f = d->n_f;
     tv.ld_g = d->n_g + 1; tv.ld_f = d->n_f + 1;
     tv.ntypes = d->n_types;
@@ -442,7 +446,7 @@ static int isspa_total(isspa_model *m, const float *xyzq4_d, float *f4_d, float 
 {
     const float4 *x = reinterpret_cast<const float4 *>(xyzq4_d);
     if (isspa_is_small(m)) {
-        HIPCHK(launch_window(window_args(m, x, step, step_d), m->max_win_atoms, m->max_group_pts, s));
+        HIPCHK(launch_window(window_args(m, x, step, step_d), m->max_group_pts, m->max_group_items, s));
     } else {
         CHK(isspa_field_pass(m, xyzq4_d, step, step_d, s));
         HIPCHK(launch_force(force_args(m, x), m->npblk, false, s));
@@ -1292,7 +1296,7 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
             w.nb = nonbond_args(e->nb, x4, nullptr, false);
             w.nb_blocks = e->nb->nblk_tot;
         }
-        HIPCHK(launch_window(w, m->max_win_atoms, m->max_group_pts, s));
+        HIPCHK(launch_window(w, m->max_group_pts, m->max_group_items, s));
     } else {
         PrologueArgs p{};
         p.bonded = bonded;

@@ -105,7 +105,7 @@ extern "C" int isspa_model_force_noalloc(isspa_model *m, const float *xyzq4_d, f
         WindowArgs wa = window_args(m, x, step, step_d);
         wa.pts = pts;
         wa.part = part_f;
-        HIPCHK(launch_window(wa, m->max_win_atoms, m->max_group_pts, s));
+        HIPCHK(launch_window(wa, m->max_group_pts, m->max_group_items, s));
     } else {
         HIPCHK(launch_mc_points(m->wins, m->atom_win, x, m->itype, m->rmax, m->rmax2, m->d.n_atoms,
                                 m->d.n_mc, m->d.seed, step, step_d, pts, s, m->lay.W, m->rmax_all,

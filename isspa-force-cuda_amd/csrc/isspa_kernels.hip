@@ -56,20 +56,19 @@ __host__ __device__ inline int diff_tab_floats(const TableView &t)
 // copy n floats into LDS with the whole block (n is block-uniform); eight
 // loads per thread are issued before their stores, so a small system's
 // kernel waits for the table once rather than once per 256 floats
-template <int NT = kBlock>
 __device__ __forceinline__ void stage_lds(float *dst, const float *__restrict__ src, int n)
 {
     constexpr int kU = 8;
-    for (int t0 = threadIdx.x; t0 < n; t0 += kU * NT) {
+    for (int t0 = threadIdx.x; t0 < n; t0 += kU * kBlock) {
         float v[kU];
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            const int t = t0 + u * NT;
+            const int t = t0 + u * kBlock;
             v[u] = t < n ? src[t] : 0.0f;
         }
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            const int t = t0 + u * NT;
+            const int t = t0 + u * kBlock;
             if (t < n) dst[t] = v[u];
         }
     }
@@ -829,24 +828,24 @@ __global__ __launch_bounds__(kBlock) void k_force(ForceArgs a)
 // lanes at once, and all field splits of 64 points run side by side.
 // Splits, FP32 tiles, shares and the order of every sum are those of the
 // separate launches, so the forces are the same bit for bit.
-// Whole step of 44 atoms, nMC = 100: 38.7 -> 31.1 us (prologue 6.1, field 6.5
-// and epilogue + force 10.0 us before, 17.5 us now); 22 atoms 36.1 -> 28.7 us.
+// Whole step of 44 atoms, nMC = 100, ten steps a graph: 34.5 us in separate
+// launches (prologue 6.1, field 6.5, epilogue + force 10.0 us), 22.2 us so.
 // The step's all-pairs, bonded and restraint blocks, which depend on the
 // coordinates alone, ride on the launch (work-items from 256 up leave).
 // ---------------------------------------------------------------------------
-constexpr int kWinThreads = 512;
-constexpr int kWinWaves = kWinThreads / kWave;
 constexpr int kWinMaxAtoms = 256;
 constexpr int kWinMaxPts = 256;
-// More blocks than this are throughput, not latency, and the separate
-// launches do that better: 339 blocks (22 atoms, nMC = 1,000) take 28.3
-// against 34.5 us, 303 (242 atoms, nMC = 100) 49.7 against 71.6 us, but 677
-// (44 atoms, nMC = 1,000) 50.5 against 47.5 us.
+// One round of two blocks a CU.  More blocks are throughput, not latency: a
+// step takes 29.0 us here against 37.5 in the separate launches with 474
+// blocks (44 atoms, nMC = 700), 51.1 against 55.3 with 454 (242 atoms, nMC =
+// 150), but 58.8 against 56.3 with 632 (64 umbrella windows) and 89.8 against
+// 86.4 with 908 (242 atoms, nMC = 300).
 constexpr int kWinMaxBlocks = 512;
 
 struct WindowLds {
     const float4 *atoms;
     const int *types;
+    const float *rmax, *rmax2;  // per atom
     const float2 *GE;
 };
 
@@ -860,11 +859,18 @@ __device__ __forceinline__ void window_field_span(const WindowArgs &a, const Win
         const int je = min(j1, jt + kFieldTile);
         float ax = 0.0f, ay = 0.0f, az = 0.0f;
         st.ex = st.ey = st.ez = 0.0f;
-#pragma unroll 2
-        for (int j = jt; j < je; ++j)
-            field_pair<PBC, false>(a.tab, a.e0, l.GE, nullptr, l.atoms[j],
-                                   [=]() { return l.types[j]; }, mi, p.x, p.y, p.z, p.w, ax, ay,
-                                   az, st);
+        // the next atom and its type are read while this pair is evaluated
+        float4 nx = l.atoms[jt];
+        int nt = l.types[jt];
+        for (int j = jt; j < je; ++j) {
+            const float4 x = nx;
+            const int t = nt;
+            const int jn = min(j + 1, je - 1);
+            nx = l.atoms[jn];
+            nt = l.types[jn];
+            field_pair<PBC, false>(a.tab, a.e0, l.GE, nullptr, x, [=]() { return t; }, mi, p.x,
+                                   p.y, p.z, p.w, ax, ay, az, st);
+        }
         fs.sx += (double)ax;
         fs.sy += (double)ay;
         fs.sz += (double)az;
@@ -875,16 +881,13 @@ __device__ __forceinline__ void window_field_span(const WindowArgs &a, const Win
 }
 
 // the points [m0, m0 + np) of window W into LDS and memory; D lanes a point
-// try D consecutive draws at a time, the first accepted one counts
+// (lt, of atom il) try D consecutive draws at a time, the first accepted one
+// counts
 __device__ __forceinline__ void window_points(const WindowArgs &a, const WinDesc &W, int m0, int np,
-                                              int lt, int sub, int D, const float4 *atoms,
-                                              const int *types, float4 *lrec, int *best)
+                                              int lt, int il, int sub, int D, uint32_t step,
+                                              const WindowLds &l, float4 *lrec, int *best)
 {
-    const uint32_t step = a.step_d ? *a.step_d : a.step;
     const bool mine = lt < np && sub < D;
-    const int il = mine ? (m0 + lt) / a.nmc : 0;
-    if (mine && sub == 0) best[lt] = kMcMaxAttempts;
-    __syncthreads();
     for (int base = 0;; base += D) {
         int c0 = 0, c1 = 0, c2 = 0;
         const int d = base + sub;
@@ -897,9 +900,8 @@ __device__ __forceinline__ void window_points(const WindowArgs &a, const WinDesc
         // the winner, or, after the last draw, the point at its atom
         const bool none = mine && last && sub == 0 && b == kMcMaxAttempts;
         if ((ok && b == d) || none) {
-            const int t = types[il];
-            const float4 p = none ? mc_place(atoms[il], a.rmax[t], a.rmax2[t], 0, 0, 0)
-                                  : mc_place(atoms[il], a.rmax[t], a.rmax2[t], c0, c1, c2);
+            const float4 p = none ? mc_place(l.atoms[il], l.rmax[il], l.rmax2[il], 0, 0, 0)
+                                  : mc_place(l.atoms[il], l.rmax[il], l.rmax2[il], c0, c1, c2);
             lrec[4 * lt] = p;
             a.pts[(long long)W.a0 * a.nmc + m0 + lt] = p;
         }
@@ -908,7 +910,9 @@ __device__ __forceinline__ void window_points(const WindowArgs &a, const WinDesc
     }
 }
 
-__global__ __launch_bounds__(kWinThreads, 4) void k_window(WindowArgs a)
+// NT: work-items of a block, a multiple of 512
+template <int NT>
+__global__ __launch_bounds__(NT, 4) void k_window(WindowArgs a)
 {
     extern __shared__ __align__(16) float lds_tab[];
     int b = blockIdx.x;
@@ -931,42 +935,63 @@ __global__ __launch_bounds__(kWinThreads, 4) void k_window(WindowArgs a)
                  a.us.com, true, reinterpret_cast<double (*)[kTermBlock]>(lds_tab));
         return;
     }
-    const int4 bt = a.blocks[b];
-    const WinDesc W = a.wins[bt.x];
     const int tid = threadIdx.x, lane = tid % kWave;
     const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int n = W.n, P = n * a.nmc;
-    const int span = force_group(n) * W.ppc;
-    const int m0 = min(P, bt.z * span), np = min(P, m0 + span) - m0;
-    // LDS: F table, atoms and types, point records (until they are written the
-    // points, in each record's first entry, and the draws' counters), then an
-    // area that holds the g and E tables and the splits' field sums, later the
-    // shares' force sums
-    const int nf = force_tab_floats(a.tab), nge = field_tab_floats(a.tab);
+    // LDS: g/E and F tables; atoms; point records (until they are written the
+    // points, in each record's first entry, and the draws' counters); then the
+    // splits' field sums, later the shares' force sums
     float4 *atoms = reinterpret_cast<float4 *>(lds_tab + a.off_atoms);
     int *types = reinterpret_cast<int *>(atoms + kWinMaxAtoms);
+    float *rmax = reinterpret_cast<float *>(types + kWinMaxAtoms), *rmax2 = rmax + kWinMaxAtoms;
     float4 *lrec = reinterpret_cast<float4 *>(lds_tab + a.off_pts);
     float4 *laux = lrec + 4 * a.cap_pts;
     int *best = reinterpret_cast<int *>(laux);
     float *area = lds_tab + a.off_x;
-    FieldXchg *xc = reinterpret_cast<FieldXchg *>(area + ((nge + 3) & ~3));
-    for (int i = tid; i < n; i += kWinThreads) {
-        atoms[i] = a.xyzq[W.a0 + i];
-        types[i] = a.itype[W.a0 + i];
-    }
-    stage_lds<kWinThreads>(lds_tab, a.tab.f, nf);
-    stage_lds<kWinThreads>(area, reinterpret_cast<const float *>(a.tab.ge), nge);
-    // (its barrier also publishes the staged data)
-    const bool pbc = needs_image<kWinThreads>(W, a.xyzq, a.rmax_all);
-    const MinImage mi = min_image_of(W.L, W.h);
-    // lt: the work-item's point, sub: its draw or field split, wave-uniform
+    FieldXchg *xc = reinterpret_cast<FieldXchg *>(area);
+    __shared__ int far_flag;
+    // The loads of the tables (which depend on nothing) are in flight while
+    // the block's window is looked up and its atoms are requested.
+    const int ntab = field_tab_floats(a.tab) + force_tab_floats(a.tab);
+    const float *tab = reinterpret_cast<const float *>(a.tab.ge);  // F follows
+    constexpr int kU = 6;
+    float tv[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) tv[u] = tab[min(tid + u * NT, ntab - 1)];
+    const int4 bt = a.blocks[b];
+    const WinDesc W = a.wins[bt.x];
+    const uint32_t step = a.step_d ? *a.step_d : a.step;
+    const int n = W.n, P = n * a.nmc;
+    const float4 x = a.xyzq[W.a0 + min(tid, n - 1)], x0 = a.xyzq[W.a0];
+    const int t = a.itype[W.a0 + min(tid, n - 1)];
+    const float rm = a.rmax[t], rm2 = a.rmax2[t];
+    const int span = force_group(n) * W.ppc;
+    const int m0 = min(P, bt.z * span), np = min(P, m0 + span) - m0;
+    // lt: the work-item's point, of atom il; sub: its draw or field split, wave-uniform
     const int npr = (np + kWave - 1) & ~(kWave - 1);
-    const int D = kWinThreads / npr;
+    const int D = NT / npr;
     const int sub = __builtin_amdgcn_readfirstlane(tid / npr);
     const int lt = tid - sub * npr;
-    window_points(a, W, m0, np, lt, sub, D, atoms, types, lrec, best);
+    const int il = lt < np && sub < D ? (m0 + lt) / a.nmc : 0;
+    if (tid == 0) far_flag = 0;
+    if (tid < npr) best[tid] = kMcMaxAttempts;
+#pragma unroll
+    for (int u = 0; u < kU; ++u)
+        if (tid + u * NT < ntab) lds_tab[tid + u * NT] = tv[u];
+    for (int k = tid + kU * NT; k < ntab; k += NT) lds_tab[k] = tab[k];
+    if (tid < n) {
+        atoms[tid] = x;
+        types[tid] = t;
+        rmax[tid] = rm;
+        rmax2[tid] = rm2;
+    }
+    __syncthreads();
+    if (atoms_far(W, x, x0, a.rmax_all)) far_flag = 1;
+    const WindowLds l{atoms, types, rmax, rmax2, reinterpret_cast<const float2 *>(lds_tab)};
+    // (its barriers also publish the flag)
+    window_points(a, W, m0, np, lt, il, sub, D, step, l, lrec, best);
+    const bool pbc = far_flag != 0;
+    const MinImage mi = min_image_of(W.L, W.h);
     // field: D splits side by side, added in order, groups of W.fg at a time
-    const WindowLds l{atoms, types, reinterpret_cast<const float2 *>(area)};
     const float4 p = lt < np ? lrec[4 * lt] : make_float4(0.0f, 0.0f, 0.0f, -1.0f);
     double g = 1.0, s0[3] = {0, 0, 0}, ei[3] = {0, 0, 0};
     double gg = 1.0, gs[3] = {0, 0, 0}, ge[3] = {0, 0, 0};
@@ -1003,7 +1028,7 @@ __global__ __launch_bounds__(kWinThreads, 4) void k_window(WindowArgs a)
                     for (int c = 0; c < 3; ++c) { s0[c] += gs[c]; ei[c] += ge[c]; }
                 }
             }
-        __syncthreads();
+        if (sp + D < W.splits) __syncthreads();
     }
     if (tid < np) {
         PointRecord pr;
@@ -1012,34 +1037,48 @@ __global__ __launch_bounds__(kWinThreads, 4) void k_window(WindowArgs a)
         laux[tid] = pr.aux;
     }
     __syncthreads();
-    // force: units of 64 receivers and one share, over the eight waves
+    // force: up to 128 receivers, a wave for each 64 and share; above, a wave
+    // for each 64 and pair of shares.  The wave of the first share keeps its
+    // sums and adds the others' from LDS, in share order.
     ForceArgs fa{};
     fa.tab = a.tab;
     fa.part = a.part;
     const int nrw = (n + kWave - 1) / kWave;
-    double *sh = reinterpret_cast<double *>(area);  // [share][receiver][6]
+    const int per = nrw <= 2 ? 1 : 2;  // shares of a wave
+    const int rg = wv * per / 4, q0 = wv * per % 4;
+    const int ir = rg * kWave + lane;  // the lane's receiver
+    double *sh = reinterpret_cast<double *>(area);  // [share - per][receiver][6]
     const DiffFParams fp{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int u = wv; u < 4 * nrw; u += kWinWaves) {
-        const int share = u & 3, il = (u >> 2) * kWave + lane;
-        int ms, me;
-        share_range(W, P, bt.z, share, ms, me);
-        const float4 xi = atoms[min(il, n - 1)];
-        const int ti = types[min(il, n - 1)];
-        const float R2 = il < n ? a.rmax2[ti] : -1.0f;
-        ForceAcc acc{0, 0, 0, 0, 0, 0, 0, 0, 0};
-        force_chunk<false, false, false>(fa, lrec, laux, ms - m0, me - m0, W, pbc, xi, R2,
-                                         lds_tab + ti * a.tab.ld_f, fp, acc);
-        double *d = sh + 6 * ((size_t)share * nrw * kWave + il);
-        d[0] = acc.ex; d[1] = acc.ey; d[2] = acc.ez;
-        d[3] = acc.lx; d[4] = acc.ly; d[5] = acc.lz;
+    ForceAcc own{0, 0, 0, 0, 0, 0, 0, 0, 0};
+    if (rg < nrw) {
+        const int ic = min(ir, n - 1);
+        const float4 xi = atoms[ic];
+        const float R2 = ir < n ? rmax2[ic] : -1.0f;
+        const float *F = lds_tab + field_tab_floats(a.tab) + types[ic] * a.tab.ld_f;
+        for (int q = q0; q < q0 + per; ++q) {
+            int ms, me;
+            share_range(W, P, bt.z, q, ms, me);
+            ForceAcc acc{0, 0, 0, 0, 0, 0, 0, 0, 0};
+            force_chunk<false, false, false>(fa, lrec, laux, ms - m0, me - m0, W, pbc, xi, R2, F, fp,
+                                             acc);
+            if (q0 == 0) {
+                own.ex += acc.ex; own.ey += acc.ey; own.ez += acc.ez;
+                own.lx += acc.lx; own.ly += acc.ly; own.lz += acc.lz;
+            } else {
+                double *d = sh + 6 * ((size_t)(q - per) * nrw * kWave + ir);
+                d[0] = acc.ex; d[1] = acc.ey; d[2] = acc.ez;
+                d[3] = acc.lx; d[4] = acc.ly; d[5] = acc.lz;
+            }
+        }
     }
     __syncthreads();
-    if (tid >= n) return;
-    double f[6];
-    for (int k = 0; k < 6; ++k) f[k] = sh[6 * tid + k];
-    for (int q = 1; q < 4; ++q)
-        for (int k = 0; k < 6; ++k) f[k] += sh[6 * ((size_t)q * nrw * kWave + tid) + k];
-    write_force_entry<false>(fa, W, bt.z, tid, ForceAcc{f[0], f[1], f[2], f[3], f[4], f[5], 0, 0, 0});
+    if (q0 != 0 || ir >= n) return;
+    for (int q = per; q < 4; ++q) {
+        const double *d = sh + 6 * ((size_t)(q - per) * nrw * kWave + ir);
+        own.ex += d[0]; own.ey += d[1]; own.ez += d[2];
+        own.lx += d[3]; own.ly += d[4]; own.lz += d[5];
+    }
+    write_force_entry<false>(fa, W, bt.z, ir, own);
 }
 
 // F_i = -q_i vtot_i S_e - vtot_i S_lj over the chunk partials, summed in the
@@ -1137,22 +1176,18 @@ hipError_t launch_epilogue(const EpilogueArgs &a, hipStream_t s)
     return hipGetLastError();
 }
 
-// LDS of k_window in floats: F table, atoms, points; then the shared area
-static int window_lds(const TableView &t, int max_atoms, int max_points, WindowArgs *a)
+// LDS of k_window in floats: tables, atoms, point records, then the splits' or
+// the shares' sums
+static int window_lds(const TableView &t, int nt, int max_points, WindowArgs &a)
 {
-    const int off_atoms = (force_tab_floats(t) + 3) & ~3;
-    const int off_pts = off_atoms + 5 * kWinMaxAtoms;
-    const int cap_pts = (max_points + kWave - 1) / kWave * kWave;
-    const int off_x = off_pts + (kRecFloats + kAuxFloats) * cap_pts;
-    const int nxc = ((field_tab_floats(t) + 3) & ~3) + kWinThreads * (int)(sizeof(FieldXchg) / 4);
-    const int nsh = 4 * 6 * 2 * ((max_atoms + kWave - 1) / kWave) * kWave;
-    if (a) {
-        a->off_atoms = off_atoms;
-        a->off_pts = off_pts;
-        a->off_x = off_x;
-        a->cap_pts = cap_pts;
-    }
-    return off_x + std::max(nxc, nsh);
+    const int tab = (field_tab_floats(t) + force_tab_floats(t) + 3) & ~3;
+    a.off_atoms = tab;
+    a.off_pts = a.off_atoms + 7 * kWinMaxAtoms;
+    a.cap_pts = (max_points + kWave - 1) / kWave * kWave;
+    a.off_x = a.off_pts + (kRecFloats + kAuxFloats) * a.cap_pts;
+    const int nxc = nt * (int)(sizeof(FieldXchg) / sizeof(float));
+    const int nsh = 2 * 6 * std::max(3 * 2 * kWave, 2 * 4 * kWave);
+    return a.off_x + std::max(nxc, nsh);
 }
 
 bool window_fits(const TableView &t, int max_atoms, int max_points, int nblocks)
@@ -1161,16 +1196,24 @@ bool window_fits(const TableView &t, int max_atoms, int max_points, int nblocks)
            field_tab_floats(t) <= kTabLdsFloats && force_tab_floats(t) <= kTabLdsFloats;
 }
 
-hipError_t launch_window(const WindowArgs &a0, int max_atoms, int max_points, hipStream_t s)
+hipError_t launch_window(const WindowArgs &a0, int max_points, int max_items, hipStream_t s)
 {
     WindowArgs a = a0;
-    size_t lds = sizeof(float) * window_lds(a.tab, max_atoms, max_points, &a);
+    // sixteen waves where a pass of eight holds less than a group's field
+    // splits and a CU has a block to itself (242 atoms, nMC = 20, 72 blocks: a
+    // step takes 36.7 against 41.2 us; but nMC = 100, 303 blocks, 63.5
+    // against 49.4 us)
+    const int nt = max_items > 512 && a.nblocks <= 256 ? 1024 : 512;
+    size_t lds = sizeof(float) * window_lds(a.tab, nt, max_points, a);
     if (a.nb_blocks) lds = std::max(lds, nonbond_lds_bytes(a.nb.T, false));
     const long terms = (long)a.bonded.nb + a.bonded.na + a.bonded.nd;
     a.bonded_blocks = a.bonded.contrib ? blocks_for(terms) : 0;
     const int grid = a.nblocks + a.nb_blocks + a.bonded_blocks + a.us.nres;
     if (grid == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_window, dim3(grid), dim3(kWinThreads), lds, s, a);
+    if (nt == 512)
+        hipLaunchKernelGGL(k_window<512>, dim3(grid), dim3(nt), lds, s, a);
+    else
+        hipLaunchKernelGGL(k_window<1024>, dim3(grid), dim3(nt), lds, s, a);
     return hipGetLastError();
 }
 

@@ -48,7 +48,7 @@ inline int field_group(int splits) { return splits % 4 == 0 ? 4 : (splits % 2 ==
 // 16-byte read (E rows beyond the g table are never read).
 struct TableView {
     const float2 *ge;
-    const float *f;
+    const float *f;  // directly behind ge
     int n_g, n_f;    // logical rows
     int ld_g, ld_f;  // padded rows per type
     int ntypes;
@@ -295,9 +295,10 @@ hipError_t launch_mc_points(const WinDesc *wins, const int *atom_win, const floa
 hipError_t launch_field(const FieldArgs &a, int nblocks, hipStream_t s);
 hipError_t launch_epilogue(const EpilogueArgs &a, hipStream_t s);
 // k_window: whether a model's windows, chunk groups and tables fit it, and the
-// launch (max_atoms, max_points: of the largest window and chunk group)
+// launch (max_atoms, max_points: of the largest window and chunk group;
+// max_items: the most (point, field split) pairs of a group)
 bool window_fits(const TableView &t, int max_atoms, int max_points, int nblocks);
-hipError_t launch_window(const WindowArgs &a, int max_atoms, int max_points, hipStream_t s);
+hipError_t launch_window(const WindowArgs &a, int max_points, int max_items, hipStream_t s);
 hipError_t launch_force(const ForceArgs &a, int nblocks, bool split, hipStream_t s);
 hipError_t launch_force_reduce(const ReduceArgs &a, bool split, hipStream_t s);
 

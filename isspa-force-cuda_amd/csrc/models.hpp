@@ -38,8 +38,7 @@ struct isspa_model {
     float rmax_all = 0.f;
     int *itype = nullptr, *atom_win = nullptr;
     float *rmax = nullptr, *rmax2 = nullptr, *vtot = nullptr;
-    float2 *ge = nullptr;
-    float *f = nullptr;
+    float2 *ge = nullptr;  // {g, E} table, then the F table
     float4 *pts = nullptr;
     float *rec = nullptr;  // [P][kRecFloats] records, then [P] float4 aux
     double *g_out = nullptr, *E_out = nullptr, *E0_out = nullptr;
@@ -59,7 +58,8 @@ struct isspa_model {
     int4 *wblk = nullptr;  // k_window: {w, -, chunk group, -}
     int nwblk = 0;
     int max_fg = 1;  // the largest splits-per-field-block of the windows
-    int max_win_atoms = 0, max_group_pts = 0;  // over the windows, for the fused force launch
+    // over the windows, for the small-window launch
+    int max_win_atoms = 0, max_group_pts = 0, max_group_items = 0;
     double *part_g = nullptr;
     int *part_cnt = nullptr;
     double *part_s0 = nullptr, *part_ein = nullptr;

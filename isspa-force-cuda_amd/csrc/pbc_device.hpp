@@ -44,22 +44,26 @@ __device__ inline void pbc_flag_block(const WinDesc &W, const float4 *__restrict
     }
 }
 
-// The same decision taken by a block's first NT work-items for its own use,
-// with two barriers and no memory: false only if every atom lies within
-// (L/2 - rmax - margin) / 2 of the first one on every axis.  It may say true
-// where the flag says 0; the image loop then shifts nothing.
+// The same decision taken by a block for its own use, atom by atom: none of
+// the window's atoms is far from the first one, x0, if every one lies within
+// (L/2 - rmax - margin) / 2 of it on every axis.  It may say far where the
+// flag says 0; the image loop then shifts nothing.
+__device__ __forceinline__ bool atoms_far(const WinDesc &W, float4 x, float4 x0, float rmax_all)
+{
+    const float lim = 0.5f * (W.h - rmax_all - 1.0e-2f);
+    // NaN -> far
+    return !(fabsf(x.x - x0.x) < lim && fabsf(x.y - x0.y) < lim && fabsf(x.z - x0.z) < lim);
+}
+
+// for the whole window, by a block's first NT work-items (two barriers)
 template <int NT>
 __device__ __forceinline__ bool needs_image(const WinDesc &W, const float4 *__restrict__ xyzq,
                                             float rmax_all)
 {
-    const float lim = 0.5f * (W.h - rmax_all - 1.0e-2f);
-    const float4 o = xyzq[W.a0];
-    int far = 0;
-    for (int i = threadIdx.x; i < W.n; i += NT) {
-        const float4 x = xyzq[W.a0 + i];
-        // NaN -> far
-        far |= !(fabsf(x.x - o.x) < lim && fabsf(x.y - o.y) < lim && fabsf(x.z - o.z) < lim);
-    }
+    const float4 x0 = xyzq[W.a0];
+    bool far = false;
+    for (int i = threadIdx.x; i < W.n; i += NT)
+        far = far || atoms_far(W, xyzq[W.a0 + i], x0, rmax_all);
     __shared__ int need;
     if (threadIdx.x == 0) need = 0;
     __syncthreads();

@@ -77,6 +77,15 @@ def test_groups_and_splits(n, n_mc, tiling):
     _check(_atoms(n, n_mc), tiling)
 
 
+@pytest.mark.parametrize("n,n_mc,tiling", [
+    (64, 8, (8, 8)), (57, 9, (1, 57)), (242, 20, (4, 22)), (242, 19, (13, 242)), (130, 1, (9, 61))])
+def test_sixteen_waves(n, n_mc, tiling):
+    """Field items of a group on both sides of a pass of eight waves (512): the
+    block has sixteen above it, with receiver groups of one wave, a share pair
+    and more units than waves."""
+    _check(_atoms(n, n_mc), tiling)
+
+
 @pytest.mark.parametrize("pairs,small,big", [(3, 2, 1), (0, 1, 2), (5, 0, 0)])
 def test_batch_engine(pairs, small, big):
     """A batch that takes the launch: engine steps equal graph replays, and its
