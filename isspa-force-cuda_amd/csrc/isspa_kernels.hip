@@ -182,18 +182,21 @@ template <bool PBC, bool AN>
 __device__ __forceinline__ void field_tile(const FieldArgs &a, const float2 *GE,
                                            const DiffType *dtypes, int j0, int j1,
                                            const MinImage &mi, float px, float py, float pz,
-                                           float R2, float &ax, float &ay, float &az,
-                                           FieldRare &st)
+                                           float R2, const Progress &pr, float &ax, float &ay,
+                                           float &az, FieldRare &st)
 {
     // the tile's atoms by a pointer that advances 16 bytes an atom (an index
     // recomputed from j costs the scalar unit a sign extension and a shift
     // before every load)
     const auto *xq = read_only(reinterpret_cast<const float *>(a.xyzq + j0));
     const auto *ity = read_only(a.itype);
+    for (int j = j0; j < j1;) {
+        const int stop = j0 + pr.rank(j - j0, j1 - j0);
 #pragma unroll 2
-    for (int j = j0; j < j1; ++j, xq += 4)  // wave-uniform
-        field_pair<PBC, AN>(a.tab, a.e0, GE, dtypes, make_float4(xq[0], xq[1], xq[2], xq[3]),
-                            [=]() { return ity[j]; }, mi, px, py, pz, R2, ax, ay, az, st);
+        for (; j < stop; ++j, xq += 4)  // wave-uniform
+            field_pair<PBC, AN>(a.tab, a.e0, GE, dtypes, make_float4(xq[0], xq[1], xq[2], xq[3]),
+                                [=]() { return ity[j]; }, mi, px, py, pz, R2, ax, ay, az, st);
+    }
 }
 
 // a point's sums over atoms [j0, j1) of its split
@@ -209,14 +212,18 @@ __device__ __forceinline__ void field_span(const FieldArgs &a, const float2 *GE,
 {
     FieldRare &st = fs.st;
     const MinImage mi = min_image_of(W.L, W.h);
+    Progress pr(a.ranked_from, j1 - j0);
     for (int jt = j0; jt < j1; jt += kFieldTile) {
         const int je = min(j1, jt + kFieldTile);
+        pr.done = jt - j0;
         float ax = 0.0f, ay = 0.0f, az = 0.0f;
         st.ex = st.ey = st.ez = 0.0f;
         if (pbc)
-            field_tile<true, AN>(a, GE, dtypes, jt, je, mi, p.x, p.y, p.z, p.w, ax, ay, az, st);
+            field_tile<true, AN>(a, GE, dtypes, jt, je, mi, p.x, p.y, p.z, p.w, pr, ax, ay, az,
+                                 st);
         else
-            field_tile<false, AN>(a, GE, dtypes, jt, je, mi, p.x, p.y, p.z, p.w, ax, ay, az, st);
+            field_tile<false, AN>(a, GE, dtypes, jt, je, mi, p.x, p.y, p.z, p.w, pr, ax, ay, az,
+                                  st);
         fs.sx += (double)ax;
         fs.sy += (double)ay;
         fs.sz += (double)az;
@@ -555,11 +562,12 @@ struct TileSums {
 };
 
 // Rec: const float4 * (records in LDS) or ScalarRecords (in memory)
-template <bool PBC, bool SPLIT, bool AN, typename Rec>
+template <bool PBC, bool SPLIT, bool AN, bool RANK, typename Rec>
 __device__ __forceinline__ void force_tile(const ForceArgs &a, Rec rec, Rec aux, int m0, int m1,
                                            const MinImage &mi, float xi, float yi, float zi,
                                            float R2, const float *Ftab,
-                                           const DiffFParams &fp, TileSums &ts, ForceAcc &acc)
+                                           const DiffFParams &fp, const Progress &pr, TileSums &ts,
+                                           ForceAcc &acc)
 {
     float &sx = ts.sx, &sy = ts.sy, &sz = ts.sz;
     // the next point's record (wave-uniform) is fetched while this one is
@@ -571,86 +579,89 @@ __device__ __forceinline__ void force_tile(const ForceArgs &a, Rec rec, Rec aux,
     // a sign extension and shifts before every load)
     Rec nr = rec + 4 * m0, nx = aux + m0;
     float4 n0 = nr[0], n1 = nr[1], n2 = nr[2], n3 = nr[3], na = nx[0];
+    for (int m = m0; m < m1;) {
+        const int stop = RANK ? pr.rank(m, m1) : m1;
 #pragma unroll 2
-    for (int m = m0; m < m1; ++m) {
-        const float4 q0 = n0, q1 = n1, q2 = n2, q3 = n3, c4 = na;
-        if (m + 1 < m1) {
-            nr = nr + 4;
-            nx = nx + 1;
-        }
-        n0 = nr[0];
-        n1 = nr[1];
-        n2 = nr[2];
-        n3 = nr[3];
-        na = nx[0];
-        const float Ex = q0.w, Ey = q1.x, Ez = q1.y;
-        const float Vx = q1.z, Vy = q1.w, Vz = q2.x;
-        const float Dx = q2.y, Dy = q2.z, Dz = q2.w;
-        const float A2 = q3.x, A2x3 = q3.y, A3 = q3.z, w = q3.w;
-        float rx = q0.x - xi, ry = q0.y - yi, rz = q0.z - zi;
-        if (PBC) {
-            rx = min_image1(rx, mi);
-            ry = min_image1(ry, mi);
-            rz = min_image1(rz, mi);
-        }
-        const float d2 = dist2_f32(rx, ry, rz);
-        const float rinv = rsqrt_f32(d2);
-        const float e = __builtin_fmaf(Ez, rz, __builtin_fmaf(Ey, ry, Ex * rx));
-        const float rinv2 = rinv * rinv;
-        const float t = e * rinv2;
-        const float u2 = e * t;
-        const float P2 = __builtin_fmaf(7.5f, u2, -1.5f);
-        const float P3p = __builtin_fmaf(17.5f, u2, -7.5f);
-        const float rinv3 = rinv2 * rinv;
-        const float rinv5 = rinv3 * rinv2;
-        const float k = __builtin_fmaf(A2x3, e, A3 * P2) * rinv5;
-        const bool in = d2 <= R2;
-        if (!SPLIT) {
-            const float dr = __builtin_fmaf(Dz, rz, __builtin_fmaf(Dy, ry, Dx * rx));
-            const float alpha = __builtin_fmaf(A2, P2, __builtin_fmaf(A3, P3p * t, dr)) * rinv5;
-            sx = __builtin_fmaf(alpha, rx, sx);
-            sy = __builtin_fmaf(alpha, ry, sy);
-            sz = __builtin_fmaf(alpha, rz, sz);
-            sx = __builtin_fmaf(-rinv3, Vx, sx);
-            sy = __builtin_fmaf(-rinv3, Vy, sy);
-            sz = __builtin_fmaf(-rinv3, Vz, sz);
-            sx = __builtin_fmaf(-k, Ex, sx);
-            sy = __builtin_fmaf(-k, Ey, sy);
-            sz = __builtin_fmaf(-k, Ez, sz);
-        } else {
-            // polarisation alone: alpha_p r - (d^-3 A1 + k) Ehat, alpha_p
-            // being alpha without the E0c.r part
-            const float A1 = c4.w;
-            const float ap =
-                __builtin_fmaf(A2, P2, __builtin_fmaf(A3, P3p * t, (3.0f * A1) * e)) * rinv5;
-            const float bp = __builtin_fmaf(rinv3, A1, k);
-            sx = __builtin_fmaf(ap, rx, __builtin_fmaf(-bp, Ex, sx));
-            sy = __builtin_fmaf(ap, ry, __builtin_fmaf(-bp, Ey, sy));
-            sz = __builtin_fmaf(ap, rz, __builtin_fmaf(-bp, Ez, sz));
-            if (!in) {
-                const float3 c = cdd_term(c4, rx, ry, rz, rinv3, rinv5);
-                acc.cx += (double)c.x;
-                acc.cy += (double)c.y;
-                acc.cz += (double)c.z;
+        for (; m < stop; ++m) {
+            const float4 q0 = n0, q1 = n1, q2 = n2, q3 = n3, c4 = na;
+            if (m + 1 < m1) {
+                nr = nr + 4;
+                nx = nx + 1;
             }
-        }
-        if (in) {
-            float fs;
-            if (AN) {
-                fs = diff_F(fp, d2 * rinv, rinv) * w;
-            } else {
-                fs = table_force(a.tab, Ftab, d2, rinv) * w;
+            n0 = nr[0];
+            n1 = nr[1];
+            n2 = nr[2];
+            n3 = nr[3];
+            na = nx[0];
+            const float Ex = q0.w, Ey = q1.x, Ez = q1.y;
+            const float Vx = q1.z, Vy = q1.w, Vz = q2.x;
+            const float Dx = q2.y, Dy = q2.z, Dz = q2.w;
+            const float A2 = q3.x, A2x3 = q3.y, A3 = q3.z, w = q3.w;
+            float rx = q0.x - xi, ry = q0.y - yi, rz = q0.z - zi;
+            if (PBC) {
+                rx = min_image1(rx, mi);
+                ry = min_image1(ry, mi);
+                rz = min_image1(rz, mi);
             }
-            const float fl = fs * rinv;
-            ts.lx = __builtin_fmaf(fl, rx, ts.lx);
-            ts.ly = __builtin_fmaf(fl, ry, ts.ly);
-            ts.lz = __builtin_fmaf(fl, rz, ts.lz);
+            const float d2 = dist2_f32(rx, ry, rz);
+            const float rinv = rsqrt_f32(d2);
+            const float e = __builtin_fmaf(Ez, rz, __builtin_fmaf(Ey, ry, Ex * rx));
+            const float rinv2 = rinv * rinv;
+            const float t = e * rinv2;
+            const float u2 = e * t;
+            const float P2 = __builtin_fmaf(7.5f, u2, -1.5f);
+            const float P3p = __builtin_fmaf(17.5f, u2, -7.5f);
+            const float rinv3 = rinv2 * rinv;
+            const float rinv5 = rinv3 * rinv2;
+            const float k = __builtin_fmaf(A2x3, e, A3 * P2) * rinv5;
+            const bool in = d2 <= R2;
             if (!SPLIT) {
-                // remove the CDD part taken in the main path
-                const float3 c = cdd_term(c4, rx, ry, rz, rinv3, rinv5);
-                sx -= c.x;
-                sy -= c.y;
-                sz -= c.z;
+                const float dr = __builtin_fmaf(Dz, rz, __builtin_fmaf(Dy, ry, Dx * rx));
+                const float alpha = __builtin_fmaf(A2, P2, __builtin_fmaf(A3, P3p * t, dr)) * rinv5;
+                sx = __builtin_fmaf(alpha, rx, sx);
+                sy = __builtin_fmaf(alpha, ry, sy);
+                sz = __builtin_fmaf(alpha, rz, sz);
+                sx = __builtin_fmaf(-rinv3, Vx, sx);
+                sy = __builtin_fmaf(-rinv3, Vy, sy);
+                sz = __builtin_fmaf(-rinv3, Vz, sz);
+                sx = __builtin_fmaf(-k, Ex, sx);
+                sy = __builtin_fmaf(-k, Ey, sy);
+                sz = __builtin_fmaf(-k, Ez, sz);
+            } else {
+                // polarisation alone: alpha_p r - (d^-3 A1 + k) Ehat, alpha_p
+                // being alpha without the E0c.r part
+                const float A1 = c4.w;
+                const float ap =
+                    __builtin_fmaf(A2, P2, __builtin_fmaf(A3, P3p * t, (3.0f * A1) * e)) * rinv5;
+                const float bp = __builtin_fmaf(rinv3, A1, k);
+                sx = __builtin_fmaf(ap, rx, __builtin_fmaf(-bp, Ex, sx));
+                sy = __builtin_fmaf(ap, ry, __builtin_fmaf(-bp, Ey, sy));
+                sz = __builtin_fmaf(ap, rz, __builtin_fmaf(-bp, Ez, sz));
+                if (!in) {
+                    const float3 c = cdd_term(c4, rx, ry, rz, rinv3, rinv5);
+                    acc.cx += (double)c.x;
+                    acc.cy += (double)c.y;
+                    acc.cz += (double)c.z;
+                }
+            }
+            if (in) {
+                float fs;
+                if (AN) {
+                    fs = diff_F(fp, d2 * rinv, rinv) * w;
+                } else {
+                    fs = table_force(a.tab, Ftab, d2, rinv) * w;
+                }
+                const float fl = fs * rinv;
+                ts.lx = __builtin_fmaf(fl, rx, ts.lx);
+                ts.ly = __builtin_fmaf(fl, ry, ts.ly);
+                ts.lz = __builtin_fmaf(fl, rz, ts.lz);
+                if (!SPLIT) {
+                    // remove the CDD part taken in the main path
+                    const float3 c = cdd_term(c4, rx, ry, rz, rinv3, rinv5);
+                    sx -= c.x;
+                    sy -= c.y;
+                    sz -= c.z;
+                }
             }
         }
     }
@@ -691,19 +702,21 @@ __device__ __forceinline__ void force_chunk(const ForceArgs &a, const float4 *__
                                             ForceAcc &acc)
 {
     const MinImage mi = min_image_of(W.L, W.h);
+    Progress pr(AHEAD ? a.ranked_from : kUnranked, m1 - m0);
     for (int mt = m0; mt < m1; mt += kForceTile) {
         const int me = min(m1, mt + kForceTile);
+        pr.done = mt - m0;
         TileLines next;
         if (AHEAD) request_tile(rec, aux, me, m1, next);
         TileSums ts{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
         // tile-local point indices from the tile's first record
         auto tile = [&](auto r, auto x) {
             if (pbc)
-                force_tile<true, SPLIT, AN>(a, r, x, 0, me - mt, mi, xi.x, xi.y, xi.z, R2, Ftab, fp,
-                                            ts, acc);
+                force_tile<true, SPLIT, AN, AHEAD>(a, r, x, 0, me - mt, mi, xi.x, xi.y, xi.z, R2,
+                                                   Ftab, fp, pr, ts, acc);
             else
-                force_tile<false, SPLIT, AN>(a, r, x, 0, me - mt, mi, xi.x, xi.y, xi.z, R2, Ftab,
-                                             fp, ts, acc);
+                force_tile<false, SPLIT, AN, AHEAD>(a, r, x, 0, me - mt, mi, xi.x, xi.y, xi.z, R2,
+                                                    Ftab, fp, pr, ts, acc);
         };
         if constexpr (AHEAD)
             tile(ScalarRecords{read_only(reinterpret_cast<const float *>(rec + 4 * mt))},
@@ -1143,6 +1156,7 @@ hipError_t launch_field(const FieldArgs &a0, int nblocks, hipStream_t s)
 {
     FieldArgs a = a0;
     a.nfield = nblocks;
+    a.ranked_from = ranked_from(nblocks);
     if (a.dtypes) {
         if (nblocks == 0) return hipSuccess;
         const int nt = diff_tab_floats(a.tab);
@@ -1225,6 +1239,7 @@ hipError_t launch_force(const ForceArgs &a, int nblocks, bool split, hipStream_t
     ForceArgs b = a;
     const int nt = force_tab_floats(a.tab);
     b.red_off = (!a.dtypes && nt <= kTabLdsFloats) ? (nt + 3) & ~3 : 0;
+    b.ranked_from = ranked_from(nblocks);
     const size_t lds = (size_t)(b.red_off + 2 * force_share_doubles(split)) * sizeof(float);
     const dim3 g(nblocks), t(kBlock);
     switch ((a.dtypes ? 2 : 0) + (split ? 1 : 0)) {

@@ -123,6 +123,7 @@ struct FieldArgs {
     // (tables only, nb_blocks = 0: none); nfield is set by the launcher
     NonbondArgs nb;
     int nb_blocks, nfield;
+    int ranked_from;  // blocks from here on rank their waves by progress (set at launch)
     int max_fg;  // the largest W.fg of the launch (its LDS holds the split exchange if > 1)
 };
 
@@ -162,6 +163,68 @@ struct ForceArgs {
     long long C;
     int xcd_runs;         // 1: each XCD takes a contiguous run of the table (equal work items)
     int red_off;          // float offset of the share-sum area in the dynamic LDS (set at launch)
+    int ranked_from;      // blocks from here on rank their waves by progress (set at launch)
+};
+
+// The first block of a launch of nb whose waves rank themselves by progress
+// (Progress, device_common.hpp); the blocks before it have the top priority.
+//   nb <= 512:   none; with one or two waves a SIMD there is little to even
+//                out (field of 550 atoms, 430 blocks: 9.8 us, ranked 10.1).
+//   nb <= 1536:  all; they run at once (6 to 7 blocks fit a CU).
+//   above:       the last 1,280, 5 a CU: those before must leave in turn, so
+//                that the rest find room early.  Force pass of 4,510 atoms
+//                (2,272 blocks): 195 us unranked, 175 with the last 1,280, 183
+//                with 1,536, 198 with 1,664 and 199 with 2,048; 187 with 768.
+constexpr int kUnranked = 0x7fffffff;
+constexpr int kRankMin = 512, kRankAll = 1536, kRankLast = 1280;
+inline int ranked_from(int nb)
+{
+    return nb <= kRankMin ? kUnranked : (nb <= kRankAll ? 0 : nb - kRankLast);
+}
+
+// A wave's issue priority by its progress.  The arbiter serves the oldest of a
+// SIMD's waves first, so of four that start together the first is done at half
+// the time of the last, which ends up alone, at a third of the SIMD's rate.
+// Here a wave with three quarters of its work to go outranks one with two:
+// they stay within a quarter of each other and end together.
+// Against the arbiter alone: force pass of 1,100 atoms (nMC = 20) 37.5 ->
+// 32.7 us, of 2,200 (nMC = 10) 69 -> 59, of 6,600 359 -> 335, of 19,998 (nMC =
+// 20) 5,420 -> 5,320 us; field pass of 1,100 atoms 22.9 -> 22.3, of 2,200 36.4
+// -> 32.3, of 6,600 166 -> 153, of 19,998 2,268 -> 2,265 us.  (Looking at the
+// rank every 16 records instead of at the quarters: field of 19,998 atoms
+// 2,335 us.)
+struct Progress {
+    int done = 0;     // work before the tile
+    int quarter = 0;  // of the wave's work, rounded up; 0: not ranked
+    __device__ __forceinline__ Progress(int from, int work)
+    {
+        if (from == kUnranked) return;
+        if ((int)blockIdx.x < from)
+            __builtin_amdgcn_s_setprio(3);
+        else
+            quarter = (work + 3) / 4;
+    }
+    // ranks the wave at place m of the tile; returns where the rank changes
+    // next, at most m1
+    __device__ __forceinline__ int rank(int m, int m1) const
+    {
+        if (quarter == 0) return m1;
+        const int x = done + m;
+        int next = quarter;
+        if (x < quarter) {
+            __builtin_amdgcn_s_setprio(3);
+        } else if (x < 2 * quarter) {
+            __builtin_amdgcn_s_setprio(2);
+            next = 2 * quarter;
+        } else if (x < 3 * quarter) {
+            __builtin_amdgcn_s_setprio(1);
+            next = 3 * quarter;
+        } else {
+            __builtin_amdgcn_s_setprio(0);
+            return m1;
+        }
+        return min(m1, next - done);
+    }
 };
 
 // A force block's four waves serve the same 64 receivers, each with its own
