@@ -245,7 +245,7 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     VjpArgs va{};
     va.wins = im->wins;
     va.atom_win = im->atom_win;
-    va.fblk = im->fblk;
+    va.gblk = im->gblk;
     va.vblk = im->vblk;
     va.nmc = im->d.n_mc;
     va.Ptot = im->P;
@@ -257,7 +257,6 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     va.itype = im->itype;
     va.rmax2 = im->rmax2;
     va.dtypes = m->dtypes;
-    va.ntypes = m->T;
     va.pbc_flag = im->pbc_flag;
     va.g_out = im->g_out;
     va.E_out = im->E_out;
@@ -271,7 +270,7 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     va.prec = m->prec;
     va.apart = m->apart;
     va.C = im->V;
-    HIPCHK(launch_vjp_points(va, im->nfblk, s));
+    HIPCHK(launch_vjp_points(va, im->ngblk, s));
     HIPCHK(launch_vjp_epilogue(va, s));
     HIPCHK(launch_vjp_atoms(va, im->nvblk, s));
     HIPCHK(launch_pbc_flag(nb->wins, nb->lay.W, m->xq, 0.0f, nb->pbc_flag, s));

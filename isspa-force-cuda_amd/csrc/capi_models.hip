@@ -98,7 +98,7 @@ static void isspa_free(isspa_model *m)
     dfree(m->itype); dfree(m->atom_win); dfree(m->rmax); dfree(m->rmax2); dfree(m->vtot);
     dfree(m->ge);
     dfree(m->pts); dfree(m->rec); dfree(m->g_out); dfree(m->E_out); dfree(m->E0_out);
-    dfree(m->cnt_out); dfree(m->pbc_flag); dfree(m->wins); dfree(m->fblk); dfree(m->gblk);
+    dfree(m->cnt_out); dfree(m->pbc_flag); dfree(m->wins); dfree(m->gblk);
     dfree(m->pblk); dfree(m->vblk); dfree(m->wblk);
     dfree(m->part_g); dfree(m->part_cnt); dfree(m->part_s0); dfree(m->part_ein); dfree(m->part_f);
     dfree(m->prof_f);
@@ -121,7 +121,7 @@ static int isspa_tile(isspa_model *m)
     m->max_win_atoms = m->max_group_pts = m->max_group_items = 0;
     m->max_fg = 1;
     long long F = 0, C = 0, V = 0;
-    std::vector<std::pair<long long, int4>> fb, gb, pb, vb, wb;
+    std::vector<std::pair<long long, int4>> gb, pb, vb, wb;
     for (int w = 0; w < L.W; ++w) {
         WinDesc d = base_desc(L, w);
         const long long n = L.n[w], P = n * nmc;
@@ -151,14 +151,12 @@ static int isspa_tile(isspa_model *m)
         d.fpo = F;
         d.ppo = C;
         d.vpo = V;
-        F += (long long)d.splits * P;
+        d.fg = field_group(d.splits);
+        F += (long long)(d.splits / d.fg) * P;
         C += (long long)d.fents * n;
         V += (long long)d.vents * n;
-        const int pblocks = (int)((P + 255) / 256), rblocks = (int)((n + 63) / 64);
-        for (int b = 0; b < pblocks; ++b)
-            for (int sp = 0; sp < d.splits; ++sp) fb.push_back({(long long)d.aps, make_int4(w, b, sp, 0)});
+        const int rblocks = (int)((n + 63) / 64);
         // the field pass: fg splits of the same 256 / fg points a block
-        d.fg = field_group(d.splits);
         m->max_fg = std::max(m->max_fg, d.fg);
         const int gpts = 256 / d.fg, gblocks = (int)((P + gpts - 1) / gpts);
         for (int b = 0; b < gblocks; ++b)
@@ -180,26 +178,22 @@ static int isspa_tile(isspa_model *m)
     auto by_work = [](const std::pair<long long, int4> &a, const std::pair<long long, int4> &b) {
         return a.first > b.first;
     };
-    std::stable_sort(fb.begin(), fb.end(), by_work);
     std::stable_sort(gb.begin(), gb.end(), by_work);
     std::stable_sort(pb.begin(), pb.end(), by_work);
     std::stable_sort(vb.begin(), vb.end(), by_work);
     std::stable_sort(wb.begin(), wb.end(), by_work);
-    std::vector<int4> fbv, gbv, pbv, vbv, wbv;
-    for (auto &x : fb) fbv.push_back(x.second);
+    std::vector<int4> gbv, pbv, vbv, wbv;
     for (auto &x : gb) gbv.push_back(x.second);
     for (auto &x : pb) pbv.push_back(x.second);
     for (auto &x : vb) vbv.push_back(x.second);
     for (auto &x : wb) wbv.push_back(x.second);
     dfree(m->wblk);
-    dfree(m->wins); dfree(m->fblk); dfree(m->gblk); dfree(m->pblk); dfree(m->vblk);
+    dfree(m->wins); dfree(m->gblk); dfree(m->pblk); dfree(m->vblk);
     CHK(upload(&m->wins, m->wins_h.data(), m->wins_h.size()));
-    CHK(upload(&m->fblk, fbv.data(), fbv.size()));
     CHK(upload(&m->gblk, gbv.data(), gbv.size()));
     CHK(upload(&m->pblk, pbv.data(), pbv.size()));
     CHK(upload(&m->vblk, vbv.data(), vbv.size()));
     CHK(upload(&m->wblk, wbv.data(), wbv.size()));
-    m->nfblk = (int)fbv.size();
     m->ngblk = (int)gbv.size();
     m->npblk = (int)pbv.size();
     m->nvblk = (int)vbv.size();

@@ -142,4 +142,16 @@ __device__ __forceinline__ const __attribute__((address_space(4))) T *read_only(
     return (const __attribute__((address_space(4))) T *)p;
 }
 
+// float4s read through the constant address space: scalar loads, whatever the
+// compiler knows about the kernel's stores and asm statements
+struct ScalarRecords {
+    const __attribute__((address_space(4))) float *p;
+    __device__ __forceinline__ ScalarRecords operator+(int k) const { return {p + 4 * k}; }
+    __device__ __forceinline__ float4 operator[](int k) const
+    {
+        const auto *q = p + 4 * k;
+        return make_float4(q[0], q[1], q[2], q[3]);
+    }
+};
+
 }  // namespace isspa

@@ -127,25 +127,6 @@ __global__ __launch_bounds__(kB) void k_diff_reduce(DiffReduceArgs a)
 // ---------------------------------------------------------------------------
 // adjoint, point side: lanes own MC points, receivers stream (wave-uniform)
 // ---------------------------------------------------------------------------
-// per-type records of the analytic model in LDS for the in-sphere branches
-// when they fit (at most kDtLdsFloats floats); the whole block calls this
-constexpr int kDtLdsFloats = 4096;
-__host__ __device__ inline int dtype_floats(int ntypes)
-{
-    return ntypes * (int)(sizeof(DiffType) / sizeof(float));
-}
-
-__device__ __forceinline__ const DiffType *stage_dtypes(const VjpArgs &a)
-{
-    extern __shared__ float lds_dt[];
-    const int nf = dtype_floats(a.ntypes);
-    if (nf > kDtLdsFloats) return a.dtypes;
-    const float *src = reinterpret_cast<const float *>(a.dtypes);
-    for (int t = threadIdx.x; t < nf; t += kB) lds_dt[t] = src[t];
-    __syncthreads();
-    return reinterpret_cast<const DiffType *>(lds_dt);
-}
-
 struct PointBar {
     float hx, hy, hz;   // E-hat bar
     float a1, a2, a3;   // A1..A3 bar
@@ -154,70 +135,92 @@ struct PointBar {
 };
 
 template <bool PBC>
-__device__ __forceinline__ void vjp_points_tile(const VjpArgs &a, const DiffType *dtypes, int j0,
-                                                int j1, const MinImage &mi, float px, float py,
-                                                float pz, float Ex, float Ey, float Ez, float A1,
-                                                float A2, float A3, PointBar &b)
+__device__ __forceinline__ void vjp_points_tile(const VjpArgs &a, int j0, int j1,
+                                                const MinImage &mi, float px, float py, float pz,
+                                                float Ex, float Ey, float Ez, float A1, float A2,
+                                                float A3, const Progress &pg, PointBar &b)
 {
-    const float4 *__restrict__ ar = a.arec;
-    for (int j = j0; j < j1; ++j) {
-        const float4 r0 = ar[4 * j + 0];  // wave-uniform
-        const float4 r1 = ar[4 * j + 1];
-        const float4 r2 = ar[4 * j + 2];
-        float rx = px - r0.x, ry = py - r0.y, rz = pz - r0.z;
-        if (PBC) {
-            rx = min_image1(rx, mi);
-            ry = min_image1(ry, mi);
-            rz = min_image1(rz, mi);
-        }
-        const float d2 = dist2_f32(rx, ry, rz);
-        const float rinv = rsqrt_f32(d2);
-        const float u = __builtin_fmaf(Ez, rz, __builtin_fmaf(Ey, ry, Ex * rx)) * rinv;
-        const float u2 = u * u;
-        const float P2 = __builtin_fmaf(7.5f, u2, -1.5f);
-        const float P3 = __builtin_fmaf(17.5f, u2, -7.5f) * u;
-        const float dP2 = 15.0f * u;
-        const float dP3 = __builtin_fmaf(52.5f, u2, -7.5f);
-        const float rinv2 = rinv * rinv;
-        const float rinv3 = rinv2 * rinv;
-        const float rinv4 = rinv2 * rinv2;
-        const float rinv5 = rinv4 * rinv;
-        const float rinv6 = rinv4 * rinv2;
-        const float la = __builtin_fmaf(r1.z, rz, __builtin_fmaf(r1.y, ry, r1.x * rx));  // Lambda.r
-        const float lb = __builtin_fmaf(r1.z, Ez, __builtin_fmaf(r1.y, Ey, r1.x * Ex));  // Lambda.E-hat
-        const float u3 = 3.0f * u;
-        b.a1 += la * u3 * rinv4 - lb * rinv3;
-        b.a2 += la * rinv5 * P2 - lb * u3 * rinv4;
-        b.a3 += la * rinv6 * P3 - lb * rinv5 * P2;
-        const float dal = 3.0f * A1 * rinv4 + A2 * dP2 * rinv5 + A3 * dP3 * rinv6;
-        const float dk = 3.0f * A2 * rinv4 + dP2 * A3 * rinv5;
-        const float k = u3 * A2 * rinv4 + P2 * A3 * rinv5;
-        const float cu = (la * dal - lb * dk) * rinv;
-        const float ce = -(rinv3 * A1 + k);
-        b.hx += cu * rx + ce * r1.x;
-        b.hy += cu * ry + ce * r1.y;
-        b.hz += cu * rz + ce * r1.z;
-        if (d2 > r0.w) {
-            const float c5 = rinv5 * la, c3 = rinv3 * (1.0f / 3.0f);
-            b.cx += c5 * rx - c3 * r1.x;
-            b.cy += c5 * ry - c3 * r1.y;
-            b.cz += c5 * rz - c3 * r1.z;
-        } else {
-            const float lp = __builtin_fmaf(r2.z, rz, __builtin_fmaf(r2.y, ry, r2.x * rx));
-            const int ti = __float_as_int(r1.w);
-            b.w += diff_F(dtypes[ti], d2 * rinv, rinv) * lp * rinv;
+    // wave-uniform records, the next one requested while this one is used
+    ScalarRecords nr{read_only(reinterpret_cast<const float *>(a.arec + 4 * j0))};
+    float4 n0 = nr[0], n1 = nr[1], n2 = nr[2];
+    for (int j = j0; j < j1;) {
+        const int stop = j0 + pg.rank(j - j0, j1 - j0);
+        for (; j < stop; ++j) {
+            const float4 r0 = n0, r1 = n1, r2 = n2;
+            if (j + 1 < j1) nr = nr + 4;
+            n0 = nr[0];
+            n1 = nr[1];
+            n2 = nr[2];
+            float rx = px - r0.x, ry = py - r0.y, rz = pz - r0.z;
+            if (PBC) {
+                rx = min_image1(rx, mi);
+                ry = min_image1(ry, mi);
+                rz = min_image1(rz, mi);
+            }
+            const float d2 = dist2_f32(rx, ry, rz);
+            const float rinv = rsqrt_f32(d2);
+            const float u = __builtin_fmaf(Ez, rz, __builtin_fmaf(Ey, ry, Ex * rx)) * rinv;
+            const float u2 = u * u;
+            const float P2 = __builtin_fmaf(7.5f, u2, -1.5f);
+            const float P3 = __builtin_fmaf(17.5f, u2, -7.5f) * u;
+            const float dP2 = 15.0f * u;
+            const float dP3 = __builtin_fmaf(52.5f, u2, -7.5f);
+            const float rinv2 = rinv * rinv;
+            const float rinv3 = rinv2 * rinv;
+            const float rinv4 = rinv2 * rinv2;
+            const float rinv5 = rinv4 * rinv;
+            const float rinv6 = rinv4 * rinv2;
+            const float la = __builtin_fmaf(r1.z, rz, __builtin_fmaf(r1.y, ry, r1.x * rx));  // Lambda.r
+            const float lb = __builtin_fmaf(r1.z, Ez, __builtin_fmaf(r1.y, Ey, r1.x * Ex));  // Lambda.E-hat
+            const float u3 = 3.0f * u;
+            b.a1 += la * u3 * rinv4 - lb * rinv3;
+            b.a2 += la * rinv5 * P2 - lb * u3 * rinv4;
+            b.a3 += la * rinv6 * P3 - lb * rinv5 * P2;
+            const float dal = 3.0f * A1 * rinv4 + A2 * dP2 * rinv5 + A3 * dP3 * rinv6;
+            const float dk = 3.0f * A2 * rinv4 + dP2 * A3 * rinv5;
+            const float k = u3 * A2 * rinv4 + P2 * A3 * rinv5;
+            const float cu = (la * dal - lb * dk) * rinv;
+            const float ce = -(rinv3 * A1 + k);
+            b.hx += cu * rx + ce * r1.x;
+            b.hy += cu * ry + ce * r1.y;
+            b.hz += cu * rz + ce * r1.z;
+            if (d2 > r0.w) {
+                const float c5 = rinv5 * la, c3 = rinv3 * (1.0f / 3.0f);
+                b.cx += c5 * rx - c3 * r1.x;
+                b.cy += c5 * ry - c3 * r1.y;
+                b.cz += c5 * rz - c3 * r1.z;
+            } else {
+                const float lp = __builtin_fmaf(r2.z, rz, __builtin_fmaf(r2.y, ry, r2.x * rx));
+                // the atom's type is wave-uniform: its constants come by scalar loads
+                const auto *T = read_only(reinterpret_cast<const float *>(
+                    a.dtypes + __builtin_amdgcn_readfirstlane(__float_as_int(r1.w))));
+                const DiffFParams fp{T[offsetof(DiffType, sts) / 4], T[offsetof(DiffType, ets) / 4],
+                                     T[offsetof(DiffType, rlo) / 4], T[offsetof(DiffType, idel) / 4]};
+                b.w += diff_F(fp, d2 * rinv, rinv) * lp * rinv;
+            }
         }
     }
 }
 
+// A block takes W.fg splits of the same 256 / fg points and adds their FP64
+// sums in split order through LDS, as the field pass: the epilogue, which is
+// bound by the partials it reads, takes 39 us instead of 117 at 32 x 1,100
+// atoms (nMC = 20) and 7.4 instead of 11.2 at 550.  The loop issues some 70
+// VALU operations a pair; the next atom's record is requested one atom ahead,
+// which hides the scalar load where few waves share a SIMD (550 atoms: 28.0 ->
+// 24.6 us) and costs nothing where many do (1,130 us at 32 x 1,100).
 __global__ __launch_bounds__(kB) void k_vjp_points(VjpArgs a)
 {
-    const int4 bt = a.fblk[blockIdx.x];
+    __shared__ double red[10][3 * kWave];  // fg = 4: 3 splits of 64 points
+    const int4 bt = a.gblk[blockIdx.x];
     const WinDesc W = a.wins[bt.x];
     const int P = W.n * a.nmc;
-    const int m = bt.y * kB + threadIdx.x;
-    const int split = bt.z;
-    const int j0 = W.a0 + split * W.aps;
+    const int fg = W.fg, np = kB / fg;
+    // wave-uniform, so the atom range stays on scalar loads
+    const int sub = __builtin_amdgcn_readfirstlane((int)threadIdx.x / np);
+    const int lt = (int)threadIdx.x - sub * np;
+    const int m = bt.y * np + lt;
+    const int j0 = W.a0 + (bt.z * fg + sub) * W.aps;
     const int j1 = min(W.a0 + W.n, j0 + W.aps);
     const bool valid = m < P;
     const long long gp = (long long)W.a0 * a.nmc + (valid ? m : 0);
@@ -226,26 +229,33 @@ __global__ __launch_bounds__(kB) void k_vjp_points(VjpArgs a)
     const float4 q3 = a.rec4[4 * gp + 3];  // A2, 3 A2, A3, w
     const float A1 = a.aux4[gp].w;
     const bool pbc = a.pbc_flag[bt.x] != 0;
-    const DiffType *dtypes = stage_dtypes(a);
     const MinImage mi = min_image_of(W.L, W.h);
     double acc[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    Progress pg(a.ranked_from, j1 - j0);
     for (int jt = j0; jt < j1; jt += kTile) {
         const int je = min(j1, jt + kTile);
+        pg.done = jt - j0;
         PointBar b{0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         if (pbc)
-            vjp_points_tile<true>(a, dtypes, jt, je, mi, q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, A1,
-                                  q3.x, q3.z, b);
+            vjp_points_tile<true>(a, jt, je, mi, q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, A1, q3.x,
+                                  q3.z, pg, b);
         else
-            vjp_points_tile<false>(a, dtypes, jt, je, mi, q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, A1,
-                                   q3.x, q3.z, b);
+            vjp_points_tile<false>(a, jt, je, mi, q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, A1, q3.x,
+                                   q3.z, pg, b);
         acc[0] += b.hx; acc[1] += b.hy; acc[2] += b.hz;
         acc[3] += b.a1; acc[4] += b.a2; acc[5] += b.a3;
         acc[6] += b.cx; acc[7] += b.cy; acc[8] += b.cz;
         acc[9] += b.w;
     }
-    if (!valid) return;
-    const long long o = W.fpo + (long long)split * P + m;
-    for (int k = 0; k < 10; ++k) a.ppart[k * a.F + o] = acc[k];
+    if (sub > 0)
+        for (int k = 0; k < 10; ++k) red[k][(sub - 1) * np + lt] = acc[k];
+    __syncthreads();
+    if (sub > 0 || !valid) return;
+    const long long o = W.fpo + (long long)bt.z * P + m;
+    for (int k = 0; k < 10; ++k) {
+        for (int w = 0; w + 1 < fg; ++w) acc[k] += red[k][w * np + lt];
+        a.ppart[k * a.F + o] = acc[k];
+    }
 }
 
 // Langevin moments and their derivatives, as the forward epilogue
@@ -295,7 +305,7 @@ __global__ __launch_bounds__(kB) void k_vjp_epilogue(VjpArgs a)
     const int P = W.n * a.nmc;
     const long long m = gp - (long long)W.a0 * a.nmc;
     double b[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    for (int s = 0; s < W.splits; ++s) {
+    for (int s = 0; s < W.splits / W.fg; ++s) {
         const long long o = W.fpo + (long long)s * P + m;
         for (int k = 0; k < 10; ++k) b[k] += a.ppart[k * a.F + o];
     }
@@ -333,40 +343,50 @@ template <bool PBC>
 __device__ __forceinline__ void vjp_atoms_tile(const VjpArgs &a, const float4 *__restrict__ pr,
                                                const DiffType &Tj, int m0, int m1,
                                                const MinImage &mi, float4 xj, float R2j, float lpx,
-                                               float lpy, float lpz, float &qb, double tb[5])
+                                               float lpy, float lpz, const Progress &pg, float &qb,
+                                               double tb[5])
 {
     const float e0 = a.e0;
-    for (int m = m0; m < m1; ++m) {
-        const float4 p = pr[4 * m + 0];  // wave-uniform
-        const float4 eb = pr[4 * m + 1];
-        const float4 e0b = pr[4 * m + 2];
-        float rx = p.x - xj.x, ry = p.y - xj.y, rz = p.z - xj.z;
-        if (PBC) {
-            rx = min_image1(rx, mi);
-            ry = min_image1(ry, mi);
-            rz = min_image1(rz, mi);
-        }
-        const float d2 = dist2_f32(rx, ry, rz);
-        const float rinv = rsqrt_f32(d2);
-        const float er = __builtin_fmaf(eb.z, rz, __builtin_fmaf(eb.y, ry, eb.x * rx));
-        const float e0r = __builtin_fmaf(e0b.z, rz, __builtin_fmaf(e0b.y, ry, e0b.x * rx));
-        const bool in_own = d2 <= p.w;
-        const bool in_rec = d2 <= R2j;
-        const float s = -e0 * rinv * rinv * rinv;
-        qb = __builtin_fmaf(s, in_own ? er : er + e0r, qb);
-        if (in_own || in_rec) {
-            const float d = d2 * rinv;
-            float v[3], dv[15];
-            diff_all(Tj, d, rinv, v, dv);
-            if (in_own) {
-                const float ce = er * rinv;
-                const float cg = (eb.w != 0.0f && v[0] != 0.0f) ? eb.w / v[0] : 0.0f;
-                for (int k = 0; k < 5; ++k) tb[k] += (double)(ce * dv[5 + k] + cg * dv[k]);
+    // wave-uniform records, the next one requested while this one is used
+    ScalarRecords nr{read_only(reinterpret_cast<const float *>(pr + 4 * m0))};
+    float4 n0 = nr[0], n1 = nr[1], n2 = nr[2];
+    for (int m = m0; m < m1;) {
+        const int stop = m0 + pg.rank(m - m0, m1 - m0);
+#pragma unroll 2
+        for (; m < stop; ++m) {
+            const float4 p = n0, eb = n1, e0b = n2;
+            if (m + 1 < m1) nr = nr + 4;
+            n0 = nr[0];
+            n1 = nr[1];
+            n2 = nr[2];
+            float rx = p.x - xj.x, ry = p.y - xj.y, rz = p.z - xj.z;
+            if (PBC) {
+                rx = min_image1(rx, mi);
+                ry = min_image1(ry, mi);
+                rz = min_image1(rz, mi);
             }
-            if (in_rec) {
-                const float lp = __builtin_fmaf(lpz, rz, __builtin_fmaf(lpy, ry, lpx * rx));
-                const float cf = e0b.w * lp * rinv;
-                for (int k = 0; k < 5; ++k) tb[k] += (double)(cf * dv[10 + k]);
+            const float d2 = dist2_f32(rx, ry, rz);
+            const float rinv = rsqrt_f32(d2);
+            const float er = __builtin_fmaf(eb.z, rz, __builtin_fmaf(eb.y, ry, eb.x * rx));
+            const float e0r = __builtin_fmaf(e0b.z, rz, __builtin_fmaf(e0b.y, ry, e0b.x * rx));
+            const bool in_own = d2 <= p.w;
+            const bool in_rec = d2 <= R2j;
+            const float s = -e0 * rinv * rinv * rinv;
+            qb = __builtin_fmaf(s, in_own ? er : er + e0r, qb);
+            if (in_own || in_rec) {
+                const float d = d2 * rinv;
+                float v[3], dv[15];
+                diff_all(Tj, d, rinv, v, dv);
+                if (in_own) {
+                    const float ce = er * rinv;
+                    const float cg = (eb.w != 0.0f && v[0] != 0.0f) ? eb.w / v[0] : 0.0f;
+                    for (int k = 0; k < 5; ++k) tb[k] += (double)(ce * dv[5 + k] + cg * dv[k]);
+                }
+                if (in_rec) {
+                    const float lp = __builtin_fmaf(lpz, rz, __builtin_fmaf(lpy, ry, lpx * rx));
+                    const float cf = e0b.w * lp * rinv;
+                    for (int k = 0; k < 5; ++k) tb[k] += (double)(cf * dv[10 + k]);
+                }
             }
         }
     }
@@ -375,8 +395,14 @@ __device__ __forceinline__ void vjp_atoms_tile(const VjpArgs &a, const float4 *_
 // A block's four waves take the same 64 atoms and one chunk each, and add
 // their FP64 sums in chunk order through LDS (as the force pass): a quarter of
 // the partials to write and to sum, and no idle wave in a window's last block.
-// 32 x 1,100 atoms: 1,016 -> 989 us, and k_vjp_finish behind it 81 -> 24 us.
-__global__ __launch_bounds__(kB) void k_vjp_atoms(VjpArgs a)
+// 32 x 1,100 atoms: k_vjp_finish behind it 81 -> 24 us.
+// Bounded by the in-sphere branch, some 200 operations for the few lanes of a
+// wave that are in a sphere.  The lane's type record stays in registers (read
+// from LDS through a flat pointer in the branch, each read waited for both
+// memories) and the next point is requested one point ahead: 52.8 -> 36 us at
+// 550 atoms, 985 -> 880 us at 32 x 1,100.  Six waves a SIMD: held to seven or
+// eight the branch spills (934 us and worse), left alone it takes five (1,006).
+__global__ __launch_bounds__(kB, 6) void k_vjp_atoms(VjpArgs a)
 {
     __shared__ double red[3][6][kWave];
     const int4 bt = a.vblk[blockIdx.x];
@@ -397,20 +423,21 @@ __global__ __launch_bounds__(kB) void k_vjp_atoms(VjpArgs a)
     const float R2j = valid ? a.rmax2[tj] : -1.0f;
     const float4 lp = a.arec[4 * (size_t)j + 2];  // Lambda' = -vtot lambda
     const bool pbc = a.pbc_flag[bt.x] != 0;
-    const DiffType &Tj = stage_dtypes(a)[tj];
+    const DiffType Tj = a.dtypes[tj];
     const MinImage mi = min_image_of(W.L, W.h);
-    double acc[6] = {0, 0, 0, 0, 0, 0};  // q, theta(5)
-    double tb[5] = {0, 0, 0, 0, 0};
+    double qsum = 0.0, tb[5] = {0, 0, 0, 0, 0};  // q, theta
+    Progress pg(a.ranked_from, m1 - m0);
     for (int mt = m0; mt < m1; mt += kTile) {
         const int me = min(m1, mt + kTile);
+        pg.done = mt - m0;
         float qb = 0.0f;
         if (pbc)
-            vjp_atoms_tile<true>(a, pr, Tj, mt, me, mi, xj, R2j, lp.x, lp.y, lp.z, qb, tb);
+            vjp_atoms_tile<true>(a, pr, Tj, mt, me, mi, xj, R2j, lp.x, lp.y, lp.z, pg, qb, tb);
         else
-            vjp_atoms_tile<false>(a, pr, Tj, mt, me, mi, xj, R2j, lp.x, lp.y, lp.z, qb, tb);
-        acc[0] += (double)qb;
+            vjp_atoms_tile<false>(a, pr, Tj, mt, me, mi, xj, R2j, lp.x, lp.y, lp.z, pg, qb, tb);
+        qsum += (double)qb;
     }
-    for (int k = 0; k < 5; ++k) acc[1 + k] = tb[k];
+    double acc[6] = {qsum, tb[0], tb[1], tb[2], tb[3], tb[4]};
     if (wv > 0)
         for (int k = 0; k < 6; ++k) red[wv - 1][k][lane] = acc[k];
     __syncthreads();
@@ -611,9 +638,9 @@ hipError_t launch_diff_reduce(const DiffReduceArgs &a, hipStream_t s)
 hipError_t launch_vjp_points(const VjpArgs &a, int nblocks, hipStream_t s)
 {
     if (nblocks == 0) return hipSuccess;
-    const int nf = dtype_floats(a.ntypes);
-    const size_t lds = nf <= kDtLdsFloats ? (size_t)nf * sizeof(float) : 0;
-    hipLaunchKernelGGL(k_vjp_points, dim3(nblocks), dim3(kB), lds, s, a);
+    VjpArgs b = a;
+    b.ranked_from = ranked_from(nblocks);
+    hipLaunchKernelGGL(k_vjp_points, dim3(nblocks), dim3(kB), 0, s, b);
     return hipGetLastError();
 }
 
@@ -627,9 +654,9 @@ hipError_t launch_vjp_epilogue(const VjpArgs &a, hipStream_t s)
 hipError_t launch_vjp_atoms(const VjpArgs &a, int nblocks, hipStream_t s)
 {
     if (nblocks == 0) return hipSuccess;
-    const int nf = dtype_floats(a.ntypes);
-    const size_t lds = nf <= kDtLdsFloats ? (size_t)nf * sizeof(float) : 0;
-    hipLaunchKernelGGL(k_vjp_atoms, dim3(nblocks), dim3(kB), lds, s, a);
+    VjpArgs b = a;
+    b.ranked_from = ranked_from(nblocks);
+    hipLaunchKernelGGL(k_vjp_atoms, dim3(nblocks), dim3(kB), 0, s, b);
     return hipGetLastError();
 }
 

@@ -542,18 +542,6 @@ __device__ __forceinline__ float table_force(const TableView &tb, const float *F
     return b == row ? f : 0.0f;
 }
 
-// float4s read through the constant address space: scalar loads, whatever the
-// compiler knows about the kernel's stores and asm statements
-struct ScalarRecords {
-    const __attribute__((address_space(4))) float *p;
-    __device__ __forceinline__ ScalarRecords operator+(int k) const { return {p + 4 * k}; }
-    __device__ __forceinline__ float4 operator[](int k) const
-    {
-        const auto *q = p + 4 * k;
-        return make_float4(q[0], q[1], q[2], q[3]);
-    }
-};
-
 // FP32 sums of one tile: the electrostatic (or, split, polarisation) sum s and
 // the in-sphere LJ sum l; flushed into the FP64 ForceAcc per tile
 struct TileSums {

@@ -463,14 +463,14 @@ struct DiffReduceArgs {
 struct VjpArgs {
     const WinDesc *wins;
     const int *atom_win;
-    const int4 *fblk, *vblk;   // point-lane and atom-lane block tables
+    const int4 *gblk, *vblk;   // point-lane and atom-lane block tables
     int nmc;
     long long Ptot;
     const float4 *pts, *rec4, *aux4, *arec, *xq;
     const int *itype;
     const float *rmax2;
     const DiffType *dtypes;
-    int ntypes;
+    int ranked_from;           // as ForceArgs (set at launch)
     const int *pbc_flag;
     const double *g_out, *E_out;
     const int *cnt_out;

@@ -49,10 +49,9 @@ struct isspa_model {
     long target_waves = 0;  // 0: automatic (kPointsPerWave)
     std::vector<WinDesc> wins_h;
     WinDesc *wins = nullptr;
-    // field blocks: gblk (fg splits a block, the field pass) and fblk (one
-    // split a block, the adjoint's point pass)
-    int4 *fblk = nullptr, *pblk = nullptr, *gblk = nullptr;
-    int nfblk = 0, npblk = 0, ngblk = 0;
+    // gblk: the field pass's and the adjoint's point pass's blocks, fg splits each
+    int4 *pblk = nullptr, *gblk = nullptr;
+    int npblk = 0, ngblk = 0;
     int4 *vblk = nullptr;  // the adjoint's atom pass: {w, 64 atoms, four chunks, -}
     int nvblk = 0;
     int4 *wblk = nullptr;  // k_window: {w, -, chunk group, -}

@@ -60,3 +60,21 @@ def test_type_sums_over_atom_ranges(chains):
         mine = ga[s.isspa.isspa_type == t]
         tol = max(1, len(mine)) * 2.0 ** -52 * np.abs(mine).sum(axis=0)
         assert np.all(np.abs(gt[t] - mine.sum(axis=0)) <= tol), t
+
+
+@pytest.mark.parametrize("chains,n_mc,splits,chunks", [
+    (3, 1, 1, 1), (3, 1, 2, 66), (3, 2, 6, 5), (3, 2, 8, 132), (3, 1, 66, 3), (12, 2, 4, 24),
+    (12, 2, 264, 420), (12, 5, 132, 1300)])
+def test_adjoint_split_groups(chains, n_mc, splits, chunks):
+    """One, two and four splits a block, points that fill no block, spans of
+    one atom or record, and launches of up to 512, 1,536 and more blocks."""
+    s = _system(chains, n_mc)
+    prm = DiffParams.from_system(s)
+    m = DiffForces(s, prm, step=2)
+    m.set_tiling(splits, chunks)
+    print(f"{s.n_atoms} atoms, {splits} splits, {chunks} chunks", flush=True)
+    lam = np.random.default_rng(5).normal(size=(s.n_atoms, 3))
+    gq, gt = m.vjp(_t(prm.q), _t(prm.theta), _t(lam))
+    rq, rt = po.diff_vjp(s, prm, po.mc_points(s, step=2), lam)
+    assert max_abs_rel_rms(gq.cpu().numpy(), rq) <= 1e-4
+    assert max_abs_rel_rms(gt.cpu().numpy(), rt) <= 1e-4
