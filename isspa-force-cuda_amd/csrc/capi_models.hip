@@ -1242,10 +1242,10 @@ extern "C" int md_engine_set_step(md_engine *e, uint32_t step, void *stream)
     return ISSPA_OK;
 }
 
-// One prologue launch computes everything that depends only on the
-// coordinates (IS-SPA minimum-image flags, bonded terms, restraint forces and
-// centres of mass, MC points); the IS-SPA passes and the all-pairs partials
-// follow, and one assembly launch forms f = bonded + IS-SPA + all-pairs +
+// One prologue launch computes what depends only on the coordinates (IS-SPA
+// minimum-image flags, MC points, and, where the epilogue does not take them,
+// bonded terms, restraint forces and centres of mass); the IS-SPA passes and
+// the all-pairs partials follow, and one assembly launch forms f = bonded + IS-SPA + all-pairs +
 // restraint -- bit for bit what zeroing f and calling bonded_force,
 // isspa_model_force, nonbond_force and us_force in that order give.
 static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
@@ -1292,9 +1292,13 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
         }
         HIPCHK(launch_window(w, m->max_group_pts, m->max_group_items, s));
     } else {
+        const RiderArgs riders{x4, bonded, 0, us};
+        const bool late = m && epilogue_takes_riders(m->P, riders);
         PrologueArgs p{};
-        p.bonded = bonded;
-        p.us = us;
+        if (!late) {
+            p.bonded = bonded;
+            p.us = us;
+        }
         p.pts.xyzq = x4;
         p.step_d = e->step_d;
         if (m) {
@@ -1302,7 +1306,8 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
             p.rmax_all = m->rmax_all;
             p.flag = m->pbc_flag;
             p.pts = PointsArgs{m->wins, m->atom_win, x4, m->itype, m->rmax, m->rmax2,
-                               m->d.n_atoms, m->d.n_mc, m->d.seed, 0u, e->step_d + kStepNext, m->pts};
+                               m->d.n_atoms, m->d.n_mc, m->d.seed, 0u, e->step_d + kStepNext, m->pts,
+                               m->lay.W};
         }
         HIPCHK(launch_step_prologue(p, s));
         if (m) {
@@ -1313,7 +1318,10 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
                 fa.nb_blocks = e->nb->nblk_tot;
             }
             HIPCHK(launch_field(fa, m->ngblk, s));
-            HIPCHK(launch_epilogue(epilogue_args(m, false), s));
+            if (late)
+                HIPCHK(launch_step_epilogue(epilogue_args(m, false), riders, s));
+            else
+                HIPCHK(launch_epilogue(epilogue_args(m, false), s));
             HIPCHK(launch_force(force_args(m, x4), m->npblk, false, s));
         }
     }

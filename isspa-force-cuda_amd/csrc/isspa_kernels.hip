@@ -75,7 +75,7 @@ __device__ __forceinline__ void stage_lds(float *dst, const float *__restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// A.1 MC points: one lane per point (mc_point).  The first nflag blocks (one
+// A.1 MC points (mc_points_block).  The first nflag blocks (one
 // per window, none when nflag = 0) compute instead the per-window
 // minimum-image flags that the field and force passes read, which saves a
 // launch.
@@ -88,9 +88,7 @@ __global__ __launch_bounds__(kBlock) void k_mc_points(PointsArgs a, int nflag, f
         pbc_flag_block(W, a.xyzq, rmax_all, flag + blockIdx.x);
         return;
     }
-    const long long gp = (long long)(blockIdx.x - nflag) * kBlock + threadIdx.x;
-    if (gp >= (long long)a.ntot * a.nmc) return;
-    mc_point(a, gp);
+    mc_points_block(a, blockIdx.x - nflag);
 }
 
 // ---------------------------------------------------------------------------
@@ -474,7 +472,7 @@ __device__ __forceinline__ void epilogue_point(const EpilogueArgs &a, const WinD
 constexpr int kEpiWideGrid = 256;
 
 template <int B>
-__global__ __launch_bounds__(kBlock) void k_field_epilogue(EpilogueArgs a)
+__device__ __forceinline__ void epilogue_block(const EpilogueArgs &a)
 {
     const long long gp = (long long)blockIdx.x * kBlock + threadIdx.x;
     if (gp >= a.Ptot) return;
@@ -491,6 +489,32 @@ __global__ __launch_bounds__(kBlock) void k_field_epilogue(EpilogueArgs a)
         for (int c = 0; c < 3; ++c) a.E_out[3 * gp + c] = pr.E[c];
     if (a.E0_out)
         for (int c = 0; c < 3; ++c) a.E0_out[3 * gp + c] = pr.E0[c];
+}
+
+template <int B>
+__global__ __launch_bounds__(kBlock) void k_field_epilogue(EpilogueArgs a)
+{
+    epilogue_block<B>(a);
+}
+
+// The wide epilogue with an engine step's bonded and restraint blocks behind
+// its own: they depend on the coordinates alone, and a bonded block, a chain of
+// FP64 operations about as long as a point's epilogue, was the longest block of
+// the launch before the field pass (5.3 us at 1,100 atoms, the points 3.1).
+__global__ __launch_bounds__(kBlock) void k_step_epilogue(EpilogueArgs a, RiderArgs r, int nepi)
+{
+    __shared__ double red[6][kTermBlock];
+    int b = (int)blockIdx.x - nepi;
+    if (b < 0) {
+        epilogue_block<8>(a);
+        return;
+    }
+    if (b < r.bonded_blocks) {
+        bonded_one(r.bonded, b * kBlock + (int)threadIdx.x);
+        return;
+    }
+    us_block(b - r.bonded_blocks, r.us.boff, r.us.us_atoms, r.us.us_mass, r.us.kx, r.us.Ls, r.xyzq,
+             r.us.fus, r.us.com, true, red);
 }
 
 // ---------------------------------------------------------------------------
@@ -1134,8 +1158,8 @@ hipError_t launch_mc_points(const WinDesc *wins, const int *atom_win, const floa
     const long long P = (long long)ntot * nmc;
     const int nflag = flag ? nwin : 0;
     if (P == 0 && nflag == 0) return hipSuccess;
-    const PointsArgs a{wins, atom_win, xyzq, itype, rmax, rmax2, ntot, nmc, seed, step, step_d, pts};
-    hipLaunchKernelGGL(k_mc_points, dim3(blocks_for(P) + nflag), dim3(kBlock), 0, s, a, nflag,
+    const PointsArgs a{wins, atom_win, xyzq, itype, rmax, rmax2, ntot, nmc, seed, step, step_d, pts, nwin};
+    hipLaunchKernelGGL(k_mc_points, dim3((unsigned)((P + kMcBlockPts - 1) / kMcBlockPts) + nflag), dim3(kBlock), 0, s, a, nflag,
                        rmax_all, flag);
     return hipGetLastError();
 }
@@ -1164,6 +1188,27 @@ hipError_t launch_field(const FieldArgs &a0, int nblocks, hipStream_t s)
             hipLaunchKernelGGL((k_field<false, false>), dim3(nblocks), dim3(kBlock), lds, s, a);
         }
     }
+    return hipGetLastError();
+}
+
+static int rider_blocks(const RiderArgs &r)
+{
+    return r.bonded.contrib ? (int)blocks_for((long)r.bonded.nb + r.bonded.na + r.bonded.nd) : 0;
+}
+
+// a block a CU: with a second round the step of 64 umbrella windows (184
+// blocks and 104 riders) takes 57.0 us, with the riders before the field 56.0
+bool epilogue_takes_riders(long long P, const RiderArgs &r)
+{
+    return P > 0 && blocks_for(P) + rider_blocks(r) + r.us.nres <= kEpiWideGrid;
+}
+
+hipError_t launch_step_epilogue(const EpilogueArgs &a, RiderArgs r, hipStream_t s)
+{
+    const int eb = (int)blocks_for(a.Ptot);
+    r.bonded_blocks = rider_blocks(r);
+    const int grid = eb + r.bonded_blocks + r.us.nres;
+    hipLaunchKernelGGL(k_step_epilogue, dim3(grid), dim3(kBlock), 0, s, a, r, eb);
     return hipGetLastError();
 }
 

@@ -288,6 +288,7 @@ struct PointsArgs {
     uint32_t step;            // used when step_d is null
     const uint32_t *step_d;
     float4 *pts;
+    int nwin;
 };
 
 // bonded terms (window-agnostic: they carry global atom indices)
@@ -320,6 +321,15 @@ struct RestraintArgs {
     const float *Ls;
     float4 *fus;  // bias forces stored (w = 1)
     double *com;
+};
+
+// Bonded terms and restraints riding on another launch of an engine step, after
+// its own blocks (each part skipped when empty).
+struct RiderArgs {
+    const float4 *xyzq;
+    BondedArgs bonded;
+    int bonded_blocks;      // set by the launcher
+    RestraintArgs us;
 };
 
 // The IS-SPA pass of a model of small windows in one launch (k_window), with
@@ -357,6 +367,9 @@ hipError_t launch_mc_points(const WinDesc *wins, const int *atom_win, const floa
                             int *flag = nullptr);
 hipError_t launch_field(const FieldArgs &a, int nblocks, hipStream_t s);
 hipError_t launch_epilogue(const EpilogueArgs &a, hipStream_t s);
+// the epilogue with riders, where it is short of blocks
+bool epilogue_takes_riders(long long P, const RiderArgs &r);
+hipError_t launch_step_epilogue(const EpilogueArgs &a, RiderArgs r, hipStream_t s);
 // k_window: whether a model's windows, chunk groups and tables fit it, and the
 // launch (max_atoms, max_points: of the largest window and chunk group;
 // max_items: the most (point, field split) pairs of a group)

@@ -425,8 +425,7 @@ __global__ __launch_bounds__(kBlk) void k_step_prologue(PrologueArgs a)
         return;
     }
     b -= a.us.nres;
-    const long long gp = (long long)b * kBlk + threadIdx.x;
-    if (gp < (long long)a.pts.ntot * a.pts.nmc) mc_point(a.pts, gp);
+    if (a.pts.ntot > 0) mc_points_block(a.pts, b);
 }
 
 hipError_t launch_step_prologue(PrologueArgs a, hipStream_t s)
@@ -434,7 +433,7 @@ hipError_t launch_step_prologue(PrologueArgs a, hipStream_t s)
     const long nterms = (long)a.bonded.nb + a.bonded.na + a.bonded.nd;
     a.bonded_blocks = a.bonded.contrib ? nblocks(nterms) : 0;
     const long long P = (long long)a.pts.ntot * a.pts.nmc;
-    const long long grid = (long long)a.nflag + a.bonded_blocks + a.us.nres + (P + kBlk - 1) / kBlk;
+    const long long grid = (long long)a.nflag + a.bonded_blocks + a.us.nres + (P + kMcBlockPts - 1) / kMcBlockPts;
     // at least one block: the first one hands the step on
     hipLaunchKernelGGL(k_step_prologue, dim3((unsigned)std::max(grid, 1LL)), dim3(kBlk), 0, s, a);
     return hipGetLastError();

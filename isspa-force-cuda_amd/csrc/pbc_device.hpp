@@ -13,31 +13,37 @@ namespace isspa {
 __device__ inline void pbc_flag_block(const WinDesc &W, const float4 *__restrict__ xyzq,
                                       float rmax_all, int *flag)
 {
-    __shared__ float lo[3][256], hi[3][256];
+    constexpr int kU = 8;  // atoms in flight a work-item
     float l[3] = {3.0e38f, 3.0e38f, 3.0e38f}, u[3] = {-3.0e38f, -3.0e38f, -3.0e38f};
-    for (int i = W.a0 + (int)threadIdx.x; i < W.a0 + W.n; i += 256) {
-        const float4 x = xyzq[i];
-        l[0] = fminf(l[0], x.x); u[0] = fmaxf(u[0], x.x);
-        l[1] = fminf(l[1], x.y); u[1] = fmaxf(u[1], x.y);
-        l[2] = fminf(l[2], x.z); u[2] = fmaxf(u[2], x.z);
+    for (int i0 = threadIdx.x; i0 < W.n; i0 += kU * 256) {
+        float4 x[kU];
+#pragma unroll
+        for (int k = 0; k < kU; ++k) x[k] = xyzq[W.a0 + min(i0 + k * 256, W.n - 1)];
+#pragma unroll
+        for (int k = 0; k < kU; ++k) {
+            l[0] = fminf(l[0], x[k].x); u[0] = fmaxf(u[0], x[k].x);
+            l[1] = fminf(l[1], x[k].y); u[1] = fmaxf(u[1], x[k].y);
+            l[2] = fminf(l[2], x[k].z); u[2] = fmaxf(u[2], x[k].z);
+        }
     }
-    for (int k = 0; k < 3; ++k) {
-        lo[k][threadIdx.x] = l[k];
-        hi[k][threadIdx.x] = u[k];
-    }
+    // the waves by shuffles, their extents through LDS
+    __shared__ float lo[3][4], hi[3][4];
+    for (int w = kWave / 2; w > 0; w >>= 1)
+        for (int k = 0; k < 3; ++k) {
+            l[k] = fminf(l[k], __shfl_xor(l[k], w));
+            u[k] = fmaxf(u[k], __shfl_xor(u[k], w));
+        }
+    if (threadIdx.x % kWave == 0)
+        for (int k = 0; k < 3; ++k) {
+            lo[k][threadIdx.x / kWave] = l[k];
+            hi[k][threadIdx.x / kWave] = u[k];
+        }
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int k = 0; k < 3; ++k) {
-                lo[k][threadIdx.x] = fminf(lo[k][threadIdx.x], lo[k][threadIdx.x + w]);
-                hi[k][threadIdx.x] = fmaxf(hi[k][threadIdx.x], hi[k][threadIdx.x + w]);
-            }
-        __syncthreads();
-    }
     if (threadIdx.x == 0) {
         int need = 0;
         for (int k = 0; k < 3; ++k) {
-            const float ext = hi[k][0] - lo[k][0];
+            const float ext = fmaxf(fmaxf(hi[k][0], hi[k][1]), fmaxf(hi[k][2], hi[k][3])) -
+                              fminf(fminf(lo[k][0], lo[k][1]), fminf(lo[k][2], lo[k][3]));
             if (!(ext + rmax_all + 1.0e-2f < W.h)) need = 1;  // NaN -> need
         }
         *flag = need;
