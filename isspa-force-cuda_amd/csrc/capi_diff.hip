@@ -273,7 +273,8 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     HIPCHK(launch_vjp_points(va, im->ngblk, s));
     HIPCHK(launch_vjp_epilogue(va, s));
     HIPCHK(launch_vjp_atoms(va, im->nvblk, s));
-    HIPCHK(launch_pbc_flag(nb->wins, nb->lay.W, m->xq, 0.0f, nb->pbc_flag, s));
+    const int *nb_flag = nullptr;
+    CHK(nonbond_flags(nb, m->xq, &nb_flag, s));
     VjpNbArgs na{};
     na.wins = nb->wins;
     na.blocks = nb->blk;
@@ -284,7 +285,7 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     na.excl_ptr = nb->excl_ptr;
     na.excl_idx = nb->excl_idx;
     na.cfar = nb->cfar;
-    na.pbc_flag = nb->pbc_flag;
+    na.pbc_flag = nb_flag;
     na.ld = m->nb_ld;
     na.T = m->T;
     na.part = nb->part;

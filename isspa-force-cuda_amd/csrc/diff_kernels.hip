@@ -470,7 +470,7 @@ __global__ __launch_bounds__(kB) void k_vjp_nonbond(VjpNbArgs a)
     const float4 li4 = a.arec[4 * (size_t)i + 3];
     uint32_t ex[4];
     for (int k = 0; k < 4; ++k) ex[k] = a.excl[4 * i + k];
-    const bool pbc = a.pbc_flag[bt.x] != 0;
+    const bool pbc = !a.pbc_flag || a.pbc_flag[bt.x] != 0;
     const MinImage mi = min_image_of(W.L, W.h);
     const int wave_lo = W.a0 + bt.y * kB + (threadIdx.x & ~(kWave - 1));
     const float4 *ldrow = lds_ld + ti * a.T;

@@ -80,6 +80,7 @@ struct nonbond_model {
     uint32_t *excl = nullptr;
     int *excl_ptr = nullptr, *excl_idx = nullptr;
     int *pbc_flag = nullptr, *atom_win = nullptr;
+    bool all_images = false;  // every pair takes its image, no flags (nonbond_flags)
     std::vector<WinDesc> wins_h;
     WinDesc *wins = nullptr;
     // split components: every pair in both orders, one entry per partner chunk
@@ -118,5 +119,6 @@ int nonbond_run(nonbond_model *m, const float *xyzq4_d, bool split, float4 *f, d
 // to compute them here
 int nonbond_partials(nonbond_model *m, const float *xyzq4_d, bool split, hipStream_t s,
                      const int *pbc_flag = nullptr);
+int nonbond_flags(nonbond_model *m, const float4 *x, const int **flag, hipStream_t s);
 int nonbond_reduce(nonbond_model *m, bool split, float4 *f, double *o0, double *o1, double *o2,
                    hipStream_t s);

@@ -320,6 +320,12 @@ __device__ __forceinline__ void nonbond_supertile(const NonbondArgs &a, const Wi
     }
 }
 
+// window w's minimum-image flag; without flags every window takes its images
+__device__ __forceinline__ bool nonbond_images(const int *pbc_flag, int w)
+{
+    return !pbc_flag || pbc_flag[w] != 0;
+}
+
 // block blk of the all-pairs grid; lds_lj holds T*T float2 (dynamic LDS),
 // followed, with SYM, by kSymLdsDoubles doubles (8-byte aligned).  SPLIT
 // writes the ordered layout (npo, one entry per partner chunk); the total
@@ -340,7 +346,7 @@ __device__ __forceinline__ void nonbond_block(const NonbondArgs &a, int blk, flo
         double *jl = reinterpret_cast<double *>(lds_lj + ((a.T * a.T + 1) & ~1));
         for (int t = threadIdx.x; t < kSymLdsDoubles; t += kNbBlock) jl[t] = 0.0;
         __syncthreads();
-        if (a.pbc_flag[bt.x] != 0)
+        if (nonbond_images(a.pbc_flag, bt.x))
             nonbond_supertile<true>(a, W, bt.y, bt.z, lds_lj, jl);
         else
             nonbond_supertile<false>(a, W, bt.y, bt.z, lds_lj, jl);
@@ -351,7 +357,7 @@ __device__ __forceinline__ void nonbond_block(const NonbondArgs &a, int blk, flo
         pbc = needs_image<kNbBlock>(W, a.xyzq, 0.0f);  // and the barrier for the table
     } else {
         __syncthreads();
-        pbc = a.pbc_flag[bt.x] != 0;
+        pbc = nonbond_images(a.pbc_flag, bt.x);
     }
     const bool near_kind = SYM && bt.w == kNbKindNear;
     // partners: a chunk, or (near kind) 256-atom block bt.z, the receivers'
