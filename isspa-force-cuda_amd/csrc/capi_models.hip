@@ -650,10 +650,10 @@ extern "C" int nonbond_model_create_batch(int n, int T, const int *ityp, const i
         const double tgt = std::max(1.0, kWaveSlots * ((double)nw * nw / work_tot));
         const int c = auto_pieces(nw, nw, kMinNonbondPartners, tgt);
         d.apc = (int)((nw + c - 1) / c);
-        d.nbc = (int)((nw + d.apc - 1) / d.apc);
+        d.nbc = (int)((nw + (long long)kNbGroup * d.apc - 1) / ((long long)kNbGroup * d.apc));
         d.npo = B;
         B += (long long)d.nbc * nw;
-        for (int b = 0; b < (int)((nw + 255) / 256); ++b)
+        for (int b = 0; b < (int)((nw + 63) / 64); ++b)
             for (int ch = 0; ch < d.nbc; ++ch) bl.push_back({(long long)d.apc, make_int4(w, b, ch, 0)});
         m->wins_h[w] = d;
     }
@@ -685,7 +685,7 @@ extern "C" int nonbond_model_create_batch(int n, int T, const int *ityp, const i
         d.spo = Bt;
         Bt += (long long)d.nte * nw;
         if (!sym) {
-            for (int b = 0; b < nsb; ++b)
+            for (int b = 0; b < (nw + 63) / 64; ++b)
                 for (int ch = 0; ch < d.nbc; ++ch)
                     blt.push_back({(long long)d.apc, make_int4(w, b, ch, kNbKindChunk)});
             continue;

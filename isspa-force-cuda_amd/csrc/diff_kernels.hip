@@ -454,13 +454,16 @@ __global__ __launch_bounds__(kB, 6) void k_vjp_atoms(VjpArgs a)
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kB) void k_vjp_nonbond(VjpNbArgs a)
 {
-    extern __shared__ float4 lds_ld[];
+    extern __shared__ __align__(16) float4 lds_ld[];
     for (int t = threadIdx.x; t < a.T * a.T; t += kB) lds_ld[t] = a.ld[t];
     __syncthreads();
     const int4 bt = a.blocks[blockIdx.x];
     const WinDesc W = a.wins[bt.x];
-    const int il = bt.y * kB + threadIdx.x;
-    const int j0 = W.a0 + bt.z * W.apc;
+    const int lane = (int)threadIdx.x % kWave;
+    // read from the first lane, so the compiler knows it is wave-uniform
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int il = bt.y * kWave + lane;
+    const int j0 = W.a0 + min(W.n, (kNbGroup * bt.z + wv) * W.apc);
     const int j1 = min(W.a0 + W.n, j0 + W.apc);
     const bool valid = il < W.n;
     const int i = W.a0 + (valid ? il : W.n - 1);
@@ -472,7 +475,7 @@ __global__ __launch_bounds__(kB) void k_vjp_nonbond(VjpNbArgs a)
     for (int k = 0; k < 4; ++k) ex[k] = a.excl[4 * i + k];
     const bool pbc = !a.pbc_flag || a.pbc_flag[bt.x] != 0;
     const MinImage mi = min_image_of(W.L, W.h);
-    const int wave_lo = W.a0 + bt.y * kB + (threadIdx.x & ~(kWave - 1));
+    const int wave_lo = W.a0 + bt.y * kWave;
     const float4 *ldrow = lds_ld + ti * a.T;
     double qacc = 0.0, sacc = 0.0, eacc = 0.0;
     for (int jt = j0; jt < j1; jt += kTile) {
@@ -526,7 +529,24 @@ __global__ __launch_bounds__(kB) void k_vjp_nonbond(VjpNbArgs a)
         sacc += (double)sb;
         eacc += (double)eb;
     }
-    if (!valid) return;
+    // the chunks' sums in order, as the forward blocks; every wave is done
+    // with the table
+    double *red = reinterpret_cast<double *>(lds_ld) + lane;
+    __syncthreads();
+    if (wv > 0) {
+        double *d = red + (wv - 1) * 3 * kWave;
+        d[0] = qacc;
+        d[kWave] = sacc;
+        d[2 * kWave] = eacc;
+    }
+    __syncthreads();
+    if (wv > 0 || !valid) return;
+    for (int w = 0; w < kNbGroup - 1; ++w) {
+        const double *d = red + w * 3 * kWave;
+        qacc += d[0];
+        sacc += d[kWave];
+        eacc += d[2 * kWave];
+    }
     const long long o = W.npo + (long long)bt.z * W.n + il;
     a.part[o] = qacc;
     a.part[a.B + o] = sacc;
@@ -663,7 +683,7 @@ hipError_t launch_vjp_atoms(const VjpArgs &a, int nblocks, hipStream_t s)
 hipError_t launch_vjp_nonbond(const VjpNbArgs &a, int nblocks, hipStream_t s)
 {
     if (nblocks == 0) return hipSuccess;
-    const size_t lds = sizeof(float4) * a.T * a.T;
+    const size_t lds = std::max(sizeof(float4) * a.T * a.T, nonbond_share_bytes(3));
     hipLaunchKernelGGL(k_vjp_nonbond, dim3(nblocks), dim3(kB), lds, s, a);
     return hipGetLastError();
 }

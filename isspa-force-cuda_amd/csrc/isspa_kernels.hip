@@ -1181,7 +1181,7 @@ hipError_t launch_field(const FieldArgs &a0, int nblocks, hipStream_t s)
         size_t lds = std::max<size_t>(nt <= kTabLdsFloats ? (size_t)nt * sizeof(float) : 0,
                                       a.max_fg > 1 ? kFieldXchgBytes : 0);
         if (a.nb_blocks) {
-            lds = std::max(lds, sizeof(float2) * a.nb.T * a.nb.T);
+            lds = std::max(lds, nonbond_lds_bytes(a.nb.T, false));
             hipLaunchKernelGGL((k_field<false, true>), dim3(nblocks + a.nb_blocks), dim3(kBlock),
                                lds, s, a);
         } else {

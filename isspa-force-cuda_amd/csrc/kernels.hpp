@@ -20,10 +20,10 @@ struct WinDesc {
     int a0, n;          // atoms of the window
     int splits, aps;    // field pass: atom splits, atoms per split
     int chunks, ppc;    // force pass: point chunks, points per chunk
-    int nbc, apc;       // nonbond: partner chunks, atoms per chunk
+    int nbc, apc;       // nonbond: groups of kNbGroup partner chunks, atoms per chunk
     long long fpo;      // field partial offset:  sum over earlier windows of splits * P
     long long ppo;      // force partial offset:  sum of fents * n
-    long long npo;      // nonbond partial offset: sum of nbc * n
+    long long npo;      // nonbond partial offset: sum of nbc * n (nbc entries per atom)
     uint32_t sys;       // Philox counter word 3
     float L, h;         // box length and half length
     int nte;            // nonbond total force: entries per atom (nbc, or the
@@ -95,12 +95,19 @@ struct NonbondArgs {
     int sym;               // the block table holds super-tiles
 };
 
+// chunks of a block: one a wave, all for the same 64 receivers
+constexpr int kNbGroup = 4;
+constexpr size_t nonbond_share_bytes(int comps) { return sizeof(double) * 3 * 64 * comps; }
+
 // dynamic LDS of an all-pairs block: the T x T LJ table, then (super-tiles)
-// the partner sums on an 8-byte boundary
-inline size_t nonbond_lds_bytes(int T, bool sym)
+// the partner sums on an 8-byte boundary; the chunks' sums take the table's place
+inline size_t nonbond_lds_bytes(int T, bool sym, bool split = false)
 {
-    return sym ? sizeof(float) * 2 * (((size_t)T * T + 1) & ~(size_t)1) + sizeof(double) * kSymLdsDoubles
-               : sizeof(float) * 2 * (size_t)T * T;
+    const size_t tab = sym ? sizeof(float) * 2 * (((size_t)T * T + 1) & ~(size_t)1) +
+                                 sizeof(double) * kSymLdsDoubles
+                           : sizeof(float) * 2 * (size_t)T * T;
+    const size_t sums = nonbond_share_bytes(split ? 9 : 3);
+    return tab > sums ? tab : sums;
 }
 
 struct FieldArgs {

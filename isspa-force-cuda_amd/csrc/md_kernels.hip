@@ -31,7 +31,7 @@ __global__ __launch_bounds__(kBlk) void k_nonbond(NonbondArgs a)
 hipError_t launch_nonbond(const NonbondArgs &a, int nb, bool split, hipStream_t s)
 {
     if (nb == 0) return hipSuccess;
-    const size_t lds = nonbond_lds_bytes(a.T, a.sym != 0);
+    const size_t lds = nonbond_lds_bytes(a.T, a.sym != 0, split);
     if (split)
         hipLaunchKernelGGL(k_nonbond<true>, dim3(nb), dim3(kBlk), lds, s, a);
     else

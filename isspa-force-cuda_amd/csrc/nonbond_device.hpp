@@ -360,12 +360,21 @@ __device__ __forceinline__ void nonbond_block(const NonbondArgs &a, int blk, flo
         pbc = nonbond_images(a.pbc_flag, bt.x);
     }
     const bool near_kind = SYM && bt.w == kNbKindNear;
-    // partners: a chunk, or (near kind) 256-atom block bt.z, the receivers'
-    // own block or a neighbour; both write entry bt.z
-    const int j0 = W.a0 + bt.z * (near_kind ? kNbBlock : W.apc);
+    const int lane = (int)threadIdx.x % kWave;
+    // read from the first lane, so the compiler knows it is wave-uniform
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    // Chunk kind: the block's waves take the same 64 receivers and a chunk
+    // each, and the block adds the chunks' sums in order: a quarter of the
+    // partials to write and to sum of a block of 256 receivers and one chunk,
+    // and fewer idle lanes.  Launch and sum behind it: 1,100 atoms 10.0 -> 9.4
+    // us, 2,222 periodic atoms 16.0 -> 12.2, 3,982 atoms 26.7 -> 22.0 us.
+    // Near kind: 256 receivers and the 256-atom block bt.z, their own or a
+    // neighbour.
+    const int chunk = kNbGroup * bt.z + wv;
+    const int j0 = W.a0 + min(W.n, near_kind ? bt.z * kNbBlock : chunk * W.apc);
     const int j1 = min(W.a0 + W.n, j0 + (near_kind ? kNbBlock : W.apc));
-    const int entry = bt.z;
-    const int il = bt.y * kNbBlock + threadIdx.x;
+    const int first = near_kind ? bt.y * kNbBlock + wv * kWave : bt.y * kWave;  // of the wave
+    const int il = first + lane;
     const bool valid = il < W.n;
     const int i = W.a0 + (valid ? il : W.n - 1);  // idle lanes mirror the last atom, results dropped
     const float4 xi = a.xyzq[i];
@@ -373,8 +382,7 @@ __device__ __forceinline__ void nonbond_block(const NonbondArgs &a, int blk, flo
     uint32_t ex[4];
     for (int k = 0; k < 4; ++k) ex[k] = a.excl[4 * i + k];
     const MinImage mi = min_image_of(W.L, W.h);
-    // first receiver of this wave, for the near-diagonal test
-    const int wave_lo = W.a0 + bt.y * kNbBlock + (threadIdx.x & ~(kWave - 1));
+    const int wave_lo = W.a0 + first;  // for the near-diagonal test
     double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     const float2 *ljrow = lds_lj + ti * a.T;
     constexpr int kTile = 64;
@@ -399,9 +407,19 @@ __device__ __forceinline__ void nonbond_block(const NonbondArgs &a, int blk, flo
                 nonbond_tile<false, SPLIT, kFast>(a, i, jt, je, mi, xi, ex, ljrow, acc);
         }
     }
+    constexpr int comps = SPLIT ? 9 : 3;
+    if (!near_kind) {
+        double *red = reinterpret_cast<double *>(lds_lj);  // every wave is done with the table
+        __syncthreads();
+        if (wv > 0)
+            for (int k = 0; k < comps; ++k) red[((wv - 1) * comps + k) * kWave + lane] = acc[k];
+        __syncthreads();
+        if (wv > 0) return;
+        for (int w = 0; w < kNbGroup - 1; ++w)
+            for (int k = 0; k < comps; ++k) acc[k] += red[(w * comps + k) * kWave + lane];
+    }
     if (!valid) return;
-    const long long o = (SPLIT ? W.npo : W.spo) + (long long)entry * W.n + il;
-    const int comps = SPLIT ? 9 : 3;
+    const long long o = (SPLIT ? W.npo : W.spo) + (long long)bt.z * W.n + il;
     for (int k = 0; k < comps; ++k) a.part[k * a.B + o] = acc[k];
 }
 
