@@ -104,6 +104,39 @@ static void isspa_free(isspa_model *m)
     dfree(m->prof_f);
 }
 
+// Puts the blocks that pair atoms with their own points before the others of a
+// window's equal items: they hold most of the in-sphere pairs and take about
+// twice the time, so each should find a CU of its own, and no round of a large
+// launch should end on one.  The field blocks go round the XCDs one by one; each
+// XCD's contiguous run of force blocks (xcd_run_entry) is ordered by itself.
+// Force pass of 550 atoms 10.9 -> 10.2 us, 1,540 atoms 37.1 -> 35.0, 6,600 atoms
+// 333 -> 321; field pass of 4,510 periodic atoms 118 -> 116 us.
+static void own_atoms_first(const WinDesc &d, long long nmc,
+                            std::vector<std::pair<long long, int4>> &gb,
+                            std::vector<std::pair<long long, int4>> &pb)
+{
+    // points [p0, p1) against atoms [a0, a1)
+    auto meets = [nmc](long long p0, long long p1, long long a0, long long a1) {
+        return p0 < a1 * nmc && p1 > a0 * nmc;
+    };
+    const long long gpts = 256 / d.fg, gats = (long long)d.fg * d.aps;
+    std::stable_partition(gb.begin(), gb.end(), [&](const std::pair<long long, int4> &x) {
+        const int4 &b = x.second;
+        return meets(b.y * gpts, (b.y + 1) * gpts, b.z * gats, (b.z + 1) * gats);
+    });
+    const long long span = (long long)force_group(d.n) * d.ppc;
+    auto own = [&](const std::pair<long long, int4> &x) {
+        const int4 &b = x.second;
+        return meets(b.z * span, (b.z + 1) * span, b.y * 64LL, (b.y + 1) * 64LL);
+    };
+    auto run = pb.begin();
+    for (size_t x = 0; x < 8; ++x) {
+        const auto end = run + (pb.size() / 8 + (x < pb.size() % 8 ? 1 : 0));
+        std::stable_partition(run, end, own);
+        run = end;
+    }
+}
+
 // per-window splits/chunks, partial offsets and the block work tables; blocks
 // are ordered by decreasing work so the longest ones start first
 static int isspa_tile(isspa_model *m)
@@ -182,6 +215,7 @@ static int isspa_tile(isspa_model *m)
     std::stable_sort(pb.begin(), pb.end(), by_work);
     std::stable_sort(vb.begin(), vb.end(), by_work);
     std::stable_sort(wb.begin(), wb.end(), by_work);
+    if (L.W == 1) own_atoms_first(m->wins_h[0], nmc, gb, pb);
     std::vector<int4> gbv, pbv, vbv, wbv;
     for (auto &x : gb) gbv.push_back(x.second);
     for (auto &x : pb) pbv.push_back(x.second);
