@@ -162,7 +162,6 @@ static int diff_prepare(isspa_diff *m, const float *xyz4_d, const double *q_d,
     pa.types = m->dtypes;
     pa.nb_lj = m->nb->lj;
     pa.nb_ld = m->nb_ld;
-    HIPCHK(launch_diff_prep_types(pa, s));
     DiffAtomArgs aa{};
     aa.n = m->n;
     aa.xyz = reinterpret_cast<const float4 *>(xyz4_d);
@@ -173,14 +172,16 @@ static int diff_prepare(isspa_diff *m, const float *xyz4_d, const double *q_d,
     aa.rmax2 = m->im->rmax2;
     aa.xq = m->xq;
     aa.arec = m->arec;
-    HIPCHK(launch_diff_prep_atoms(aa, s));
+    HIPCHK(launch_diff_prep(pa, aa, s));
     return ISSPA_OK;
 }
 
-// points, field, epilogue, force partials, then F and S_e
-static int diff_isspa_forward(isspa_diff *m, const double *q_d, double *f_d, hipStream_t s)
+// points, field, epilogue, force partials, then F and S_e; with pairs also the
+// all-pairs partials, which F then includes
+static int diff_forward(isspa_diff *m, const double *q_d, double *f_d, bool pairs, hipStream_t s)
 {
     isspa_model *im = m->im;
+    nonbond_model *nb = m->nb;
     HIPCHK(launch_mc_points(im->wins, im->atom_win, m->xq, im->itype, im->rmax, im->rmax2,
                             im->d.n_atoms, im->d.n_mc, im->d.seed, m->step, nullptr, im->pts, s,
                             im->lay.W, im->rmax_all, im->pbc_flag));
@@ -188,7 +189,19 @@ static int diff_isspa_forward(isspa_diff *m, const double *q_d, double *f_d, hip
     fa.dtypes = m->dtypes;
     HIPCHK(launch_field(fa, im->ngblk, s));
     // the adjoint reads the per-point g, count and E
-    HIPCHK(launch_epilogue(epilogue_args(im, true), s));
+    RiderArgs riders{};
+    if (pairs) {
+        const int *flag = nullptr;
+        CHK(nonbond_flags(nb, m->xq, &flag, s));
+        riders.nb = nonbond_args(nb, m->xq, flag, false);
+        riders.nb_blocks = nb->nblk_tot;
+    }
+    if (pairs && !nb->any_sym && epilogue_takes_riders(im->P, riders)) {
+        HIPCHK(launch_step_epilogue(epilogue_args(im, true), riders, s));
+    } else {
+        HIPCHK(launch_epilogue(epilogue_args(im, true), s));
+        if (pairs) HIPCHK(launch_nonbond(riders.nb, riders.nb_blocks, false, s));
+    }
     ForceArgs ka = force_args(im, m->xq);
     ka.dtypes = m->dtypes;
     HIPCHK(launch_force(ka, im->npblk, false, s));
@@ -204,6 +217,11 @@ static int diff_isspa_forward(isspa_diff *m, const double *q_d, double *f_d, hip
     ra.q = q_d;
     ra.se = m->se;
     ra.f = f_d;
+    if (pairs) {
+        ra.nb_wins = nb->wins;
+        ra.nb_part = nb->part;
+        ra.nb_B = nb->B_tot;
+    }
     HIPCHK(launch_diff_reduce(ra, s));
     return ISSPA_OK;
 }
@@ -217,9 +235,7 @@ extern "C" int isspa_diff_forces(isspa_diff *m, const float *xyz4_d, const doubl
     m->fwd_valid = false;
     CHK(diff_buffers(m));
     CHK(diff_prepare(m, xyz4_d, q_d, theta_d, nullptr, s));
-    CHK(diff_isspa_forward(m, q_d, f_d, s));
-    CHK(nonbond_run(m->nb, reinterpret_cast<const float *>(m->xq), false, nullptr, f_d, nullptr,
-                    nullptr, s));
+    CHK(diff_forward(m, q_d, f_d, true, s));
     m->fwd_x = xyz4_d;
     m->fwd_q = q_d;
     m->fwd_theta = theta_d;
@@ -240,7 +256,7 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     CHK(diff_prepare(m, xyz4_d, q_d, theta_d, lam_d, s));
     if (run_forward) {
         m->fwd_valid = false;  // ftmp, not the caller's forces, holds this forward
-        CHK(diff_isspa_forward(m, q_d, m->ftmp, s));
+        CHK(diff_forward(m, q_d, m->ftmp, false, s));
     }
     VjpArgs va{};
     va.wins = im->wins;
@@ -271,8 +287,6 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     va.apart = m->apart;
     va.C = im->V;
     HIPCHK(launch_vjp_points(va, im->ngblk, s));
-    HIPCHK(launch_vjp_epilogue(va, s));
-    HIPCHK(launch_vjp_atoms(va, im->nvblk, s));
     const int *nb_flag = nullptr;
     CHK(nonbond_flags(nb, m->xq, &nb_flag, s));
     VjpNbArgs na{};
@@ -290,7 +304,8 @@ static int diff_vjp(isspa_diff *m, const float *xyz4_d, const double *q_d, const
     na.T = m->T;
     na.part = nb->part;
     na.B = nb->B;
-    HIPCHK(launch_vjp_nonbond(na, nb->nblk, s));
+    HIPCHK(launch_vjp_epilogue_nonbond(va, na, nb->nblk, s));
+    HIPCHK(launch_vjp_atoms(va, im->nvblk, s));
     VjpFinishArgs fa{};
     fa.n = m->n;
     fa.wins = im->wins;

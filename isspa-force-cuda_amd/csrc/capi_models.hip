@@ -796,7 +796,7 @@ extern "C" int nonbond_model_destroy(nonbond_model *m)
 }
 
 // split: the components' block table and partial layout; otherwise the total force's
-static NonbondArgs nonbond_args(nonbond_model *m, const float4 *x, const int *pbc_flag, bool split)
+NonbondArgs nonbond_args(nonbond_model *m, const float4 *x, const int *pbc_flag, bool split)
 {
     NonbondArgs a{};
     a.wins = m->wins; a.blocks = split ? m->blk : m->blk_tot; a.xyzq = x; a.aux = m->aux;
@@ -1346,7 +1346,7 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
         }
         HIPCHK(launch_window(w, m->max_group_pts, m->max_group_items, s));
     } else {
-        const RiderArgs riders{x4, bonded, 0, us};
+        const RiderArgs riders{x4, bonded, 0, us, NonbondArgs{}, 0};
         const bool late = m && epilogue_takes_riders(m->P, riders);
         PrologueArgs p{};
         if (!late) {

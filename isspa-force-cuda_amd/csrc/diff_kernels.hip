@@ -35,7 +35,7 @@ static inline int nblk(long long n) { return (int)((n + kB - 1) / kB); }
 // ---------------------------------------------------------------------------
 // parameters -> per-type constants and LJ pair tables
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kB) void k_diff_prep_types(DiffPrepArgs a)
+__device__ __forceinline__ void diff_prep_types(const DiffPrepArgs &a)
 {
     const int T = a.T;
     for (int t = threadIdx.x; t < T; t += kB) {
@@ -79,9 +79,9 @@ __global__ __launch_bounds__(kB) void k_diff_prep_types(DiffPrepArgs a)
 }
 
 // positions with the charges as FP32 .w; receiver records for the adjoint
-__global__ __launch_bounds__(kB) void k_diff_prep_atoms(DiffAtomArgs a)
+__device__ __forceinline__ void diff_prep_atoms(const DiffAtomArgs &a, int block)
 {
-    const int i = blockIdx.x * kB + threadIdx.x;
+    const int i = block * kB + (int)threadIdx.x;
     if (i >= a.n) return;
     const float4 x = a.xyz[i];
     const double q = a.q[i];
@@ -98,29 +98,43 @@ __global__ __launch_bounds__(kB) void k_diff_prep_atoms(DiffAtomArgs a)
     r[3] = make_float4((float)l0, (float)l1, (float)l2, 0.0f);
 }
 
-// F_i = -q_i vtot_i S_e - vtot_i S_lj (overwrites f), S_e kept for the adjoint.
+// the types by the first block, the atoms by the others
+__global__ __launch_bounds__(kB) void k_diff_prep(DiffPrepArgs t, DiffAtomArgs a)
+{
+    if (blockIdx.x == 0)
+        diff_prep_types(t);
+    else
+        diff_prep_atoms(a, (int)blockIdx.x - 1);
+}
+
+// F_i = -q_i vtot_i S_e - vtot_i S_lj, plus the all-pairs sum where its partials
+// are given (overwrites f); S_e kept for the adjoint.
 // Latency bound: a block of 16 atoms x 16 entry slices (reduce_device.hpp) with
 // eight entries in flight a slice.  One lane per atom over all chunks
 // took 53.9 us at 550 atoms (3 blocks, 181 dependent rounds) and 121 us for
 // 32 x 1,100 atoms; now 7.4 and 16 us (86 MB, 5.4 TB/s).
 __global__ __launch_bounds__(kB) void k_diff_reduce(DiffReduceArgs a)
 {
-    __shared__ double red[kSumSlices][6][kSumAtoms];
+    __shared__ double red[kSumSlices][9][kSumAtoms];
     const int al = threadIdx.x % kSumAtoms, sl = threadIdx.x / kSumAtoms;
     const int i = blockIdx.x * kSumAtoms + al;
     const bool valid = i < a.n;
-    double s[6] = {0, 0, 0, 0, 0, 0};
+    double s[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};  // S_e, S_lj; all pairs
     if (valid) {
         const WinDesc W = window_of(a.wins, a.nwin, a.atom_win, i);
         sum_batches<6, 8>(ForceEntry<6>(W, a.part, i), sl, W.fents, s);
+        if (a.nb_part) {
+            const WinDesc Wn = window_of(a.nb_wins, a.nwin, a.atom_win, i);
+            sum_batches<3, 4>(nonbond_entry<3>(Wn, a.nb_part, a.nb_B, i), sl, Wn.nte, s + 6);
+        }
     }
-    combine_slices<6>(red, al, sl, s);
+    combine_slices<9>(red, al, sl, s);
     if (sl != 0 || !valid) return;
     const double vt = a.vtot[a.itype[i]];
     const double qv = -a.q[i] * vt;
     for (int c = 0; c < 3; ++c) {
         a.se[3 * i + c] = s[c];
-        a.f[3 * i + c] = qv * s[c] - vt * s[3 + c];
+        a.f[3 * i + c] = qv * s[c] - vt * s[3 + c] + s[6 + c];
     }
 }
 
@@ -297,7 +311,7 @@ __device__ __forceinline__ void moments_derivs(double x, double m[3], double dm[
     dm[2] = dm[0] - 5.0 * dm[1] / x + 5.0 * m[1] / (x * x);
 }
 
-__global__ __launch_bounds__(kB) void k_vjp_epilogue(VjpArgs a)
+__device__ __forceinline__ void vjp_epilogue_block(const VjpArgs &a)
 {
     const long long gp = (long long)blockIdx.x * kB + threadIdx.x;
     if (gp >= a.Ptot) return;
@@ -452,12 +466,11 @@ __global__ __launch_bounds__(kB, 6) void k_vjp_atoms(VjpArgs a)
 // ---------------------------------------------------------------------------
 // adjoint of the all-pairs term: lanes own receivers i, partners stream
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kB) void k_vjp_nonbond(VjpNbArgs a)
+__device__ __forceinline__ void vjp_nonbond_block(const VjpNbArgs &a, int block, float4 *lds_ld)
 {
-    extern __shared__ __align__(16) float4 lds_ld[];
     for (int t = threadIdx.x; t < a.T * a.T; t += kB) lds_ld[t] = a.ld[t];
     __syncthreads();
-    const int4 bt = a.blocks[blockIdx.x];
+    const int4 bt = a.blocks[block];
     const WinDesc W = a.wins[bt.x];
     const int lane = (int)threadIdx.x % kWave;
     // read from the first lane, so the compiler knows it is wave-uniform
@@ -553,6 +566,29 @@ __global__ __launch_bounds__(kB) void k_vjp_nonbond(VjpNbArgs a)
     a.part[2 * a.B + o] = eacc;
 }
 
+__global__ __launch_bounds__(kB) void k_vjp_epilogue(VjpArgs a)
+{
+    vjp_epilogue_block(a);
+}
+
+__global__ __launch_bounds__(kB) void k_vjp_nonbond(VjpNbArgs a)
+{
+    extern __shared__ __align__(16) float4 lds_ld[];
+    vjp_nonbond_block(a, blockIdx.x, lds_ld);
+}
+
+// The epilogue with the all-pairs blocks behind its own where a block a CU
+// holds both: each is a chain that leaves the chip idle (550 atoms: 7.4 us
+// with 43 blocks and 8.7 with 81).
+__global__ __launch_bounds__(kB) void k_vjp_epilogue_nonbond(VjpArgs a, VjpNbArgs n, int nepi)
+{
+    extern __shared__ __align__(16) float4 lds_ld[];
+    if ((int)blockIdx.x < nepi)
+        vjp_epilogue_block(a);
+    else
+        vjp_nonbond_block(n, (int)blockIdx.x - nepi, lds_ld);
+}
+
 // Per atom: the chunk partials + the direct charge term.  Latency bound like
 // k_diff_reduce and split the same way, four entries in flight a slice: one lane per atom took 74.7 us at 550 atoms and
 // 133 us for 32 x 1,100 atoms; now 9.2 and 24 us.
@@ -635,16 +671,9 @@ __global__ __launch_bounds__(kB) void k_type_sum(const double *__restrict__ part
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-hipError_t launch_diff_prep_types(const DiffPrepArgs &a, hipStream_t s)
+hipError_t launch_diff_prep(const DiffPrepArgs &t, const DiffAtomArgs &a, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_diff_prep_types, dim3(1), dim3(kB), 0, s, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_diff_prep_atoms(const DiffAtomArgs &a, hipStream_t s)
-{
-    if (a.n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_diff_prep_atoms, dim3(nblk(a.n)), dim3(kB), 0, s, a);
+    hipLaunchKernelGGL(k_diff_prep, dim3(1 + nblk(a.n)), dim3(kB), 0, s, t, a);
     return hipGetLastError();
 }
 
@@ -664,10 +693,20 @@ hipError_t launch_vjp_points(const VjpArgs &a, int nblocks, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_vjp_epilogue(const VjpArgs &a, hipStream_t s)
+// the point epilogue and the all-pairs adjoint, in one launch up to a block a CU
+hipError_t launch_vjp_epilogue_nonbond(const VjpArgs &a, const VjpNbArgs &n, int nb_blocks,
+                                       hipStream_t s)
 {
-    if (a.Ptot == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_vjp_epilogue, dim3(nblk(a.Ptot)), dim3(kB), 0, s, a);
+    const int nepi = nblk(a.Ptot);
+    const size_t lds = std::max(sizeof(float4) * n.T * n.T, nonbond_share_bytes(3));
+    if (nepi + nb_blocks <= 256) {
+        if (nepi + nb_blocks > 0)
+            hipLaunchKernelGGL(k_vjp_epilogue_nonbond, dim3(nepi + nb_blocks), dim3(kB), lds, s, a,
+                               n, nepi);
+        return hipGetLastError();
+    }
+    if (nepi > 0) hipLaunchKernelGGL(k_vjp_epilogue, dim3(nepi), dim3(kB), 0, s, a);
+    if (nb_blocks > 0) hipLaunchKernelGGL(k_vjp_nonbond, dim3(nb_blocks), dim3(kB), lds, s, n);
     return hipGetLastError();
 }
 
@@ -677,14 +716,6 @@ hipError_t launch_vjp_atoms(const VjpArgs &a, int nblocks, hipStream_t s)
     VjpArgs b = a;
     b.ranked_from = ranked_from(nblocks);
     hipLaunchKernelGGL(k_vjp_atoms, dim3(nblocks), dim3(kB), 0, s, b);
-    return hipGetLastError();
-}
-
-hipError_t launch_vjp_nonbond(const VjpNbArgs &a, int nblocks, hipStream_t s)
-{
-    if (nblocks == 0) return hipSuccess;
-    const size_t lds = std::max(sizeof(float4) * a.T * a.T, nonbond_share_bytes(3));
-    hipLaunchKernelGGL(k_vjp_nonbond, dim3(nblocks), dim3(kB), lds, s, a);
     return hipGetLastError();
 }
 

@@ -497,13 +497,16 @@ __global__ __launch_bounds__(kBlock) void k_field_epilogue(EpilogueArgs a)
     epilogue_block<B>(a);
 }
 
-// The wide epilogue with an engine step's bonded and restraint blocks behind
-// its own: they depend on the coordinates alone, and a bonded block, a chain of
-// FP64 operations about as long as a point's epilogue, was the longest block of
-// the launch before the field pass (5.3 us at 1,100 atoms, the points 3.1).
+// The wide epilogue with other blocks behind its own.  An engine step's bonded
+// and restraint blocks depend on the coordinates alone, and a bonded block, a
+// chain of FP64 operations about as long as a point's epilogue, was the longest
+// block of the launch before the field pass (5.3 us at 1,100 atoms, the points
+// 3.1).  The differentiable model's all-pairs blocks were a launch of 6.4 us at
+// 550 atoms.
 __global__ __launch_bounds__(kBlock) void k_step_epilogue(EpilogueArgs a, RiderArgs r, int nepi)
 {
     __shared__ double red[6][kTermBlock];
+    extern __shared__ __align__(16) float2 lds_lj[];
     int b = (int)blockIdx.x - nepi;
     if (b < 0) {
         epilogue_block<8>(a);
@@ -513,8 +516,13 @@ __global__ __launch_bounds__(kBlock) void k_step_epilogue(EpilogueArgs a, RiderA
         bonded_one(r.bonded, b * kBlock + (int)threadIdx.x);
         return;
     }
-    us_block(b - r.bonded_blocks, r.us.boff, r.us.us_atoms, r.us.us_mass, r.us.kx, r.us.Ls, r.xyzq,
-             r.us.fus, r.us.com, true, red);
+    b -= r.bonded_blocks;
+    if (b < r.us.nres) {
+        us_block(b, r.us.boff, r.us.us_atoms, r.us.us_mass, r.us.kx, r.us.Ls, r.xyzq, r.us.fus,
+                 r.us.com, true, red);
+        return;
+    }
+    nonbond_block<false, false, false>(r.nb, b - r.us.nres, lds_lj);
 }
 
 // ---------------------------------------------------------------------------
@@ -1200,15 +1208,16 @@ static int rider_blocks(const RiderArgs &r)
 // blocks and 104 riders) takes 57.0 us, with the riders before the field 56.0
 bool epilogue_takes_riders(long long P, const RiderArgs &r)
 {
-    return P > 0 && blocks_for(P) + rider_blocks(r) + r.us.nres <= kEpiWideGrid;
+    return P > 0 && blocks_for(P) + rider_blocks(r) + r.us.nres + r.nb_blocks <= kEpiWideGrid;
 }
 
 hipError_t launch_step_epilogue(const EpilogueArgs &a, RiderArgs r, hipStream_t s)
 {
     const int eb = (int)blocks_for(a.Ptot);
     r.bonded_blocks = rider_blocks(r);
-    const int grid = eb + r.bonded_blocks + r.us.nres;
-    hipLaunchKernelGGL(k_step_epilogue, dim3(grid), dim3(kBlock), 0, s, a, r, eb);
+    const int grid = eb + r.bonded_blocks + r.us.nres + r.nb_blocks;
+    const size_t lds = r.nb_blocks ? nonbond_lds_bytes(r.nb.T, false) : 0;
+    hipLaunchKernelGGL(k_step_epilogue, dim3(grid), dim3(kBlock), lds, s, a, r, eb);
     return hipGetLastError();
 }
 

@@ -330,13 +330,15 @@ struct RestraintArgs {
     double *com;
 };
 
-// Bonded terms and restraints riding on another launch of an engine step, after
-// its own blocks (each part skipped when empty).
+// Bonded terms, restraints and all-pairs blocks (no super-tiles) riding on the
+// epilogue, after its own blocks (each part skipped when empty).
 struct RiderArgs {
     const float4 *xyzq;
     BondedArgs bonded;
     int bonded_blocks;      // set by the launcher
     RestraintArgs us;
+    NonbondArgs nb;
+    int nb_blocks;
 };
 
 // The IS-SPA pass of a model of small windows in one launch (k_window), with
@@ -479,6 +481,9 @@ struct DiffReduceArgs {
     const double *q;
     double *se;            // out [N][3]
     double *f;             // out [N][3] (overwritten)
+    const WinDesc *nb_wins;  // all-pairs partials added to f, or null
+    const double *nb_part;
+    long long nb_B;
 };
 struct VjpArgs {
     const WinDesc *wins;
@@ -529,13 +534,12 @@ struct VjpFinishArgs {
     double *gq;                // out [N]
     double *gatom;             // out [N][5]
 };
-hipError_t launch_diff_prep_types(const DiffPrepArgs &a, hipStream_t s);
-hipError_t launch_diff_prep_atoms(const DiffAtomArgs &a, hipStream_t s);
+hipError_t launch_diff_prep(const DiffPrepArgs &t, const DiffAtomArgs &a, hipStream_t s);
 hipError_t launch_diff_reduce(const DiffReduceArgs &a, hipStream_t s);
 hipError_t launch_vjp_points(const VjpArgs &a, int nblocks, hipStream_t s);
-hipError_t launch_vjp_epilogue(const VjpArgs &a, hipStream_t s);
+hipError_t launch_vjp_epilogue_nonbond(const VjpArgs &a, const VjpNbArgs &n, int nb_blocks,
+                                       hipStream_t s);
 hipError_t launch_vjp_atoms(const VjpArgs &a, int nblocks, hipStream_t s);
-hipError_t launch_vjp_nonbond(const VjpNbArgs &a, int nblocks, hipStream_t s);
 hipError_t launch_vjp_finish(const VjpFinishArgs &a, hipStream_t s);
 // part: scratch of 5 T type_reduce_ranges(n) doubles
 int type_reduce_ranges(int n);

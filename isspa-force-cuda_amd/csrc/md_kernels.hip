@@ -40,7 +40,7 @@ hipError_t launch_nonbond(const NonbondArgs &a, int nb, bool split, hipStream_t 
 }
 
 // sum [comps][B] partials over the window's chunks in order; comps == 3:
-// f += sum (or, with f null, o0 += sum in FP64); comps == 9: three FP64 outputs
+// f += sum; comps == 9: three FP64 outputs
 // sum over the partner chunks in the fixed slice order of reduce_device.hpp
 template <int COMPS>
 __global__ __launch_bounds__(kBlk) void k_chunk_reduce3(const WinDesc *__restrict__ wins,
@@ -63,15 +63,11 @@ __global__ __launch_bounds__(kBlk) void k_chunk_reduce3(const WinDesc *__restric
     combine_slices<COMPS>(red, al, sl, s);
     if (sl != 0 || !valid) return;
     if constexpr (COMPS == 3) {
-        if (f) {
-            float4 v = f[i];
-            v.x += (float)s[0];
-            v.y += (float)s[1];
-            v.z += (float)s[2];
-            f[i] = v;
-        } else {
-            for (int k = 0; k < 3; ++k) o0[3 * i + k] += s[k];
-        }
+        float4 v = f[i];
+        v.x += (float)s[0];
+        v.y += (float)s[1];
+        v.z += (float)s[2];
+        f[i] = v;
     } else {
         for (int k = 0; k < 3; ++k) {
             o0[3 * i + k] = s[k];

@@ -110,7 +110,7 @@ WindowArgs window_args(isspa_model *m, const float4 *x, uint32_t step, const uin
 ReduceArgs reduce_args(isspa_model *m, const float4 *x, float4 *f, double *flj, double *fpol,
                        double *fcdd);
 // the all-pairs term for positions x: split -> three FP64 component outputs;
-// otherwise f (float4, +=) or, with f null, o0 (double[N*3], +=)
+// otherwise f (float4, +=)
 int nonbond_run(nonbond_model *m, const float *xyzq4_d, bool split, float4 *f, double *o0,
                 double *o1, double *o2, hipStream_t s);
 // the same in two halves: per-chunk partials, then their fixed-order sum
@@ -119,6 +119,7 @@ int nonbond_run(nonbond_model *m, const float *xyzq4_d, bool split, float4 *f, d
 // to compute them here
 int nonbond_partials(nonbond_model *m, const float *xyzq4_d, bool split, hipStream_t s,
                      const int *pbc_flag = nullptr);
+NonbondArgs nonbond_args(nonbond_model *m, const float4 *x, const int *pbc_flag, bool split);
 int nonbond_flags(nonbond_model *m, const float4 *x, const int **flag, hipStream_t s);
 int nonbond_reduce(nonbond_model *m, bool split, float4 *f, double *o0, double *o1, double *o2,
                    hipStream_t s);
