@@ -91,48 +91,82 @@ __device__ __forceinline__ float diff_F(const DiffType &T, float d, float rinv)
     return 24.0f * T.ets * rinv * (2.0f * sr6 * sr6 - sr6) * diff_switch(T, d).S;
 }
 
-// values {g, E, F} and derivatives dv[5k + p]
-__device__ __forceinline__ void diff_all(const DiffType &T, float d, float rinv, float v[3],
-                                         float dv[15])
+// x / b for r = 1 / b rounded: a product, then two of Markstein's corrections
+// by the exact remainder (P. Markstein, IBM J. Res. Dev. 34, 1990), which leave
+// the correctly rounded quotient; 5 operations against 11 of the division
+__device__ __forceinline__ float div_by(float x, float b, float r)
 {
-    const DiffSwitch sw = diff_switch(T, d);
-    float dS[5];
-#pragma unroll
-    for (int p = 0; p < 5; ++p) dS[p] = -sw.dSdz * T.idel * T.drlo[p];
-#pragma unroll
-    for (int k = 0; k < 15; ++k) dv[k] = 0.0f;
+    float q = x * r;
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, x), r, q);
+    return __builtin_fmaf(__builtin_fmaf(-b, q, x), r, q);
+}
+
+// What the adjoint needs of a lane's type, kept in registers: the constants,
+// the reciprocals of the two it divides by, and d r_lo / d theta but for eps,
+// on which r_lo never depends.
+struct DiffVjpType {
+    float sts, ets, x0, g0, al, c, rlo, rhi, idel;
+    float eps2;            // 2 eps
+    float rsts, reps2;     // 1 / sts, 1 / (2 eps)
+    float d0, d2, d3, d4;  // d r_lo / d {sigma, x0, g0, al}
+    __device__ __forceinline__ explicit DiffVjpType(const DiffType &T)
+        : sts(T.sts), ets(T.ets), x0(T.x0), g0(T.g0), al(T.al), c(T.c), rlo(T.rlo), rhi(T.rhi),
+          idel(T.idel), eps2(2.0f * T.eps), rsts(1.0f / T.sts), reps2(1.0f / (2.0f * T.eps)),
+          d0(T.drlo[0]), d2(T.drlo[2]), d3(T.drlo[3]), d4(T.drlo[4])
+    {
+    }
+};
+
+// g and the derivatives of g, E and F by {sigma, x0, g0, al}, and of F by eps
+struct DiffDerivs {
+    float g;
+    float dg[4], dE[4], dF[4], dFeps;
+};
+
+__device__ __forceinline__ DiffDerivs diff_derivs(const DiffVjpType &T, float d, float rinv)
+{
+    DiffDerivs o;
+    const float z = (d - T.rlo) * T.idel + 1.0f;
+    float S = 0.0f, dSdz = 0.0f;
+    if (z >= 1.0f) {
+        S = 1.0f;
+    } else if (!(z <= 0.0f)) {  // NaN stays
+        S = z * z * (3.0f - 2.0f * z);
+        dSdz = 6.0f * z * (1.0f - z);
+    }
+    const float dS = -dSdz * T.idel;
+    const float dS0 = dS * T.d0, dS2 = dS * T.d2, dS3 = dS * T.d3, dS4 = dS * T.d4;
     const float u = d - T.x0;
-    // g
-    if (d >= T.rhi) {
-        v[0] = 1.0f;
-    } else {
+    o.g = 1.0f;
+    o.dg[0] = o.dg[1] = o.dg[2] = o.dg[3] = 0.0f;
+    if (!(d >= T.rhi)) {
         const float P = T.g0 - T.al * u * u;
-        if (P <= 0.0f) {
-            v[0] = 0.0f;
-        } else {
-            v[0] = sw.S * P;
-            const float dP[5] = {0.0f, 0.0f, 2.0f * T.al * u, 1.0f, -u * u};
-#pragma unroll
-            for (int p = 0; p < 5; ++p) dv[p] = dS[p] * P + sw.S * dP[p];
+        o.g = 0.0f;
+        if (!(P <= 0.0f)) {
+            o.g = S * P;
+            o.dg[0] = dS0 * P;
+            o.dg[1] = dS2 * P + S * (2.0f * T.al * u);
+            o.dg[2] = dS3 * P + S;
+            o.dg[3] = dS4 * P - S * (u * u);
         }
     }
-    // E
     const float Er = T.c * expf(-0.5f * u * u);
-    v[1] = Er * sw.S;
-#pragma unroll
-    for (int p = 0; p < 5; ++p) dv[5 + p] = Er * dS[p];
-    dv[7] += Er * u * sw.S;
-    // F
+    o.dE[0] = Er * dS0;
+    o.dE[1] = Er * dS2 + Er * u * S;
+    o.dE[2] = Er * dS3;
+    o.dE[3] = Er * dS4;
     const float sr = T.sts * rinv;
     const float sr2 = sr * sr;
     const float sr6 = sr2 * sr2 * sr2;
     const float FLJ = 24.0f * T.ets * rinv * (2.0f * sr6 * sr6 - sr6);
-    const float dFds = 24.0f * T.ets * rinv * (24.0f * sr6 * sr6 - 6.0f * sr6) / T.sts;
-    v[2] = FLJ * sw.S;
-#pragma unroll
-    for (int p = 0; p < 5; ++p) dv[10 + p] = FLJ * dS[p];
-    dv[10] += 0.5f * dFds * sw.S;
-    dv[11] += FLJ / (2.0f * T.eps) * sw.S;
+    const float dFds =
+        div_by(24.0f * T.ets * rinv * (24.0f * sr6 * sr6 - 6.0f * sr6), T.sts, T.rsts);
+    o.dF[0] = FLJ * dS0 + 0.5f * dFds * S;
+    o.dF[1] = FLJ * dS2;
+    o.dF[2] = FLJ * dS3;
+    o.dF[3] = FLJ * dS4;
+    o.dFeps = div_by(FLJ, T.eps2, T.reps2) * S;
+    return o;
 }
 
 }  // namespace isspa

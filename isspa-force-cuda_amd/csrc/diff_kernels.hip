@@ -355,7 +355,7 @@ __device__ __forceinline__ void vjp_epilogue_block(const VjpArgs &a)
 // ---------------------------------------------------------------------------
 template <bool PBC>
 __device__ __forceinline__ void vjp_atoms_tile(const VjpArgs &a, const float4 *__restrict__ pr,
-                                               const DiffType &Tj, int m0, int m1,
+                                               const DiffVjpType &Tj, int m0, int m1,
                                                const MinImage &mi, float4 xj, float R2j, float lpx,
                                                float lpy, float lpz, const Progress &pg, float &qb,
                                                double tb[5])
@@ -389,17 +389,19 @@ __device__ __forceinline__ void vjp_atoms_tile(const VjpArgs &a, const float4 *_
             qb = __builtin_fmaf(s, in_own ? er : er + e0r, qb);
             if (in_own || in_rec) {
                 const float d = d2 * rinv;
-                float v[3], dv[15];
-                diff_all(Tj, d, rinv, v, dv);
+                const DiffDerivs D = diff_derivs(Tj, d, rinv);
                 if (in_own) {
                     const float ce = er * rinv;
-                    const float cg = (eb.w != 0.0f && v[0] != 0.0f) ? eb.w / v[0] : 0.0f;
-                    for (int k = 0; k < 5; ++k) tb[k] += (double)(ce * dv[5 + k] + cg * dv[k]);
+                    const float cg = (eb.w != 0.0f && D.g != 0.0f) ? eb.w / D.g : 0.0f;
+                    tb[0] += (double)(ce * D.dE[0] + cg * D.dg[0]);
+                    for (int k = 1; k < 4; ++k) tb[k + 1] += (double)(ce * D.dE[k] + cg * D.dg[k]);
                 }
                 if (in_rec) {
                     const float lp = __builtin_fmaf(lpz, rz, __builtin_fmaf(lpy, ry, lpx * rx));
                     const float cf = e0b.w * lp * rinv;
-                    for (int k = 0; k < 5; ++k) tb[k] += (double)(cf * dv[10 + k]);
+                    tb[0] += (double)(cf * D.dF[0]);
+                    tb[1] += (double)(cf * D.dFeps);
+                    for (int k = 1; k < 4; ++k) tb[k + 1] += (double)(cf * D.dF[k]);
                 }
             }
         }
@@ -414,7 +416,9 @@ __device__ __forceinline__ void vjp_atoms_tile(const VjpArgs &a, const float4 *_
 // wave that are in a sphere.  The lane's type record stays in registers (read
 // from LDS through a flat pointer in the branch, each read waited for both
 // memories) and the next point is requested one point ahead: 52.8 -> 36 us at
-// 550 atoms, 985 -> 880 us at 32 x 1,100.  Six waves a SIMD: held to seven or
+// 550 atoms, 985 -> 880 us at 32 x 1,100.  Without the terms that are zero for
+// every type, and with the divisions by the type's constants as products
+// (div_by), 32 and 840 us.  Six waves a SIMD: held to seven or
 // eight the branch spills (934 us and worse), left alone it takes five (1,006).
 __global__ __launch_bounds__(kB, 6) void k_vjp_atoms(VjpArgs a)
 {
@@ -437,7 +441,7 @@ __global__ __launch_bounds__(kB, 6) void k_vjp_atoms(VjpArgs a)
     const float R2j = valid ? a.rmax2[tj] : -1.0f;
     const float4 lp = a.arec[4 * (size_t)j + 2];  // Lambda' = -vtot lambda
     const bool pbc = a.pbc_flag[bt.x] != 0;
-    const DiffType Tj = a.dtypes[tj];
+    const DiffVjpType Tj(a.dtypes[tj]);
     const MinImage mi = min_image_of(W.L, W.h);
     double qsum = 0.0, tb[5] = {0, 0, 0, 0, 0};  // q, theta
     Progress pg(a.ranked_from, m1 - m0);
