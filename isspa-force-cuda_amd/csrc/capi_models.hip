@@ -1029,9 +1029,10 @@ extern "C" int bonded_force(bonded_model *m, int terms, const float *xyzq4_d, fl
     if (!m || !xyzq4_d || !f4_d) return fail(ISSPA_ERR_ARG, "bonded_force: null argument");
     hipStream_t s = S(stream);
     CHK(bonded_terms(m, terms, xyzq4_d, s));
-    HIPCHK(launch_bonded_gather(m->contrib, m->gptr, m->gidx, m->n,
-                                reinterpret_cast<float4 *>(f4_d), s));
-    if (energies_d) HIPCHK(launch_bonded_energy(m->energy, m->nb, m->na, m->nd, energies_d, s));
+    HIPCHK(launch_bonded_gather(BondedSumArgs{m->contrib, m->gptr, m->gidx, m->n,
+                                              reinterpret_cast<float4 *>(f4_d), m->energy, m->nb,
+                                              m->na, m->nd, energies_d},
+                                s));
     return ISSPA_OK;
 }
 

@@ -429,8 +429,17 @@ hipError_t launch_chunk_reduce3(const WinDesc *wins, int nwin, const int *atom_w
 
 // ---- bonded ----
 hipError_t launch_bonded_terms(const BondedArgs &a, hipStream_t s);
-hipError_t launch_bonded_gather(const float4 *contrib, const int *ptr, const int *idx, int n,
-                                float4 *f, hipStream_t s);
+// the terms' forces summed per atom into f and, with energy, their energies
+struct BondedSumArgs {
+    const float4 *contrib;
+    const int *ptr, *idx;   // an atom's contribution slots
+    int n;
+    float4 *f;
+    const double *eterm;
+    int nb, na, nd;
+    double *energy;         // out [5], or null
+};
+hipError_t launch_bonded_gather(const BondedSumArgs &g, hipStream_t s);
 // The MD engine's step prologue: every launch of a step that depends only on
 // the coordinates, in one grid.  Each part is skipped when empty (nflag 0,
 // bonded.contrib null, us.nres 0, pts.ntot 0).
@@ -446,8 +455,6 @@ struct PrologueArgs {
 };
 hipError_t launch_step_prologue(PrologueArgs a, hipStream_t s);
 
-hipError_t launch_bonded_energy(const double *eterm, int nb, int na, int nd, double *out5,
-                                hipStream_t s);
 
 // ---- differentiable model: parameter preparation, forward reduction, adjoint ----
 struct DiffPrepArgs {
