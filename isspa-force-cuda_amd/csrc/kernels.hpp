@@ -21,7 +21,7 @@ struct WinDesc {
     int splits, aps;    // field pass: atom splits, atoms per split
     int chunks, ppc;    // force pass: point chunks, points per chunk
     int nbc, apc;       // nonbond: groups of kNbGroup partner chunks, atoms per chunk
-    long long fpo;      // field partial offset:  sum over earlier windows of splits * P
+    long long fpo;      // field partial offset:  sum over earlier windows of splits / fg * P
     long long ppo;      // force partial offset:  sum of fents * n
     long long npo;      // nonbond partial offset: sum of nbc * n (nbc entries per atom)
     uint32_t sys;       // Philox counter word 3
@@ -440,8 +440,8 @@ struct BondedSumArgs {
     double *energy;         // out [5], or null
 };
 hipError_t launch_bonded_gather(const BondedSumArgs &g, hipStream_t s);
-// The MD engine's step prologue: every launch of a step that depends only on
-// the coordinates, in one grid.  Each part is skipped when empty (nflag 0,
+// The MD engine's step prologue: what of a step depends only on the coordinates
+// and does not ride on the epilogue, in one grid.  Each part is skipped when empty (nflag 0,
 // bonded.contrib null, us.nres 0, pts.ntot 0).
 struct PrologueArgs {
     int nflag;              // minimum-image flags of the IS-SPA windows

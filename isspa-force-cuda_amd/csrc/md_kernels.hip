@@ -414,10 +414,10 @@ hipError_t launch_us(int nres, const int *boff, const int2 *atoms, const float *
 }
 
 // ---------------------------------------------------------------------------
-// MD engine step prologue: the launches of a step that depend only on the
-// coordinates, as block ranges of one grid -- minimum-image flags (one block
-// per window), bonded terms (256 terms a block), restraints (one block each,
-// bias forces stored for the force assembly) and the MC points.
+// MD engine step prologue: what of a step depends only on the coordinates and
+// does not ride on the epilogue, as block ranges of one grid -- minimum-image
+// flags (one block per window), bonded terms (256 terms a block), restraints
+// (one block each, bias forces stored for the force assembly) and the MC points.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kBlk) void k_step_prologue(PrologueArgs a)
 {

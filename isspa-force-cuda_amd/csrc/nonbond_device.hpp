@@ -328,7 +328,7 @@ __device__ __forceinline__ bool nonbond_images(const int *pbc_flag, int w)
 
 // block blk of the all-pairs grid; lds_lj holds T*T float2 (dynamic LDS),
 // followed, with SYM, by kSymLdsDoubles doubles (8-byte aligned).  SPLIT
-// writes the ordered layout (npo, one entry per partner chunk); the total
+// writes the ordered layout (npo, one entry per group of partner chunks); the total
 // force writes the total-mode layout (spo, nte entries per atom).  SYM
 // compiles the super-tile kinds in (the field launch that carries the
 // all-pairs blocks of small systems has none).

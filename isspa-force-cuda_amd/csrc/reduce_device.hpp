@@ -120,7 +120,7 @@ struct PlanarEntry {
 };
 
 // all-pairs partials of atom i (COMPS = 3: the total force, entries of the
-// total-force layout; 9: the split components, one entry per partner chunk)
+// total-force layout; 9: the split components, one per group of partner chunks)
 template <int COMPS>
 __device__ __forceinline__ PlanarEntry<COMPS> nonbond_entry(const WinDesc &W, const double *part,
                                                             long long B, int i)
