@@ -1336,8 +1336,11 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
     // without the side stream the all-pairs blocks ride on the small-window or
     // the field launch (which carry partner-chunk blocks only: windows large
     // enough for super-tiles always have the side stream)
-    const bool nb_rides = m && e->nb && !fork && !e->nb->any_sym;
-    if (m && isspa_is_small(m)) {
+    const bool small = m && isspa_is_small(m);
+    // (k_window has LDS of its own beside the LJ table: over 128 LJ types the
+    // all-pairs term keeps its launch there)
+    const bool nb_rides = m && e->nb && !fork && !e->nb->any_sym && (!small || e->nb->T <= 128);
+    if (small) {
         WindowArgs w = window_args(m, x4, 0u, e->step_d + kStepNext);
         w.step_now = e->step_d + kStepNow;
         w.bonded = bonded;

@@ -441,7 +441,7 @@ __global__ __launch_bounds__(kBlk) void k_step_prologue(PrologueArgs a)
         return;
     }
     b -= a.us.nres;
-    if (a.pts.ntot > 0) mc_points_block(a.pts, b);
+    if ((long long)a.pts.ntot * a.pts.nmc > 0) mc_points_block(a.pts, b);
 }
 
 hipError_t launch_step_prologue(PrologueArgs a, hipStream_t s)

@@ -168,7 +168,10 @@ class GpuSystem:
 
     def isspa_components(self, step: int = 0):
         n = self.system.n_atoms
-        out = [torch.zeros((n, 3), dtype=torch.float64, device=self.dev) for _ in range(3)]
+        # written whole by the call, so not filled first (as in the calls below):
+        # the six fills of the two component calls were a tenth of their time at
+        # 1,100 atoms
+        out = [torch.empty((n, 3), dtype=torch.float64, device=self.dev) for _ in range(3)]
         check(capi.lib.isspa_model_force_components(self.isspa, ptr(self.x), ptr(out[0]),
                                                     ptr(out[1]), ptr(out[2]), step, self.stream()),
               "isspa_model_force_components")
@@ -176,11 +179,11 @@ class GpuSystem:
 
     def field(self):
         P = self.system.n_points
-        o = dict(pts=torch.zeros((P, 4), dtype=torch.float32, device=self.dev),
-                 g=torch.zeros(P, dtype=torch.float64, device=self.dev),
-                 cnt=torch.zeros(P, dtype=torch.int32, device=self.dev),
-                 E=torch.zeros((P, 3), dtype=torch.float64, device=self.dev),
-                 E0=torch.zeros((P, 3), dtype=torch.float64, device=self.dev))
+        o = dict(pts=torch.empty((P, 4), dtype=torch.float32, device=self.dev),
+                 g=torch.empty(P, dtype=torch.float64, device=self.dev),
+                 cnt=torch.empty(P, dtype=torch.int32, device=self.dev),
+                 E=torch.empty((P, 3), dtype=torch.float64, device=self.dev),
+                 E0=torch.empty((P, 3), dtype=torch.float64, device=self.dev))
         check(capi.lib.isspa_model_get_field(self.isspa, ptr(o["pts"]), ptr(o["g"]), ptr(o["cnt"]),
                                              ptr(o["E"]), ptr(o["E0"]), self.stream()))
         return o
@@ -211,7 +214,7 @@ class GpuSystem:
 
     def nonbond_components(self):
         n = self.system.n_atoms
-        out = [torch.zeros((n, 3), dtype=torch.float64, device=self.dev) for _ in range(3)]
+        out = [torch.empty((n, 3), dtype=torch.float64, device=self.dev) for _ in range(3)]
         check(capi.lib.nonbond_force_components(self.nonbond, ptr(self.x), ptr(out[0]),
                                                 ptr(out[1]), ptr(out[2]), self.stream()),
               "nonbond_force_components")
@@ -219,7 +222,7 @@ class GpuSystem:
 
     def bonded_force(self, terms: int = capi.TERM_ALL, f: Optional[torch.Tensor] = None):
         f = self.f if f is None else f
-        e = torch.zeros(5, dtype=torch.float64, device=self.dev)
+        e = torch.empty(5, dtype=torch.float64, device=self.dev)
         check(capi.lib.bonded_force(self.bonded, terms, ptr(self.x), ptr(f), ptr(e),
                                     self.stream()), "bonded_force")
         return f, e
