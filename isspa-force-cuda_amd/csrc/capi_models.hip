@@ -441,7 +441,7 @@ ReduceArgs reduce_args(isspa_model *m, const float4 *x, float4 *f, double *flj, 
 // whether the total force runs as k_window (small windows)
 bool isspa_is_small(const isspa_model *m)
 {
-    return window_fits(m->tv, m->max_win_atoms, m->max_group_pts, m->nwblk);
+    return window_fits(m->tv, m->lay.W, m->max_win_atoms, m->max_group_pts, m->nwblk);
 }
 
 WindowArgs window_args(isspa_model *m, const float4 *x, uint32_t step, const uint32_t *step_d)

@@ -1,6 +1,6 @@
 """The small-window launch (points, field, epilogue and force in one block) on
 both sides of its limits and at its edges: window sizes around 64, 128, 192 and
-256 atoms (256 is the largest it takes), chunk groups of one point, of a whole
+256 atoms (144 is the largest it takes of a window alone, 256 of a batch), chunk groups of one point, of a whole
 number of waves and one more, and of the largest 256 points; every split count
 from one to more than a pass holds; boxes with and without images.
 
@@ -84,6 +84,35 @@ def test_sixteen_waves(n, n_mc, tiling):
     block has sixteen above it, with receiver groups of one wave, a share pair
     and more units than waves."""
     _check(_atoms(n, n_mc), tiling)
+
+
+@pytest.mark.parametrize("n", [143, 144, 145, 192, 193, 255, 256, 257])
+@pytest.mark.parametrize("n_mc,tiling", [(3, None), (1, (5, 9)), (2, (32, 40))])
+def test_two_windows(n, n_mc, tiling):
+    """The launch of a batch, forces against the component pass and the oracle
+    of each window, and against the window alone at the same tiling, which
+    above 144 atoms takes the separate launches: the same bit for bit."""
+    w = _atoms(n, n_mc)
+    m = batch.merge_windows([w, w], [0, 1])
+    # (the cut chain's exclusions reach past its window: no all-pairs term)
+    g = GpuSystem(m, "cuda:0", us=False, nonbond=False)
+    if tiling:
+        g.set_tiling(*tiling)
+    print(f"2 x {n} atoms, nMC={n_mc}, tiling {g.tiling()}", flush=True)
+    g.zero_forces()
+    tot = g.isspa_force(step=4).clone()
+    comp = g.isspa_components(step=4)
+    part = comp["lj"] + comp["pol"] + comp["cdd"]
+    assert max_abs_rel_rms(tot[:, :3].double().cpu().numpy(), part.cpu().numpy()) <= 2e-6
+    if tiling:
+        h = GpuSystem(w, "cuda:0", us=False, nonbond=False)
+        h.set_tiling(*tiling)
+        h.zero_forces()
+        assert torch.equal(h.isspa_force(step=4)[:, :3], tot[:n, :3])
+        h.close()
+    ref = po.isspa_total(w, step=4)["total"]
+    assert max_abs_rel_rms(tot[:n, :3].double().cpu().numpy(), ref) <= 1e-5
+    g.close()
 
 
 @pytest.mark.parametrize("pairs,small,big", [(3, 2, 1), (0, 1, 2), (5, 0, 0)])
