@@ -866,14 +866,15 @@ __global__ __launch_bounds__(kBlock) void k_force(ForceArgs a)
 // The step's all-pairs, bonded and restraint blocks, which depend on the
 // coordinates alone, ride on the launch (work-items from 256 up leave).
 // ---------------------------------------------------------------------------
-// A window alone, above 144 atoms, gains nothing from having each group of
-// points in one block: the blocks are few and the separate passes spread the
+// Where every window has more than 144 atoms, having each group of points in one
+// block gains nothing: the blocks are few and the separate passes spread the
 // same chains over the chip.  Engine step of 132 atoms, nMC = 20, 25.5 us here
 // and 29.3 in the separate launches, of 154 atoms 32.6 and 30.9, of 242 atoms
 // 36.5 and 33.6; their solvent force 23.0 and 26.7, 28.2 and 24.2, 32.1 and
-// 27.4.  A batch has the blocks: 39.7 and 44.4 us with four windows of 242 atoms
-// beside eight small ones.
-constexpr int kWinMaxAtoms = 256, kWinLoneAtoms = 144;
+// 27.4; three windows of 242 atoms, nMC = 40, 49.6 and 45.1.  With smaller
+// windows among them the launch wins again: 37.5 and 40.8 us for four windows of
+// 242 atoms and one of 44.
+constexpr int kWinMaxAtoms = 256, kWinMinAtoms = 144;
 constexpr int kWinMaxPts = 256;
 // One round of two blocks a CU.  More blocks are throughput, not latency: a
 // step takes 29.0 us here against 37.5 in the separate launches with 474
@@ -1253,9 +1254,9 @@ static int window_lds(const TableView &t, int nt, int max_points, WindowArgs &a)
     return a.off_x + std::max(nxc, nsh);
 }
 
-bool window_fits(const TableView &t, int nwin, int max_atoms, int max_points, int nblocks)
+bool window_fits(const TableView &t, int min_atoms, int max_atoms, int max_points, int nblocks)
 {
-    return max_atoms <= (nwin == 1 ? kWinLoneAtoms : kWinMaxAtoms) && max_points <= kWinMaxPts &&
+    return min_atoms <= kWinMinAtoms && max_atoms <= kWinMaxAtoms && max_points <= kWinMaxPts &&
            nblocks <= kWinMaxBlocks && field_tab_floats(t) <= kTabLdsFloats &&
            force_tab_floats(t) <= kTabLdsFloats;
 }

@@ -382,7 +382,7 @@ hipError_t launch_step_epilogue(const EpilogueArgs &a, RiderArgs r, hipStream_t 
 // k_window: whether a model's windows, chunk groups and tables fit it, and the
 // launch (max_atoms, max_points: of the largest window and chunk group;
 // max_items: the most (point, field split) pairs of a group)
-bool window_fits(const TableView &t, int nwin, int max_atoms, int max_points, int nblocks);
+bool window_fits(const TableView &t, int min_atoms, int max_atoms, int max_points, int nblocks);
 hipError_t launch_window(const WindowArgs &a, int max_points, int max_items, hipStream_t s);
 hipError_t launch_force(const ForceArgs &a, int nblocks, bool split, hipStream_t s);
 hipError_t launch_force_reduce(const ReduceArgs &a, bool split, hipStream_t s);

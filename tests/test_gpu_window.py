@@ -1,6 +1,6 @@
 """The small-window launch (points, field, epilogue and force in one block) on
 both sides of its limits and at its edges: window sizes around 64, 128, 192 and
-256 atoms (144 is the largest it takes of a window alone, 256 of a batch), chunk groups of one point, of a whole
+256 atoms (it takes windows up to 256 atoms if one has at most 144), chunk groups of one point, of a whole
 number of waves and one more, and of the largest 256 points; every split count
 from one to more than a pass holds; boxes with and without images.
 
@@ -89,16 +89,17 @@ def test_sixteen_waves(n, n_mc, tiling):
 @pytest.mark.parametrize("n", [143, 144, 145, 192, 193, 255, 256, 257])
 @pytest.mark.parametrize("n_mc,tiling", [(3, None), (1, (5, 9)), (2, (32, 40))])
 def test_two_windows(n, n_mc, tiling):
-    """The launch of a batch, forces against the component pass and the oracle
-    of each window, and against the window alone at the same tiling, which
-    above 144 atoms takes the separate launches: the same bit for bit."""
+    """A window and a small one, which bring both into the launch up to 256
+    atoms: forces against the component pass and the oracle, and against the
+    window alone at the same tiling, which above 144 atoms takes the separate
+    launches: the same bit for bit."""
     w = _atoms(n, n_mc)
-    m = batch.merge_windows([w, w], [0, 1])
+    m = batch.merge_windows([w, _atoms(22, n_mc)], [0, 1])
     # (the cut chain's exclusions reach past its window: no all-pairs term)
     g = GpuSystem(m, "cuda:0", us=False, nonbond=False)
     if tiling:
         g.set_tiling(*tiling)
-    print(f"2 x {n} atoms, nMC={n_mc}, tiling {g.tiling()}", flush=True)
+    print(f"{n} and 22 atoms, nMC={n_mc}, tiling {g.tiling()}", flush=True)
     g.zero_forces()
     tot = g.isspa_force(step=4).clone()
     comp = g.isspa_components(step=4)
