@@ -763,13 +763,12 @@ extern "C" int nonbond_model_create_batch(int n, int T, const int *ityp, const i
         TRY(upload(&m->excl_idx, fidx.data(), std::max<size_t>(1, fidx.size())));
     }
     TRY(dalloc(&m->pbc_flag, Ly.W));
-    double pairs = 0.0;
     m->all_images = true;
     for (int w = 0; w < Ly.W; ++w) {
-        pairs += (double)Ly.n[w] * Ly.n[w];
+        m->pairs += (double)Ly.n[w] * Ly.n[w];
         m->all_images = m->all_images && std::isfinite(Ly.L[w]);
     }
-    m->all_images = m->all_images && pairs <= 4096.0 * 4096.0;
+    m->all_images = m->all_images && m->pairs <= kManyPairs;
     TRY(upload(&m->atom_win, Ly.atom_win.data(), Ly.atom_win.size()));
     TRY(upload(&m->wins, m->wins_h.data(), m->wins_h.size()));
     TRY(upload(&m->blk, blv.data(), blv.size()));
@@ -1161,7 +1160,7 @@ extern "C" int us_force(us_model *m, const float *xyzq4_d, float *f4_d, double *
 // ---------------------------------------------------------------------------
 // MD engine: one step = zero f, bonded, IS-SPA, nonbond, US, leap-frog, step++
 // (order of src/total_force_cuda.cpp:109-153), as five launches: prologue,
-// field (+ all-pairs below kForkMinAtoms), epilogue (+ bonded, restraints),
+// field (+ all-pairs below kManyPairs), epilogue (+ bonded, restraints),
 // force, assembly, or, for small windows, two: k_window and the assembly (which
 // also integrates and advances the step); see engine_forces.
 // ---------------------------------------------------------------------------
@@ -1194,8 +1193,6 @@ struct md_engine {
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
 };
-
-constexpr int kForkMinAtoms = 4096;
 
 // Destroys the executable graph and its graph once the last replay has ended
 // (a replay still in flight reads the executable's kernel arguments).
@@ -1268,9 +1265,10 @@ extern "C" int md_engine_create(isspa_model *isspa, nonbond_model *nb, bonded_mo
         if (he == hipSuccess) he = hipEventCreateWithFlags(&e->ev_replayed, hipEventDisableTiming);
         if (he != hipSuccess) rc = fail(ISSPA_ERR_HIP, "md_engine_create: %s", hipGetErrorString(he));
     }
-    // below a few thousand atoms the all-pairs kernel is a few microseconds and
-    // the fork and join would cost more than the overlap saves
-    if (rc == ISSPA_OK && isspa && nb && n >= kForkMinAtoms) {
+    // up to 4,096^2 pairs the all-pairs kernel is a few microseconds and the fork
+    // and join cost more than the overlap saves: 56 umbrella windows, 5,632 atoms
+    // but 1.0e6 pairs, take 67.7 us a step beside the field pass and 58.2 riding on it
+    if (rc == ISSPA_OK && isspa && nb && nb->pairs >= kManyPairs) {
         hipError_t he = hipStreamCreateWithFlags(&e->side, hipStreamNonBlocking);
         if (he == hipSuccess) he = hipEventCreateWithFlags(&e->ev_fork, hipEventDisableTiming);
         if (he == hipSuccess) he = hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming);

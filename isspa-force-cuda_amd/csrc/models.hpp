@@ -71,6 +71,9 @@ struct isspa_model {
     unsigned generation = 0;
 };
 
+// from here on the all-pairs term has flags, and in an engine step a stream, of its own
+constexpr double kManyPairs = 4096.0 * 4096.0;
+
 struct nonbond_model {
     Windows lay;
     int n = 0, T = 0;
@@ -80,6 +83,7 @@ struct nonbond_model {
     uint32_t *excl = nullptr;
     int *excl_ptr = nullptr, *excl_idx = nullptr;
     int *pbc_flag = nullptr, *atom_win = nullptr;
+    double pairs = 0.0;       // ordered pairs, over the windows
     bool all_images = false;  // every pair takes its image, no flags (nonbond_flags)
     std::vector<WinDesc> wins_h;
     WinDesc *wins = nullptr;

@@ -66,7 +66,8 @@ def test_riders_around_256_blocks(chains, n_mc):
     _check(s)
 
 
-@pytest.mark.parametrize("pairs,small,big", [(0, 3, 2), (2, 40, 4), (40, 16, 8)])
+@pytest.mark.parametrize("pairs,small,big", [(0, 3, 2), (2, 40, 4), (40, 16, 8), (0, 40, 16)])
 def test_riders_with_restraints(pairs, small, big):
-    """Restraint blocks behind the epilogue, or, with many windows, before."""
+    """Restraint blocks behind the epilogue, or, with many windows, before; the
+    last batch has more than 4,096 atoms, its all-pairs blocks ride all the same."""
     _check(batch.merge_windows(batch.umbrella_windows(pairs, small, big, n_mc=20)))
