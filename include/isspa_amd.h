@@ -161,9 +161,12 @@ int isspa_model_get_field(isspa_model *m, float *pts4_d, double *g_d, int *cnt_d
                           double *E0_d, void *stream);
 /* Stage timing for tuning and roofline accounting (no reference counterpart;
  * the reference times whole wrappers with events, src/timing_class.cpp):
- * runs each stage once untimed and then `reps` times back to back between
- * two events on `stream`, and returns the mean milliseconds per launch in
- * ms[5] = {points, field, epilogue, force, force reduction}.  Uses the
+ * runs each launch of isspa_model_force once untimed and then `reps` times back
+ * to back between two events on `stream`, and returns the mean milliseconds per
+ * launch in ms[5] = {points, field, epilogue, force, force reduction}.  Where
+ * the model's windows take the small-window launch, which does the first four
+ * stages at once, its time is in the force entry and the three before it are 0.
+ * Which launches run depends on the tiling (isspa_model_set_tiling).  Uses the
  * positions xyzq4_d; leaves caller buffers untouched.  Synchronous. */
 int isspa_model_profile(isspa_model *m, const float *xyzq4_d, int reps, float *ms, void *stream);
 /* Tuning knobs (0 = automatic): atom splits of the field pass, point chunks of

@@ -527,8 +527,14 @@ extern "C" int isspa_model_profile(isspa_model *m, const float *xyzq4_d, int rep
     HIPCHK(hipEventCreate(&ev[0]));
     HIPCHK(hipEventCreate(&ev[1]));
     int rc = ISSPA_OK;
-    hipError_t e = launch_pbc_flag(m->wins, m->lay.W, x, m->rmax_all, m->pbc_flag, s);
+    const bool small = isspa_is_small(m);  // the route of isspa_total
+    hipError_t e = hipSuccess;
+    if (!small) e = launch_pbc_flag(m->wins, m->lay.W, x, m->rmax_all, m->pbc_flag, s);
     for (int stage = 0; stage < 5 && rc == ISSPA_OK && e == hipSuccess; ++stage) {
+        if (small && stage < 3) {
+            ms[stage] = 0.f;  // inside the small-window launch
+            continue;
+        }
         // one untimed launch, then `reps` timed back-to-back launches
         for (int r = 0; r <= reps && e == hipSuccess; ++r) {
             if (r == 1) e = hipEventRecord(ev[0], s);
@@ -540,7 +546,11 @@ extern "C" int isspa_model_profile(isspa_model *m, const float *xyzq4_d, int rep
                 break;
             case 1: e = launch_field(field_args(m, x), m->ngblk, s); break;
             case 2: e = launch_epilogue(epilogue_args(m, false), s); break;
-            case 3: e = launch_force(force_args(m, x), m->npblk, false, s); break;
+            case 3:
+                e = small ? launch_window(window_args(m, x, 0u, nullptr), m->max_group_pts,
+                                          m->max_group_items, s)
+                          : launch_force(force_args(m, x), m->npblk, false, s);
+                break;
             default:
                 e = launch_force_reduce(reduce_args(m, x, m->prof_f, nullptr, nullptr, nullptr),
                                         false, s);

@@ -9,7 +9,10 @@ the wave targets tried are multiples of a round.  The library's automatic
 choice aims at a target wave count shared among windows in proportion to
 their work; this tuner measures
 candidates on the device with isspa_model_profile (HIP events around
-back-to-back launches of each stage) and keeps the fastest.
+back-to-back launches of each stage) and keeps the fastest.  The profile times
+the launches that the force calls make at that tiling: the separate passes, or
+the small-window launch, and the tiling itself can move a model of small
+windows from one to the other.
 
 Two candidate families:
   * target wave counts (the automatic per-window choice at several targets),
@@ -18,7 +21,8 @@ Two candidate families:
     the best wave target, plus the pair of the best split count and the best
     chunk count found separately.  The field pass and its epilogue depend only
     on the split count and the force pass and its reduction only on the chunk
-    count, so each is searched on its own stages: for a single system over
+    count, so each is searched on its own stages (on whole passes where a
+    candidate runs as one launch): for a single system over
     counts whose grid fills at least 85% of its last round of wave slots, for
     a batch over x0.25..x2 of the largest window's counts (an explicit tiling
     applies to every window, clamped to its size).
@@ -40,7 +44,9 @@ import dataclasses
 import math
 from typing import List, Optional, Sequence, Tuple
 
-PASS_STAGES = ("field", "epilogue", "force", "reduce")
+# the whole pass, so that a tiling that runs as the small-window launch (reported
+# as the force stage, with 0 before it) compares with one that runs in separate passes
+PASS_STAGES = ("points", "field", "epilogue", "force", "reduce")
 FIELD_STAGES = ("field", "epilogue")
 FORCE_STAGES = ("force", "reduce")
 WAVE_SLOTS = 8192        # 256 CUs x 4 SIMDs x 8 resident waves
@@ -56,9 +62,9 @@ class TuneResult:
     measure: str = "IS-SPA pass"  # what `ms` times: "IS-SPA pass" or the confirmation's measure
 
 
-def _measure(g, reps: int, stages=PASS_STAGES) -> float:
+def _measure(g, reps: int) -> float:
     prof = g.profile(reps)
-    return sum(prof[k] for k in stages)
+    return sum(prof[k] for k in PASS_STAGES)
 
 
 def engine_forces_ms(g, reps: int) -> float:
@@ -178,10 +184,15 @@ def tune(g, reps: int = 3, waves: Sequence[int] = (8192, 16384, 24576, 32768, 49
         for kind, cands, stages, pick in (
                 ("field-splits", split_c, FIELD_STAGES, lambda v: (v, c0)),
                 ("force-chunks", chunk_c, FORCE_STAGES, lambda v: (s0, v))):
-            stage_ms = []
+            profs = []
             for v in cands:
                 g.set_tiling(*pick(v))
-                ms = _measure(g, reps, stages)
+                profs.append(g.profile(reps))
+            if any(prof["field"] == 0.0 for prof in profs):
+                stages = PASS_STAGES  # some run as one launch: whole passes compare
+            stage_ms = []
+            for v, prof in zip(cands, profs):
+                ms = sum(prof[k] for k in stages)
                 stage_ms.append((ms, v))
                 table.append((kind, (v,), ms))
                 if log:

@@ -189,7 +189,8 @@ class GpuSystem:
         return o
 
     def profile(self, reps: int = 5):
-        """Mean ms per launch of {points, field, epilogue, force, reduce}."""
+        """Mean ms per launch of {points, field, epilogue, force, reduce} of
+        isspa_force; the first three are 0 where one launch does the four."""
         ms = (C.c_float * 5)()
         check(capi.lib.isspa_model_profile(self.isspa, ptr(self.x), reps, ms, self.stream()),
               "isspa_model_profile")
