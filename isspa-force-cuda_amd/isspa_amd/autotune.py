@@ -126,7 +126,15 @@ def effective_pieces(n: int, pieces: int) -> int:
     return -(-n // per)
 
 
-def round_fill(blocks: int, pieces: int) -> float:
+def force_blocks(n: int) -> float:
+    """Blocks of the force pass per point chunk of an n-atom window: a block's four
+    waves take the same 64 atoms and a share each, a share being a whole chunk, or
+    a half (quarter) of one in windows of at most 128 (64) atoms."""
+    shares = 4 if n <= 64 else 2 if n <= 128 else 1
+    return -(-n // 64) * shares / WAVES_PER_BLOCK
+
+
+def round_fill(blocks: float, pieces: int) -> float:
     """Fraction of the last round of wave slots that a grid of blocks x pieces
     256-thread blocks fills (1.0 = whole rounds)."""
     rounds = blocks * pieces * WAVES_PER_BLOCK / WAVE_SLOTS
@@ -134,7 +142,7 @@ def round_fill(blocks: int, pieces: int) -> float:
     return 1.0 if last == 0.0 else last
 
 
-def round_aligned(n: int, blocks: int, base: int, lo: float = 0.5, hi: float = 2.0,
+def round_aligned(n: int, blocks: float, base: int, lo: float = 0.5, hi: float = 2.0,
                   min_fill: float = 0.85, limit: int = 6) -> List[int]:
     """Piece counts of `n` items between lo*base and hi*base whose grid
     (`blocks` blocks per piece) fills at least `min_fill` of its last round,
@@ -176,7 +184,7 @@ def tune(g, reps: int = 3, waves: Sequence[int] = (8192, 16384, 24576, 32768, 49
         if g.windows is None:
             n, P = g.system.n_atoms, g.system.n_points
             split_c = round_aligned(n, -(-P // 256), s0)
-            chunk_c = round_aligned(P, -(-n // 256), c0)
+            chunk_c = round_aligned(P, force_blocks(n), c0)
         else:
             split_c = sorted({max(1, s0 // 4), max(1, s0 // 2), s0, 2 * s0})
             chunk_c = sorted({max(1, c0 // 4), max(1, c0 // 2), c0, 2 * c0})

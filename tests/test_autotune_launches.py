@@ -1,9 +1,25 @@
 """The autotuner on models whose force call takes the small-window launch at some
 tilings (no GPU): isspa_model_profile then reports that launch as the force stage
 and the passes inside it as 0."""
+import math
+
 import pytest
 
 from isspa_amd import autotune
+
+
+@pytest.mark.parametrize("n", [1, 44, 64, 65, 128, 129, 1100, 4510, 19998])
+def test_force_blocks_follow_the_grid(n):
+    """The force pass launches ceil(n / 64) blocks for each group of chunks; four
+    chunks are four groups with four shares of a chunk a block, two with two."""
+    shares = 4 if n <= 64 else 2 if n <= 128 else 1
+    assert 4 * autotune.force_blocks(n) == math.ceil(n / 64) * shares
+    if n == 19998:
+        # whole groups of four chunks: the grid of the candidate counts
+        for c in autotune.round_aligned(n * 20, autotune.force_blocks(n), 208)[:-1]:
+            if c % 4 == 0 and c != 208:
+                rounds = math.ceil(n / 64) * (c // 4) * 4 / 8192
+                assert rounds == int(rounds) or rounds % 1 >= 0.85
 
 
 class _Model:
