@@ -152,7 +152,6 @@ static int isspa_tile(isspa_model *m)
                                std::max(kMinAutoWaves, (long)(m->P / kPointsPerWave)));
     m->wins_h.assign(L.W, WinDesc{});
     m->max_win_atoms = m->max_group_pts = m->max_group_items = 0;
-    m->min_win_atoms = m->d.n_atoms;
     m->max_fg = 1;
     long long F = 0, C = 0, V = 0;
     std::vector<std::pair<long long, int4>> gb, pb, vb, wb;
@@ -175,7 +174,6 @@ static int isspa_tile(isspa_model *m)
         d.ppc = (int)((P + c - 1) / c);
         d.chunks = (int)((P + d.ppc - 1) / d.ppc);
         m->max_win_atoms = std::max(m->max_win_atoms, (int)n);
-        m->min_win_atoms = std::min(m->min_win_atoms, (int)n);
         const int group = force_group((int)n), shares = force_shares((int)n);
         m->max_group_pts = std::max(m->max_group_pts, (int)std::min(P, (long long)group * d.ppc));
         m->max_group_items = std::max<long long>(
@@ -234,6 +232,7 @@ static int isspa_tile(isspa_model *m)
     m->npblk = (int)pbv.size();
     m->nvblk = (int)vbv.size();
     m->nwblk = (int)wbv.size();
+    m->win_pays = window_pays(m->wins_h.data(), L.W, nmc, m->nwblk, m->max_group_items);
     m->F = F;
     m->C = C;
     m->V = V;
@@ -443,7 +442,7 @@ ReduceArgs reduce_args(isspa_model *m, const float4 *x, float4 *f, double *flj, 
 // whether the total force runs as k_window (small windows)
 bool isspa_is_small(const isspa_model *m)
 {
-    return window_fits(m->tv, m->min_win_atoms, m->max_win_atoms, m->max_group_pts, m->nwblk);
+    return m->win_pays && window_fits(m->tv, m->max_win_atoms, m->max_group_pts, m->nwblk);
 }
 
 WindowArgs window_args(isspa_model *m, const float4 *x, uint32_t step, const uint32_t *step_d)

@@ -866,15 +866,13 @@ __global__ __launch_bounds__(kBlock) void k_force(ForceArgs a)
 // The step's all-pairs, bonded and restraint blocks, which depend on the
 // coordinates alone, ride on the launch (work-items from 256 up leave).
 // ---------------------------------------------------------------------------
-// Where every window has more than 144 atoms, having each group of points in one
-// block gains nothing: the blocks are few and the separate passes spread the
-// same chains over the chip.  Engine step of 132 atoms, nMC = 20, 25.5 us here
-// and 29.3 in the separate launches, of 154 atoms 32.6 and 30.9, of 242 atoms
-// 36.5 and 33.6; their solvent force 23.0 and 26.7, 28.2 and 24.2, 32.1 and
-// 27.4; three windows of 242 atoms, nMC = 40, 49.6 and 45.1.  With smaller
-// windows among them the launch wins again: 37.5 and 40.8 us for four windows of
-// 242 atoms and one of 44.
-constexpr int kWinMaxAtoms = 256, kWinMinAtoms = 144;
+// Windows alone of more than 144 atoms gain nothing from having each group of points
+// in one block: the blocks are few and the separate passes spread the same chains over
+// the chip.  Engine step of 132 atoms, nMC = 20, 25.5 us here and 29.3 in the separate
+// launches, of 154 atoms 32.6 and 30.9, of 242 atoms 36.5 and 33.6; their solvent force
+// 23.0 and 26.7, 28.2 and 24.2, 32.1 and 27.4.  Batches with windows on both sides
+// follow window_pays.
+constexpr int kWinMaxAtoms = 256, kWinSmallAtoms = 144;
 constexpr int kWinMaxPts = 256;
 // One round of two blocks a CU.  More blocks are throughput, not latency: a
 // step takes 29.0 us here against 37.5 in the separate launches with 474
@@ -1254,21 +1252,71 @@ static int window_lds(const TableView &t, int nt, int max_points, WindowArgs &a)
     return a.off_x + std::max(nxc, nsh);
 }
 
-bool window_fits(const TableView &t, int min_atoms, int max_atoms, int max_points, int nblocks)
+bool window_fits(const TableView &t, int max_atoms, int max_points, int nblocks)
 {
-    return min_atoms <= kWinMinAtoms && max_atoms <= kWinMaxAtoms && max_points <= kWinMaxPts &&
-           nblocks <= kWinMaxBlocks && field_tab_floats(t) <= kTabLdsFloats &&
-           force_tab_floats(t) <= kTabLdsFloats;
+    return max_atoms <= kWinMaxAtoms && max_points <= kWinMaxPts && nblocks <= kWinMaxBlocks &&
+           field_tab_floats(t) <= kTabLdsFloats && force_tab_floats(t) <= kTabLdsFloats;
+}
+
+// Work-items of a k_window block: sixteen waves where a pass of eight holds less
+// than a group's field splits and a CU has a block to itself (242 atoms, nMC = 20,
+// 72 blocks: a step takes 36.7 against 41.2 us; but nMC = 100, 303 blocks, 63.5
+// against 49.4 us).
+static int window_threads(int max_items, int nblocks)
+{
+    return max_items > 512 && nblocks <= 256 ? 1024 : 512;
+}
+
+// Whether k_window is the faster route for windows that fit it.
+//
+// With windows on both sides of kWinSmallAtoms it depends on where the longest chains
+// are.  k_window lasts as long as its longest block, which makes its field passes one
+// after the other (each a split's atoms a lane) and then its waves' shares of the
+// force: a least-squares fit gives the solvent force 14 us + 0.3 us an atom of those
+// passes + 0.2 us a point of those shares.  The separate passes pay their launches,
+// wait for the longest share of any window and take longer with more pairs: 23 us + 0.14
+// us a point of that share + 2.3 us a million pairs; in an engine step, whose other terms
+// ride on k_window, both take 5 us more.  The rule is that comparison in units of 0.3 us,
+// its constants moved to where the measured times divide best.
+//
+// Measured on 382 batches drawn from windows of 2 to 242 atoms, nMC 3 to 100, both
+// routes each: where the rule takes k_window (206), the step is 10% and the solvent
+// force alone 2.2% faster than in separate passes; where it does not (176), k_window
+// would take the same time for the step (0.3% less) and 9.8% more for the force.  Four
+// windows of 220 atoms, nMC = 10: with two pairs of atoms the step takes 35.1 us separate
+// and 36.6 here, the force 28.4 and 32.8; with two chains of 22 atoms, whose shares are
+// the longest, 41.1 and 37.7, and 33.8 and 32.6.
+bool window_pays(const WinDesc *w, int nwin, int nmc, int nblocks, int max_items)
+{
+    int lo = w[0].n, hi = w[0].n;
+    for (int k = 1; k < nwin; ++k) {
+        lo = std::min(lo, w[k].n);
+        hi = std::max(hi, w[k].n);
+    }
+    if (hi <= kWinSmallAtoms) return true;
+    if (lo > kWinSmallAtoms) return false;
+    const int nt = window_threads(max_items, nblocks);
+    double chain = 0.0, longest = 0.0, pairs = 0.0;
+    for (int k = 0; k < nwin; ++k) {
+        const WinDesc &d = w[k];
+        const long long P = (long long)d.n * nmc;
+        const long long np = std::min(P, (long long)force_group(d.n) * d.ppc);
+        if (np > kWinMaxPts) return false;
+        const int side = nt / (int)((np + kWave - 1) / kWave * kWave);  // splits of a pass
+        const int passes = (d.splits + side - 1) / side;
+        const int shares = force_shares(d.n), share = (d.ppc + shares - 1) / shares;
+        const int per = d.n <= 2 * kWave ? 1 : 2;  // shares of a wave
+        chain = std::max(chain, passes * d.aps + 0.6 * per * share);
+        longest = std::max(longest, (double)share);
+        pairs += (double)d.n * (double)P;
+    }
+    return chain <= 28.0 + 0.6 * longest + 6.0e-6 * pairs;
 }
 
 hipError_t launch_window(const WindowArgs &a0, int max_points, int max_items, hipStream_t s)
 {
     WindowArgs a = a0;
-    // sixteen waves where a pass of eight holds less than a group's field
-    // splits and a CU has a block to itself (242 atoms, nMC = 20, 72 blocks: a
-    // step takes 36.7 against 41.2 us; but nMC = 100, 303 blocks, 63.5
-    // against 49.4 us)
-    const int nt = max_items > 512 && a.nblocks <= 256 ? 1024 : 512;
+    const int nt = window_threads(max_items, a.nblocks);
     size_t lds = sizeof(float) * window_lds(a.tab, nt, max_points, a);
     if (a.nb_blocks) lds = std::max(lds, nonbond_lds_bytes(a.nb.T, false));
     const long terms = (long)a.bonded.nb + a.bonded.na + a.bonded.nd;

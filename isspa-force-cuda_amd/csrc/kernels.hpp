@@ -379,10 +379,12 @@ hipError_t launch_epilogue(const EpilogueArgs &a, hipStream_t s);
 // the epilogue with riders, where it is short of blocks
 bool epilogue_takes_riders(long long P, const RiderArgs &r);
 hipError_t launch_step_epilogue(const EpilogueArgs &a, RiderArgs r, hipStream_t s);
-// k_window: whether a model's windows, chunk groups and tables fit it, and the
-// launch (max_atoms, max_points: of the largest window and chunk group;
-// max_items: the most (point, field split) pairs of a group)
-bool window_fits(const TableView &t, int min_atoms, int max_atoms, int max_points, int nblocks);
+// k_window: whether a model's windows, chunk groups and tables fit it, whether it is
+// the faster route (windows w of the present tiling), and the launch (max_atoms,
+// max_points: of the largest window and chunk group; max_items: the most (point,
+// field split) pairs of a group)
+bool window_fits(const TableView &t, int max_atoms, int max_points, int nblocks);
+bool window_pays(const WinDesc *w, int nwin, int nmc, int nblocks, int max_items);
 hipError_t launch_window(const WindowArgs &a, int max_points, int max_items, hipStream_t s);
 hipError_t launch_force(const ForceArgs &a, int nblocks, bool split, hipStream_t s);
 hipError_t launch_force_reduce(const ReduceArgs &a, bool split, hipStream_t s);

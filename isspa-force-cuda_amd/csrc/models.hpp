@@ -58,7 +58,8 @@ struct isspa_model {
     int nwblk = 0;
     int max_fg = 1;  // the largest splits-per-field-block of the windows
     // over the windows, for the small-window launch
-    int min_win_atoms = 0, max_win_atoms = 0, max_group_pts = 0, max_group_items = 0;
+    int max_win_atoms = 0, max_group_pts = 0, max_group_items = 0;
+    bool win_pays = false;
     double *part_g = nullptr;
     int *part_cnt = nullptr;
     double *part_s0 = nullptr, *part_ein = nullptr;
