@@ -833,14 +833,11 @@ int nonbond_flags(nonbond_model *m, const float4 *x, const int **flag, hipStream
     return ISSPA_OK;
 }
 
-int nonbond_partials(nonbond_model *m, const float *xyzq4_d, bool split, hipStream_t s,
-                     const int *pbc_flag)
+int nonbond_partials(nonbond_model *m, const float *xyzq4_d, bool split, hipStream_t s)
 {
     const float4 *x = reinterpret_cast<const float4 *>(xyzq4_d);
-    // A flag set with a larger margin only sends a window through the
-    // minimum-image loop when no image is needed, where that loop's shift
-    // (fma(-L, 0, r)) returns r unchanged: the result is the same bit for bit.
-    if (!pbc_flag) CHK(nonbond_flags(m, x, &pbc_flag, s));
+    const int *pbc_flag = nullptr;
+    CHK(nonbond_flags(m, x, &pbc_flag, s));
     HIPCHK(launch_nonbond(nonbond_args(m, x, pbc_flag, split), split ? m->nblk : m->nblk_tot,
                           split, s));
     return ISSPA_OK;
@@ -1346,9 +1343,7 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
     // the field launch (which carry partner-chunk blocks only: windows large
     // enough for super-tiles always have the side stream)
     const bool small = m && isspa_is_small(m);
-    // (k_window has LDS of its own beside the LJ table: over 128 LJ types the
-    // all-pairs term keeps its launch there)
-    const bool nb_rides = m && e->nb && !fork && !e->nb->any_sym && (!small || e->nb->T <= 128);
+    const bool nb_rides = m && e->nb && !fork && !e->nb->any_sym;
     if (small) {
         WindowArgs w = window_args(m, x4, 0u, e->step_d + kStepNext);
         w.step_now = e->step_d + kStepNow;
@@ -1381,7 +1376,9 @@ static int engine_forces(md_engine *e, hipStream_t s, bool integrate)
         if (m) {
             FieldArgs fa = field_args(m, x4);
             if (nb_rides) {
-                // with the prologue's IS-SPA minimum-image flags
+                // with the prologue's IS-SPA minimum-image flags: their margin is larger,
+                // which only sends a window through images it does not need, and those
+                // change no bit
                 fa.nb = nonbond_args(e->nb, x4, m->pbc_flag, false);
                 fa.nb_blocks = e->nb->nblk_tot;
             }

@@ -27,25 +27,11 @@ struct DiffType {
     float pad;
 };
 
-struct DiffSwitch {
-    float S, dSdz;
-};
-
-__device__ __forceinline__ DiffSwitch diff_switch(const DiffType &T, float d)
+// S(d)
+__device__ __forceinline__ float diff_switch(const DiffType &T, float d)
 {
     const float z = (d - T.rlo) * T.idel + 1.0f;
-    DiffSwitch o;
-    if (z <= 0.0f) {
-        o.S = 0.0f;
-        o.dSdz = 0.0f;
-    } else if (z >= 1.0f) {
-        o.S = 1.0f;
-        o.dSdz = 0.0f;
-    } else {
-        o.S = z * z * (3.0f - 2.0f * z);
-        o.dSdz = 6.0f * z * (1.0f - z);
-    }
-    return o;
+    return z <= 0.0f ? 0.0f : (z >= 1.0f ? 1.0f : z * z * (3.0f - 2.0f * z));
 }
 
 __device__ __forceinline__ float diff_g(const DiffType &T, float d)
@@ -54,13 +40,13 @@ __device__ __forceinline__ float diff_g(const DiffType &T, float d)
     const float u = d - T.x0;
     const float P = T.g0 - T.al * u * u;
     if (P <= 0.0f) return 0.0f;
-    return diff_switch(T, d).S * P;
+    return diff_switch(T, d) * P;
 }
 
 __device__ __forceinline__ float diff_E(const DiffType &T, float d)
 {
     const float u = d - T.x0;
-    return T.c * expf(-0.5f * u * u) * diff_switch(T, d).S;
+    return T.c * expf(-0.5f * u * u) * diff_switch(T, d);
 }
 
 // the four constants diff_F needs, held in registers by the force pass
@@ -81,14 +67,6 @@ __device__ __forceinline__ float diff_F(const DiffFParams &T, float d, float rin
     const float sr2 = sr * sr;
     const float sr6 = sr2 * sr2 * sr2;
     return 24.0f * T.ets * rinv * (2.0f * sr6 * sr6 - sr6) * S;
-}
-
-__device__ __forceinline__ float diff_F(const DiffType &T, float d, float rinv)
-{
-    const float sr = T.sts * rinv;
-    const float sr2 = sr * sr;
-    const float sr6 = sr2 * sr2 * sr2;
-    return 24.0f * T.ets * rinv * (2.0f * sr6 * sr6 - sr6) * diff_switch(T, d).S;
 }
 
 // x / b for r = 1 / b rounded: a product, then two of Markstein's corrections

@@ -119,11 +119,7 @@ ReduceArgs reduce_args(isspa_model *m, const float4 *x, float4 *f, double *flj, 
 int nonbond_run(nonbond_model *m, const float *xyzq4_d, bool split, float4 *f, double *o0,
                 double *o1, double *o2, hipStream_t s);
 // the same in two halves: per-chunk partials, then their fixed-order sum
-// pbc_flag: per-window minimum-image flags already computed on stream s with a
-// margin at least as large as the all-pairs one (the IS-SPA model's), or null
-// to compute them here
-int nonbond_partials(nonbond_model *m, const float *xyzq4_d, bool split, hipStream_t s,
-                     const int *pbc_flag = nullptr);
+int nonbond_partials(nonbond_model *m, const float *xyzq4_d, bool split, hipStream_t s);
 NonbondArgs nonbond_args(nonbond_model *m, const float4 *x, const int *pbc_flag, bool split);
 int nonbond_flags(nonbond_model *m, const float4 *x, const int **flag, hipStream_t s);
 int nonbond_reduce(nonbond_model *m, bool split, float4 *f, double *o0, double *o1, double *o2,

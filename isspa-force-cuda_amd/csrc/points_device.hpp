@@ -50,7 +50,8 @@ __device__ __forceinline__ float4 mc_place(float4 x, float R, float R2, int v0, 
 // rounds, is a chain of some 150 dependent operations: with one lane a point
 // that was seven draws in a row, now it is two, the same work in four times
 // the waves.  The owner's position and radii are requested before the first
-// draw, and the owner is found by a 32-bit division where that is enough.
+// draw, and the owner is found by a 32-bit division (a model has fewer than 2^29
+// points).
 // Launch of 1,100 atoms, nMC = 20: 5.6 -> 3.1 us; 19,998 atoms 12.7 -> 11.9 us.
 constexpr int kMcLanes = 4, kMcBlockPts = 256 / kMcLanes;
 
@@ -61,8 +62,7 @@ __device__ __forceinline__ void mc_points_block(const PointsArgs &a, long long b
     const int sub = threadIdx.x % kMcLanes;
     const long long at = block * kMcBlockPts + threadIdx.x / kMcLanes;
     const long long gp = min(at, total - 1);
-    const int k = total <= 0x7fffffffll ? (int)((uint32_t)gp / (uint32_t)a.nmc)
-                                        : (int)(gp / a.nmc);
+    const int k = (int)((uint32_t)gp / (uint32_t)a.nmc);
     const float4 x = a.xyzq[k];
     const int t = a.itype[k];
     const WinDesc W = a.nwin == 1 ? a.wins[0] : a.wins[a.atom_win[k]];
