@@ -70,9 +70,9 @@ struct TableView {
 constexpr int kRecFloats = 16;
 constexpr int kAuxFloats = 4;
 
-// all-pairs blocks: 256 receivers; kinds of the block table's .w
+// all-pairs blocks of 256 work-items; kinds of the block table's .w
 constexpr int kNbBlock = 256;
-constexpr int kNbKindChunk = 0;  // receivers x a partner chunk, every pair in both orders
+constexpr int kNbKindChunk = 0;  // 64 receivers x kNbGroup partner chunks, every pair in both orders
 constexpr int kNbKindNear = 1;   // receiver block x itself or a neighbouring block, ordered
 constexpr int kNbKindSym = 2;    // super-tile: receiver block x partner block, each pair once
 constexpr int kSymMinAtoms = 4096;            // windows that take each pair once
@@ -80,7 +80,7 @@ constexpr int kSymLdsDoubles = 3 * kNbBlock;  // a super-tile's partner sums in 
 
 struct NonbondArgs {
     const WinDesc *wins;
-    const int4 *blocks;    // {w, receiver block, partner chunk or block, kind}
+    const int4 *blocks;    // {w, receiver block, group of partner chunks or block, kind}
     const float4 *xyzq;
     const float4 *aux;     // per atom j: {4 R_j^2, cA_j, cB_j, LJ type (int bits)}
     const float2 *lj;      // [T*T] {12A, 6B}
@@ -174,7 +174,7 @@ struct ForceArgs {
 };
 
 // The first block of a launch of nb whose waves rank themselves by progress
-// (Progress, device_common.hpp); the blocks before it have the top priority.
+// (Progress, below); the blocks before it have the top priority.
 //   nb <= 512:   none; with one or two waves a SIMD there is little to even
 //                out (field of 550 atoms, 430 blocks: 9.8 us, ranked 10.1).
 //   nb <= 1536:  all; they run at once (6 to 7 blocks fit a CU).
@@ -182,6 +182,21 @@ struct ForceArgs {
 //                that the rest find room early.  Force pass of 4,510 atoms
 //                (2,272 blocks): 195 us unranked, 175 with the last 1,280, 183
 //                with 1,536, 198 with 1,664 and 199 with 2,048; 187 with 768.
+// The split force pass, the analytic field and force passes and both sides of the
+// adjoint follow the same lines, though they hold four to seven blocks a CU.  Measured
+// none / this rule / all ranked / the last 1,280, in us:
+//   split force   414 blocks   21.9 /  22.2 /  22.3 /  22.1;  990  48.5 / 44.5 / 44.4 / 44.5;
+//               2,135         146.6 / 136.0 / 140.7 / 135.6; 3,328 424 / 405 / 413 / 408
+//   analytic field 516         19.7 /  20.2 /  20.2 /  20.2; 1,116 30.2 / 28.8 / 28.7 / 28.9;
+//               2,064          33.9 /  34.7 /  34.9 /  34.7; 8,256 99.2 / 99.2 / 101.9 / 97.9
+//   analytic force 384         10.3 /  10.5 /  11.4 /  11.1;  975  33.7 / 31.2 / 31.2 / 31.0;
+//               2,484          52.2 /  50.3 /  54.7 /  50.2; 7,920 195.5 / 194.5 / 196.0 / 192.3
+//   adjoint, points 416        15.2 /  15.3 /  15.5 /  15.3; 1,032 38.2 / 34.0 / 33.7 / 33.8;
+//               2,064          59.9 /  55.2 /  58.8 /  55.1; 8,256 245 / 243 / 245 / 240
+//   adjoint, atoms  384        17.0 /  17.1 /  17.3 /  17.3;  828  41.7 / 37.7 / 37.3 / 37.6;
+//               2,484          78.3 /  70.7 /  71.7 /  70.9; 29,376 838 / 830 / 850 / 831
+// Over 62 launches of 315 to 29,376 blocks the rule is within 2.6% of the best of the
+// four, and up to 12% faster than unranked.
 constexpr int kUnranked = 0x7fffffff;
 constexpr int kRankMin = 512, kRankAll = 1536, kRankLast = 1280;
 inline int ranked_from(int nb)
