@@ -54,6 +54,9 @@ FLOP_FIELD_PAIR = 24      # field pass, per (point, atom), outside rmax
 FLOP_NB_PAIR = 36         # nonbond, per unordered pair
 
 
+# HBM-side traffic of a k_force launch; TRAFFIC_JSON is the profile of its former
+# blocks (256 receivers and one chunk each, a partial for every chunk)
+FORCE_TRAFFIC_JSON = "k_force_shares_19998atoms_nmc20_traffic.json"
 TRAFFIC_JSON = "k_force_19998atoms_nmc20_traffic.json"
 COUNTERS_JSON = "isspa_passes_19998atoms_nmc20_valu_counters.json"
 
@@ -66,9 +69,9 @@ def traffic_at(chunks, path):
     """HBM-side bytes of one k_force launch at `chunks` force chunks, from the
     committed FETCH_SIZE / WRITE_SIZE passes (copy-calibrated) at several
     chunk counts.  k_force reads the point records and writes 6 FP64 partials
-    per (chunk, atom): its WRITE_SIZE is linear in the chunk count and its
-    FETCH_SIZE nearly constant, so both are interpolated linearly between the
-    two profiled counts around `chunks`.  Returns (bytes or None outside the
+    per atom and group of chunks: its WRITE_SIZE is linear in the chunk count and
+    its FETCH_SIZE nearly constant, so both are interpolated linearly between
+    the two profiled counts around `chunks`.  Returns (bytes or None outside the
     profiled range, note, summary file), or None without the file."""
     if not os.path.exists(path):
         return None
@@ -87,6 +90,14 @@ def traffic_at(chunks, path):
                     f"{hi['chunks']} force chunks (this run {chunks})")
             break
     return traffic, note, tr["summary"]
+
+
+def force_grid(n_atoms, chunks):
+    """Work-items of a k_force launch on one system: a block of 256 for each 64
+    receivers and group of chunks (four; two of at most 128 atoms, one of at most
+    64)."""
+    group = 1 if n_atoms <= 64 else 2 if n_atoms <= 128 else 4
+    return -(-n_atoms // 64) * -(-chunks // group) * 256
 
 
 def counter_check(path):
@@ -414,13 +425,13 @@ def main():
     log("stage ms: " + ", ".join(f"{k} {v:.4f}" for k, v in prof.items()))
     if args.traffic_sweep:
         # k_force launches at other chunk counts, told apart in a counter pass
-        # by their grid (chunks x receiver blocks x 256 work-items)
-        rblocks = (s.n_atoms + 255) // 256
+        # by their grid
         for c in (int(v) for v in args.traffic_sweep.split(",")):
             g.set_tiling(splits, c)
             _, c_eff = g.tiling()
             g.profile(1)
-            log(f"traffic sweep: {c_eff} force chunks, k_force grid {c_eff * rblocks * 256}")
+            log(f"traffic sweep: {c_eff} force chunks, "
+                f"k_force grid {force_grid(s.n_atoms, c_eff)}")
         g.set_tiling(splits, chunks)
     N, P = s.n_atoms, s.n_points
     force_flop = FLOP_FORCE_PAIR * N * P
@@ -471,7 +482,7 @@ def main():
     # HBM-side bytes per k_force launch and the VALU-instruction counter pass
     # of the same kernels, from the committed profiles
     if args.workload == 2:
-        tr = traffic_at(chunks, os.path.join(ROOT, "profiles", TRAFFIC_JSON))
+        tr = traffic_at(chunks, os.path.join(ROOT, "profiles", FORCE_TRAFFIC_JSON))
         if tr is not None:
             out["roofline"]["traffic"], out["roofline"]["traffic_note"], \
                 out["roofline"]["traffic_source"] = tr
