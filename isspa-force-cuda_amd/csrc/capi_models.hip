@@ -89,6 +89,26 @@ static int auto_pieces(long long lanes, long long work, long long min_work, doub
     return (int)std::max(1LL, s);
 }
 
+// Partner chunks of an all-pairs window of nw atoms, a wave each.  Where many
+// windows share the waves, a window's share alone would be one to a few chunks, and
+// a block takes kNbGroup of them: waves without one would wait for the others at the
+// block's sums and hold their places meanwhile.  So such a window gets whole groups,
+// and as many as chunks of a tile (64 partners) give, up to 16: the partial entries
+// stay few, and the last round of blocks ends in short ones.
+// nonbond_force of 256 x 1,100 atoms 743 us with the one chunk of the share, 312 with
+// four, 294 with eight, 284 with 16 and 293 with 24; of 128 x 2,200 atoms 1,380, 519,
+// 479, 464 and 473; of 512 x 550 atoms (8) 433 -> 179, of 1,024 x 220 (4) 125 -> 93.
+// (In blocks of 256 receivers and one chunk these took 350, 627, 226 and 77 us.)
+static int nonbond_chunks(long long nw, double target)
+{
+    const long long c = auto_pieces(nw, nw, kMinNonbondPartners, target);
+    const long long most = std::max(1LL, nw / kMinNonbondPartners);
+    if (c >= most || c >= 3 * kNbGroup) return (int)c;
+    auto groups = [](long long k) { return (k + kNbGroup - 1) / kNbGroup * kNbGroup; };
+    const long long tiles = groups(std::max(1LL, std::min(4LL * kNbGroup, nw / 64)));
+    return (int)std::min(most, std::max(groups(c), tiles));
+}
+
 // ---------------------------------------------------------------------------
 // IS-SPA model
 // ---------------------------------------------------------------------------
@@ -693,7 +713,7 @@ extern "C" int nonbond_model_create_batch(int n, int T, const int *ityp, const i
         WinDesc d = base_desc(Ly, w);
         const long long nw = Ly.n[w];
         const double tgt = std::max(1.0, kWaveSlots * ((double)nw * nw / work_tot));
-        const int c = auto_pieces(nw, nw, kMinNonbondPartners, tgt);
+        const int c = nonbond_chunks(nw, tgt);
         d.apc = (int)((nw + c - 1) / c);
         d.nbc = (int)((nw + (long long)kNbGroup * d.apc - 1) / ((long long)kNbGroup * d.apc));
         d.npo = B;

@@ -1,0 +1,77 @@
+"""Batches of more windows than the launches have waves for: the time of a window
+must not rise with their number, and every window's result stays that of the
+oracle, or of the window alone at the same tiling."""
+import dataclasses
+
+import numpy as np
+import pytest
+import torch
+
+import pyoracle as po
+from isspa_amd import batch, synth
+from isspa_amd.engine import GpuSystem
+from isspa_amd.system import max_abs_rel_rms
+
+pytestmark = pytest.mark.gpu
+
+
+def _frames(n, chains, n_mc, lbox=200.0):
+    """n windows of one lattice with thermal noise."""
+    base = synth.make_lattice(chains, 64.0, 4, lbox, seed=31)
+    base.n_mc, base.seed, base.temperature_k, base.pnu = n_mc, 17, 298.0, 0.01
+    rng = np.random.default_rng(5)
+    ws = []
+    for _ in range(n):
+        f = dataclasses.replace(base)
+        f.xyzq = base.xyzq.copy()
+        f.xyzq[:, :3] += rng.normal(scale=0.1, size=(base.n_atoms, 3)).astype(np.float32)
+        ws.append(f)
+    return ws
+
+
+def _ms(fn, reps=10):
+    fn()
+    best = 1e9
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(reps):
+            fn()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) / reps)
+    return best
+
+
+def test_all_pairs_time_a_window():
+    """The all-pairs force of 256 windows of 1,100 atoms against 32 of them, per window:
+    0.7 times as long measured, 1.8 with a single partner chunk a window."""
+    t = {}
+    for n in (32, 256):
+        g = GpuSystem(batch.merge_windows(_frames(n, 50, 5)), "cuda:0", us=False, bonded=False)
+        t[n] = _ms(g.nonbond_force) / n
+        g.close()
+    print(f"us a window: {1e3 * t[32]:.2f} of 32, {1e3 * t[256]:.2f} of 256", flush=True)
+    assert t[256] <= 1.2 * t[32]
+
+
+@pytest.mark.parametrize("n,chains", [(130, 50), (256, 50), (400, 9), (420, 14), (900, 6)])
+@pytest.mark.parametrize("lbox", [200.0, 62.0])
+def test_all_pairs_of_many_windows(n, chains, lbox):
+    """Few chunks a window, with and without images, totals and components."""
+    ws = _frames(n, chains, 2, lbox)
+    g = GpuSystem(batch.merge_windows(ws), "cuda:0", us=False, bonded=False)
+    print(f"{n} x {ws[0].n_atoms} atoms, box {lbox}", flush=True)
+    g.zero_forces()
+    f = g.nonbond_force()[:, :3].double().cpu().numpy()
+    c = g.nonbond_components()
+    part = (c["lj"] + c["coul"] + c["pair"]).cpu().numpy()
+    assert max_abs_rel_rms(f, part) <= 2e-6
+    sl = batch.window_slices(g.system)
+    for w in (0, n // 2, n - 1):
+        ref = po.nonbond(ws[w])
+        a, b = sl[w]
+        for k in ("lj", "coul", "pair"):
+            assert max_abs_rel_rms(c[k][a:b].cpu().numpy(), ref[k]) <= 1e-5, (w, k)
+        assert max_abs_rel_rms(f[a:b], ref["lj"] + ref["coul"] + ref["pair"]) <= 1e-5, w
+    g.close()
