@@ -75,3 +75,35 @@ def test_all_pairs_of_many_windows(n, chains, lbox):
             assert max_abs_rel_rms(c[k][a:b].cpu().numpy(), ref[k]) <= 1e-5, (w, k)
         assert max_abs_rel_rms(f[a:b], ref["lj"] + ref["coul"] + ref["pair"]) <= 1e-5, w
     g.close()
+
+
+@pytest.mark.parametrize("n,chains,n_mc", [(700, 6, 2), (600, 7, 3), (1500, 3, 2), (300, 14, 2)])
+def test_force_of_many_windows(n, chains, n_mc):
+    """Few force chunks a window, at an automatic tiling: total and components against
+    the oracle, every window like the window alone at that tiling."""
+    ws = _frames(n, chains, n_mc)
+    g = GpuSystem(batch.merge_windows(ws), "cuda:0", us=False, bonded=False, nonbond=False)
+    g.set_target_waves(8192)
+    s, c = g.tiling()
+    atoms = ws[0].n_atoms
+    group = 4 if atoms > 128 else 2 if atoms > 64 else 1
+    print(f"{n} x {atoms} atoms, nMC={n_mc}, tiling {s, c}", flush=True)
+    assert c < 32 and c % group == 0    # whole blocks
+    g.zero_forces()
+    f = g.isspa_force(step=2)[:, :3].clone()
+    comp = g.isspa_components(step=2)
+    sl = batch.window_slices(g.system)
+    for w in (0, 1, n // 2, n - 1):
+        a, b = sl[w]
+        h = GpuSystem(batch.merge_windows([ws[w]], [w]), "cuda:0", us=False, bonded=False,
+                      nonbond=False)
+        h.set_tiling(s, c)
+        h.zero_forces()
+        assert torch.equal(h.isspa_force(step=2)[:, :3], f[a:b]), w
+        hc = h.isspa_components(step=2)
+        assert all(torch.equal(hc[k], comp[k][a:b]) for k in comp), w
+        h.close()
+        ref = po.isspa_total(ws[w], step=2, sys_id=w)
+        for k in ("lj", "pol", "cdd"):
+            assert max_abs_rel_rms(comp[k][a:b].cpu().numpy(), ref[k]) <= 1e-5, (w, k)
+    g.close()
