@@ -807,7 +807,7 @@ __device__ __forceinline__ void write_force_entry(const ForceArgs &a, const WinD
 template <bool SPLIT, bool AN>
 __global__ __launch_bounds__(kBlock) void k_force(ForceArgs a)
 {
-    const int4 bt = a.blocks[a.xcd_runs ? xcd_run_entry(blockIdx.x, gridDim.x) : blockIdx.x];
+    const int4 bt = a.blocks[xcd_run_entry(blockIdx.x, gridDim.x)];
     const WinDesc W = a.wins[bt.x];
     const int lane = (int)threadIdx.x % kWave;
     // the wave index read from the first lane, so the compiler knows it is

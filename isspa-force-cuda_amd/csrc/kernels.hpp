@@ -168,7 +168,6 @@ struct ForceArgs {
     const int *pbc_flag;
     double *part;         // [C][stride]: (S_e, S_lj), or (pol, lj, cdd, pad) split
     long long C;
-    int xcd_runs;         // 1: each XCD takes a contiguous run of the table (equal work items)
     int red_off;          // float offset of the share-sum area in the dynamic LDS (set at launch)
     int ranked_from;      // blocks from here on rank their waves by progress (set at launch)
 };
@@ -267,10 +266,9 @@ __host__ __device__ constexpr int force_share_doubles(bool split)
     return 3 * 64 * (split ? 9 : 6);
 }
 
-// Workgroup b of a launch goes to XCD b % 8 (round-robin).  With xcd_runs the
-// table entry of workgroup b is the (b / 8)-th of XCD b % 8's contiguous run,
-// so the receiver blocks of one chunk share an L2 instead of being dealt to
-// all eight.  A bijection on [0, nb) for any nb.
+// Workgroup b of a launch goes to XCD b % 8 (round-robin).  The force table's entry of
+// workgroup b is the (b / 8)-th of XCD b % 8's contiguous run, so the receiver
+// blocks of one group of chunks share an L2 instead of being dealt to all eight.  A bijection on [0, nb) for any nb.
 __device__ __forceinline__ int xcd_run_entry(int b, int nb)
 {
     const int q = nb >> 3, r = nb & 7, x = b & 7, k = b >> 3;
