@@ -211,7 +211,7 @@ static int isspa_tile(isspa_model *m)
             : (double)std::min(kMaxAutoWaves,
                                std::max(kMinAutoWaves, (long)(m->P / kPointsPerWave)));
     m->wins_h.assign(L.W, WinDesc{});
-    m->max_win_atoms = m->max_group_pts = m->max_group_items = 0;
+    m->max_win_atoms = m->max_group_pts = m->max_group_items = m->max_fents = 0;
     m->max_fg = 1;
     long long F = 0, C = 0, V = 0;
     std::vector<std::pair<long long, int4>> gb, pb, vb, wb;
@@ -238,6 +238,7 @@ static int isspa_tile(isspa_model *m)
             d.splits * ((std::min(P, (long long)group * d.ppc) + 63) / 64 * 64));
         d.fents = (d.chunks + group - 1) / group;
         d.vents = (d.chunks + 3) / 4;
+        m->max_fents = std::max(m->max_fents, d.fents);
         d.fpo = F;
         d.ppo = C;
         d.vpo = V;
@@ -490,7 +491,7 @@ ReduceArgs reduce_args(isspa_model *m, const float4 *x, float4 *f, double *flj, 
 {
     ReduceArgs ra{};
     ra.wins = m->wins; ra.nwin = m->lay.W; ra.atom_win = m->atom_win; ra.part = m->part_f; ra.C = m->C;
-    ra.ntot = m->d.n_atoms; ra.xyzq = x; ra.itype = m->itype; ra.vtot = m->vtot; ra.f = f;
+    ra.max_fents = m->max_fents; ra.ntot = m->d.n_atoms; ra.xyzq = x; ra.itype = m->itype; ra.vtot = m->vtot; ra.f = f;
     ra.f_lj = flj; ra.f_pol = fpol; ra.f_cdd = fcdd;
     return ra;
 }
@@ -783,6 +784,8 @@ extern "C" int nonbond_model_create_batch(int n, int T, const int *ityp, const i
         const bool sym = !fallback && lj_sym && sym_lds_ok && nw >= kSymMinAtoms;
         const int nsb = (nw + kNbBlock - 1) / kNbBlock;
         d.nte = sym ? nsb : d.nbc;
+        m->max_nbc = std::max(m->max_nbc, d.nbc);
+        m->max_nte = std::max(m->max_nte, d.nte);
         d.spo = Bt;
         Bt += (long long)d.nte * nw;
         if (!sym) {
@@ -902,8 +905,9 @@ int nonbond_partials(nonbond_model *m, const float *xyzq4_d, bool split, hipStre
 int nonbond_reduce(nonbond_model *m, bool split, float4 *f, double *o0, double *o1, double *o2,
                    hipStream_t s)
 {
-    HIPCHK(launch_chunk_reduce3(m->wins, m->lay.W, m->atom_win, m->part, split ? m->B : m->B_tot, m->n,
-                                split ? 9 : 3, f, o0, o1, o2, s));
+    HIPCHK(launch_chunk_reduce3(m->wins, m->lay.W, m->atom_win, m->part, split ? m->B : m->B_tot,
+                                split ? m->max_nbc : m->max_nte, m->n, split ? 9 : 3, f, o0, o1, o2,
+                                s));
     return ISSPA_OK;
 }
 

@@ -1120,25 +1120,10 @@ __global__ __launch_bounds__(NT, 4) void k_window(WindowArgs a)
     write_force_entry<false>(fa, W, bt.z, ir, own);
 }
 
-// F_i = -q_i vtot_i S_e - vtot_i S_lj over the chunk partials, summed in the
-// fixed slice order of reduce_device.hpp (kSumAtoms atoms x kSumSlices chunk
-// slices a block).
+// the force of atom i, or its components, from its summed partials
 template <bool SPLIT>
-__global__ __launch_bounds__(kBlock) void k_force_reduce(ReduceArgs a)
+__device__ __forceinline__ void write_force(const ReduceArgs &a, int i, const double *s)
 {
-    constexpr int comps = SPLIT ? 9 : 6;
-    __shared__ double red[kSumSlices][comps][kSumAtoms];
-    const int al = threadIdx.x % kSumAtoms, sl = threadIdx.x / kSumAtoms;
-    const int i = blockIdx.x * kSumAtoms + al;
-    const bool valid = i < a.ntot;
-    double s[comps];
-    for (int k = 0; k < comps; ++k) s[k] = 0.0;
-    if (valid) {
-        const WinDesc W = window_of(a.wins, a.nwin, a.atom_win, i);
-        sum_batches<comps, 8>(ForceEntry<comps>(W, a.part, i), sl, W.fents, s);
-    }
-    combine_slices<comps>(red, al, sl, s);
-    if (sl != 0 || !valid) return;
     if (!SPLIT) {
         const float3 fi = isspa_atom_force(a.xyzq[i].w, a.vtot[a.itype[i]], s);
         float4 f = a.f[i];
@@ -1156,6 +1141,35 @@ __global__ __launch_bounds__(kBlock) void k_force_reduce(ReduceArgs a)
             a.f_lj[3 * i + c] = -vt * s[3 + c];
             a.f_cdd[3 * i + c] = qv * s[6 + c];
         }
+    }
+}
+
+// F_i = -q_i vtot_i S_e - vtot_i S_lj over the chunk partials, summed in the
+// fixed slice order of reduce_device.hpp (kSumAtoms atoms x kSumSlices chunk
+// slices a block).  FEW: an atom a work-item (few_entries).
+template <bool SPLIT, bool FEW>
+__global__ __launch_bounds__(kBlock) void k_force_reduce(ReduceArgs a)
+{
+    constexpr int comps = SPLIT ? 9 : 6;
+    double s[comps];
+    for (int k = 0; k < comps; ++k) s[k] = 0.0;
+    if constexpr (FEW) {
+        const int i = blockIdx.x * kBlock + threadIdx.x;
+        if (i >= a.ntot) return;
+        const WinDesc W = window_of(a.wins, a.nwin, a.atom_win, i);
+        sum_batches<comps, kFewBatch, 1>(ForceEntry<comps>(W, a.part, i), 0, W.fents, s);
+        write_force<SPLIT>(a, i, s);
+    } else {
+        __shared__ double red[kSumSlices][comps][kSumAtoms];
+        const int al = threadIdx.x % kSumAtoms, sl = threadIdx.x / kSumAtoms;
+        const int i = blockIdx.x * kSumAtoms + al;
+        const bool valid = i < a.ntot;
+        if (valid) {
+            const WinDesc W = window_of(a.wins, a.nwin, a.atom_win, i);
+            sum_batches<comps, 8>(ForceEntry<comps>(W, a.part, i), sl, W.fents, s);
+        }
+        combine_slices<comps>(red, al, sl, s);
+        if (sl == 0 && valid) write_force<SPLIT>(a, i, s);
     }
 }
 
@@ -1353,11 +1367,15 @@ hipError_t launch_force(const ForceArgs &a, int nblocks, bool split, hipStream_t
 hipError_t launch_force_reduce(const ReduceArgs &a, bool split, hipStream_t s)
 {
     if (a.ntot == 0) return hipSuccess;
-    const int nb = (a.ntot + kSumAtoms - 1) / kSumAtoms;
-    if (split)
-        hipLaunchKernelGGL(k_force_reduce<true>, dim3(nb), dim3(kBlock), 0, s, a);
-    else
-        hipLaunchKernelGGL(k_force_reduce<false>, dim3(nb), dim3(kBlock), 0, s, a);
+    const bool few = few_entries(a.max_fents, a.ntot);
+    const int atoms = few ? kBlock : kSumAtoms;
+    const dim3 g((a.ntot + atoms - 1) / atoms), t(kBlock);
+    switch ((few ? 2 : 0) + (split ? 1 : 0)) {
+    case 0: hipLaunchKernelGGL((k_force_reduce<false, false>), g, t, 0, s, a); break;
+    case 1: hipLaunchKernelGGL((k_force_reduce<true, false>), g, t, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_force_reduce<false, true>), g, t, 0, s, a); break;
+    default: hipLaunchKernelGGL((k_force_reduce<true, true>), g, t, 0, s, a); break;
+    }
     return hipGetLastError();
 }
 

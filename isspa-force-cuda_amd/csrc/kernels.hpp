@@ -287,6 +287,7 @@ struct ReduceArgs {
     const int *atom_win;
     const double *part;
     long long C;
+    int max_fents;        // the most entries of a window
     int ntot;
     const float4 *xyzq;
     const int *itype;
@@ -438,9 +439,10 @@ constexpr int kStepNext = 0, kStepNow = 1;
 
 // ---- nonbond ----
 hipError_t launch_nonbond(const NonbondArgs &a, int nblocks, bool split, hipStream_t s);
+// max_entries: the most entries of a window
 hipError_t launch_chunk_reduce3(const WinDesc *wins, int nwin, const int *atom_win, const double *part,
-                                long long B, int ntot, int comps, float4 *f, double *o0,
-                                double *o1, double *o2, hipStream_t s);
+                                long long B, int max_entries, int ntot, int comps, float4 *f,
+                                double *o0, double *o1, double *o2, hipStream_t s);
 
 // ---- bonded ----
 hipError_t launch_bonded_terms(const BondedArgs &a, hipStream_t s);

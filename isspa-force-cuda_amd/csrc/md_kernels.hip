@@ -39,10 +39,10 @@ hipError_t launch_nonbond(const NonbondArgs &a, int nb, bool split, hipStream_t 
     return hipGetLastError();
 }
 
-// sum [comps][B] partials over the window's chunks in order; comps == 3:
-// f += sum; comps == 9: three FP64 outputs
-// sum over the partner chunks in the fixed slice order of reduce_device.hpp
-template <int COMPS>
+// sum [comps][B] partials over the window's groups of partner chunks in the fixed
+// slice order of reduce_device.hpp; comps == 3: f += sum; comps == 9: three FP64
+// outputs.  FEW: an atom a work-item (few_entries).
+template <int COMPS, bool FEW>
 __global__ __launch_bounds__(kBlk) void k_chunk_reduce3(const WinDesc *__restrict__ wins,
                                                         int nwin,
                                                         const int *__restrict__ atom_win,
@@ -50,17 +50,21 @@ __global__ __launch_bounds__(kBlk) void k_chunk_reduce3(const WinDesc *__restric
                                                         long long B, int ntot, float4 *f,
                                                         double *o0, double *o1, double *o2)
 {
-    __shared__ double red[kSumSlices][COMPS][kSumAtoms];
-    const int al = threadIdx.x % kSumAtoms, sl = threadIdx.x / kSumAtoms;
-    const int i = blockIdx.x * kSumAtoms + al;
+    constexpr int kAtoms = FEW ? kBlk : kSumAtoms;
+    const int al = threadIdx.x % kAtoms, sl = threadIdx.x / kAtoms;
+    const int i = blockIdx.x * kAtoms + al;
     const bool valid = i < ntot;
     double s[COMPS];
     for (int k = 0; k < COMPS; ++k) s[k] = 0.0;
     if (valid) {
         const WinDesc W = window_of(wins, nwin, atom_win, i);
-        sum_batches<COMPS, 4>(nonbond_entry<COMPS>(W, part, B, i), sl, COMPS == 3 ? W.nte : W.nbc, s);
+        sum_batches<COMPS, FEW ? kFewBatch : 4, FEW ? 1 : kSumSlices>(nonbond_entry<COMPS>(W, part, B, i), sl,
+                                                    COMPS == 3 ? W.nte : W.nbc, s);
     }
-    combine_slices<COMPS>(red, al, sl, s);
+    if constexpr (!FEW) {
+        __shared__ double red[kSumSlices][COMPS][kSumAtoms];
+        combine_slices<COMPS>(red, al, sl, s);
+    }
     if (sl != 0 || !valid) return;
     if constexpr (COMPS == 3) {
         float4 v = f[i];
@@ -78,17 +82,23 @@ __global__ __launch_bounds__(kBlk) void k_chunk_reduce3(const WinDesc *__restric
 }
 
 hipError_t launch_chunk_reduce3(const WinDesc *wins, int nwin, const int *atom_win,
-                                const double *part, long long B, int ntot, int comps, float4 *f, double *o0,
-                                double *o1, double *o2, hipStream_t s)
+                                const double *part, long long B, int max_entries, int ntot,
+                                int comps, float4 *f, double *o0, double *o1, double *o2,
+                                hipStream_t s)
 {
     if (ntot == 0) return hipSuccess;
-    const dim3 grid((ntot + kSumAtoms - 1) / kSumAtoms);
-    if (comps == 3)
-        hipLaunchKernelGGL(k_chunk_reduce3<3>, grid, dim3(kBlk), 0, s, wins, nwin, atom_win, part, B,
-                           ntot, f, o0, o1, o2);
-    else
-        hipLaunchKernelGGL(k_chunk_reduce3<9>, grid, dim3(kBlk), 0, s, wins, nwin, atom_win, part, B,
-                           ntot, f, o0, o1, o2);
+    const bool few = few_entries(max_entries, ntot);
+    const int atoms = few ? kBlk : kSumAtoms;
+    const dim3 g((ntot + atoms - 1) / atoms), t(kBlk);
+#define REDUCE(C, F) \
+    hipLaunchKernelGGL((k_chunk_reduce3<C, F>), g, t, 0, s, wins, nwin, atom_win, part, B, ntot, f, o0, o1, o2)
+    switch ((few ? 2 : 0) + (comps == 3 ? 0 : 1)) {
+    case 0: REDUCE(3, false); break;
+    case 1: REDUCE(9, false); break;
+    case 2: REDUCE(3, true); break;
+    default: REDUCE(9, true); break;
+    }
+#undef REDUCE
     return hipGetLastError();
 }
 

@@ -60,6 +60,7 @@ struct isspa_model {
     // over the windows, for the small-window launch
     int max_win_atoms = 0, max_group_pts = 0, max_group_items = 0;
     bool win_pays = false;
+    int max_fents = 0;  // the most force entries of a window
     double *part_g = nullptr;
     int *part_cnt = nullptr;
     double *part_s0 = nullptr, *part_ein = nullptr;
@@ -98,6 +99,7 @@ struct nonbond_model {
     int nblk_tot = 0;
     long long B_tot = 0;
     bool any_sym = false;
+    int max_nbc = 0, max_nte = 0;  // the most entries of a window in either layout
     double *part = nullptr;  // max(9 B, 3 B_tot) doubles, shared by both layouts
 };
 

@@ -59,30 +59,45 @@ __device__ __forceinline__ WinDesc window_of(const WinDesc *__restrict__ wins, i
 // below n), the loads of all of them issued before the first is used.  The
 // missing ones read entry n - 1 again and count as zero, so the last batch
 // waits once, as every other.  load(entry, v) reads an entry's COMPS values.
-template <int COMPS, int B, typename Load>
+// S = 1: one slice, every entry in turn.
+template <int COMPS, int B, int S = kSumSlices, typename Load>
 __device__ __forceinline__ void load_batch(Load load, int c, int n, double (&v)[B][COMPS])
 {
 #pragma unroll
-    for (int u = 0; u < B; ++u) load(min(c + u * kSumSlices, n - 1), v[u]);
+    for (int u = 0; u < B; ++u) load(min(c + u * S, n - 1), v[u]);
 }
-template <int COMPS, int B>
+template <int COMPS, int B, int S = kSumSlices>
 __device__ __forceinline__ void add_batch(int c, int n, const double (&v)[B][COMPS], double *s)
 {
 #pragma unroll
     for (int u = 0; u < B; ++u) {
-        const bool in = c + u * kSumSlices < n;
+        const bool in = c + u * S < n;
 #pragma unroll
         for (int k = 0; k < COMPS; ++k) s[k] += in ? v[u][k] : 0.0;
     }
 }
-template <int COMPS, int B, typename Load>
+template <int COMPS, int B, int S = kSumSlices, typename Load>
 __device__ __forceinline__ void sum_batches(Load load, int c, int n, double *s)
 {
-    for (; c < n; c += B * kSumSlices) {
+    for (; c < n; c += B * S) {
         double v[B][COMPS];
-        load_batch<COMPS, B>(load, c, n, v);
-        add_batch<COMPS, B>(c, n, v, s);
+        load_batch<COMPS, B, S>(load, c, n, v);
+        add_batch<COMPS, B, S>(c, n, v, s);
     }
+}
+
+// Sums of few entries for many atoms: one work-item an atom, kFewBatch entries in
+// flight.  With at most kSumSlices entries a slice holds one entry or none, so the
+// entries in turn give the slices' sum bit for bit; and most of sixteen work-items an
+// atom would have nothing to read, behind two barriers.  From 8,192 atoms on the atoms
+// alone hide the latency: the force reduction of 3,520 atoms and 16 entries takes 4.2 us
+// so and 3.5 in slices, of 8,800 atoms 4.2 and 4.8 (one entry 3.0 and 3.5), of 160,600
+// atoms and 4 entries 7.1 and 25.7, of 440,000 atoms 17.7 (4.8 TB/s) and 66.6; components
+// of 160,600 atoms 227 and 266 us a call.
+constexpr int kFewAtoms = 8192, kFewBatch = 4;
+inline bool few_entries(int entries, int atoms)
+{
+    return entries <= kSumSlices && atoms >= kFewAtoms;
 }
 
 // Reads the COMPS components (6, or 9 in split mode) of the force partial of
