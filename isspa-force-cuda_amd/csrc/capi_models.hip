@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "models.hpp"
+#include "xcd_runs.hpp"
 
 using namespace isspa;
 
@@ -170,31 +171,6 @@ static void own_atoms_first(const WinDesc &d, long long nmc,
         std::stable_partition(run, end, own);
         run = end;
     }
-}
-
-// Deals the force blocks of a batch, longest first, to the eight XCDs by whole chunk
-// groups: the receiver blocks of a group read the same records, and an L2 that holds
-// them serves them all.  Every XCD's contiguous run (xcd_run_entry) is still longest
-// first.  In one list over all XCDs the 4 to 18 receiver blocks of a group went to as
-// many L2s, which fetched its records each.  Solvent force of 256 x 1,100 atoms, nMC =
-// 20, 9,042 -> 7,424 us (8,657 with 5 blocks of 256 receivers), nMC = 5, 2,387 -> 2,017,
-// 32 x 1,100, nMC = 20, 1,118 -> 1,050, 4 x 1,100 172 -> 162, 80 x 220 232 -> 230; 64
-// umbrella windows 53 -> 51.
-static void groups_to_xcds(std::vector<std::pair<long long, int4>> &pb)
-{
-    std::vector<std::pair<long long, int4>> run[8];
-    for (auto it = pb.begin(); it != pb.end();) {
-        const int4 g = it->second;
-        const auto end = std::find_if(it, pb.end(), [&](const std::pair<long long, int4> &x) {
-            return x.second.x != g.x || x.second.z != g.z;
-        });
-        auto *shortest = std::min_element(
-            run, run + 8, [](const auto &a, const auto &b) { return a.size() < b.size(); });
-        shortest->insert(shortest->end(), it, end);
-        it = end;
-    }
-    pb.clear();
-    for (const auto &r : run) pb.insert(pb.end(), r.begin(), r.end());
 }
 
 // per-window splits/chunks, partial offsets and the block work tables; blocks

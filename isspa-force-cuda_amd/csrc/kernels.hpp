@@ -13,6 +13,7 @@
 #include <stdint.h>
 
 #include "diff_device.hpp"
+#include "xcd_runs.hpp"
 
 namespace isspa {
 
@@ -264,15 +265,6 @@ __host__ __device__ constexpr int force_group(int n) { return 4 / force_shares(n
 __host__ __device__ constexpr int force_share_doubles(bool split)
 {
     return 3 * 64 * (split ? 9 : 6);
-}
-
-// Workgroup b of a launch goes to XCD b % 8 (round-robin).  The force table's entry of
-// workgroup b is the (b / 8)-th of XCD b % 8's contiguous run, so the receiver
-// blocks of one group of chunks share an L2 instead of being dealt to all eight.  A bijection on [0, nb) for any nb.
-__device__ __forceinline__ int xcd_run_entry(int b, int nb)
-{
-    const int q = nb >> 3, r = nb & 7, x = b & 7, k = b >> 3;
-    return x * q + (x < r ? x : r) + k;
 }
 
 // The force pass's partials are stored entry by entry, entry
