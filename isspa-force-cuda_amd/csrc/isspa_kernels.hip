@@ -1288,18 +1288,23 @@ static int window_threads(int max_items, int nblocks)
 // after the other (each a split's atoms a lane) and then its waves' shares of the
 // force: a least-squares fit gives the solvent force 14 us + 0.3 us an atom of those
 // passes + 0.2 us a point of those shares.  The separate passes pay their launches,
-// wait for the longest share of any window and take longer with more pairs: 23 us + 0.14
-// us a point of that share + 2.3 us a million pairs; in an engine step, whose other terms
-// ride on k_window, both take 5 us more.  The rule is that comparison in units of 0.3 us,
-// its constants moved to where the measured times divide best.
+// wait for the longest share of any window, read a point's partial fields one after the
+// other and take longer with more pairs: 20 us + 0.14 us a point of that share + 0.3 us
+// an entry of the longest row of partial fields + 2.7 us a million pairs; in an engine
+// step, whose other terms ride on k_window, both take 5 to 8 us more.  The rule is that
+// comparison in units of 0.3 us, its constants moved to where the measured times divide
+// best.
 //
 // Measured on 382 batches drawn from windows of 2 to 242 atoms, nMC 3 to 100, both
-// routes each: where the rule takes k_window (206), the step is 10% and the solvent
-// force alone 2.2% faster than in separate passes; where it does not (176), k_window
-// would take the same time for the step (0.3% less) and 9.8% more for the force.  Four
-// windows of 220 atoms, nMC = 10: with two pairs of atoms the step takes 35.1 us separate
-// and 36.6 here, the force 28.4 and 32.8; with two chains of 22 atoms, whose shares are
-// the longest, 41.1 and 37.7, and 33.8 and 32.6.
+// routes each: where the rule takes k_window (212), the step is 10% and the solvent
+// force alone 2.6% faster than in separate passes; where it does not (170), k_window
+// would take the same time for the step and 10.8% more for the force.  Without the term
+// of the entries, which a window of 22 splits has 11 of and one of 20 five, batches of a
+// single 220-atom window were sent the slower way: 39 pairs and 40 chains of 22 atoms
+// beside it (nMC = 20), a step of 35.9 us instead of 32.1.  Four windows of 220 atoms,
+// nMC = 10: with two pairs of atoms the step takes 35.1 us separate and 36.6 here, the
+// force 28.4 and 32.8; with two chains of 22 atoms, whose shares are the longest, 41.1
+// and 37.7, and 33.8 and 32.6.
 bool window_pays(const WinDesc *w, int nwin, int nmc, int nblocks, int max_items)
 {
     int lo = w[0].n, hi = w[0].n;
@@ -1310,7 +1315,7 @@ bool window_pays(const WinDesc *w, int nwin, int nmc, int nblocks, int max_items
     if (hi <= kWinSmallAtoms) return true;
     if (lo > kWinSmallAtoms) return false;
     const int nt = window_threads(max_items, nblocks);
-    double chain = 0.0, longest = 0.0, pairs = 0.0;
+    double chain = 0.0, longest = 0.0, entries = 0.0, pairs = 0.0;
     for (int k = 0; k < nwin; ++k) {
         const WinDesc &d = w[k];
         const long long P = (long long)d.n * nmc;
@@ -1322,9 +1327,10 @@ bool window_pays(const WinDesc *w, int nwin, int nmc, int nblocks, int max_items
         const int per = d.n <= 2 * kWave ? 1 : 2;  // shares of a wave
         chain = std::max(chain, passes * d.aps + 0.6 * per * share);
         longest = std::max(longest, (double)share);
+        entries = std::max(entries, (double)(d.splits / d.fg));
         pairs += (double)d.n * (double)P;
     }
-    return chain <= 28.0 + 0.6 * longest + 6.0e-6 * pairs;
+    return chain <= 20.0 + 0.6 * longest + 0.8 * entries + 8.0e-6 * pairs;
 }
 
 hipError_t launch_window(const WindowArgs &a0, int max_points, int max_items, hipStream_t s)

@@ -32,14 +32,14 @@ def _one_launch(g):
 # chains, nMC, (splits, chunks): the largest group's (point, split) pairs and the
 # waves of a block
 CASES = [
-    (7, 4, (8, 52)),      # 154 atoms: 512 pairs, 8 waves
+    (7, 2, (8, 103)),     # 154 atoms: 512 pairs, 8 waves
     (7, 4, (9, 52)),      # 576, 16 waves
     (11, 4, (16, 61)),    # 242 atoms: 1,024, 16 waves
     (11, 4, (32, 61)),    # 1,984, two passes
     (9, 4, (61, 50)),     # 198 atoms: 3,200, four passes
-    (11, 20, (8, 1210)),  # 343 blocks: 512, 8 waves
-    (11, 20, (16, 1210)),  # 1,024, 8 waves, two passes
-    (9, 20, (20, 990)),   # 1,280, 8 waves, three passes
+    (8, 20, (8, 1174)),   # 176 atoms, 304 blocks: 512, 8 waves
+    (10, 20, (16, 1100)),  # 220 atoms: 1,024, 8 waves, two passes
+    (9, 20, (24, 990)),   # 1,408, 8 waves, three passes
 ]
 
 

@@ -59,13 +59,14 @@ def _expected(ns, n_mc, splits, chunks):
         return max(ns) <= 144
     items = max(t[3] * math.ceil(p / 64) * 64 for t, p in zip(w, pts))
     nt = 1024 if items > 512 and blocks <= 256 else 512
-    chain = longest = 0.0
+    chain = longest = entries = 0.0
     for (n, P, aps, s, ppc, sh, _), p in zip(w, pts):
         passes = math.ceil(s / (nt // (math.ceil(p / 64) * 64)))
         share = math.ceil(ppc / sh)
         chain = max(chain, passes * aps + 0.6 * (1 if n <= 128 else 2) * share)
         longest = max(longest, share)
-    return chain <= 28 + 0.6 * longest + 6e-6 * sum(n * P for n, P, *_ in w)
+        entries = max(entries, s // (4 if s % 4 == 0 else 2 if s % 2 == 0 else 1))
+    return chain <= 20 + 0.6 * longest + 0.8 * entries + 8e-6 * sum(n * P for n, P, *_ in w)
 
 
 @pytest.mark.parametrize("sizes,n_mc,one_launch", [
@@ -74,6 +75,8 @@ def _expected(ns, n_mc, splits, chunks):
     ([9] * 6 + [0], 20, False),           # 36.4, 41.6
     ([10] * 4 + [1] * 20, 10, True),      # 35.8, 30.3
     ([10] * 2 + [1] * 8 + [0] * 32, 20, True),
+    ([10] + [1] * 40 + [0] * 39, 20, True),  # step 35.9 us separate, 32.1 as one launch
+    ([10] + [1] * 12 + [0] * 4, 10, False),  # 35.3, 37.2
     ([6] * 3 + [0], 10, True),
     ([7, 8], 10, False)])
 def test_where_the_work_is(sizes, n_mc, one_launch):
